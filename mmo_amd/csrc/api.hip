@@ -139,6 +139,7 @@ struct mmo_ctx {
   int scan_xsub = 8;
   int scan_chunk = 4;
   int row_filter = 1;
+  int scan_split = 12288;     // row-list scans of at most this many tiles split the atoms
   CellGrid cgs{};
   DevBuf<int> d_cells;
   DevBuf<RecPos> rpos_s;
@@ -172,6 +173,7 @@ struct mmo_ctx {
   DevBuf<double4> s_ppar;
   DevBuf<int> s_int;
   DevBuf<Tile> s_tile;
+  DevBuf<double> s_scan_part;   // row-list scans of few tiles: energies per atom and pose
   DevBuf<double> s_scan;   // rotations + translations of the last scan
   DevBuf<int> s_tperm;
   // receptor on the host (rows x, y, z; atomic numbers) for host-side set-ups
@@ -455,6 +457,8 @@ InterLaunch inter_launch(mmo_ctx* c, int mode, const LigInfo* ligs, const LigAto
   L.row_chunk = c->scan_chunk;
   L.row_filter = c->row_filter;
   L.atom_order = nullptr;
+  L.n_atoms = 0;
+  L.part = nullptr;
   L.cg = c->cg;
   L.fr = c->fr;
   L.rpos = c->rpos.p;
@@ -572,6 +576,24 @@ InterLaunch scan_launch(mmo_ctx* c, int mode, int scan_cull) {
   return L;
 }
 
+// Row-list scans of few tiles (64 poses each): one ligand atom per wavefront, its energies
+// going to scratch that k_scan_sum adds up.  A wavefront that takes all of a tile's atoms
+// waits for one atom's receptor reads after the other's (36 us an atom whatever the scan's
+// size below 2,000 tiles, 8 wavefronts per SIMD being 8,192 of them).  Whole against split,
+// the 75-atom ligand and the 3000-atom receptor, ms per launch: 125 tiles 2.70 / 0.14, 1,000
+// 2.74 / 0.77, 4,000 3.91 / 2.73, 8,000 6.61 / 5.39, 12,000 9.30 / 8.08; the filtered scan
+// of one tile 2.7 / 0.08.  Beyond that the scratch (8 bytes per atom and pose) costs more
+// memory than the last, partly filled round of wavefronts is worth.
+int split_scan(mmo_ctx* c, InterLaunch& L, int lig_id, size_t ntiles) {
+  constexpr size_t kMaxPart = (size_t)1 << 26;   // doubles (512 MiB)
+  L.n_atoms = c->ligs[lig_id].n;
+  if (L.cull < 4 || ntiles > (size_t)c->scan_split || L.n_atoms * ntiles * kWave > kMaxPart)
+    return MMO_OK;
+  HIPCHK(c, c->s_scan_part.ensure(L.n_atoms * ntiles * kWave));
+  L.part = c->s_scan_part.p;
+  return MMO_OK;
+}
+
 // translations in Morton order of their per-axis ranks: 64 consecutive slots form a
 // compact brick (a 4x4x4 block of a lattice)
 std::vector<int> morton_translations(const double* trans, int ntrans) {
@@ -665,7 +687,7 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     c->d_rb_left.release(); c->d_rb_right.release(); c->d_rg_off.release(); c->d_rg_atoms.release();
     c->s_xyz.release(); c->s_e.release(); c->s_g.release(); c->s_part.release();
     c->s_lig.release(); c->s_latom.release(); c->s_pij.release(); c->s_ppar.release();
-    c->s_int.release(); c->s_tile.release(); c->s_scan.release(); c->s_tperm.release();
+    c->s_int.release(); c->s_tile.release(); c->s_scan.release(); c->s_scan_part.release(); c->s_tperm.release();
     c->d_cell.release(); c->d_cellp.release(); c->d_mask.release(); c->s_skip.release();
     c->s_tk_st.release(); c->s_tk_u.release(); c->s_keep.release(); c->s_select.release();
     c->s_list.release(); c->s_nkept.release(); c->d_desolv.release(); c->d_rec64.release();
@@ -1490,6 +1512,7 @@ int mmo_scan_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, int nrot,
     timer_end(c, "interp", s);
   } else {
     InterLaunch L = scan_launch(c, mode, c->scan_cull);
+    if ((r = split_scan(c, L, lig_id, (size_t)nrot * ((ntrans + kWave - 1) / kWave)))) return r;
     timer_begin(c, "inter", s);
     HIPCHK(c, launch_inter_scan(L, lig_id, d_rot, nrot, d_trans, c->s_tperm.p, ntrans, e_out, s));
     timer_end(c, "inter", s);
@@ -2314,6 +2337,7 @@ int mmo_scan_filtered_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, 
       // the scan's own culled kernel (the list form has no unculled one): the kept poses'
       // energies are those of mmo_scan_dev, bit for bit
       InterLaunch L = scan_launch(c, MMO_SHIFTED, c->scan_cull ? c->scan_cull : 2);
+      if ((r = split_scan(c, L, lig_id, ((size_t)nk + kWave - 1) / kWave))) return r;
       timer_begin(c, "inter", s);
       HIPCHK(c, launch_inter_scan_list(L, lig_id, a.rots, a.trans, c->s_tperm.p, ntrans, c->s_list.p,
                                        nk, e_out, s));
@@ -2594,6 +2618,7 @@ int mmo_tune_set(mmo_ctx* c, const char* key, double v) {
   else if (k == "scan_xsub" && iv >= 1 && iv <= 16) c->scan_xsub = iv;
   else if (k == "scan_chunk" && (iv == 4 || iv == 8)) c->scan_chunk = iv;
   else if (k == "row_filter" && (iv == 0 || iv == 1)) c->row_filter = iv;
+  else if (k == "scan_split" && iv >= 0 && iv <= (1 << 20)) c->scan_split = iv;
   else if (k == "grid_pack" && (iv == 0 || iv == 1)) c->grid_pack = iv;
   else if (k == "mc_waves_per_cu" && iv >= 1 && iv <= 32) c->mc_waves_per_cu = iv;
   else if (k == "mc_wg_waves" && iv >= 1 && iv <= 16) c->mc_wg_waves = iv;
@@ -2623,6 +2648,7 @@ double mmo_tune_get(mmo_ctx* c, const char* key) {
   if (k == "scan_xsub") return c->scan_xsub;
   if (k == "scan_chunk") return c->scan_chunk;
   if (k == "row_filter") return c->row_filter;
+  if (k == "scan_split") return c->scan_split;
   if (k == "grid_pack") return c->grid_pack;
   if (k == "pose_waves") return c->pose_waves;
   if (k == "scan_cull") return c->scan_cull;

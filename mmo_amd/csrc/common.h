@@ -217,7 +217,7 @@ __device__ __forceinline__ LigPt lig_pt(double x, double y, double z, const Fram
   l.x = to_fixed(x, fr.ox, fr.scale, fr.lim, sat);
   l.y = to_fixed(y, fr.oy, fr.scale, fr.lim, sat);
   l.z = to_fixed(z, fr.oz, fr.scale, fr.lim, sat);
-  const double is = 1.0 / fr.scale;
+  const double is = (double)fr.inv_s;   // 2^-k, exact in both types
   l.rx = quant_residual(x, fr.ox, is, l.x);
   l.ry = quant_residual(y, fr.oy, is, l.y);
   l.rz = quant_residual(z, fr.oz, is, l.z);

@@ -111,6 +111,10 @@ struct InterArgs {
   int rslice;         // receptor atoms per gridDim.y slice
   int npose_total;    // for partial outputs when gridDim.y > 1
   const int* atom_order;   // nullable: per ligand at atom_base, the sweeps' atom order
+  // k_scan_rows with few tiles: gridDim.y = the ligand's atoms, one per wavefront, their
+  // energies to part[(atom * ntiles + tile) * 64 + lane] for k_scan_sum (nullptr: one
+  // wavefront sums all atoms of its tile)
+  double* part;
 };
 
 // --------------------------------------------------------------- pair arithmetic
@@ -423,14 +427,14 @@ k_inter_cull(InterArgs<Src> a, CellGrid cg) {
   }
 }
 
-// Rigid scan over the row lists of a finer cell grid (row_sweep): one pose per lane, K
-// ligand atoms at a time (consecutive atoms of the ligand's sweep order, a walk of its
-// bond graph, so the K atoms are close and the wavefront's box grows little).  RMODE bit
-// 0 clear: receptor read in place (uniform addresses, scalar cache); set: receptor
+// Rigid scan over the row lists of a finer cell grid (row_sweep): one pose per lane, one
+// ligand atom after the other.  RMODE bit 0 clear: receptor read in place (uniform addresses, scalar cache); set: receptor
 // positions and LJ factors staged in LDS.  Bit 1: the far rows' atoms are tested against
 // the box grown by the cutoff before the sweep (row_sweep's FILT).  The cell table stays
-// in global memory (it is read per lane, once per candidate row).
-template <int RMODE, int CHUNK, int K, class Src>
+// in global memory (it is read per lane, once per candidate row).  SPLIT: one ligand atom
+// per wavefront (blockIdx.y), for scans of too few tiles to fill the chip; the pose's sum
+// runs over the atoms' energies in atom order either way, so both forms give the same bits.
+template <int RMODE, int CHUNK, bool SPLIT, class Src>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8)))
 k_scan_rows(InterArgs<Src> a, CellGrid cg) {
   extern __shared__ __align__(16) char smem[];
@@ -457,51 +461,54 @@ k_scan_rows(InterArgs<Src> a, CellGrid cg) {
   const int pose = pose_ok ? a.src.pose_id(t.pose0 + lane) : 0;
   const LigInfo li = a.ligs[t.lig];
   const Frame fr = a.fr;
-  double e_el = 0.0, e_vd = 0.0;
+  const int j_begin = SPLIT ? blockIdx.y : 0, j_end = SPLIT ? j_begin + 1 : li.n_atoms;
+  double e = 0.0;
   int sat = 0;
-  for (int j0 = 0; j0 < li.n_atoms; j0 += K) {
-    LigPt l[K];
-    bool valid[K];
-    double cq[K], ca[K], cb[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      valid[k] = pose_ok && j0 + k < li.n_atoms;
-      cq[k] = ca[k] = cb[k] = 0.0;
-      l[k] = lig_pt_far();
-      if (j0 + k < li.n_atoms) {
-        const int j = (K > 1 && a.atom_order) ? a.atom_order[li.atom_base + j0 + k] : j0 + k;
-        const LigAtom la = a.latoms[li.atom_base + j];
-        if (pose_ok) {
-          double x, y, z;
-          a.src.pos(pose, lane, j, li, a.latoms, a.lig_xyz, x, y, z);
-          l[k] = lig_pt(x, y, z, fr, &sat);
-          cq[k] = la.keq; ca[k] = la.a; cb[k] = la.b;
-        }
-      }
+  for (int j = j_begin; j < j_end; ++j) {
+    const LigAtom la = a.latoms[li.atom_base + j];
+    LigPt l[1];
+    const bool valid[1] = {pose_ok};
+    l[0] = lig_pt_far();   // a lane without a pose: its pairs weigh exactly 0
+    if (pose_ok) {
+      double x, y, z;
+      a.src.pos(pose, lane, j, li, a.latoms, a.lig_xyz, x, y, z);
+      l[0] = lig_pt(x, y, z, fr, &sat);
     }
+    // the atom's energy is summed from zero, then added to the pose's: the same sum in the
+    // same order whether one wavefront takes all atoms or each its own
+    double ej = 0.0;
     float qx, qy, qz, hx, hy, hz;
-    if (!wave_box<K>(l, valid, fr.inv_s, qx, qy, qz, hx, hy, hz)) continue;
-    row_sweep<(RMODE & 1) == 0, CHUNK, K, (RMODE & 2) != 0>(cg, s_pos, s_ab, a.rres, fr.inv_s, fr.inv_s2, qx, qy, qz, hx,
-                                    hy, hz, l,
-                                    [&](const float (&sq)[K], const float (&s12)[K],
-                                        const float (&s6)[K]) {
-#pragma unroll
-                                      for (int k = 0; k < K; ++k) {
-                                        e_el = fma((double)sq[k], cq[k], e_el);
-                                        e_vd = fma((double)s12[k], ca[k], e_vd);
-                                        e_vd = fma(-2.0 * (double)s6[k], cb[k], e_vd);
-                                      }
-                                    });
+    if (wave_box<1>(l, valid, fr.inv_s, qx, qy, qz, hx, hy, hz))
+      row_sweep<(RMODE & 1) == 0, CHUNK, (RMODE & 2) != 0>(
+          cg, s_pos, s_ab, a.rres, fr.inv_s, fr.inv_s2, qx, qy, qz, hx, hy, hz, l[0],
+          [&](float sq, float s12, float s6) {
+            ej = fma((double)sq, la.keq, ej);
+            ej = fma((double)s12, la.a, ej);
+            ej = fma(-2.0 * (double)s6, la.b, ej);
+          });
+    e += ej;
   }
   (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
-  if (pose_ok) {
-    const size_t o = (size_t)pose * a.e_stride;
-    a.e_out[o] = e_el + e_vd;
-    if (a.e_comp) {
-      a.e_comp[o + 2] = e_el;
-      a.e_comp[o + 3] = e_vd;
-    }
-  }
+  // (stores only here: one inside the loop would take the receptor's reads off the scalar
+  // cache, which the compiler uses for memory that nothing before them may have written)
+  if (SPLIT) a.part[((size_t)blockIdx.y * a.ntiles + tidx) * kWave + lane] = e;
+  else if (pose_ok) a.e_out[(size_t)pose * a.e_stride] = e;
+}
+
+// the poses' energies from a split k_scan_rows: the atoms' parts in atom order
+template <class Src>
+__global__ void __launch_bounds__(256) k_scan_sum(InterArgs<Src> a) {
+  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
+  const int tidx = slot / kWave, lane = slot & (kWave - 1);
+  if (tidx >= a.ntiles) return;
+  const Tile t = a.src.tile(tidx);
+  if (lane >= t.npose) return;
+  const int n = a.ligs[t.lig].n_atoms;
+  const size_t stride = (size_t)a.ntiles * kWave;
+  double e = 0.0;
+#pragma unroll 4
+  for (int j = 0; j < n; ++j) e += a.part[j * stride + slot];
+  a.e_out[(size_t)a.src.pose_id(t.pose0 + lane) * a.e_stride] = e;
 }
 
 // The cell-packed copy of the grids (GridDev::cells): one thread per (type, cell) gathers
@@ -886,6 +893,7 @@ hipError_t launch_inter_coords(const InterLaunch& L, const Tile* tiles, const in
   a.ntiles = ntiles; a.fr = L.fr; a.rpos = L.rpos; a.rab = L.rab; a.rres = L.rres; a.nrec = L.nrec;
   a.rtile = L.rtile; a.ligs = L.ligs; a.latoms = L.latoms; a.lig_xyz = L.lig_xyz;
   a.e_stride = e_stride; a.grad = grad; a.write_e = write_e; a.atom_order = nullptr;
+  a.part = nullptr;
   a.rslice = L.rslice > 0 ? L.rslice : L.nrec;
   a.npose_total = npose;
   if (L.cull && !grad) {
@@ -914,30 +922,36 @@ static hipError_t launch_rows(const InterLaunch& L, const InterArgs<Src>& a, hip
     if (blocks == 0) return hipSuccess;
     const size_t lds =
         L.cull == 5 ? (size_t)(a.nrec + kRowChunk) * (sizeof(RecPos) + sizeof(RecAB)) : 0;
-#define MMO_ROWS(RM, CH, KK)                                                                   \
+#define MMO_ROWS_AS(RM, CH, SP)                                                                \
   {                                                                                            \
     if (lds > 0) {                                                                             \
       hipError_t e = hipFuncSetAttribute(                                                      \
-          reinterpret_cast<const void*>(&k_scan_rows<RM, CH, KK, Src>),                        \
+          reinterpret_cast<const void*>(&k_scan_rows<RM, CH, SP, Src>),                        \
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                               \
       if (e != hipSuccess) return e;                                                           \
     }                                                                                          \
-    hipLaunchKernelGGL((k_scan_rows<RM, CH, KK, Src>), dim3(blocks), dim3(waves * kWave), lds, \
-                       s, a, L.cg);                                                            \
+    hipLaunchKernelGGL((k_scan_rows<RM, CH, SP, Src>), dim3(blocks, SP ? L.n_atoms : 1),       \
+                       dim3(waves * kWave), lds, s, a, L.cg);                                  \
   }
+#define MMO_ROWS(RM, CH)                                                                       \
+  { if (a.part) MMO_ROWS_AS(RM, CH, true) else MMO_ROWS_AS(RM, CH, false) }
     // one ligand atom per lane: two (bonded neighbours of the sweep order) were measured
     // 15-20% slower on the 36.9M-pose scan, whichever receptor path
     const int rm = (L.cull == 5 ? 1 : 0) | (L.row_filter ? 2 : 0);
     if (rm == 0) {
-      if (L.row_chunk == 4) MMO_ROWS(0, 4, 1) else MMO_ROWS(0, 8, 1)
+      if (L.row_chunk == 4) MMO_ROWS(0, 4) else MMO_ROWS(0, 8)
     } else if (rm == 1) {
-      if (L.row_chunk == 4) MMO_ROWS(1, 4, 1) else MMO_ROWS(1, 8, 1)
+      if (L.row_chunk == 4) MMO_ROWS(1, 4) else MMO_ROWS(1, 8)
     } else if (rm == 2) {
-      if (L.row_chunk == 4) MMO_ROWS(2, 4, 1) else MMO_ROWS(2, 8, 1)
+      if (L.row_chunk == 4) MMO_ROWS(2, 4) else MMO_ROWS(2, 8)
     } else {
-      if (L.row_chunk == 4) MMO_ROWS(3, 4, 1) else MMO_ROWS(3, 8, 1)
+      if (L.row_chunk == 4) MMO_ROWS(3, 4) else MMO_ROWS(3, 8)
     }
+#undef MMO_ROWS_AS
 #undef MMO_ROWS
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess || !a.part) return err;
+    hipLaunchKernelGGL((k_scan_sum<Src>), dim3((a.ntiles * kWave + 255) / 256), dim3(256), 0, s, a);
     return hipGetLastError();
   }
 }
@@ -992,6 +1006,7 @@ hipError_t launch_inter_scan(const InterLaunch& L, int lig, const double* rots, 
   a.nrec = L.nrec; a.rtile = L.rtile; a.ligs = L.ligs; a.latoms = L.latoms;
   a.lig_xyz = L.lig_xyz; a.e_out = e_out; a.e_stride = 1; a.e_comp = nullptr; a.grad = nullptr;
   a.write_e = 1; a.rslice = L.nrec; a.npose_total = nrot * ntrans; a.atom_order = L.atom_order;
+  a.part = L.part;
   if (L.cull) return launch_cull(L, a, s);
   return launch_inter_any(L.mode, L.k, false, a, L.waves, s);
 }
@@ -1007,6 +1022,7 @@ hipError_t launch_inter_scan_list(const InterLaunch& L, int lig, const double* r
   a.rres = L.rres; a.nrec = L.nrec; a.rtile = L.rtile; a.ligs = L.ligs; a.latoms = L.latoms;
   a.lig_xyz = L.lig_xyz; a.e_out = e_out; a.e_stride = 1; a.e_comp = nullptr; a.grad = nullptr;
   a.write_e = 1; a.rslice = L.nrec; a.npose_total = nlist; a.atom_order = L.atom_order;
+  a.part = L.part;
   return launch_cull(L, a, s);
 }
 
