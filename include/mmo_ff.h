@@ -243,8 +243,8 @@ int mmo_topk_dev(mmo_ctx* ctx, const double* e, int64_t n, int k, double* e_out,
                  void* stream);
 /* mmo_topk_dev without any allocation: no counterpart in the reference; for callers that
  * cannot allocate device memory (code under HIP graph capture, serving loops).  The
- * kernels' scratch (radix state, histogram, counters, per-chunk counts) is a static
- * device array of 132 KiB per GPU, set up by mmo_ctx_create, so n <= 134,217,728
+ * kernels' scratch (radix state, histogram, candidates, per-chunk counts) is a static
+ * device array of 353 KiB per GPU, set up by mmo_ctx_create, so n <= 134,217,728
  * (larger n -> MMO_ERR_BAD_ARG); same results as mmo_topk_dev.  All calls on one GPU
  * share that array: calls that overlap on one GPU (other streams, other contexts,
  * other threads) race and must be ordered by the caller. */

@@ -30,14 +30,16 @@ std::string g_last_error;
 
 // ----------------------------------------------- no-allocation top-k (mmo_topk_dev_noalloc)
 // Scratch of the top-k kernels in a file-scope device array instead of library
-// allocations: radix state (3 x u64) at byte 0, histogram (256 x u32) at 256, counter
-// (u32) at 1280, per-chunk counts (u32) from 1536.  Each GPU holds its own copy for the
-// life of the process; host code uses the per-device address from hipGetSymbolAddress,
-// never the array's name.  Every call on one GPU reuses its copy: the kernels clear the
-// state, histogram and counter themselves and write every chunk count before reading it.
+// allocations (topk_scratch: state, histogram, candidates, per-chunk counts).  Each GPU
+// holds its own copy for the life of the process; host code uses the per-device address
+// from hipGetSymbolAddress, never the array's name.  Every call on one GPU reuses its copy:
+// the kernels clear the state and the histogram themselves and write every candidate and
+// chunk count before reading it.
 constexpr size_t kTopkChunk = 4096;                       // energies per chunk count
 constexpr size_t kTopkNoallocChunks = 32768;              // -> at most 134,217,728 energies
-constexpr size_t kTopkNoallocBytes = 1536 + 4 * kTopkNoallocChunks;
+constexpr size_t kTopkCandAt = 512 + sizeof(unsigned) * kTopkHist;
+constexpr size_t kTopkChunksAt = kTopkCandAt + 16 * (size_t)kTopkCand;
+constexpr size_t kTopkNoallocBytes = kTopkChunksAt + 4 * kTopkNoallocChunks;
 static __device__ __align__(256) unsigned char scratch[kTopkNoallocBytes];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -53,6 +55,14 @@ void scratch_setup(int device) {
   const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
   g_scratch_err[device] = e;
   if (e == hipSuccess) g_scratch_ptr[device] = p;
+}
+
+TopkScratch topk_scratch(unsigned char* b) {
+  static_assert((kTopkPasses + 1) * sizeof(TopkState) <= 448, "top-k scratch layout");
+  double* cand = reinterpret_cast<double*>(b + kTopkCandAt);
+  return TopkScratch{reinterpret_cast<TopkState*>(b), reinterpret_cast<unsigned*>(b + 448),
+                     reinterpret_cast<unsigned*>(b + 512), reinterpret_cast<unsigned*>(b + kTopkChunksAt),
+                     cand, reinterpret_cast<int64_t*>(cand + kTopkCand), kTopkChunk};
 }
 
 struct Uff { double x, d; };
@@ -198,8 +208,7 @@ struct mmo_ctx {
   DevBuf<double> s_dpart;
   DevBuf<uint32_t> d_mask;
   DevBuf<uint8_t> s_skip;
-  DevBuf<uint64_t> s_tk_st;
-  DevBuf<unsigned> s_tk_u;
+  DevBuf<unsigned char> s_tk;   // top-k scratch (topk_scratch)
   // filtered scan: keep flags and compacted slots of the scan's pose order, the kept
   // count, the compaction's scratch
   DevBuf<uint8_t> s_keep, s_select;
@@ -689,7 +698,7 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     c->s_lig.release(); c->s_latom.release(); c->s_pij.release(); c->s_ppar.release();
     c->s_int.release(); c->s_tile.release(); c->s_scan.release(); c->s_scan_part.release(); c->s_tperm.release();
     c->d_cell.release(); c->d_cellp.release(); c->d_mask.release(); c->s_skip.release();
-    c->s_tk_st.release(); c->s_tk_u.release(); c->s_keep.release(); c->s_select.release();
+    c->s_tk.release(); c->s_keep.release(); c->s_select.release();
     c->s_list.release(); c->s_nkept.release(); c->d_desolv.release(); c->d_rec64.release();
     c->s_dvox.release(); c->s_datoms.release(); c->s_dpart.release();
     for (auto& kv : c->ev) {
@@ -2357,12 +2366,8 @@ int mmo_topk_dev(mmo_ctx* c, const double* e, int64_t n, int k, double* e_out, i
     return fail(c, MMO_ERR_BAD_ARG, "bad top-k arguments (n %lld, k %d, k <= %d)", (long long)n,
                 k, kTopkMax);
   const int kk = (int)std::min<int64_t>(k, n);
-  const size_t chunk = kTopkChunk;
-  const size_t nb = ((size_t)n + chunk - 1) / chunk;
-  HIPCHK(c, c->s_tk_st.ensure(3));
-  HIPCHK(c, c->s_tk_u.ensure(256 + 1 + nb));
-  TopkScratch w{c->s_tk_st.p, c->s_tk_u.p, c->s_tk_u.p + 256, c->s_tk_u.p + 257, chunk};
-  HIPCHK(c, launch_topk(e, (size_t)n, kk, e_out, idx_out, w, (hipStream_t)stream));
+  HIPCHK(c, c->s_tk.ensure(kTopkChunksAt + 4 * (((size_t)n + kTopkChunk - 1) / kTopkChunk)));
+  HIPCHK(c, launch_topk(e, (size_t)n, kk, e_out, idx_out, topk_scratch(c->s_tk.p), (hipStream_t)stream));
   return MMO_OK;
 }
 
@@ -2390,12 +2395,9 @@ int mmo_topk_dev_noalloc(mmo_ctx* c, const double* e, int64_t n, int k, double* 
   if (!base)
     return fail(c, MMO_ERR_DEVICE, "top-k scratch of device %d unavailable: %s", c->device,
                 hipGetErrorString(se));
-  unsigned char* b = static_cast<unsigned char*>(base);
   const int kk = (int)std::min<int64_t>(k, n);
-  TopkScratch w{reinterpret_cast<uint64_t*>(b), reinterpret_cast<unsigned*>(b + 256),
-                reinterpret_cast<unsigned*>(b + 1280), reinterpret_cast<unsigned*>(b + 1536),
-                kTopkChunk};
-  HIPCHK(c, launch_topk(e, (size_t)n, kk, e_out, idx_out, w, (hipStream_t)stream));
+  HIPCHK(c, launch_topk(e, (size_t)n, kk, e_out, idx_out,
+                        topk_scratch(static_cast<unsigned char*>(base)), (hipStream_t)stream));
   return MMO_OK;
 }
 

@@ -215,11 +215,22 @@ hipError_t select_flagged_slots(const uint8_t* flags, int n, int* out, int* n_ou
                                 size_t* temp_bytes, hipStream_t s);
 
 constexpr int kTopkMax = 2048;
+constexpr int kTopkCand = 4096;   // keys the select leaves to the final sort (>= kTopkMax)
+constexpr int kTopkPasses = 5;       // digits of the select
+constexpr int kTopkHist = kTopkPasses * 8192;
+struct TopkState {
+  uint64_t prefix, mask;      // the selected high bits and which they are
+  uint64_t rem, k;            // keys still to be taken among those matching the prefix; of k
+  unsigned done;              // the keys at or below the prefix fit the candidate list
+  unsigned pad;
+};
 struct TopkScratch {
-  uint64_t* st;               // 3
-  unsigned* hist;             // 256
-  unsigned* cnt;              // 1
+  TopkState* st;              // kTopkPasses + 1
+  unsigned* count;            // candidates gathered
+  unsigned* hist;             // kTopkHist: the counts of each pass
   unsigned* bcnt;             // one per chunk
+  double* cand_e;             // kTopkCand
+  int64_t* cand_i;            // kTopkCand
   size_t chunk;
 };
 hipError_t launch_topk(const double* e, size_t n, int k, double* out_e, int64_t* out_i,

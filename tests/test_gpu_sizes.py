@@ -47,3 +47,39 @@ def test_split_scan_equals_whole_scan(sys0, nrot, ntrans, scan_cull):
         x = _rows(lig) @ rots[a].T + trans[b]
         sums.append(inter_abs_sum(rec, x, lig, True))
     assert_energy(got[1][pick], want, sums, what="split scan")
+
+
+def _topk_input(kind, n, rng):
+    if kind == "ties":          # 7 values: far more equal keys than the candidate list holds
+        return rng.integers(-3, 4, n).astype(np.float64)
+    if kind == "inf":           # a filtered scan: a few finite energies
+        e = np.full(n, np.inf)
+        e[rng.choice(n, 50, replace=False)] = rng.normal(-20, 30, 50)
+        return e
+    if kind == "close":         # keys that share their first 40 bits
+        return -1.0 - rng.integers(0, 1 << 20, n) * 2.0 ** -52
+    e = rng.normal(0, 1, n) * 10.0 ** rng.uniform(-300, 300, n)
+    e[rng.choice(n, 5, replace=False)] = [np.nan, -np.inf, 0.0, -0.0, 5e-324]
+    return e
+
+
+@pytest.mark.parametrize("kind", ["ties", "inf", "close", "wide"])
+@pytest.mark.parametrize("n,k", [(4096, 2048), (4097, 2048), (4097, 1), (300_001, 100), (300_001, 2048)])
+def test_topk_edges(sys0, kind, n, k):
+    """The top-k at the sizes where its path changes (the candidate list holds 4,096), on
+    ties beyond the list, +inf but for a few, keys that differ in their last bits only and
+    the whole range of doubles: exactly the (energy, index) order, on an input that is not
+    16-byte aligned."""
+    import torch
+    ctx, _, _ = sys0
+    rng = np.random.default_rng(n + k)
+    e = _topk_input(kind, n, rng)
+    d = torch.empty(n + 1, dtype=torch.float64, device="cuda:0")[1:]
+    d.copy_(torch.tensor(e))
+    v, i = ctx.topk(d, k)
+    bits = e.view(np.int64)
+    key = np.where(bits < 0, ~bits.view(np.uint64), bits.view(np.uint64) | np.uint64(1 << 63))
+    key[np.isnan(e)] = np.uint64(0xFFFFFFFFFFFFFFFF)
+    want = np.lexsort((np.arange(n), key))[:k]
+    assert np.array_equal(i.cpu().numpy(), want)
+    assert np.array_equal(v.cpu().numpy(), e[want], equal_nan=True)
