@@ -102,6 +102,7 @@ struct LigHost {
   std::vector<uint32_t> pair_ij;
   std::vector<int> rb_left, rb_right, rg_off, rg_atoms;
   std::vector<int> sweep;   // order in which the per-atom sweeps take the atoms
+  std::vector<int> clash;   // order in which the scan filters test them (farthest first)
 };
 
 }  // namespace
@@ -174,6 +175,7 @@ struct mmo_ctx {
   DevBuf<uint32_t> d_pair_ij;
   DevBuf<double4> d_pair_par;
   DevBuf<int> d_sweep;          // per ligand at atom_base: the sweeps' atom order
+  DevBuf<int> d_clash;          // the same: the scan filters' order
   DevBuf<int> d_rb_left, d_rb_right, d_rg_off, d_rg_atoms;
   // scratch for the plain (one ligand) forms
   DevBuf<double> s_xyz, s_e, s_g, s_part;
@@ -206,13 +208,13 @@ struct mmo_ctx {
   DevBuf<int> s_dvox;
   DevBuf<double4> s_datoms;
   DevBuf<double> s_dpart;
-  DevBuf<uint32_t> d_mask;
+  DevBuf<uint32_t> d_mask, d_mask_cells;
   DevBuf<uint8_t> s_skip;
   DevBuf<unsigned char> s_tk;   // top-k scratch (topk_scratch)
-  // filtered scan: keep flags and compacted slots of the scan's pose order, the kept
-  // count, the compaction's scratch
-  DevBuf<uint8_t> s_keep, s_select;
-  DevBuf<int> s_list, s_nkept;
+  // filtered scan: keep flags of the scan's pose order, kept slots and their number
+  DevBuf<uint64_t> s_keep;
+  DevBuf<unsigned> s_nkept;
+  DevBuf<int> s_list;
   // tuning
   int inter_k = 4, inter_waves = 4, inter_rtile = 2048;
   std::map<std::string, std::pair<hipEvent_t, hipEvent_t>> ev;
@@ -357,6 +359,24 @@ std::vector<uint32_t> intra_pairs(const int32_t* dists, int n) {
   return out;
 }
 
+// Order of the atoms for the scan filters, which stop at a pose's first clash: farthest from
+// the centre first, since those reach the protein around a pocket soonest.
+std::vector<int> clash_order(const std::vector<double>& xyz, int n) {
+  double c[3] = {0.0, 0.0, 0.0};
+  for (int j = 0; j < n; ++j)
+    for (int k = 0; k < 3; ++k) c[k] += xyz[3 * j + k] / n;
+  std::vector<std::pair<double, int>> far(n);
+  for (int j = 0; j < n; ++j) {
+    double d2 = 0.0;
+    for (int k = 0; k < 3; ++k) d2 += (xyz[3 * j + k] - c[k]) * (xyz[3 * j + k] - c[k]);
+    far[j] = {std::isfinite(d2) ? -d2 : 0.0, j};
+  }
+  std::sort(far.begin(), far.end());
+  std::vector<int> order(n);
+  for (int j = 0; j < n; ++j) order[j] = far[j].second;
+  return order;
+}
+
 int pair_params(mmo_ctx* c, const std::vector<uint32_t>& pij, const double* q,
                 const int32_t* anum, std::vector<double4>& out) {
   out.resize(pij.size());
@@ -400,7 +420,7 @@ int sync_ligands(mmo_ctx* c) {
   std::vector<double> xyz;
   std::vector<uint32_t> pij;
   std::vector<double4> ppar;
-  std::vector<int> rbl, rbr, rgo, rga, swp;
+  std::vector<int> rbl, rbr, rgo, rga, swp, clash;
   c->max_atoms = 0;
   for (const LigHost& h : c->ligs) {
     LigInfo li{};
@@ -421,6 +441,7 @@ int sync_ligands(mmo_ctx* c) {
     }
     xyz.insert(xyz.end(), h.xyz.begin(), h.xyz.end());
     swp.insert(swp.end(), h.sweep.begin(), h.sweep.end());
+    clash.insert(clash.end(), h.clash.begin(), h.clash.end());
     std::vector<double4> pp;
     int r = pair_params(c, h.pair_ij, h.q.data(), h.anum.data(), pp);
     if (r) return r;
@@ -446,6 +467,7 @@ int sync_ligands(mmo_ctx* c) {
   if ((r = upload(c, c->d_rg_off, rgo.data(), rgo.size(), s))) return r;
   if ((r = upload(c, c->d_rg_atoms, rga.data(), rga.size(), s))) return r;
   if ((r = upload(c, c->d_sweep, swp.data(), swp.size(), s))) return r;
+  if ((r = upload(c, c->d_clash, clash.data(), clash.size(), s))) return r;
   HIPCHK(c, hipStreamSynchronize(s));
   c->lig_dirty = false;
   ++c->lig_version;
@@ -692,13 +714,13 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     c->grid_cells.release();
     c->rpos_s.release(); c->rab_s.release(); c->rres_s.release(); c->d_cells.release();
     c->d_ligs.release(); c->d_latoms.release(); c->d_lig_xyz.release();
-    c->d_pair_ij.release(); c->d_pair_par.release(); c->d_sweep.release();
+    c->d_pair_ij.release(); c->d_pair_par.release(); c->d_sweep.release(); c->d_clash.release();
     c->d_rb_left.release(); c->d_rb_right.release(); c->d_rg_off.release(); c->d_rg_atoms.release();
     c->s_xyz.release(); c->s_e.release(); c->s_g.release(); c->s_part.release();
     c->s_lig.release(); c->s_latom.release(); c->s_pij.release(); c->s_ppar.release();
     c->s_int.release(); c->s_tile.release(); c->s_scan.release(); c->s_scan_part.release(); c->s_tperm.release();
     c->d_cell.release(); c->d_cellp.release(); c->d_mask.release(); c->s_skip.release();
-    c->s_tk.release(); c->s_keep.release(); c->s_select.release();
+    c->s_tk.release(); c->s_keep.release(); c->d_mask_cells.release();
     c->s_list.release(); c->s_nkept.release(); c->d_desolv.release(); c->d_rec64.release();
     c->s_dvox.release(); c->s_datoms.release(); c->s_dpart.release();
     for (auto& kv : c->ev) {
@@ -1148,6 +1170,7 @@ int mmo_ligand_add(mmo_ctx* c, const double* xs, const double* ys, const double*
   }
   h.pair_ij = intra_pairs(dists, n);
   h.sweep = sweep_order(dists, n);
+  h.clash = clash_order(h.xyz, n);
   for (int k = 0; k < nrb; ++k) {
     if (rb_left[k] < 0 || rb_left[k] >= n || rb_right[k] < 0 || rb_right[k] >= n ||
         rb_left[k] == rb_right[k])
@@ -2076,8 +2099,8 @@ int scan_filter_setup(mmo_ctx* c, int lig_id, const double* rots, int nrot, cons
   a.rots = c->s_scan.p; a.trans = c->s_scan.p + 9 * (size_t)nrot; a.nrot = nrot; a.ntrans = ntrans;
   size_t base = 0;
   for (int l = 0; l < lig_id; ++l) base += (size_t)c->ligs[l].n;   // LigInfo.atom_base
-  a.lig = c->d_lig_xyz.p + 3 * base; a.n_atoms = h.n;
-  a.mask = c->has_mask ? c->d_mask.p : nullptr;
+  a.lig = c->d_lig_xyz.p + 3 * base; a.order = c->d_clash.p + base; a.n_atoms = h.n;
+  a.cells = c->has_mask ? c->d_mask_cells.p : nullptr;
   a.ox = c->mask_o[0]; a.oy = c->mask_o[1]; a.oz = c->mask_o[2];
   a.inv_step = c->has_mask ? 1.0 / c->mask_step : 0.0;
   a.nx = c->mask_n[0]; a.ny = c->mask_n[1]; a.nz = c->mask_n[2];
@@ -2106,6 +2129,8 @@ int mmo_set_vdw_mask(mmo_ctx* c, const double* radii, double step, int nx, int n
     bitmask_atom(mask, dims, o, step, &c->rec_host[3 * (size_t)a], rad, true);
   }
   if ((r = upload(c, c->d_mask, mask.data(), mask.size(), c->stream))) return r;
+  HIPCHK(c, c->d_mask_cells.ensure(mask.size()));
+  HIPCHK(c, launch_mask_cells(c->d_mask.p, c->d_mask_cells.p, nx, ny, nz, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->mask_host.swap(mask);
   c->mask_step = step;
@@ -2321,19 +2346,17 @@ int mmo_scan_filtered_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, 
   const std::vector<int> tperm = morton_translations(trans, ntrans);
   if ((r = upload(c, c->s_tperm, tperm.data(), tperm.size(), s))) return r;
   const int n = nrot * ntrans;
-  HIPCHK(c, c->s_keep.ensure(n));
+  const size_t groups = scan_keep_groups(nrot, ntrans);
+  HIPCHK(c, c->s_keep.ensure(groups * (kKeepSlots / 64)));
   HIPCHK(c, c->s_list.ensure(n));
-  HIPCHK(c, c->s_nkept.ensure(1));
-  // keep flags in the scan's pose order, then the kept slots compacted in that order (so
-  // that consecutive kept poses stay in the scan's bricks)
-  HIPCHK(c, launch_scan_keep(a, c->s_tperm.p, c->s_keep.p, s));
-  size_t tb = 0;
-  HIPCHK(c, select_flagged_slots(c->s_keep.p, n, c->s_list.p, c->s_nkept.p, nullptr, &tb, s));
-  HIPCHK(c, c->s_select.ensure(tb));
-  HIPCHK(c, select_flagged_slots(c->s_keep.p, n, c->s_list.p, c->s_nkept.p, c->s_select.p, &tb, s));
-  HIPCHK(c, launch_fill(e_out, (size_t)n, __builtin_inf(), s));
+  HIPCHK(c, c->s_nkept.ensure(groups + 1));
+  // the kept slots in the scan's pose order (so that consecutive kept poses stay in the
+  // scan's bricks); every energy +inf until it is scored
+  a.e = e_out;
+  HIPCHK(c, launch_scan_keep(a, c->s_tperm.p,
+                             KeepScratch{c->s_keep.p, c->s_nkept.p, c->s_nkept.p + groups, c->s_list.p}, s));
   int nk = 0;
-  HIPCHK(c, hipMemcpyAsync(&nk, c->s_nkept.p, sizeof(int), hipMemcpyDeviceToHost, s));
+  HIPCHK(c, hipMemcpyAsync(&nk, c->s_nkept.p + groups, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(c, hipStreamSynchronize(s));
   if (nk > 0) {
     if (mode == MMO_INTERP) {

@@ -198,21 +198,30 @@ struct ScanFilterArgs {
   int nrot, ntrans;
   const double* lig;          // centred conformer rows (x, y, z)
   int n_atoms;
-  const uint32_t* mask;       // protein vdW volume bitmask, voxel i + j*nx + k*nx*ny
+  const int* order;           // the order in which its atoms are tested
+  const uint32_t* cells;      // protein vdW volume by cell (launch_mask_cells), i + j*nx + k*nx*ny
   double ox, oy, oz, inv_step;
   int nx, ny, nz;
   const uint8_t* skip;        // per translation: 1 = skipped (ROI / centre clash)
   int atom_clash;             // test every atom's 8 corners
-  double* e;                  // scan energies, set to +inf for skipped poses
+  double* e;                  // scan energies, set to +inf for skipped poses (all, before scoring)
 };
 hipError_t launch_scan_filter(const ScanFilterArgs& a, hipStream_t s);
-// keep[slot] = 1 for the poses the filters keep, over the scan's pose order (rotation r,
-// translation tperm[slot - r * ntrans])
-hipError_t launch_scan_keep(const ScanFilterArgs& a, const int* tperm, uint8_t* keep, hipStream_t s);
-// out[0 .. *n_out) = the slots whose flag is set, in order (n_out: device); temp: device
-// scratch of *temp_bytes (with temp == nullptr only *temp_bytes is set)
-hipError_t select_flagged_slots(const uint8_t* flags, int n, int* out, int* n_out, void* temp,
-                                size_t* temp_bytes, hipStream_t s);
+// the bitmask's cells: bit (i, j, k) set when one of the cell's 8 corners is
+hipError_t launch_mask_cells(const uint32_t* mask, uint32_t* cells, int nx, int ny, int nz,
+                             hipStream_t s);
+// Filter before scoring: list[0 .. *total) = the slots of the scan's pose order (rotation r,
+// translation tperm[slot - r * ntrans]) that the filters keep, in order; every a.e = +inf.
+constexpr int kKeepSlots = 2048;   // slots of one workgroup
+size_t scan_keep_groups(int nrot, int ntrans);
+struct KeepScratch {
+  uint64_t* words;            // kKeepSlots / 64 per workgroup: keep flags
+  unsigned* count;            // per workgroup
+  unsigned* total;
+  int* list;
+};
+hipError_t launch_scan_keep(const ScanFilterArgs& a, const int* tperm, const KeepScratch& w,
+                            hipStream_t s);
 
 constexpr int kTopkMax = 2048;
 constexpr int kTopkCand = 4096;   // keys the select leaves to the final sort (>= kTopkMax)

@@ -83,3 +83,45 @@ def test_topk_edges(sys0, kind, n, k):
     want = np.lexsort((np.arange(n), key))[:k]
     assert np.array_equal(i.cpu().numpy(), want)
     assert np.array_equal(v.cpu().numpy(), e[want], equal_nan=True)
+
+
+@pytest.mark.parametrize("nrot,ntrans", [(1, 1), (40, 3), (70, 63), (3, 64), (2, 2049), (1, 4500)])
+def test_scan_filters_on_few_and_many_translations(sys0, nrot, ntrans):
+    """The clash filters with fewer than 64 translations (slots of several rotations in a
+    wavefront) and with more (one rotation per workgroup, 2,048 slots each), before and after
+    scoring: the poses that the mask's corners give, and atoms or translations that are not finite
+    never clash."""
+    import torch
+    from mmo_amd import _lib
+    ctx, lig, rec = sys0
+    small = synth.make_ligand(np.random.default_rng(5), 12, 8, 0)
+    lid = ctx.add_ligand(small)
+    rng = np.random.default_rng(nrot + ntrans)
+    rots, trans = synth.random_rotations(rng, nrot), rng.uniform(-6, 6, (ntrans, 3))
+    if ntrans > 3:
+        trans[2, 1] = np.nan
+    rxyz, step = _rows(rec), 0.375
+    origin = rxyz.min(axis=0) - 2.0
+    dims = tuple(int(v) for v in np.ceil((rxyz.max(axis=0) + 2.0 - origin) / step) + 1)
+    ctx.set_vdw_mask(step, dims, origin)
+    flags = _lib.SCAN_ATOM_CLASH
+    before, kept = ctx.scan_filtered(lid, ff.SHIFTED, rots, trans, flags=flags)
+    after = torch.zeros(nrot * ntrans, dtype=torch.float64, device="cuda:0")
+    ctx.scan_filter(lid, rots, trans, after, flags=flags)
+    skipped = np.isinf(after.cpu().numpy())
+    words = ctx.vdw_mask()
+    bit = lambda v: (words[v >> 5] >> (v & 31)) & 1   # noqa: E731
+    c = _rows(small)
+    want = np.zeros((nrot, ntrans), dtype=bool)
+    for r in range(nrot):
+        f = ((c @ rots[r].T)[None] + trans[:, None] - origin) * (1.0 / step)
+        inside = np.all((f > -1.0) & (f < np.array(dims) - 1), axis=2)
+        i = np.where(inside[..., None], np.nan_to_num(f), 0.0).astype(np.int64)
+        for q in range(8):
+            v = (i[..., 0] + (q & 1)) + dims[0] * ((i[..., 1] + ((q >> 1) & 1)) + dims[1] * (i[..., 2] + (q >> 2)))
+            want[r] |= np.any(inside & (bit(v) != 0), axis=1)
+    assert np.array_equal(skipped, want.ravel())
+    e = before.cpu().numpy()
+    assert kept == int((~skipped).sum()) and np.array_equal(np.isposinf(e) & skipped, skipped)
+    full = ctx.scan(lid, ff.SHIFTED, rots, trans).cpu().numpy()
+    assert np.array_equal(e[~skipped], full[~skipped], equal_nan=True)
