@@ -408,7 +408,9 @@ int mmo_fixed_point_bits(const mmo_ctx* ctx);
  * once: 4 or 8), "row_filter" (1: the row lists test each far row's atoms against the
  * wavefront's box grown by the cutoff and sweep only those within it; same energies),
  * "scan_split" (row-list scans of at most this many 64-pose tiles take one ligand atom per
- * wavefront; same energies), "cell_size" (applies to the next mmo_set_receptor), "mc_waves_per_cu",
+ * wavefront; same energies), "scan_lattice" (interpolated scans of translations that form a
+ * lattice: 0 the general kernel, 1 the lattice kernel by a rule on sizes, 2 whenever it can),
+ * "cell_size" (applies to the next mmo_set_receptor), "mc_waves_per_cu",
  * "pose_waves" (batches: wavefronts per workgroup), "pose_cull" (1: batches in
  * the shifted form run one wavefront per pose with a culled receptor sweep; 0: tiles of
  * poses over the whole receptor), "pose_sweep" (that sweep: 1 lanes over the receptor

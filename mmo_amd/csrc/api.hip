@@ -150,6 +150,7 @@ struct mmo_ctx {
   int scan_xsub = 8;
   int scan_chunk = 4;
   int row_filter = 1;
+  int scan_lattice = 1;       // interpolated scans of lattices: 0 general kernel, 1 by rule, 2 always
   int scan_split = 12288;     // row-list scans of at most this many tiles split the atoms
   CellGrid cgs{};
   DevBuf<int> d_cells;
@@ -653,6 +654,63 @@ std::vector<int> morton_translations(const double* trans, int ntrans) {
   for (int t = 0; t < ntrans; ++t) tperm[t] = t;
   std::stable_sort(tperm.begin(), tperm.end(), [&](int a, int b) { return key[a] < key[b]; });
   return tperm;
+}
+
+// Translations that are a product X x Y x Z listed axis by axis (any axis fastest), compared
+// value for value: the axes' values one after the other, their lengths and strides.
+bool translation_lattice(const double* trans, int ntrans, std::vector<double>& axes, int n[3],
+                         int stride[3]) {
+  static const int orders[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+  for (const auto& o : orders) {   // o[0] the fastest axis
+    const int f = o[0], m = o[1], s = o[2];
+    auto same = [&](int t, int u, int ax) { return trans[3 * (size_t)t + ax] == trans[3 * (size_t)u + ax]; };
+    int nf = 1;
+    while (nf < ntrans && same(nf, 0, m) && same(nf, 0, s)) ++nf;
+    int nm = 1;
+    while ((long long)(nm + 1) * nf <= ntrans && same(nm * nf, 0, s)) ++nm;
+    if (ntrans % ((long long)nf * nm) != 0) continue;
+    const int ns = ntrans / (nf * nm);
+    bool ok = true;
+    for (int k = 0, t = 0; k < ns && ok; ++k)
+      for (int j = 0; j < nm && ok; ++j)
+        for (int i = 0; i < nf && ok; ++i, ++t)
+          ok = same(t, i, f) && same(t, j * nf, m) && same(t, k * nm * nf, s);
+    if (!ok) continue;
+    n[f] = nf; n[m] = nm; n[s] = ns;
+    stride[f] = 1; stride[m] = nf; stride[s] = nf * nm;
+    axes.clear();
+    for (int ax = 0; ax < 3; ++ax)
+      for (int i = 0; i < n[ax]; ++i) axes.push_back(trans[3 * (size_t)i * stride[ax] + ax]);
+    return true;
+  }
+  return false;
+}
+
+// Whether an interpolated scan takes the lattice kernel (k_interp_lattice): translations that
+// form a lattice whose z ascend by at most 4 grid layers, grids within a 31-bit buffer, and
+// enough work.  SIMD cycles per ligand atom, measured on 75 atoms and 64^3 grids: a 64-pose
+// tile of the general kernel 579; a wavefront of the lattice kernel about 250 for the x, y
+// and z weights, 130 a layer (its two node pairs a lane, at 4 lanes a cycle) and 27 a z, so
+// it gains where the columns fill their wavefronts and z shares layers: ms general / lattice,
+// 4,608 rotations: 20^3 at 0.5 A 10.18 / 3.88, 16^3 at 0.25 4.02 / 1.03, 9 x 9 x 40 at 0.2
+// 3.18 / 1.07, 10^3 at 1.0 2.11 / 1.74, but 5 x 5 x 1 0.075 / 0.098.  A wavefront walks its z
+// one after the other (250 us a 20-long column), so below 2,048 wavefronts the general
+// kernel's shorter ones win: 128 rotations of 20^3 (896) 0.32 / 0.35, 512 (3,584) 1.27 / 0.53.
+bool lattice_scan(const mmo_ctx* c, int nrot, const double* trans, int ntrans,
+                  std::vector<double>& axes, LatticeArgs& la) {
+  const size_t grid_bytes = c->g.nvox * c->ntypes * sizeof(float);
+  if (!c->scan_lattice || grid_bytes >= ((size_t)1 << 31) ||
+      !translation_lattice(trans, ntrans, axes, la.n, la.stride))
+    return false;
+  la.nrot = nrot; la.ntrans = ntrans; la.g = c->g; la.grid_bytes = (uint32_t)grid_bytes;
+  const int nz = la.n[2], zc = std::min(nz, kLatticeZ);
+  const double* z = axes.data() + la.n[0] + la.n[1];
+  for (int k = 1; k < nz; ++k)   // also false for a z that is not a number
+    if (!(z[k] >= z[k - 1] && (z[k] - z[k - 1]) * c->g.ods <= 4.0)) return false;
+  if (c->scan_lattice == 2) return true;
+  const double layers = nz > 1 ? (z[nz - 1] - z[0]) * c->g.ods * (zc - 1) / (nz - 1) + 2.0 : 2.0;
+  const double units = (double)lattice_units(la), tiles = (double)nrot * ((ntrans + kWave - 1) / kWave);
+  return units >= 2048.0 && 1.15 * units * (250.0 + 130.0 * layers + 27.0 * zc) < 579.0 * tiles;
 }
 
 }  // namespace
@@ -1528,11 +1586,25 @@ int mmo_scan_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, int nrot,
     for (int t : c->ligs[lig_id].type)
       if (t >= c->ntypes) return fail(c, MMO_ERR_BAD_ARG, "ligand grid type %d >= %d", t, c->ntypes);
   hipStream_t s = (hipStream_t)stream;
-  const std::vector<int> tperm = morton_translations(trans, ntrans);
-  if ((r = upload(c, c->s_tperm, tperm.data(), tperm.size(), s))) return r;
   HIPCHK(c, c->s_scan.ensure(9 * (size_t)nrot + 3 * (size_t)ntrans));
   HIPCHK(c, hipMemcpyAsync(c->s_scan.p, rots, 9 * (size_t)nrot * sizeof(double),
                            hipMemcpyHostToDevice, s));
+  std::vector<double> axes;
+  LatticeArgs la{};
+  if (mode == MMO_INTERP && lattice_scan(c, nrot, trans, ntrans, axes, la)) {
+    la.rots = c->s_scan.p; la.axes = c->s_scan.p + 9 * (size_t)nrot;
+    la.ligs = c->d_ligs.p; la.latoms = c->d_latoms.p; la.lig_xyz = c->d_lig_xyz.p;
+    la.lig = lig_id; la.e_out = e_out;
+    HIPCHK(c, hipMemcpyAsync(c->s_scan.p + 9 * (size_t)nrot, axes.data(), axes.size() * sizeof(double),
+                             hipMemcpyHostToDevice, s));
+    timer_begin(c, "interp", s);
+    HIPCHK(c, launch_interp_lattice(la, s));
+    timer_end(c, "interp", s);
+    HIPCHK(c, hipStreamSynchronize(s));   // the host arrays have been read
+    return MMO_OK;
+  }
+  const std::vector<int> tperm = morton_translations(trans, ntrans);
+  if ((r = upload(c, c->s_tperm, tperm.data(), tperm.size(), s))) return r;
   HIPCHK(c, hipMemcpyAsync(c->s_scan.p + 9 * (size_t)nrot, trans, 3 * (size_t)ntrans * sizeof(double),
                            hipMemcpyHostToDevice, s));
   const double* d_rot = c->s_scan.p;
@@ -2643,6 +2715,7 @@ int mmo_tune_set(mmo_ctx* c, const char* key, double v) {
   else if (k == "scan_xsub" && iv >= 1 && iv <= 16) c->scan_xsub = iv;
   else if (k == "scan_chunk" && (iv == 4 || iv == 8)) c->scan_chunk = iv;
   else if (k == "row_filter" && (iv == 0 || iv == 1)) c->row_filter = iv;
+  else if (k == "scan_lattice" && iv >= 0 && iv <= 2) c->scan_lattice = iv;
   else if (k == "scan_split" && iv >= 0 && iv <= (1 << 20)) c->scan_split = iv;
   else if (k == "grid_pack" && (iv == 0 || iv == 1)) c->grid_pack = iv;
   else if (k == "mc_waves_per_cu" && iv >= 1 && iv <= 32) c->mc_waves_per_cu = iv;
@@ -2673,6 +2746,7 @@ double mmo_tune_get(mmo_ctx* c, const char* key) {
   if (k == "scan_xsub") return c->scan_xsub;
   if (k == "scan_chunk") return c->scan_chunk;
   if (k == "row_filter") return c->row_filter;
+  if (k == "scan_lattice") return c->scan_lattice;
   if (k == "scan_split") return c->scan_split;
   if (k == "grid_pack") return c->grid_pack;
   if (k == "pose_waves") return c->pose_waves;

@@ -98,4 +98,35 @@ __device__ __forceinline__ double trilin(const GridDev& g, int ty, double px, do
          G * (wlx * wly * wlz) + H * (whx * wly * wlz);
 }
 
+// The rigid scans' trilinear form (k_interp over scans, k_interp_lattice): the weights of
+// G3D.trilin factored by axis, bilinear in x and y on a layer, then linear in z.  Written in
+// fused operations, so that every scan kernel gives a pose the same bits.
+struct AxisCell { double w; int i; bool in; };   // weight of node i + 1, cell, inside the grid
+
+// p: distance from the grid's node 0 along one axis of n nodes (the cell test of trilin)
+__device__ __forceinline__ AxisCell axis_cell(const GridDev& g, double p, int n) {
+  const double f = p * g.ods;
+  AxisCell a;
+  a.in = p >= 0.0 && f < (double)(n - 1);
+  a.i = a.in ? (int)f : 0;
+  a.w = fma(-(double)a.i, g.step, p) * g.ods;
+  return a;
+}
+struct LayerWeights { double w00, w10, w11, w01; };
+__device__ __forceinline__ LayerWeights layer_weights(const AxisCell& x, const AxisCell& y) {
+  const double vx = 1.0 - x.w, vy = 1.0 - y.w;
+  return {vx * vy, x.w * vy, x.w * y.w, vx * y.w};
+}
+// nodes (i, j), (i + 1, j), (i + 1, j + 1), (i, j + 1) of a layer
+__device__ __forceinline__ double layer_value(const LayerWeights& w, float a, float b, float c, float d) {
+  return fma((double)d, w.w01, fma((double)c, w.w11, fma((double)b, w.w10, (double)a * w.w00)));
+}
+__device__ __forceinline__ double between_layers(double b0, double b1, double w) {
+  return fma(w, b1 - b0, b0);
+}
+// coordinate of R c + T along one row r of R (Rot.rotate, src/rot.ml:97-100, then translate)
+__device__ __forceinline__ double rotate_shift(const double* r, const double* c, double t) {
+  return fma(r[2], c[2], fma(r[1], c[1], r[0] * c[0])) + t;
+}
+
 }  // namespace mmo

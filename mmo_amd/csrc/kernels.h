@@ -55,6 +55,26 @@ struct InterpLaunch {
   const double* lig_xyz;
 };
 
+// interpolated rigid scan over translations X x Y x Z (k_interp_lattice)
+struct LatticeArgs {
+  const double* rots;          // nrot x 9
+  const double* axes;          // the n[0] x, n[1] y and n[2] z values
+  int nrot, ntrans, n[3], stride[3];   // translation of (i, j, k) = i stride[0] + ...
+  GridDev g;
+  uint32_t grid_bytes;         // of all types' grids together (below 2 GiB)
+  const LigInfo* ligs;
+  const LigAtom* latoms;
+  const double* lig_xyz;
+  int lig;
+  double* e_out;
+};
+constexpr int kLatticeZ = 20;   // z positions of one wavefront
+inline size_t lattice_units(const LatticeArgs& a) {
+  return (size_t)a.nrot * (((size_t)a.n[0] * a.n[1] + kWave - 1) / kWave) *
+         ((a.n[2] + kLatticeZ - 1) / kLatticeZ);
+}
+hipError_t launch_interp_lattice(const LatticeArgs& a, hipStream_t s);
+
 struct IntraArgs {
   const LigInfo* ligs;
   const uint32_t* pair_ij;

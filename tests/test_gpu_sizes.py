@@ -125,3 +125,33 @@ def test_scan_filters_on_few_and_many_translations(sys0, nrot, ntrans):
     assert kept == int((~skipped).sum()) and np.array_equal(np.isposinf(e) & skipped, skipped)
     full = ctx.scan(lid, ff.SHIFTED, rots, trans).cpu().numpy()
     assert np.array_equal(e[~skipped], full[~skipped], equal_nan=True)
+
+
+def _lattice(nx, ny, nz, step, order, rng):
+    """nx x ny x nz translations with unequal steps, listed with `order` from slow to fast."""
+    ax = [np.sort(rng.uniform(-0.5, 0.5, n)) * step * n for n in (nx, ny, nz)]
+    g = np.meshgrid(*[ax[k] for k in order], indexing="ij")
+    return np.stack([g[order.index(k)].ravel() for k in range(3)], 1)
+
+
+@pytest.mark.parametrize("dims,step,order", [
+    ((1, 1, 1), 0.5, (2, 1, 0)), ((64, 1, 1), 0.3, (2, 1, 0)), ((5, 13, 21), 0.4, (2, 1, 0)),
+    ((13, 5, 40), 0.2, (0, 1, 2)), ((7, 9, 20), 0.5, (1, 2, 0)), ((3, 4, 8), 3.0, (2, 0, 1)),
+    ((2, 2, 60), 0.9, (2, 1, 0))])
+def test_lattice_scan_equals_general_scan(sys0, dims, step, order):
+    """The interpolated scan of a translation lattice (unequal steps, any axis fastest, columns
+    that fill a wavefront or not, more and fewer z than one wavefront takes, poses that leave
+    the grid) gives the general kernel's energies bit for bit."""
+    ctx, lig, rec = sys0
+    probe_a, probe_q, types = synth.grid_types([lig], 10)
+    origin, gdims, gstep = synth.grid_spec((0.0, 0.0, 0.0), 64, 0.375)
+    ctx.compute_grids(probe_a, probe_q, gstep, gdims, origin, copy_out=False)
+    lid = ctx.add_ligand(lig, types=types[0])
+    rng = np.random.default_rng(sum(dims))
+    rots, trans = synth.random_rotations(rng, 3), _lattice(*dims, step, order, rng)
+    got = []
+    for how in (0, 2):
+        ctx.tune(scan_lattice=how)
+        got.append(ctx.scan(lid, ff.INTERP, rots, trans).cpu().numpy())
+    ctx.tune(scan_lattice=1)
+    assert np.array_equal(got[0], got[1], equal_nan=True)
