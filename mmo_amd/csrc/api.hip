@@ -139,7 +139,8 @@ struct mmo_ctx {
   int min_rec_lds = 1;        // fused minimiser: receptor in LDS when >= 8 wavefronts fit
   int mc_rec_lds = 1;         // Monte Carlo direct form: receptor in LDS when it fits
   int cull_waves = 8;          // rigid scan: wavefronts per workgroup
-  int pose_waves = 16;         // batches (one wavefront per pose): wavefronts per workgroup
+  int pose_waves = 16;         // batches (pose_sweep = 0): wavefronts per workgroup
+  int ncu = 256;               // compute units of the device
   CellGrid cg{};              // scan and grid kernels: cubic cells
   DevBuf<int> d_cell;
   CellGrid cgp{};             // pose and Monte Carlo sweeps: cells cut along x, same atom order
@@ -258,6 +259,10 @@ struct mmo_batch {
   std::vector<int> by_size, order;
   int order_waves = 0;
   DevBuf<int> d_pose_lig, d_atom_off, d_dof_off, d_perm, d_order, d_by_size;
+  // units of kUnitAtoms atoms of the shifted form's batch kernel, pose-major
+  int nunits = 0;
+  DevBuf<UnitAtom> d_units;
+  DevBuf<int> d_unit_off;
   DevBuf<Tile> d_tiles;
   DevBuf<double> d_xyz, d_e, d_g, d_part, d_conf;
 };
@@ -747,6 +752,7 @@ int mmo_ctx_create(int device, mmo_ctx** out) {
   mmo_ctx* c = new mmo_ctx();
   c->device = device;
   c->pid = getpid();
+  (void)hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device);
   if (hipStreamCreate(&c->stream) != hipSuccess) {
     delete c;
     return fail(nullptr, MMO_ERR_DEVICE, "stream creation failed");
@@ -1267,8 +1273,8 @@ static int pose_cull_waves(const mmo_ctx* c, int npose) {
   return std::max(1, std::min(c->pose_waves, (npose + 255) / 256));
 }
 
-// Deals the batch's slot order for workgroups of `waves` wavefronts (at creation, and
-// again only if the workgroup shape changes).  The host copy stays in the batch while
+// Deals the batch's slot order for workgroups of `waves` wavefronts (pose_sweep = 0; again
+// only if the workgroup shape changes).  The host copy stays in the batch while
 // the upload may be in flight; a re-deal first waits for the previous upload.
 static int deal_batch(mmo_batch* b, int waves, hipStream_t s) {
   if (b->order_waves == waves) return MMO_OK;
@@ -1324,8 +1330,24 @@ int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch**
   std::stable_sort(b->by_size.begin(), b->by_size.end(), [&](int u, int v) {
     return c->ligs[pose_lig[u]].n > c->ligs[pose_lig[v]].n;
   });
+  std::vector<UnitAtom> units;
+  std::vector<int> unit_off(npose + 1, 0);
+  {
+    std::vector<int> base(c->ligs.size() + 1, 0);   // LigInfo.atom_base
+    for (size_t l = 0; l < c->ligs.size(); ++l) base[l + 1] = base[l] + c->ligs[l].n;
+    units.reserve((size_t)na + (size_t)npose * (kUnitAtoms - 1));
+    for (int p = 0; p < npose; ++p) {
+      const LigHost& h = c->ligs[pose_lig[p]];
+      for (int j = 0; j < h.n || j % kUnitAtoms; ++j)
+        units.push_back(j < h.n ? UnitAtom{b->atom_off[p] + h.sweep[j], base[pose_lig[p]] + h.sweep[j]}
+                                : UnitAtom{-1, 0});
+      unit_off[p + 1] = (int)(units.size() / kUnitAtoms);
+    }
+    b->nunits = unit_off[npose];
+  }
   hipStream_t s = c->stream;
-  if ((r = deal_batch(b, pose_cull_waves(c, npose), s)) ||
+  if ((r = upload(c, b->d_units, units.data(), units.size(), s)) ||
+      (r = upload(c, b->d_unit_off, unit_off.data(), unit_off.size(), s)) ||
       (r = upload(c, b->d_pose_lig, b->pose_lig.data(), npose, s)) ||
       (r = upload(c, b->d_atom_off, b->atom_off.data(), npose + 1, s)) ||
       (r = upload(c, b->d_dof_off, b->dof_off.data(), npose + 1, s)) ||
@@ -1349,6 +1371,7 @@ void mmo_batch_destroy(mmo_batch* b) {
     (void)hipSetDevice(b->device);
     b->d_pose_lig.release(); b->d_atom_off.release(); b->d_dof_off.release(); b->d_perm.release();
     b->d_order.release(); b->d_by_size.release();
+    b->d_units.release(); b->d_unit_off.release();
     b->d_tiles.release(); b->d_xyz.release(); b->d_e.release(); b->d_g.release(); b->d_part.release();
     b->d_conf.release();
   }
@@ -1369,8 +1392,9 @@ int mmo_batch_dof_offsets(const mmo_batch* b, int32_t* off) {
   return MMO_OK;
 }
 
+// sum_later: the caller adds up the units' energies (b->d_part) of a shifted gradient itself
 static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out, double* grad,
-                       hipStream_t s) {
+                       hipStream_t s, bool sum_later = false) {
   mmo_ctx* c = b->ctx;
   const int inter = flags & (MMO_F_INTER_SHIFTED | MMO_F_INTER_GLOBAL | MMO_F_INTER_INTERP);
   if (inter && (inter & (inter - 1)))
@@ -1387,13 +1411,37 @@ static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out
       for (int t : h.type)
         if (t >= c->ntypes) return fail(c, MMO_ERR_BAD_ARG, "ligand grid type %d >= %d", t, c->ntypes);
   }
-  // every gradient producer adds to the buffer, except the pose kernel: when it runs it
+  // every gradient producer adds to the buffer, except the pose kernels: when one runs it
   // is the first producer and writes each atom's row once, so the buffer is not cleared
-  const bool pose_first = want_grad && (inter & MMO_F_INTER_SHIFTED) && c->pose_cull;
+  const bool pose_first = (inter & MMO_F_INTER_SHIFTED) && c->pose_cull;
+  const bool by_units = pose_first && c->pose_sweep == 1;   // writes the whole energy rows, too
   if (want_grad && !pose_first) HIPCHK(c, launch_fill(grad, 3 * (size_t)b->natoms, 0.0, s));
-  HIPCHK(c, launch_fill(e_out, 4 * (size_t)b->npose, 0.0, s));
-  if ((inter & MMO_F_INTER_SHIFTED) && c->pose_cull) {
-    // one wavefront per pose over the culled receptor (per-atom or 8-atom sub-block sweep)
+  if (!by_units) HIPCHK(c, launch_fill(e_out, 4 * (size_t)b->npose, 0.0, s));
+  const bool comp = (flags & MMO_F_COMPONENTS) != 0;
+  if (by_units) {
+    InterLaunch L = inter_launch(c, MMO_SHIFTED, c->d_ligs.p, c->d_latoms.p, c->d_lig_xyz.p);
+    L.cg = c->cgp;
+    PoseUnitArgs a{};
+    a.xyz = xyz; a.units = b->d_units.p; a.nunits = b->nunits; a.latoms = c->d_latoms.p;
+    a.rres = c->rres.p;
+    HIPCHK(c, b->d_part.ensure(2 * (size_t)b->nunits));
+    a.part = b->d_part.p;
+    timer_begin(c, "inter", s);
+    if (!want_grad || comp) {
+      a.pairs = comp ? 1 : 0;
+      HIPCHK(c, launch_pose_units(L, a, false, c->ncu, s));
+      HIPCHK(c, launch_pose_sum(a.part, b->d_unit_off.p, b->npose, comp, comp, e_out, s));
+    }
+    if (want_grad) {
+      a.grad = grad;
+      if (comp) a.part = nullptr;   // the energies are written
+      HIPCHK(c, launch_pose_units(L, a, true, c->ncu, s));
+      if (!comp && !sum_later)
+        HIPCHK(c, launch_pose_sum(a.part, b->d_unit_off.p, b->npose, false, false, e_out, s));
+    }
+    timer_end(c, "inter", s);
+  } else if (pose_first) {
+    // one wavefront per pose over the culled receptor, 8-atom sub-blocks
     InterLaunch L = inter_launch(c, MMO_SHIFTED, c->d_ligs.p, c->d_latoms.p, c->d_lig_xyz.p);
     L.cg = c->cgp;
     // the receptor goes to LDS when enough poses per workgroup amortise the copy
@@ -1401,23 +1449,21 @@ static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out
     PoseCullArgs a{};
     a.xyz = xyz; a.atom_off = b->d_atom_off.p; a.pose_lig = b->d_pose_lig.p; a.npose = b->npose;
     a.rres = c->rres.p;
-    a.ligs = c->d_ligs.p; a.latoms = c->d_latoms.p; a.atom_order = c->d_sweep.p;
+    a.ligs = c->d_ligs.p; a.latoms = c->d_latoms.p;
     a.e_out = e_out; a.e_stride = 4;
-    const bool comp = (flags & MMO_F_COMPONENTS) != 0;
     const int waves = pose_cull_waves(c, b->npose);
     if ((r = deal_batch(b, waves, s))) return r;
     a.order = b->d_order.p;
     timer_begin(c, "inter", s);
     if (!want_grad || comp) {
       a.e_comp = comp ? e_out : nullptr;
-      HIPCHK(c, launch_pose_cull(L, a, false, waves, c->pose_sweep == 1, s));
+      HIPCHK(c, launch_pose_cull(L, a, false, waves, s));
     }
     if (want_grad) {
       a.e_comp = nullptr;
       a.grad = grad;
-      a.grad_assign = 1;
       a.write_e = comp ? 0 : 1;
-      HIPCHK(c, launch_pose_cull(L, a, true, waves, c->pose_sweep == 1, s));
+      HIPCHK(c, launch_pose_cull(L, a, true, waves, s));
     }
     timer_end(c, "inter", s);
   } else if (inter & (MMO_F_INTER_SHIFTED | MMO_F_INTER_GLOBAL)) {
@@ -1435,7 +1481,6 @@ static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out
     L.rtile = std::min(L.rtile, L.rslice);
     nslice = (c->nrec + L.rslice - 1) / L.rslice;
     if (nslice > 1) HIPCHK(c, b->d_part.ensure((size_t)nslice * b->npose * 4));
-    const bool comp = (flags & MMO_F_COMPONENTS) != 0;
     timer_begin(c, "inter", s);
     if (!want_grad || comp)
       HIPCHK(c, launch_inter_coords(L, b->d_tiles.p, b->d_perm.p, b->ntiles, b->npose, xyz,
@@ -1555,8 +1600,13 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
         }
       }
     }
-    if ((r = batch_score(b, bflags, xyz, e_out, gx, s))) return r;
+    const bool sum_later = g && (score_flags & MMO_F_INTER_SHIFTED) && c->pose_cull && c->pose_sweep == 1;
+    if ((r = batch_score(b, bflags, xyz, e_out, gx, s, sum_later))) return r;
     if (g) {
+      if (sum_later) {
+        a.part = b->d_part.p; a.unit_off = b->d_unit_off.p; a.e_sum = e_out;
+        a.clear_intra = (score_flags & MMO_F_INTRA) ? 0 : 1;
+      }
       a.grad_xyz = gx;
       a.gdof = gdof;
       HIPCHK(c, launch_dof_grad(a, s));

@@ -151,6 +151,12 @@ __device__ __forceinline__ double wave_sum(double v) {
   v += dpp_d<0x143, 0xc>(v, 0.0);
   return readlane_d(v, 63);
 }
+// sum of v[i0 .. i1) over one wavefront (uniform): lane l adds v[i0 + l], v[i0 + l + 64], ...
+__device__ __forceinline__ double wave_sum_range(const double* v, int i0, int i1, int stride) {
+  double s = 0.0;
+  for (int i = i0 + (int)(threadIdx.x & (kWave - 1)); i < i1; i += kWave) s += v[(size_t)i * stride];
+  return wave_sum(s);
+}
 __device__ __forceinline__ double wave_max(double v) {
   v = fmax(v, dpp_d<0x111>(v, v));
   v = fmax(v, dpp_d<0x112>(v, v));
@@ -232,25 +238,31 @@ __device__ __forceinline__ LigPt lig_pt_far() {
   return LigPt{f, f, f, 0.0f, 0.0f, 0.0f};
 }
 
-// r^2 (A^2) of receptor atom i and ligand atom l from fixed-point differences d; for
-// pairs closer than sqrt(near2) the residuals of both atoms are added (a wavefront
-// branch that is rarely taken)
+// r^2 (A^2) of a pair from its fixed-point differences
+__device__ __forceinline__ float fixed_r2(float dx, float dy, float dz, const PairK& pk) {
+  return (dx * dx + dy * dy + dz * dz) * pk.inv_s2;
+}
+// r^2 of receptor atom i and ligand atom l with the residuals of both added: the near pairs
+__device__ __forceinline__ float near_r2(float dx, float dy, float dz, const LigPt& l, int i,
+                                         const PairK& pk) {
+  // 32-bit byte offset from the (wave-uniform) base (a 24-bit multiply, full rate),
+  // formed here: the empty asm keeps the compiler from hoisting it onto every pair
+  int ii = i;
+  asm volatile("" : "+v"(ii));
+  const RecRes rr = *reinterpret_cast<const RecRes*>(
+      reinterpret_cast<const char*>(pk.rres) + __umul24((uint32_t)ii, (uint32_t)sizeof(RecRes)));
+  const float ex = fmaf(dx, pk.inv_s, rr.x - l.rx);
+  const float ey = fmaf(dy, pk.inv_s, rr.y - l.ry);
+  const float ez = fmaf(dz, pk.inv_s, rr.z - l.rz);
+  return fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+}
+// r^2 of a pair; for pairs closer than sqrt(near2) the residuals of both atoms are added (a
+// wavefront branch that is rarely taken)
 __device__ __forceinline__ float pair_r2(float dx, float dy, float dz, const LigPt& l, int i,
                                          const PairK& pk) {
-  float r2 = (dx * dx + dy * dy + dz * dz) * pk.inv_s2;
+  float r2 = fixed_r2(dx, dy, dz, pk);
   if (__builtin_expect(__ballot(r2 < pk.near2) != 0ull, 0)) {
-    if (r2 < pk.near2) {
-      // 32-bit byte offset from the (wave-uniform) base (a 24-bit multiply, full rate),
-      // formed here: the empty asm keeps the compiler from hoisting it onto every pair
-      int ii = i;
-      asm volatile("" : "+v"(ii));
-      const RecRes rr = *reinterpret_cast<const RecRes*>(
-          reinterpret_cast<const char*>(pk.rres) + __umul24((uint32_t)ii, (uint32_t)sizeof(RecRes)));
-      const float ex = fmaf(dx, pk.inv_s, rr.x - l.rx);
-      const float ey = fmaf(dy, pk.inv_s, rr.y - l.ry);
-      const float ez = fmaf(dz, pk.inv_s, rr.z - l.rz);
-      r2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
-    }
+    if (r2 < pk.near2) r2 = near_r2(dx, dy, dz, l, i, pk);
   }
   return r2;
 }
@@ -265,18 +277,9 @@ __device__ __forceinline__ float max_r2(float r2, float min_r2) {
 // is the same and the clamp costs nothing outside the rare branch.
 __device__ __forceinline__ float pair_r2_clamped(float dx, float dy, float dz, const LigPt& l,
                                                  int i, const PairK& pk) {
-  float r2 = (dx * dx + dy * dy + dz * dz) * pk.inv_s2;
+  float r2 = fixed_r2(dx, dy, dz, pk);
   if (__builtin_expect(__ballot(r2 < pk.near2) != 0ull, 0)) {
-    if (r2 < pk.near2) {
-      int ii = i;
-      asm volatile("" : "+v"(ii));
-      const RecRes rr = *reinterpret_cast<const RecRes*>(
-          reinterpret_cast<const char*>(pk.rres) + __umul24((uint32_t)ii, (uint32_t)sizeof(RecRes)));
-      const float ex = fmaf(dx, pk.inv_s, rr.x - l.rx);
-      const float ey = fmaf(dy, pk.inv_s, rr.y - l.ry);
-      const float ez = fmaf(dz, pk.inv_s, rr.z - l.rz);
-      r2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
-    }
+    if (r2 < pk.near2) r2 = near_r2(dx, dy, dz, l, i, pk);
     r2 = max_r2(r2, pk.min_r2);
   }
   return r2;

@@ -26,6 +26,20 @@ __device__ __forceinline__ float shift_t_exact(const RecPos& p, const LigPt& l, 
   return (float)fmin(fmax(t, 0.0), 1.0);
 }
 
+// shifted-form receptor sums of one pair at r^2 (clamped)
+__device__ __forceinline__ void pair_sums(const RecPos& p, const RecAB& ab, float r2c, float t, float& sq,
+                                          float& s12, float& s6) {
+  const float ir = __builtin_amdgcn_rsqf(r2c);
+  const float u = inv_r2(ir, r2c);
+  const float u3 = u * (u * u);
+  // w u^3 serves both LJ terms: 9 multiplies and FMAs after u^3 instead of 10
+  const float w = t * t;
+  const float v = w * u3;
+  sq = fmaf(p.q, w * ir, sq);
+  s6 = fmaf(ab.b, v, s6);
+  s12 = fmaf(ab.a, v * u3, s12);
+}
+
 // EXACT_T: the shift t from shift_t_exact (single-probe sums: the grid precompute)
 template <int MODE, bool NEAR = true, bool EXACT_T = false>
 __device__ __forceinline__ void pair_energy(const RecPos& p, const RecAB& ab, const LigPt& l,
@@ -33,20 +47,13 @@ __device__ __forceinline__ void pair_energy(const RecPos& p, const RecAB& ab, co
                                             float& s6) {
   const float dx = (float)(p.x - l.x), dy = (float)(p.y - l.y), dz = (float)(p.z - l.z);
   // NEAR: the clamp is applied in the near-pair branch (pair_r2_clamped); else not needed
-  const float r2c = NEAR ? pair_r2_clamped(dx, dy, dz, l, i, pk)
-                         : (dx * dx + dy * dy + dz * dz) * pk.inv_s2;
-  const float ir = __builtin_amdgcn_rsqf(r2c);
-  const float u = inv_r2(ir, r2c);
-  const float u3 = u * (u * u);
+  const float r2c = NEAR ? pair_r2_clamped(dx, dy, dz, l, i, pk) : fixed_r2(dx, dy, dz, pk);
   if (MODE == MMO_SHIFTED) {
-    // w u^3 serves both LJ terms: 9 multiplies and FMAs after u^3 instead of 10
-    const float t = EXACT_T ? shift_t_exact(p, l, i, pk) : shift_t(r2c, pk);
-    const float w = t * t;
-    const float v = w * u3;
-    sq = fmaf(p.q, w * ir, sq);
-    s6 = fmaf(ab.b, v, s6);
-    s12 = fmaf(ab.a, v * u3, s12);
+    pair_sums(p, ab, r2c, EXACT_T ? shift_t_exact(p, l, i, pk) : shift_t(r2c, pk), sq, s12, s6);
   } else {
+    const float ir = __builtin_amdgcn_rsqf(r2c);
+    const float u = inv_r2(ir, r2c);
+    const float u3 = u * (u * u);
     sq = fmaf(p.q, ir, sq);
     s12 = fmaf(ab.a, u3 * u3, s12);
     s6 = fmaf(ab.b, u3, s6);
@@ -57,12 +64,9 @@ __device__ __forceinline__ void pair_energy(const RecPos& p, const RecAB& ab, co
 // coef * (x_rec - x_lig) in fixed-point units (the caller scales by -2 * 2^-k).
 // F = ke qi qj / r + Aij u^6 - 2 Bij u^3, dF/dr2 = -u (ke qi qj / (2 r) + 6 Aij u^6 - 6 Bij u^3),
 // w = t^2 with t = 1 - r2/144, dw/dr2 = -t/72.
-__device__ __forceinline__ void pair_grad_shifted(const RecPos& p, const RecAB& ab, const LigPt& l,
-                                                  int i, const PairK& pk, float c1, float aj,
-                                                  float bj, float& e, float& gx, float& gy,
-                                                  float& gz) {
-  const float dx = (float)(p.x - l.x), dy = (float)(p.y - l.y), dz = (float)(p.z - l.z);
-  const float r2 = pair_r2(dx, dy, dz, l, i, pk);
+__device__ __forceinline__ void pair_grad_at(const RecPos& p, const RecAB& ab, float dx, float dy,
+                                             float dz, float r2, const PairK& pk, float c1, float aj,
+                                             float bj, float& e, float& gx, float& gy, float& gz) {
   const float r2c = max_r2(r2, pk.min_r2);
   const float ir = __builtin_amdgcn_rsqf(r2c);
   const float u = inv_r2(ir, r2c);
@@ -81,6 +85,13 @@ __device__ __forceinline__ void pair_grad_shifted(const RecPos& p, const RecAB& 
   gz = fmaf(coef, dz, gz);
 }
 
+__device__ __forceinline__ void pair_grad_shifted(const RecPos& p, const RecAB& ab, const LigPt& l,
+                                                  int i, const PairK& pk, float c1, float aj,
+                                                  float bj, float& e, float& gx, float& gy,
+                                                  float& gz) {
+  const float dx = (float)(p.x - l.x), dy = (float)(p.y - l.y), dz = (float)(p.z - l.z);
+  pair_grad_at(p, ab, dx, dy, dz, pair_r2(dx, dy, dz, l, i, pk), pk, c1, aj, bj, e, gx, gy, gz);
+}
 // ------------------------------------------------------- inter kernel, culled
 // Shifted form only.  The whole receptor sits in LDS sorted by 4 A cells.  For each
 // block of K atoms per lane the wavefront takes the bounding box of its lanes' atom
@@ -708,6 +719,176 @@ __device__ __forceinline__ int in_vgpr_i(int x) {
   return x;
 }
 
+// One pass of the per-atom sweep: NA ligand atoms lu (uniform) against the receptor atoms near
+// any of them; the lanes' FP32 sums (energy form: sq, s12, s6 per atom; GRAD: fe and the
+// gradient f in fixed-point units).  pk: pair_k; c1, fa, fb: the atoms' parameters (GRAD).
+// MERGED: the pass's pairs share one test for a near pair instead of one each.  The pairs
+// are then straight-line code, which holds more registers: measured for the energies of
+// batches 316 against 340 us (2,500 poses, 15,000-atom receptor in global memory), but no gain
+// for the chains (23.8 against 23.4 ms), the gradient (280 / 278 us) or the minimiser (22.0
+// against 20.8 ms), which keep one test a pair.
+template <bool GRAD, bool NEAR, int NA, bool MERGED>
+__device__ __forceinline__ void sweep_pass(const CellGrid& cg, const int* __restrict__ s_cell,
+                                           const RecPos* __restrict__ s_pos,
+                                           const RecAB* __restrict__ s_ab, float inv_s, const PairK& pk,
+                                           int* wl, const LigPt (&lu)[NA], const float (&c1)[NA],
+                                           const float (&fa)[NA], const float (&fb)[NA], float (&sq)[NA],
+                                           float (&s12)[NA], float (&s6)[NA], float (&fe)[NA],
+                                           float (&fx)[NA], float (&fy)[NA], float (&fz)[NA]) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int* s_r0 = wl;                 // compacted rows: first receptor atom
+  int* s_beg = wl + kWave;        //                 first position; s_beg[nc] = total
+  int* s_cnt = wl + 2 * kWave;    // [1..63]: rows whose first segment lane is this one
+  const uint64_t below = lane ? ((1ull << lane) - 1ull) : 0ull;
+  constexpr float R = 12.05f;     // cutoff + FP32 rounding margin
+  constexpr float R2 = R * R;
+  float qx[NA], qy[NA], qz[NA];
+  LigPt lv[NA];
+  float zlo_q = 3.0e38f, zhi_q = -3.0e38f, ylo_q = 3.0e38f, yhi_q = -3.0e38f;
+#pragma unroll
+  for (int u = 0; u < NA; ++u) {
+    qx[u] = uniformf((float)lu[u].x * inv_s);
+    qy[u] = uniformf((float)lu[u].y * inv_s);
+    qz[u] = uniformf((float)lu[u].z * inv_s);
+    // the pair loop reads the (wave-uniform) ligand atoms from VGPRs: an SGPR operand
+    // would cost issue rate on every pair
+    lv[u] = LigPt{in_vgpr_i(lu[u].x), in_vgpr_i(lu[u].y), in_vgpr_i(lu[u].z), lu[u].rx,
+                  lu[u].ry, lu[u].rz};
+    zlo_q = fminf(zlo_q, qz[u]); zhi_q = fmaxf(zhi_q, qz[u]);
+    ylo_q = fminf(ylo_q, qy[u]); yhi_q = fmaxf(yhi_q, qy[u]);
+  }
+  const int cz0 = max(0, (int)floorf((zlo_q - R - cg.z0) * cg.inv_c));
+  const int cz1 = min(cg.nz - 1, (int)floorf((zhi_q + R - cg.z0) * cg.inv_c));
+  const int cy0 = max(0, (int)floorf((ylo_q - R - cg.y0) * cg.inv_c));
+  const int cy1 = min(cg.ny - 1, (int)floorf((yhi_q + R - cg.y0) * cg.inv_c));
+  const int nyc = cy1 - cy0 + 1, nzc = cz1 - cz0 + 1;
+  const int nrows = (nzc > 0 && nyc > 0) ? nzc * nyc : 0;
+  // up to 8 x 8 rows (cells of 3.5 A or more): lane = 8 z + y, no division
+  const bool grid8 = nyc <= 8 && nzc <= 8;
+#pragma unroll
+  for (int u = 0; u < NA; ++u) sq[u] = s12[u] = s6[u] = fe[u] = fx[u] = fy[u] = fz[u] = 0.0f;
+  for (int base_row = 0; base_row < nrows; base_row += kWave) {
+    int r0 = 0, len = 0;
+    const int idx = base_row + lane;
+    const bool in = grid8 ? (base_row == 0 && (lane >> 3) < nzc && (lane & 7) < nyc) : idx < nrows;
+    if (in) {
+      const int cz = grid8 ? cz0 + (lane >> 3) : cz0 + idx / nyc;
+      const int cy = grid8 ? cy0 + (lane & 7) : cy0 + idx % nyc;
+      const float zlo = cg.z0 + cz * cg.c, ylo = cg.y0 + cy * cg.c;
+      float xlo = 3.0e38f, xhi = -3.0e38f;
+#pragma unroll
+      for (int u = 0; u < NA; ++u) {
+        const float dzb = fmaxf(0.0f, fmaxf(zlo - qz[u], qz[u] - (zlo + cg.c)));
+        const float dyb = fmaxf(0.0f, fmaxf(ylo - qy[u], qy[u] - (ylo + cg.c)));
+        const float rx2 = R2 - dzb * dzb - dyb * dyb;
+        if (rx2 >= 0.0f) {
+          const float rx = bound_sqrt(rx2);
+          xlo = fminf(xlo, qx[u] - rx);
+          xhi = fmaxf(xhi, qx[u] + rx);
+        }
+      }
+      if (xlo <= xhi) {
+        const int cx0 = max(0, (int)floorf((xlo - cg.x0) * cg.inv_cx));
+        const int cx1 = min(cg.nx - 1, (int)floorf((xhi - cg.x0) * cg.inv_cx));
+        if (cx0 <= cx1) {
+          const int rowb = (cz * cg.ny + cy) * cg.nx;
+          r0 = s_cell[rowb + cx0];
+          len = s_cell[rowb + cx1 + 1] - r0;
+        }
+      }
+    }
+    // inclusive prefix sum of the row lengths: row k covers [incl - len, incl)
+    const int incl = wave_incl_scan(len);
+    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+    if (total == 0) {
+      if (grid8) break;
+      continue;
+    }
+    const uint64_t nonempty = __ballot(len > 0);
+    const int nc = __popcll(nonempty);
+    // this lane's segment [t, t_end) of the concatenation
+    const int m = (total + kWave - 1) / kWave;
+    int t = lane * m;
+    const int t_end = min(total, t + m);
+    // first lane whose segment starts at or after this row's start; only the first
+    // non-empty row starts at 0 (lane 0), and a row that no segment starts in (first
+    // lane 64) is reached by walking
+    const int first_lane = ceil_div_small(incl - len, m, __builtin_amdgcn_rcpf((float)m));
+    wave_lds_sync();            // the previous rows' readers are done
+    if (len > 0) {
+      const int c = __popcll(nonempty & below);
+      s_r0[c] = r0;
+      s_beg[c] = incl - len;
+    }
+    if (lane == 0) s_beg[nc] = total;
+    if (lane > 0) s_cnt[lane] = 0;
+    wave_lds_sync();
+    if (len > 0 && first_lane > 0 && first_lane < kWave) atomicAdd(&s_cnt[first_lane], 1);
+    wave_lds_sync();
+    // the row holding t: k = (rows starting at or before t) - 1, a prefix sum over
+    // the lanes of how many rows first reach each lane (1 at lane 0: row 0)
+    const int k = wave_incl_scan(lane > 0 ? s_cnt[lane] : 1) - 1;
+    int i = s_r0[k] + (t - s_beg[k]);
+    int row_end = s_beg[k + 1];
+    int kw = k;
+    for (int it = 0; it < m; ++it, ++t) {
+      if (t < t_end) {
+        if (t == row_end) {       // the next compacted row starts here
+          ++kw;
+          i = s_r0[kw];
+          row_end = s_beg[kw + 1];
+        }
+        const RecPos p = s_pos[i];
+        const RecAB ab = s_ab[i];
+        if constexpr (MERGED) {
+          // the pass's pairs share one test for a near pair (on the bit patterns: r^2 is
+          // not negative), so that they are straight-line code and overlap
+          float dx[NA], dy[NA], dz[NA], r2[NA];
+          int nearest = 0x7fffffff;
+#pragma unroll
+          for (int u = 0; u < NA; ++u) {
+            dx[u] = (float)(p.x - lv[u].x);
+            dy[u] = (float)(p.y - lv[u].y);
+            dz[u] = (float)(p.z - lv[u].z);
+            r2[u] = fixed_r2(dx[u], dy[u], dz[u], pk);
+            nearest = min(nearest, __float_as_int(r2[u]));
+          }
+          if (NEAR && __builtin_expect(__ballot(nearest < __float_as_int(pk.near2)) != 0ull, 0)) {
+#pragma unroll
+            for (int u = 0; u < NA; ++u) {
+              // the energy form takes the differences again (from copies the compiler
+              // cannot match with those above) rather than hold all of them up to here
+              int px = p.x, py = p.y, pz = p.z;
+              if (!GRAD) asm volatile("" : "+v"(px), "+v"(py), "+v"(pz));
+              if (r2[u] < pk.near2)
+                r2[u] = near_r2((float)(px - lv[u].x), (float)(py - lv[u].y), (float)(pz - lv[u].z),
+                                lv[u], i, pk);
+              if (!GRAD) r2[u] = max_r2(r2[u], pk.min_r2);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < NA; ++u) {
+            if (GRAD)
+              pair_grad_at(p, ab, dx[u], dy[u], dz[u], r2[u], pk, c1[u], fa[u], fb[u], fe[u],
+                           fx[u], fy[u], fz[u]);
+            else
+              pair_sums(p, ab, r2[u], shift_t(r2[u], pk), sq[u], s12[u], s6[u]);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < NA; ++u) {
+            if (GRAD)
+              pair_grad_shifted(p, ab, lv[u], i, pk, c1[u], fa[u], fb[u], fe[u], fx[u], fy[u], fz[u]);
+            else
+              pair_energy<MMO_SHIFTED, NEAR>(p, ab, lv[u], i, pk, sq[u], s12[u], s6[u]);
+          }
+        }
+        ++i;
+      }
+    }
+  }
+}
+
 template <bool GRAD, class AtomFn, class GradOut, bool NEAR = true, bool PRELOAD = true,
           int NA = 1>
 __device__ __forceinline__ void atom_sweep(const CellGrid& cg, const int* __restrict__ s_cell,
@@ -719,12 +900,6 @@ __device__ __forceinline__ void atom_sweep(const CellGrid& cg, const int* __rest
   static_assert(NA == 1 || (NA >= 2 && NA <= 4 && PRELOAD), "several atoms per pass need the preload");
   const PairK pk = pair_k(fr.inv_s2, fr.inv_s, rres);
   const int lane = threadIdx.x & (kWave - 1);
-  int* s_r0 = wl;                 // compacted rows: first receptor atom
-  int* s_beg = wl + kWave;        //                 first position; s_beg[nc] = total
-  int* s_cnt = wl + 2 * kWave;    // [1..63]: rows whose first segment lane is this one
-  const uint64_t below = lane ? ((1ull << lane) - 1ull) : 0ull;
-  constexpr float R = 12.05f;     // cutoff + FP32 rounding margin
-  constexpr float R2 = R * R;
   // PRELOAD: the atoms of a 64-atom chunk are fetched together, one per lane, and
   // broadcast one at a time; in GRAD the lane of an atom keeps its gradient until the
   // chunk ends, so no atom waits on its own load or gradient write.  NA > 1: NA
@@ -760,118 +935,14 @@ __device__ __forceinline__ void atom_sweep(const CellGrid& cg, const int* __rest
           atom(jb + jj, lu[u], cq[u], ca[u], cb[u]);
         }
       }
-      float qx[NA], qy[NA], qz[NA], c1[NA], fa[NA], fb[NA];
-      LigPt lv[NA];
-      float zlo_q = 3.0e38f, zhi_q = -3.0e38f, ylo_q = 3.0e38f, yhi_q = -3.0e38f;
-#pragma unroll
-      for (int u = 0; u < NA; ++u) {
-        qx[u] = uniformf((float)lu[u].x * fr.inv_s);
-        qy[u] = uniformf((float)lu[u].y * fr.inv_s);
-        qz[u] = uniformf((float)lu[u].z * fr.inv_s);
-        // the pair loop reads the (wave-uniform) ligand atoms from VGPRs: an SGPR operand
-        // would cost issue rate on every pair
-        lv[u] = LigPt{in_vgpr_i(lu[u].x), in_vgpr_i(lu[u].y), in_vgpr_i(lu[u].z), lu[u].rx,
-                      lu[u].ry, lu[u].rz};
-        c1[u] = (float)cq[u]; fa[u] = (float)ca[u]; fb[u] = (float)cb[u];
-        zlo_q = fminf(zlo_q, qz[u]); zhi_q = fmaxf(zhi_q, qz[u]);
-        ylo_q = fminf(ylo_q, qy[u]); yhi_q = fmaxf(yhi_q, qy[u]);
-      }
-      const int cz0 = max(0, (int)floorf((zlo_q - R - cg.z0) * cg.inv_c));
-      const int cz1 = min(cg.nz - 1, (int)floorf((zhi_q + R - cg.z0) * cg.inv_c));
-      const int cy0 = max(0, (int)floorf((ylo_q - R - cg.y0) * cg.inv_c));
-      const int cy1 = min(cg.ny - 1, (int)floorf((yhi_q + R - cg.y0) * cg.inv_c));
-      const int nyc = cy1 - cy0 + 1, nzc = cz1 - cz0 + 1;
-      const int nrows = (nzc > 0 && nyc > 0) ? nzc * nyc : 0;
-      // up to 8 x 8 rows (cells of 3.5 A or more): lane = 8 z + y, no division
-      const bool grid8 = nyc <= 8 && nzc <= 8;
+      float c1[NA], fa[NA], fb[NA];
       float sq[NA], s12[NA], s6[NA], fe[NA], fx[NA], fy[NA], fz[NA];
 #pragma unroll
-      for (int u = 0; u < NA; ++u) sq[u] = s12[u] = s6[u] = fe[u] = fx[u] = fy[u] = fz[u] = 0.0f;
-      for (int base_row = 0; base_row < nrows; base_row += kWave) {
-        int r0 = 0, len = 0;
-        const int idx = base_row + lane;
-        const bool in = grid8 ? (base_row == 0 && (lane >> 3) < nzc && (lane & 7) < nyc) : idx < nrows;
-        if (in) {
-          const int cz = grid8 ? cz0 + (lane >> 3) : cz0 + idx / nyc;
-          const int cy = grid8 ? cy0 + (lane & 7) : cy0 + idx % nyc;
-          const float zlo = cg.z0 + cz * cg.c, ylo = cg.y0 + cy * cg.c;
-          float xlo = 3.0e38f, xhi = -3.0e38f;
-#pragma unroll
-          for (int u = 0; u < NA; ++u) {
-            const float dzb = fmaxf(0.0f, fmaxf(zlo - qz[u], qz[u] - (zlo + cg.c)));
-            const float dyb = fmaxf(0.0f, fmaxf(ylo - qy[u], qy[u] - (ylo + cg.c)));
-            const float rx2 = R2 - dzb * dzb - dyb * dyb;
-            if (rx2 >= 0.0f) {
-              const float rx = bound_sqrt(rx2);
-              xlo = fminf(xlo, qx[u] - rx);
-              xhi = fmaxf(xhi, qx[u] + rx);
-            }
-          }
-          if (xlo <= xhi) {
-            const int cx0 = max(0, (int)floorf((xlo - cg.x0) * cg.inv_cx));
-            const int cx1 = min(cg.nx - 1, (int)floorf((xhi - cg.x0) * cg.inv_cx));
-            if (cx0 <= cx1) {
-              const int rowb = (cz * cg.ny + cy) * cg.nx;
-              r0 = s_cell[rowb + cx0];
-              len = s_cell[rowb + cx1 + 1] - r0;
-            }
-          }
-        }
-        // inclusive prefix sum of the row lengths: row k covers [incl - len, incl)
-        const int incl = wave_incl_scan(len);
-        const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
-        if (total == 0) {
-          if (grid8) break;
-          continue;
-        }
-        const uint64_t nonempty = __ballot(len > 0);
-        const int nc = __popcll(nonempty);
-        // this lane's segment [t, t_end) of the concatenation
-        const int m = (total + kWave - 1) / kWave;
-        int t = lane * m;
-        const int t_end = min(total, t + m);
-        // first lane whose segment starts at or after this row's start; only the first
-        // non-empty row starts at 0 (lane 0), and a row that no segment starts in (first
-        // lane 64) is reached by walking
-        const int first_lane = ceil_div_small(incl - len, m, __builtin_amdgcn_rcpf((float)m));
-        wave_lds_sync();            // the previous rows' readers are done
-        if (len > 0) {
-          const int c = __popcll(nonempty & below);
-          s_r0[c] = r0;
-          s_beg[c] = incl - len;
-        }
-        if (lane == 0) s_beg[nc] = total;
-        if (lane > 0) s_cnt[lane] = 0;
-        wave_lds_sync();
-        if (len > 0 && first_lane > 0 && first_lane < kWave) atomicAdd(&s_cnt[first_lane], 1);
-        wave_lds_sync();
-        // the row holding t: k = (rows starting at or before t) - 1, a prefix sum over
-        // the lanes of how many rows first reach each lane (1 at lane 0: row 0)
-        const int k = wave_incl_scan(lane > 0 ? s_cnt[lane] : 1) - 1;
-        int i = s_r0[k] + (t - s_beg[k]);
-        int row_end = s_beg[k + 1];
-        int kw = k;
-        for (int it = 0; it < m; ++it, ++t) {
-          if (t < t_end) {
-            if (t == row_end) {       // the next compacted row starts here
-              ++kw;
-              i = s_r0[kw];
-              row_end = s_beg[kw + 1];
-            }
-            const RecPos p = s_pos[i];
-            const RecAB ab = s_ab[i];
-#pragma unroll
-            for (int u = 0; u < NA; ++u) {
-              if (GRAD)
-                pair_grad_shifted(p, ab, lv[u], i, pk, c1[u], fa[u], fb[u], fe[u], fx[u], fy[u],
-                                  fz[u]);
-              else
-                pair_energy<MMO_SHIFTED, NEAR>(p, ab, lv[u], i, pk, sq[u], s12[u], s6[u]);
-            }
-            ++i;
-          }
-        }
+      for (int u = 0; u < NA; ++u) {
+        c1[u] = (float)cq[u]; fa[u] = (float)ca[u]; fb[u] = (float)cb[u];
       }
+      sweep_pass<GRAD, NEAR, NA, false>(cg, s_cell, s_pos, s_ab, fr.inv_s, pk, wl, lu, c1, fa, fb, sq,
+                                        s12, s6, fe, fx, fy, fz);
 #pragma unroll
       for (int u = 0; u < NA; ++u) {
         if (!live[u]) continue;

@@ -539,16 +539,159 @@ hipError_t launch_pack_cells(const GridDev& g, int ntypes, float* cells, hipStre
 }
 
 // ----------------------------------------------------- inter kernel, pose-culled
-// ligand atoms per pass of the per-atom sweep
-constexpr int kPoseSweepAtoms = 4;
+// Shifted form for arbitrary poses (batches, gradients, minimisation): the work is cut into
+// units of kUnitAtoms ligand atoms, consecutive in the ligand's sweep order (a walk of its
+// bond graph, so a unit is a compact piece of it), and a wavefront takes one unit at a time
+// (sweep_pass: the receptor atoms near any of the four).  The cost follows the pairs inside
+// the cutoff wherever the poses are, a few poses spread over as many wavefronts as they have
+// units, and many poses end together whatever their ligands' sizes.  Each unit's energy is
+// its own FP64 wavefront sum, added up per pose by lane and wavefront sum (k_pose_sum,
+// k_dof_grad), so a pose's bits do not depend on the batch it is in.
+// Bound: VALU issue and the latency of each unit's row listing (4 wavefronts per SIMD with
+// the gradient, 6 without).  The receptor and the cell table come from L1 and L2: a copy in
+// LDS (one persistent workgroup per CU taking blocks of units in turn) measured 191 against
+// 172 us for 4,096 poses and 722 against 643 for 16,384, as its wavefronts end unevenly where
+// the dispatcher deals out small workgroups.  One wavefront per pose, which this replaces,
+// us for gradients of 1, 64, 1,024, 4,096, 16,384 poses of library ligands: 81, 194, 181,
+// 189, 662 -> 11, 14, 55, 172, 643; on the 15,000-atom receptor 161, 378, 385, 411, 1301 ->
+// 18, 21, 95, 312, 1195.
+template <bool GRAD>
+__global__ void __launch_bounds__(256) k_pose_units(PoseUnitArgs a, Frame fr, const RecPos* rpos,
+                                                    const RecAB* rab, CellGrid cg) {
+  __shared__ int s_wl[4 * kAtomSweepInts];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  int* wl = s_wl + wave * kAtomSweepInts;
+  const PairK pk = pair_k(fr.inv_s2, fr.inv_s, a.rres);
+  constexpr int NA = kUnitAtoms;
+  // A wavefront takes a.block consecutive units (of one pose or of several): their atoms are
+  // fetched and converted together, one per lane, then broadcast unit by unit.
+  const int u0 = uniformi((blockIdx.x * 4 + wave) * a.block);
+  const int nu = min(a.block, a.nunits - u0);
+  if (nu <= 0) return;
+  {
+    UnitAtom ua{-1, 0};
+    if (lane < NA * nu) ua = a.units[(size_t)u0 * NA + lane];
+    LigPt mine = lig_pt_zero();
+    double mq = 0.0, ma = 0.0, mb = 0.0;
+    int sat = 0;
+    if (ua.row >= 0) {
+      const double* x = a.xyz + 3 * (size_t)ua.row;
+      mine = lig_pt(x[0], x[1], x[2], fr, &sat);
+      const LigAtom la = a.latoms[ua.latom];
+      mq = la.keq; ma = la.a; mb = la.b;
+    }
+    (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
+    const uint64_t valid = __ballot(ua.row >= 0);
+    float gxm = 0.0f, gym = 0.0f, gzm = 0.0f;   // GRAD: the lane's atom's
+    for (int k = 0; k < nu; ++k) {
+      const int live = __popcll((valid >> (NA * k)) & ((1ull << NA) - 1ull));
+      LigPt lu[NA];
+      double cq[NA], ca[NA], cb[NA];
+      float c1[NA], fa[NA], fb[NA];
+#pragma unroll
+      for (int u = 0; u < NA; ++u) {
+        const int ju = NA * k + (u < live ? u : 0);   // a short unit repeats its first atom
+        lu[u].x = __builtin_amdgcn_readlane(mine.x, ju);
+        lu[u].y = __builtin_amdgcn_readlane(mine.y, ju);
+        lu[u].z = __builtin_amdgcn_readlane(mine.z, ju);
+        lu[u].rx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.rx), ju));
+        lu[u].ry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.ry), ju));
+        lu[u].rz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.rz), ju));
+        cq[u] = readlane_d(mq, ju);
+        ca[u] = readlane_d(ma, ju);
+        cb[u] = readlane_d(mb, ju);
+        c1[u] = (float)cq[u]; fa[u] = (float)ca[u]; fb[u] = (float)cb[u];
+      }
+      float sq[NA], s12[NA], s6[NA], fe[NA], fx[NA], fy[NA], fz[NA];
+      sweep_pass<GRAD, true, NA, !GRAD>(cg, cg.cell_start, rpos, rab, fr.inv_s, pk, wl, lu, c1, fa, fb,
+                                        sq, s12, s6, fe, fx, fy, fz);
+      if (GRAD) {
+        double e = 0.0;
+#pragma unroll
+        for (int u = 0; u < NA; ++u) {
+          if (u < live) e += (double)fe[u];
+          const float sx = wave_sum_f(fx[u]), sy = wave_sum_f(fy[u]), sz = wave_sum_f(fz[u]);
+          gxm = lane == NA * k + u ? sx : gxm;
+          gym = lane == NA * k + u ? sy : gym;
+          gzm = lane == NA * k + u ? sz : gzm;
+        }
+        if (a.part) {
+          e = wave_sum(e);
+          if (lane == 0) a.part[u0 + k] = e;
+        }
+      } else {
+        double el = 0.0, vd = 0.0;
+#pragma unroll
+        for (int u = 0; u < NA; ++u) {
+          if (u >= live) continue;
+          el = fma((double)sq[u], cq[u], el);
+          vd = fma((double)s12[u], ca[u], vd);
+          vd = fma(-2.0 * (double)s6[u], cb[u], vd);
+        }
+        if (a.pairs) {
+          el = wave_sum(el);
+          vd = wave_sum(vd);
+          if (lane == 0) {
+            a.part[2 * (size_t)(u0 + k)] = el;
+            a.part[2 * (size_t)(u0 + k) + 1] = vd;
+          }
+        } else {
+          el = wave_sum(el + vd);
+          if (lane == 0) a.part[u0 + k] = el;
+        }
+      }
+    }
+    if (GRAD && ua.row >= 0) {
+      const double gs = -2.0 * (double)fr.inv_s;
+      double* g = a.grad + 3 * (size_t)ua.row;
+      g[0] = gs * (double)gxm; g[1] = gs * (double)gym; g[2] = gs * (double)gzm;
+    }
+  }
+}
 
-// Shifted form for arbitrary poses (batches, gradients, minimisation): one wavefront per
-// pose; the receptor is swept per 8-atom sub-block of the pose (pose_sweep) or per atom
-// (atom_sweep), so the cost follows the pairs inside the cutoff wherever the poses are.
-// With an order, slot s of the launch (workgroup s / waves, wavefront s % waves) scores
-// pose order[s]: the host deals the poses, largest ligands first, so that the SIMDs
-// receive equal shares of ligand atoms instead of whatever the batch order gives them.
-template <bool GRAD, bool LDS, bool ATOMWISE>
+hipError_t launch_pose_units(const InterLaunch& L, const PoseUnitArgs& args, bool grad, int ncu,
+                             hipStream_t s) {
+  PoseUnitArgs a = args;
+  if (a.nunits == 0) return hipSuccess;
+  // one unit a wavefront until the chip is full several times over (5,120 wavefronts at a
+  // time); then two, whose atoms are fetched and converted together: 57,000 units 176 / 172
+  // us (gradient), 229,000 665 / 643; 14,000 55 / 55.  More (632 us with 4, 630 with 8) lose
+  // as much on the 15,000-atom receptor's energies (870 us with 1, 900 with 2, 930 with 4).
+  a.block = a.nunits >= 128 * ncu ? 2 : 1;
+  const size_t groups = ((size_t)(a.nunits + a.block - 1) / a.block + 3) / 4;
+  if (grad)
+    hipLaunchKernelGGL(k_pose_units<true>, dim3((unsigned)groups), dim3(256), 0, s, a, L.fr, L.rpos, L.rab, L.cg);
+  else
+    hipLaunchKernelGGL(k_pose_units<false>, dim3((unsigned)groups), dim3(256), 0, s, a, L.fr, L.rpos, L.rab, L.cg);
+  return hipGetLastError();
+}
+
+template <bool PAIRS>
+__global__ void __launch_bounds__(256) k_pose_sum(const double* part, const int* unit_off, int npose,
+                                                  bool comp, double* e_out) {
+  const int p = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  if (p >= npose) return;
+  const int u0 = unit_off[p], u1 = unit_off[p + 1];
+  const double a = wave_sum_range(part, u0, u1, PAIRS ? 2 : 1);
+  const double b = PAIRS ? wave_sum_range(part + 1, u0, u1, 2) : 0.0;
+  const int lane = threadIdx.x & (kWave - 1);
+  if (lane < 4) e_out[4 * (size_t)p + lane] = lane == 0 ? a + b : lane == 1 || !comp ? 0.0 : lane == 2 ? a : b;
+}
+
+hipError_t launch_pose_sum(const double* part, const int* unit_off, int npose, bool pairs, bool comp,
+                           double* e_out, hipStream_t s) {
+  if (npose == 0) return hipSuccess;
+  const dim3 grid((npose + 3) / 4), block(256);
+  if (pairs) hipLaunchKernelGGL(k_pose_sum<true>, grid, block, 0, s, part, unit_off, npose, comp, e_out);
+  else hipLaunchKernelGGL(k_pose_sum<false>, grid, block, 0, s, part, unit_off, npose, comp, e_out);
+  return hipGetLastError();
+}
+
+// The earlier batch kernel (tuning key pose_sweep = 0): one wavefront per pose, the receptor
+// swept per 8-atom sub-block (pose_sweep).  With an order, slot s of the launch (workgroup
+// s / waves, wavefront s % waves) scores pose order[s]: the host deals the poses, largest
+// ligands first, so that the SIMDs receive equal shares of ligand atoms.
+template <bool GRAD, bool LDS>
 __global__ void __launch_bounds__(1024) k_pose_cull(PoseCullArgs a, Frame fr, const RecPos* rpos,
                                                     const RecAB* rab, int nrec, CellGrid cg) {
   extern __shared__ __align__(16) char smem[];
@@ -557,81 +700,61 @@ __global__ void __launch_bounds__(1024) k_pose_cull(PoseCullArgs a, Frame fr, co
   const int* s_cell;
   load_receptor<LDS>(rpos, rab, nrec, cg, s_pos, s_ab, s_cell, smem);
   const int lane = threadIdx.x & (kWave - 1);
-  // this wavefront's scratch for atom_sweep, after the receptor copy
-  int* wl = reinterpret_cast<int*>(smem + receptor_lds_bytes<LDS>(nrec, cg)) +
-            (threadIdx.x / kWave) * kAtomSweepInts;
-  auto score = [&](int p) {
-    const LigInfo li = a.ligs[a.pose_lig[p]];
-    const size_t row0 = (size_t)a.atom_off[p];
-    const double* x = a.xyz + 3 * row0;
-    int sat = 0;
-    double e_el = 0.0, e_vd = 0.0;
-    // sweep position j -> ligand atom (the per-atom sweep's order, if given)
-    auto at = [&](int j) { return (ATOMWISE && a.atom_order) ? a.atom_order[li.atom_base + j] : j; };
-    auto atom = [&](int j, LigPt& l, double& cq, double& ca, double& cb) {
-      const int ja = at(j);
-      l = lig_pt(x[3 * ja], x[3 * ja + 1], x[3 * ja + 2], fr, &sat);
-      const LigAtom la = a.latoms[li.atom_base + ja];
-      cq = la.keq; ca = la.a; cb = la.b;
-    };
-    auto gout = [&](int j, double gx, double gy, double gz) {
-      double* g = a.grad + 3 * (row0 + at(j));
-      if (a.grad_assign) {
-        g[0] = gx; g[1] = gy; g[2] = gz;
-      } else {
-        g[0] += gx; g[1] += gy; g[2] += gz;
-      }
-    };
-    if (ATOMWISE)
-      atom_sweep<GRAD, decltype(atom)&, decltype(gout)&, true, true, kPoseSweepAtoms>(
-          cg, s_cell, s_pos, s_ab, a.rres, fr, li.n_atoms, wl, atom, gout, e_el, e_vd);
-    else
-      pose_sweep<GRAD>(cg, s_cell, s_pos, s_ab, a.rres, fr, li.n_atoms, atom, gout, e_el, e_vd);
-    (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
-    // every lane of an atom slot holds part of the sums: the wavefront sum counts each
-    // pair once (lanes of one slot share the atom, split the receptor atoms)
-    e_el = wave_sum(e_el);
-    e_vd = wave_sum(e_vd);
-    if (lane == 0) {
-      const size_t o = (size_t)p * a.e_stride;
-      if (!GRAD || a.write_e) a.e_out[o] = e_el + e_vd;
-      if (!GRAD && a.e_comp) {
-        a.e_comp[o + 2] = e_el;
-        a.e_comp[o + 3] = e_vd;
-      }
-    }
-  };
   const int slot = blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
-  if (slot < a.npose) score(a.order ? a.order[slot] : slot);
+  if (slot >= a.npose) return;
+  const int p = a.order ? a.order[slot] : slot;
+  const LigInfo li = a.ligs[a.pose_lig[p]];
+  const size_t row0 = (size_t)a.atom_off[p];
+  const double* x = a.xyz + 3 * row0;
+  int sat = 0;
+  double e_el = 0.0, e_vd = 0.0;
+  auto atom = [&](int j, LigPt& l, double& cq, double& ca, double& cb) {
+    l = lig_pt(x[3 * j], x[3 * j + 1], x[3 * j + 2], fr, &sat);
+    const LigAtom la = a.latoms[li.atom_base + j];
+    cq = la.keq; ca = la.a; cb = la.b;
+  };
+  auto gout = [&](int j, double gx, double gy, double gz) {
+    double* g = a.grad + 3 * (row0 + j);
+    g[0] = gx; g[1] = gy; g[2] = gz;
+  };
+  pose_sweep<GRAD>(cg, s_cell, s_pos, s_ab, a.rres, fr, li.n_atoms, atom, gout, e_el, e_vd);
+  (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
+  // every lane of an atom slot holds part of the sums: the wavefront sum counts each
+  // pair once (lanes of one slot share the atom, split the receptor atoms)
+  e_el = wave_sum(e_el);
+  e_vd = wave_sum(e_vd);
+  if (lane == 0) {
+    const size_t o = (size_t)p * a.e_stride;
+    if (!GRAD || a.write_e) a.e_out[o] = e_el + e_vd;
+    if (!GRAD && a.e_comp) {
+      a.e_comp[o + 2] = e_el;
+      a.e_comp[o + 3] = e_vd;
+    }
+  }
 }
 
 hipError_t launch_pose_cull(const InterLaunch& L, const PoseCullArgs& a, bool grad, int waves,
-                            bool atomwise, hipStream_t s) {
+                            hipStream_t s) {
   if (a.npose == 0) return hipSuccess;
   waves = std::max(1, std::min(16, waves));
   const int blocks = (a.npose + waves - 1) / waves;
   const bool in_lds = L.cull == 1;
-  const size_t lds = (in_lds ? receptor_lds_bytes<true>(L.nrec, L.cg) : 0) +
-                     (size_t)waves * kAtomSweepInts * sizeof(int);
-#define MMO_POSE_CULL(G, A)                                                                    \
+  const size_t lds = in_lds ? receptor_lds_bytes<true>(L.nrec, L.cg) : 0;
+#define MMO_POSE_CULL(G)                                                                       \
   if (in_lds) {                                                                                \
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pose_cull<G, true, A>), \
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pose_cull<G, true>),   \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);  \
     if (e != hipSuccess) return e;                                                             \
-    hipLaunchKernelGGL((k_pose_cull<G, true, A>), dim3(blocks), dim3(waves * kWave), lds, s,   \
+    hipLaunchKernelGGL((k_pose_cull<G, true>), dim3(blocks), dim3(waves * kWave), lds, s,      \
                        a, L.fr, L.rpos, L.rab, L.nrec, L.cg);                                  \
   } else {                                                                                     \
-    hipLaunchKernelGGL((k_pose_cull<G, false, A>), dim3(blocks), dim3(waves * kWave), lds, s,  \
+    hipLaunchKernelGGL((k_pose_cull<G, false>), dim3(blocks), dim3(waves * kWave), lds, s,     \
                        a, L.fr, L.rpos, L.rab, L.nrec, L.cg);                                  \
   }
-  if (grad && atomwise) {
-    MMO_POSE_CULL(true, true)
-  } else if (grad) {
-    MMO_POSE_CULL(true, false)
-  } else if (atomwise) {
-    MMO_POSE_CULL(false, true)
+  if (grad) {
+    MMO_POSE_CULL(true)
   } else {
-    MMO_POSE_CULL(false, false)
+    MMO_POSE_CULL(false)
   }
 #undef MMO_POSE_CULL
   return hipGetLastError();

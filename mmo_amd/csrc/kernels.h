@@ -132,6 +132,12 @@ struct DofArgs {
   int e_stride;
   const uint32_t* pair_ij;
   const double4* pair_par;      // ke qi qj, Ai Aj, 2 Bi Bj
+  // nullable: the adjoint also sums the poses' units (launch_pose_sum's GRAD form) into
+  // e_sum[4 * pose] and clears the rest of the row (E_intra only with clear_intra)
+  const double* part;
+  const int* unit_off;
+  double* e_sum;
+  int clear_intra;
 };
 
 // part: scratch of (nslices * npose * e_stride) doubles when the receptor is split
@@ -188,21 +194,36 @@ struct PoseCullArgs {
   double* e_out;            // e_out[pose * e_stride] = E_inter
   int e_stride;
   double* e_comp;           // nullable: [pose*e_stride + 2] elec, [+3] vdW
-  double* grad;             // GRAD: dE/dxyz rows, added to what the buffer holds
-  int grad_assign;          // GRAD: write the rows instead (each atom's row is written once)
+  double* grad;             // GRAD: dE/dxyz rows (each atom's row is written once)
   int write_e;
   const RecRes* rres;       // receptor quantisation residuals
   // nullable: the pose of each launch slot (slot = workgroup * waves + wavefront), a
   // permutation of 0..npose-1
   const int* order;
-  // nullable: per ligand at atom_base, the order in which the per-atom sweep takes the
-  // atoms (a permutation of 0..n_atoms-1)
-  const int* atom_order;
 };
-// atomwise: lanes over the receptor atoms near each ligand atom (atom_sweep) instead of
-// 8-atom sub-blocks (pose_sweep)
 hipError_t launch_pose_cull(const InterLaunch& L, const PoseCullArgs& a, bool grad, int waves,
-                            bool atomwise, hipStream_t s);
+                            hipStream_t s);
+
+// shifted form per unit of kUnitAtoms ligand atoms (consecutive in the sweep order)
+constexpr int kUnitAtoms = 4;
+struct UnitAtom { int row, latom; };   // coordinate row, ligand-atom index; row < 0: none
+struct PoseUnitArgs {
+  const double* xyz;        // rows (x, y, z)
+  const UnitAtom* units;    // kUnitAtoms per unit, pose-major
+  int nunits;
+  const LigAtom* latoms;
+  const RecRes* rres;
+  double* part;             // per unit: E, or with `pairs` (energy form) elec and vdW; nullable (GRAD)
+  int pairs;
+  double* grad;             // GRAD: each atom's row written once
+  int block;                // units a wavefront takes (set by the launch)
+};
+hipError_t launch_pose_units(const InterLaunch& L, const PoseUnitArgs& a, bool grad, int ncu,
+                             hipStream_t s);
+// e_out[4p ..] = E_inter, 0, elec, vdW (comp) or E_inter, 0, 0, 0 from the poses' units
+// [unit_off[p], unit_off[p + 1]); pairs: part holds (elec, vdW), else E
+hipError_t launch_pose_sum(const double* part, const int* unit_off, int npose, bool pairs, bool comp,
+                           double* e_out, hipStream_t s);
 
 // LDS a workgroup may hold on gfx950
 constexpr size_t kMaxLds = 160 * 1024;

@@ -233,6 +233,10 @@ __global__ void __launch_bounds__(INTRA ? kDofWaves * kWave : kWave) k_dof_grad(
     load_conformer(a, li, sx, sy, sz);
     forward_torsions(li, t, sx, sy, sz);   // ends with a barrier
   }
+  if (a.part && tid >= (int)blockDim.x - kWave) {   // the last wavefront
+    const double e = wave_sum_range(a.part, a.unit_off[pose], a.unit_off[pose + 1], 1);
+    if (lane < 4 && (lane != 1 || a.clear_intra)) a.e_sum[4 * (size_t)pose + lane] = lane == 0 ? e : 0.0;
+  }
   if (INTRA) {
     double* gx = gi + 3 * L * (tid / kWave);
     double* gy = gx + L;

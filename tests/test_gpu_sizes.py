@@ -155,3 +155,52 @@ def test_lattice_scan_equals_general_scan(sys0, dims, step, order):
         got.append(ctx.scan(lid, ff.INTERP, rots, trans).cpu().numpy())
     ctx.tune(scan_lattice=1)
     assert np.array_equal(got[0], got[1], equal_nan=True)
+
+
+@pytest.mark.parametrize("atoms", [1, 4, 5, 75, 131])
+@pytest.mark.parametrize("n", [1, 2400])
+def test_pose_units(sys0, atoms, n):
+    """Batches by units of four ligand atoms: ligands whose last unit is full or not, one
+    pose and enough (131 atoms: 79,200 units) for two units a wavefront.  Energies, their
+    parts and gradients of sampled poses against the oracle, and each pose alone gives the
+    bits it has in the batch, also through DOF vectors."""
+    import torch
+    ctx, _, rec = sys0
+    rng = np.random.default_rng(atoms)
+    lig = synth.config0()[0] if atoms == 75 else None
+    if lig is None:
+        big = max(synth.library(24), key=lambda l: len(l["xs"]))
+        keep = np.arange(min(atoms, len(big["xs"])))
+        lig = {k: big[k][keep] for k in ("xs", "ys", "zs", "q", "anum")}
+        lig.update(dists=np.asarray(big["dists"])[np.ix_(keep, keep)], rb_left=np.zeros(0, np.int32),
+                   rb_right=np.zeros(0, np.int32), rg_off=np.zeros(1, np.int32),
+                   rg_atoms=np.zeros(0, np.int32))
+    lid = ctx.add_ligand(lig)
+    b = ctx.batch(np.full(n, lid))
+    x = np.concatenate([_rows(lig) @ r.T + rng.uniform(-4, 4, 3) for r in synth.random_rotations(rng, n)])
+    flags = ff.F_INTER_SHIFTED | ff.F_INTRA
+    e, g = b.score(x, flags | ff.F_GRAD)
+    ec, _ = b.score(x, flags | ff.F_COMPONENTS)
+    np.testing.assert_allclose(ec[:, 2] + ec[:, 3], ec[:, 0], rtol=1e-12, atol=1e-9)
+    one = ctx.batch(np.array([lid]))
+    m = len(lig["xs"])
+    for p in rng.choice(n, min(n, 6), replace=False):
+        xp = x[p * m:(p + 1) * m]
+        e1, g1 = one.score(xp, flags | ff.F_GRAD)
+        assert np.array_equal(e1[0], e[p]) and np.array_equal(g1, g[p * m:(p + 1) * m])
+        posed = dict(lig, xs=xp[:, 0].copy(), ys=xp[:, 1].copy(), zs=xp[:, 2].copy())
+        s = inter_abs_sum(rec, xp, lig, True)
+        want = oracle.ene_inter(rec, posed, shifted=True)
+        assert_energy(e[p, 0], want, s, what="units %d" % atoms)
+        assert_energy(ec[p, 0], want, s, what="units %d, parts" % atoms)
+    d = torch.tensor(np.concatenate([np.concatenate([rng.uniform(-3, 3, 6), np.zeros(len(lig["rb_left"]))])
+                                     for _ in range(n)]), device="cuda:0")
+    ed = torch.full((n, 4), 7.0, dtype=torch.float64, device="cuda:0")
+    gd = torch.empty_like(d)
+    b.score_dofs_dev(d, ed, gdof=gd, flags=ff.F_INTER_SHIFTED | ff.F_GRAD)
+    nd = len(d) // n
+    e1, g1 = torch.full((1, 4), 7.0, dtype=torch.float64, device="cuda:0"), torch.empty(nd, dtype=torch.float64, device="cuda:0")
+    one.score_dofs_dev(d[-nd:].clone(), e1, gdof=g1, flags=ff.F_INTER_SHIFTED | ff.F_GRAD)
+    torch.cuda.synchronize()
+    assert torch.equal(e1[0], ed[-1]) and torch.equal(g1, gd[-nd:])
+    assert torch.all(ed[:, 1:] == 0)   # no E_intra asked for, no parts with the gradient
