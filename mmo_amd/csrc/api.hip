@@ -94,6 +94,11 @@ struct DevBuf {
   }
 };
 
+// ligands the adjoint without a serial pass takes: a bound on the host's check, and on the
+// n^2 bits of interacting pairs (above, a pose does not fit in LDS with its E_intra)
+constexpr int kMaxFreeAtoms = 1024;
+constexpr size_t kMaxFreeWork = 1u << 24;
+
 struct LigHost {
   int n;
   std::vector<double> xyz;   // centred conformer, rows
@@ -102,6 +107,7 @@ struct LigHost {
   std::vector<uint32_t> pair_ij;
   std::vector<int> rb_left, rb_right, rg_off, rg_atoms;
   std::vector<int> sweep;   // order in which the per-atom sweeps take the atoms
+  bool free = false;        // torsions_free, and within kMaxFree*
   std::vector<int> clash;   // order in which the scan filters test them (farthest first)
 };
 
@@ -176,6 +182,8 @@ struct mmo_ctx {
   DevBuf<double> d_lig_xyz;
   DevBuf<uint32_t> d_pair_ij;
   DevBuf<double4> d_pair_par;
+  DevBuf<uint64_t> d_intra_bits;   // per atom i, bit d: the pair (i, i + d mod n) counts (free ligands)
+  DevBuf<int64_t> d_bit_base;      // per ligand, into d_intra_bits
   DevBuf<int> d_sweep;          // per ligand at atom_base: the sweeps' atom order
   DevBuf<int> d_clash;          // the same: the scan filters' order
   DevBuf<int> d_rb_left, d_rb_right, d_rg_off, d_rg_atoms;
@@ -252,6 +260,7 @@ struct mmo_batch {
   int device = 0;      // the context's, kept so that destruction never reads the context
   pid_t pid = 0;
   int npose = 0, natoms = 0, ndof = 0, ntiles = 0, max_atoms = 0, max_rb = 0, max_rg = 0;
+  bool free = true;    // every ligand's torsions are free (LigHost)
   std::vector<int> pose_lig, atom_off, dof_off, perm;
   std::vector<Tile> tiles;
   // poses by ligand size, largest first, and the pose kernel's slot order dealt from it
@@ -427,6 +436,8 @@ int sync_ligands(mmo_ctx* c) {
   std::vector<uint32_t> pij;
   std::vector<double4> ppar;
   std::vector<int> rbl, rbr, rgo, rga, swp, clash;
+  std::vector<uint64_t> bits;
+  std::vector<int64_t> bit_base;
   c->max_atoms = 0;
   for (const LigHost& h : c->ligs) {
     LigInfo li{};
@@ -453,6 +464,17 @@ int sync_ligands(mmo_ctx* c) {
     if (r) return r;
     pij.insert(pij.end(), h.pair_ij.begin(), h.pair_ij.end());
     ppar.insert(ppar.end(), pp.begin(), pp.end());
+    bit_base.push_back((int64_t)bits.size());
+    if (h.free) {
+      const uint32_t n = h.n, words = n / 128 + 1;
+      bits.resize(bits.size() + (size_t)words * n, 0ull);
+      uint64_t* w = bits.data() + bit_base.back();
+      for (uint32_t ij : h.pair_ij) {   // the pair (i, j) from the end with d <= n / 2
+        const uint32_t i = ij & 0xffff, j = ij >> 16, lo = std::min(i, j), gap = std::max(i, j) - lo;
+        const uint32_t from = gap <= n / 2 ? lo : lo + gap, d = gap <= n / 2 ? gap : n - gap;
+        w[from * words + d / 64] |= 1ull << (d % 64);
+      }
+    }
     rbl.insert(rbl.end(), h.rb_left.begin(), h.rb_left.end());
     rbr.insert(rbr.end(), h.rb_right.begin(), h.rb_right.end());
     const int ga = (int)rga.size();
@@ -468,6 +490,8 @@ int sync_ligands(mmo_ctx* c) {
   if ((r = upload(c, c->d_lig_xyz, xyz.data(), xyz.size(), s))) return r;
   if ((r = upload(c, c->d_pair_ij, pij.data(), pij.size(), s))) return r;
   if ((r = upload(c, c->d_pair_par, ppar.data(), ppar.size(), s))) return r;
+  if ((r = upload(c, c->d_intra_bits, bits.data(), bits.size(), s))) return r;
+  if ((r = upload(c, c->d_bit_base, bit_base.data(), bit_base.size(), s))) return r;
   if ((r = upload(c, c->d_rb_left, rbl.data(), rbl.size(), s))) return r;
   if ((r = upload(c, c->d_rb_right, rbr.data(), rbr.size(), s))) return r;
   if ((r = upload(c, c->d_rg_off, rgo.data(), rgo.size(), s))) return r;
@@ -778,7 +802,7 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     c->grid_cells.release();
     c->rpos_s.release(); c->rab_s.release(); c->rres_s.release(); c->d_cells.release();
     c->d_ligs.release(); c->d_latoms.release(); c->d_lig_xyz.release();
-    c->d_pair_ij.release(); c->d_pair_par.release(); c->d_sweep.release(); c->d_clash.release();
+    c->d_pair_ij.release(); c->d_pair_par.release(); c->d_intra_bits.release(); c->d_bit_base.release(); c->d_sweep.release(); c->d_clash.release();
     c->d_rb_left.release(); c->d_rb_right.release(); c->d_rg_off.release(); c->d_rg_atoms.release();
     c->s_xyz.release(); c->s_e.release(); c->s_g.release(); c->s_part.release();
     c->s_lig.release(); c->s_latom.release(); c->s_pij.release(); c->s_ppar.release();
@@ -1206,6 +1230,47 @@ int mmo_ene_intra_grad(mmo_ctx* c, const double* xs, const double* ys, const dou
 }
 
 // ------------------------------------------------------------------ ligand registry
+// Torsions whose derivatives can all be taken in the final conformer: dE/dtau_k is then the
+// torque of group k about its axis where both have come to lie.  It holds if each later
+// torsion k' either leaves group and axis k alone, carries both, or turns a part of group k
+// about an axis that turns with it (then it commutes with the rotation k):
+//   groups and ends disjoint but for common ends;
+//   group k within group k', axis k within group k' and the ends of k' (which stay);
+//   group k' within group k, axis k' within group k and the ends of k.
+// Rotation groups that are each one side of their bond, all seen from one end of the
+// molecule, are of this kind; groups facing each other are not.
+static bool torsions_free(const LigHost& h) {
+  const int R = (int)h.rb_left.size();
+  if (h.n > kMaxFreeAtoms || (size_t)R * (h.rg_atoms.size() + R + h.n) > kMaxFreeWork) return false;
+  std::vector<char> in(h.n);
+  for (int k = 0; k < R; ++k) {
+    std::fill(in.begin(), in.end(), 0);
+    for (int m = h.rg_off[k]; m < h.rg_off[k + 1]; ++m) {
+      if (in[h.rg_atoms[m]]) return false;   // an atom listed twice
+      in[h.rg_atoms[m]] = 1;
+    }
+    const int size = h.rg_off[k + 1] - h.rg_off[k];
+    const int l = h.rb_left[k], r = h.rb_right[k];
+    for (int q = k + 1; q < R; ++q) {
+      const int lq = h.rb_left[q], rq = h.rb_right[q];
+      int shared = 0;
+      bool has_l = false, has_r = false;   // ends of k in group q
+      for (int m = h.rg_off[q]; m < h.rg_off[q + 1]; ++m) {
+        shared += in[h.rg_atoms[m]];
+        has_l |= h.rg_atoms[m] == l;
+        has_r |= h.rg_atoms[m] == r;
+      }
+      const bool apart = shared == 0 && !in[lq] && !in[rq] && !has_l && !has_r;
+      const bool carried = shared == size && (has_l || l == lq || l == rq) &&
+                           (has_r || r == lq || r == rq);
+      const bool within = shared == h.rg_off[q + 1] - h.rg_off[q] && !has_l && !has_r &&
+                          (in[lq] || lq == l || lq == r) && (in[rq] || rq == l || rq == r);
+      if (!apart && !carried && !within) return false;
+    }
+  }
+  return true;
+}
+
 int mmo_ligand_add(mmo_ctx* c, const double* xs, const double* ys, const double* zs,
                    const double* q, const int32_t* anum, const int32_t* dists, int n,
                    const int32_t* rb_left, const int32_t* rb_right, const int32_t* rg_off,
@@ -1255,6 +1320,7 @@ int mmo_ligand_add(mmo_ctx* c, const double* xs, const double* ys, const double*
   } else {
     h.rg_off.assign(1, 0);
   }
+  h.free = torsions_free(h);
   c->ligs.push_back(std::move(h));
   c->lig_dirty = true;
   *lig_id = (int)c->ligs.size() - 1;
@@ -1317,6 +1383,7 @@ int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch**
     }
     b->max_atoms = std::max(b->max_atoms, c->ligs[l].n);
     b->max_rb = std::max(b->max_rb, (int)c->ligs[l].rb_left.size());
+    b->free &= c->ligs[l].free;
     b->max_rg = std::max(b->max_rg, c->ligs[l].rg_off.back());
   }
   b->atom_off[npose] = (int)na;
@@ -1578,6 +1645,7 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
                 "ligands too large for the DOF kernels: %zu bytes of LDS per pose (limit %zu)",
                 dof_lds_bytes(a, g), kMaxLds);
   HIPCHK(c, launch_apply_config(a, s));
+  a.free_torsions = g && b->free;   // after the limit, which is the general adjoint's
   const int score_flags = flags & ~MMO_F_COMPONENTS;
   if (score_flags & ~MMO_F_GRAD) {
     if (!e_out) return fail(c, MMO_ERR_BAD_ARG, "NULL energy buffer");
@@ -1594,6 +1662,9 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
         ai.e_stride = 4;
         ai.pair_ij = c->d_pair_ij.p;
         ai.pair_par = c->d_pair_par.p;
+        ai.latoms = c->d_latoms.p;
+        ai.intra_bits = c->d_intra_bits.p;
+        ai.bit_base = c->d_bit_base.p;
         if (dof_lds_bytes(ai, true) <= kMaxLds) {
           a = ai;
           bflags &= ~MMO_F_INTRA;

@@ -132,6 +132,11 @@ struct DofArgs {
   int e_stride;
   const uint32_t* pair_ij;
   const double4* pair_par;      // ke qi qj, Ai Aj, 2 Bi Bj
+  // every ligand's torsions are free (LigHost): the adjoint then needs no serial pass
+  int free_torsions;
+  const LigAtom* latoms;
+  const uint64_t* intra_bits;   // per ligand at bit_base: each atom's pairs (intra_ring)
+  const int64_t* bit_base;
   // nullable: the adjoint also sums the poses' units (launch_pose_sum's GRAD form) into
   // e_sum[4 * pose] and clears the rest of the row (E_intra only with clear_intra)
   const double* part;

@@ -1,6 +1,7 @@
 // pose_kernels.hip -- DOFs -> coordinates (Optim.apply_config, src/optim.ml:64-80) and
 // its adjoint (dE/dxyz -> dE/dDOF), one workgroup per pose (one wavefront; kDofWaves
-// when the adjoint also evaluates E_intra), FP64 throughout.
+// when the adjoint also evaluates E_intra; kFreeThreads threads where the torsions need no
+// serial pass), FP64 throughout.
 //
 // Forward: the registered centred conformer c0; for k = 0..R-1 the atoms of rotation
 // group k turn by tau_k about the axis right_k - left_k through right_k
@@ -26,6 +27,8 @@ namespace mmo {
 
 // wavefronts per pose of the adjoint when it also evaluates E_intra
 constexpr int kDofWaves = 2;
+// threads per pose of the adjoint without a serial torsion pass
+constexpr int kFreeThreads = 256;
 
 // LDS of the DOF kernels: `arrays` FP64 coordinate arrays of max_atoms entries, then the
 // staged torsion tree (TorsionLds)
@@ -332,7 +335,160 @@ __global__ void __launch_bounds__(INTRA ? kDofWaves * kWave : kWave) k_dof_grad(
   }
 }
 
+// E_intra (src/mol.ml:881-903, topo distance >= 3) of the conformer in LDS, FP64, with its
+// gradient.  Thread = (atom i, slice), over the pairs (i, i + d mod L), d = 1 + slice,
+// 1 + slice + slices, ..., L / 2: every pair once, atom i's side in registers, the other
+// side added to this wavefront's LDS copy g (3 rows of L) at lanes' distinct addresses but
+// where a wavefront holds two slices.
+// s: x, y, z, ke q, A, B of the L atoms (rows of L); bits: per atom i, bit d set if the pair
+// counts (words of 64).  Returns the thread's energy.
+__device__ double intra_ring(const double* s, const uint64_t* bits, int L, double* g) {
+  const int S = L >= kFreeThreads ? 1 : kFreeThreads / L, words = L / 128 + 1;
+  const int slice = S > 1 ? (int)threadIdx.x / L : 0;
+  double e = 0.0;
+  for (int i = (int)threadIdx.x - slice * L; i < L && slice < S; i += S > 1 ? L : kFreeThreads) {
+    const double x = s[i], y = s[L + i], z = s[2 * L + i];
+    const double q = s[3 * L + i], A = s[4 * L + i], B2 = 2.0 * s[5 * L + i];
+    double gx = 0.0, gy = 0.0, gz = 0.0;
+    int d = 1 + slice;
+    for (int w = 0; w < words; ++w) {
+      const uint64_t mine = bits[(size_t)i * words + w];
+      for (const int d1 = min(L / 2 + 1, 64 * (w + 1)); d < d1; d += S) {
+        if (!((mine >> (d & 63)) & 1ull)) continue;
+        const int j = i + d < L ? i + d : i + d - L;
+        const double dx = x - s[j], dy = y - s[L + j], dz = z - s[2 * L + j];
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const bool apart = r2 >= 1.0e-4;              // r >= 0.01 (Math.non_zero_dist)
+        const double irr = rsqrt(fmax(r2, 1.0e-4));   // no branch around the refinement
+        const double ir = apart ? irr : 100.0;        // 1 / max(r, 0.01)
+        const double u = ir * ir;
+        const double u3 = u * u * u;
+        // ke qi qj / r, Ai Aj u^6, 2 Bi Bj u^3
+        const double eq = (q * s[3 * L + j]) * (1.0 / kElecWeight) * ir,
+                     e12 = (A * s[4 * L + j]) * (u3 * u3), e6 = (B2 * s[5 * L + j]) * u3;
+        e += eq + e12 - e6;
+        // dE/dr / r = -(ke qq / r^3) - 12 AA u^7 + 6 BB2 u^4
+        const double c = apart ? u * fma(6.0, e6, fma(-12.0, e12, -eq)) : 0.0;
+        const double fx = c * dx, fy = c * dy, fz = c * dz;
+        gx += fx; gy += fy; gz += fz;
+        atomicAdd(&g[j], -fx); atomicAdd(&g[L + j], -fy); atomicAdd(&g[2 * L + j], -fz);
+      }
+    }
+    atomicAdd(&g[i], gx); atomicAdd(&g[L + i], gy); atomicAdd(&g[2 * L + i], gz);
+  }
+  return e;
+}
+
+// The adjoint when every torsion is free (torsions_free, api.hip): dE/dtau_k is the torque
+// of group k about its axis in the final conformer, so the torsions need neither an order
+// nor the earlier conformers and are shared by the wavefronts (the last one takes the
+// rigid-body sums).  The general kernel, bound by its
+// serial chain of 7 FP64 wave sums a torsion, takes 26 us for 16 poses and 81 us for 4,096
+// poses of 26 to 94 atoms; this one 8 and 55 us.  E_intra bounds it now (all pairs in FP64,
+// and three LDS additions each): every pair from either side without LDS additions was 78
+// us, 128 threads a pose 75 us.
+template <bool INTRA>
+__global__ void __launch_bounds__(kFreeThreads) k_dof_grad_free(DofArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  __shared__ double s_part[kFreeThreads / kWave];
+  __shared__ double s_sn[3], s_cs[3];
+  const int pose = blockIdx.x;
+  if (pose >= a.npose) return;
+  const int lig = a.pose_lig[pose];
+  const LigInfo li = a.ligs[lig];
+  const int L = li.n_atoms, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  double* sx = reinterpret_cast<double*>(smem);
+  double* sy = sx + L;
+  double* sz = sy + L;
+  double* hx = sz + L;   // INTRA: first the atoms' ke q, A, B
+  double* hy = hx + L;
+  double* hz = hy + L;
+  double* gi = hz + L;   // INTRA: intra_ring's copies
+  const int base = a.atom_off[pose];
+  double* gd = a.gdof + a.dof_off[pose];
+  for (int j = tid; j < L; j += kFreeThreads) {
+    const double* c = a.conf + 3 * (size_t)(base + j);   // after the torsions
+    sx[j] = c[0]; sy[j] = c[1]; sz[j] = c[2];
+    if (INTRA) {
+      const LigAtom la = a.latoms[li.atom_base + j];
+      hx[j] = la.keq; hy[j] = la.a; hz[j] = la.b;
+    }
+  }
+  if (INTRA)
+    for (int j = tid; j < 3 * L * (kFreeThreads / kWave); j += kFreeThreads) gi[j] = 0.0;
+  if (tid < 3) sincos(a.dofs[a.dof_off[pose] + 3 + tid], &s_sn[tid], &s_cs[tid]);
+  if (a.part && wave == kFreeThreads / kWave - 1) {
+    const double e = wave_sum_range(a.part, a.unit_off[pose], a.unit_off[pose + 1], 1);
+    if (lane < 4 && (lane != 1 || a.clear_intra)) a.e_sum[4 * (size_t)pose + lane] = lane == 0 ? e : 0.0;
+  }
+  __syncthreads();
+  if (INTRA) {
+    const double e = wave_sum(intra_ring(sx, a.intra_bits + a.bit_base[lig], L, gi + 3 * L * wave));
+    if (lane == 0) s_part[wave] = e;
+    __syncthreads();
+    if (tid == 0) {
+      double sum = 0.0;
+      for (int w = 0; w < kFreeThreads / kWave; ++w) sum += s_part[w];
+      a.e_intra[(size_t)pose * a.e_stride] = sum;
+    }
+  }
+  double M[9], dA[9], dB[9], dG[9];
+  rot_xyz(s_sn, s_cs, M, dA, dB, dG);
+  for (int j = tid; j < L; j += kFreeThreads) {
+    const double* g = a.grad_xyz + 3 * (size_t)(base + j);
+    double h0 = M[0] * g[0] + M[3] * g[1] + M[6] * g[2];   // M^T g
+    double h1 = M[1] * g[0] + M[4] * g[1] + M[7] * g[2];
+    double h2 = M[2] * g[0] + M[5] * g[1] + M[8] * g[2];
+    if (INTRA) {
+      const double* p = gi + j;
+      for (int w = 0; w < kFreeThreads / kWave; ++w, p += 3 * L) { h0 += p[0]; h1 += p[L]; h2 += p[2 * L]; }
+    }
+    hx[j] = h0; hy[j] = h1; hz[j] = h2;
+  }
+  __syncthreads();
+  constexpr int kTorsionWaves = kFreeThreads / kWave - 1;
+  if (wave == kTorsionWaves) {   // the last wavefront: the six rigid-body sums
+    double tx = 0.0, ty = 0.0, tz = 0.0, S[9];
+    for (int q = 0; q < 9; ++q) S[q] = 0.0;
+    for (int j = lane; j < L; j += kWave) {
+      const double* g = a.grad_xyz + 3 * (size_t)(base + j);
+      const double g0 = g[0], g1 = g[1], g2 = g[2];
+      tx += g0; ty += g1; tz += g2;
+      const double c[3] = {sx[j], sy[j], sz[j]};
+      for (int r = 0; r < 3; ++r)
+        for (int cc = 0; cc < 3; ++cc) S[3 * r + cc] += (r == 0 ? g0 : r == 1 ? g1 : g2) * c[cc];
+    }
+    double ga = 0.0, gb = 0.0, gg = 0.0;   // the matrices do not depend on the lane
+    for (int q = 0; q < 9; ++q) { ga += dA[q] * S[q]; gb += dB[q] * S[q]; gg += dG[q] * S[q]; }
+    tx = wave_sum(tx); ty = wave_sum(ty); tz = wave_sum(tz);
+    ga = wave_sum(ga); gb = wave_sum(gb); gg = wave_sum(gg);
+    if (lane == 0) { gd[0] = tx; gd[1] = ty; gd[2] = tz; gd[3] = ga; gd[4] = gb; gd[5] = gg; }
+    return;
+  }
+  for (int k = wave; k < li.nrb; k += kTorsionWaves) {
+    const int left = a.rb_left[li.rb_base + k], right = a.rb_right[li.rb_base + k];
+    const int g0 = a.rg_off[li.rg_base + k], g1 = a.rg_off[li.rg_base + k + 1];
+    const double px = sx[right], py = sy[right], pz = sz[right];
+    const double vx = px - sx[left], vy = py - sy[left], vz = pz - sz[left];
+    double tqx = 0.0, tqy = 0.0, tqz = 0.0;   // sum of (x - p) x h
+    for (int m = g0 + lane; m < g1; m += kWave) {
+      const int i = a.rg_atoms[m];
+      const double yx = sx[i] - px, yy = sy[i] - py, yz = sz[i] - pz;
+      const double h0 = hx[i], h1 = hy[i], h2 = hz[i];
+      tqx += yy * h2 - yz * h1; tqy += yz * h0 - yx * h2; tqz += yx * h1 - yy * h0;
+    }
+    const double tb = wave_sum((vx * tqx + vy * tqy + vz * tqz) * rsqrt(vx * vx + vy * vy + vz * vz));
+    if (lane == 0) gd[6 + k] = tb;
+  }
+}
+
+// LDS of k_dof_grad_free: coordinates and adjoint; with E_intra a copy per wavefront, too
+static size_t dof_free_lds_bytes(const DofArgs& a) {
+  return dof_coord_bytes(a.max_atoms, a.e_intra ? 6 + 3 * (kFreeThreads / kWave) : 6);
+}
+
 size_t dof_lds_bytes(const DofArgs& a, bool grad) {
+  if (grad && a.free_torsions) return dof_free_lds_bytes(a);
   const int arrays = grad ? (a.e_intra ? 6 + 3 * kDofWaves : 6) : 3;
   return dof_coord_bytes(a.max_atoms, arrays) + torsion_lds_bytes(a.max_rb, a.max_rg);
 }
@@ -360,7 +516,15 @@ hipError_t launch_dof_grad(const DofArgs& a, hipStream_t s) {
   if (a.npose == 0) return hipSuccess;
   const size_t lds = dof_lds_bytes(a, true);
   if (lds > kMaxLds) return hipErrorInvalidConfiguration;
-  if (a.e_intra) {
+  if (a.free_torsions && a.e_intra) {
+    hipError_t e = lds_limit(&k_dof_grad_free<true>, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_dof_grad_free<true>, dim3(a.npose), dim3(kFreeThreads), lds, s, a);
+  } else if (a.free_torsions) {
+    hipError_t e = lds_limit(&k_dof_grad_free<false>, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_dof_grad_free<false>, dim3(a.npose), dim3(kFreeThreads), lds, s, a);
+  } else if (a.e_intra) {
     hipError_t e = lds_limit(&k_dof_grad<true>, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_dof_grad<true>, dim3(a.npose), dim3(kDofWaves * kWave), lds, s, a);

@@ -204,3 +204,73 @@ def test_pose_units(sys0, atoms, n):
     torch.cuda.synchronize()
     assert torch.equal(e1[0], ed[-1]) and torch.equal(g1, gd[-nd:])
     assert torch.all(ed[:, 1:] == 0)   # no E_intra asked for, no parts with the gradient
+
+
+def _chain(n, nrb, kind, rng):
+    """A zigzag of n atoms with nrb torsions: groups that are the far side of each bond
+    ("nested"), both sides in turn ("facing"), two arms turned outwards ("arms"), or any
+    atoms at all ("any")."""
+    i = np.arange(n)
+    x = np.stack([1.25 * (i - (n - 1) / 2), 0.8 * (i % 2) + 0.3 * (i % 5), 0.5 * (i % 3)], 1)
+    left, right, groups = [], [], []
+    for k in np.sort(rng.choice(n - 1, min(nrb, n - 1), replace=False)) if n > 2 else []:
+        far, near = i[k + 2:], i[:k]
+        back = {"nested": False, "facing": len(left) % 2 == 1, "arms": k < n // 2, "any": False}[kind]
+        left.append(k + 1 if back else k)
+        right.append(k if back else k + 1)
+        groups.append(near if back else far)
+        if kind == "any":
+            rest = np.setdiff1d(i, [k, k + 1])
+            groups[-1] = np.sort(rng.choice(rest, rng.integers(0, len(rest) + 1), replace=False))
+    if kind == "arms":   # outermost last within either arm: parents before children
+        order = np.argsort([-r if l > r else r for l, r in zip(left, right)], kind="stable")
+        left, right, groups = ([v[o] for o in order] for v in (left, right, groups))
+    off = np.concatenate([[0], np.cumsum([len(g) for g in groups])]).astype(np.int32)
+    c = x - x.mean(0)
+    return {"xs": c[:, 0].copy(), "ys": c[:, 1].copy(), "zs": c[:, 2].copy(),
+            "q": rng.uniform(-0.4, 0.4, n), "anum": rng.choice([6, 7, 8, 1], n).astype(np.int32),
+            "dists": np.abs(i[:, None] - i[None, :]).astype(np.int32),
+            "rb_left": np.array(left, np.int32), "rb_right": np.array(right, np.int32), "rg_off": off,
+            "rg_atoms": np.concatenate([np.zeros(0, int)] + groups).astype(np.int32)}
+
+
+@pytest.mark.parametrize("kind", ["nested", "arms", "facing", "any"])
+@pytest.mark.parametrize("n", [1, 2, 5, 64, 65, 128, 131, 257, 1024, 1025])
+def test_dof_gradient_of_all_torsion_forms(sys0, n, kind):
+    """The DOF gradient, with and without E_intra, for torsions whose derivatives can and
+    cannot be taken in the final conformer, at the edges of the pair ring (odd and even atom
+    counts, one and several atoms a thread, words of 64 pairs, the largest ligand): against
+    the oracle's FP64 Jacobian applied to the coordinate gradient.
+    Tolerance: coordinates agree to 1e-13 A of each other, forces of pairs beyond 0.5 A
+    therefore to 14 x 1e-13 / 0.5 = 3e-12 of themselves; a few hundred partners: 1e-9."""
+    import torch
+    ctx, _, _ = sys0
+    rng = np.random.default_rng(n)
+    dev = torch.device("cuda:0")
+    for nrb in (0, 3, 9) if n <= 257 else (3,):
+        lig = _chain(n, nrb, kind, rng)
+        lid = ctx.add_ligand(lig)
+        b = ctx.batch(np.full(3, lid))
+        nrb = len(lig["rb_left"])
+        d = np.concatenate([rng.uniform(-3, 3, (3, 3)), rng.uniform(-3, 3, (3, 3)),
+                            rng.uniform(-0.3, 0.3, (3, nrb))], 1)
+        for flags in (ff.F_INTER_SHIFTED | ff.F_INTRA, ff.F_INTER_SHIFTED):
+            e = torch.empty((3, 4), dtype=torch.float64, device=dev)
+            x = torch.empty((b.natoms, 3), dtype=torch.float64, device=dev)
+            g = torch.empty(d.size, dtype=torch.float64, device=dev)
+            b.score_dofs_dev(torch.tensor(d.ravel(), device=dev), e, xyz_out=x, gdof=g,
+                             flags=flags | ff.F_GRAD)
+            torch.cuda.synchronize()
+            x, g, e = x.cpu().numpy(), g.cpu().numpy().reshape(3, -1), e.cpu().numpy()
+            _, gx = b.score(x, ff.F_INTER_SHIFTED | ff.F_GRAD)
+            for p in range(3):
+                xp, h = x[p * n:(p + 1) * n], gx[p * n:(p + 1) * n].copy()
+                posed = dict(lig, xs=xp[:, 0].copy(), ys=xp[:, 1].copy(), zs=xp[:, 2].copy())
+                if flags & ff.F_INTRA:
+                    want, gi = oracle.grad_intra(posed)
+                    h += gi
+                    assert e[p, 1] == pytest.approx(want, rel=1e-9, abs=1e-9)
+                J = oracle.apply_config_jvp(_rows(lig), lig["rb_left"], lig["rb_right"], lig["rg_off"],
+                                            lig["rg_atoms"], d[p])[2]
+                scale = np.abs(J).sum(axis=(1, 2)) * np.abs(h).max()
+                np.testing.assert_array_less(np.abs(g[p] - (J * h).sum(axis=(1, 2))), 1e-9 * scale + 1e-12)
