@@ -141,6 +141,7 @@ struct mmo_ctx {
   int mc_wg_waves = 16;       // Monte Carlo chains (wavefronts) per workgroup
   int min_fused = 1;          // minimiser: all iterations in one persistent launch
   int min_f64 = 0;            // fused minimiser: FP64 pair arithmetic (parity mode)
+  int min_pooled = 8;         // fused minimiser: poses per CU up to which workgroups pool their sweeps
   int min_waves = 16;         // fused minimiser: wavefronts per workgroup
   int min_rec_lds = 1;        // fused minimiser: receptor in LDS when >= 8 wavefronts fit
   int mc_rec_lds = 1;         // Monte Carlo direct form: receptor in LDS when it fits
@@ -2627,7 +2628,22 @@ struct mmo_min {
   DevBuf<double> x, g, d, xt, gt, e, rad, S, Y, rho, lo, hi;
   DevBuf<MinPose> st;
   DevBuf<int> queue;
+  DevBuf<float4> fe;   // pooled form: its sweep units' energies
 };
+
+// Poses a workgroup of the pooled minimiser keeps (0: this batch takes another form).  One
+// workgroup per CU; up to 6 poses each all run at once, up to 8 half of them at a time (2,000
+// poses: 4 slots 17.0 ms, 8 slots 22.0, one wavefront per pose 22.0; 1,500: 6 slots 13.4, 3
+// slots 14.9; 3,000: 4 slots 24.2, one wavefront per pose 22.7).  Their units' energies (1 KiB
+// per 4 atoms) stay within a bound.
+constexpr size_t kMinPooledBytes = 64u << 20;
+static int min_slots(const mmo_ctx* c, const mmo_batch* b) {
+  const int per_cu = (b->npose + c->ncu - 1) / c->ncu;
+  if (per_cu > c->min_pooled) return 0;
+  const int slots = per_cu <= 6 ? per_cu : (per_cu + 1) / 2;
+  const size_t bytes = (size_t)slots * c->ncu * min_units(b->max_atoms) * kWave * sizeof(float4);
+  return slots <= kMinSlots && bytes <= kMinPooledBytes ? slots : 0;
+}
 
 int mmo_min_create(mmo_batch* b, int history, int flags, const double* lo, const double* hi,
                    double max_step, double gtol, mmo_min** out) {
@@ -2663,6 +2679,10 @@ int mmo_min_create(mmo_batch* b, int history, int flags, const double* lo, const
   if (e == hipSuccess) e = z->rho.ensure((size_t)history * np);
   if (e == hipSuccess) e = z->st.ensure(np);
   if (e == hipSuccess) e = z->queue.ensure(1);
+  // without this buffer the minimiser takes another form
+  const size_t unit_fe = (size_t)min_units(b->max_atoms) * kWave;
+  if (e == hipSuccess && inter == MMO_F_INTER_SHIFTED && min_slots(c, b) > 0)
+    if (z->fe.ensure((size_t)min_slots(c, b) * c->ncu * unit_fe) != hipSuccess) (void)hipGetLastError();
   if (e == hipSuccess && b->d_by_size.n < (size_t)b->npose)
     e = b->d_by_size.ensure(b->npose) == hipSuccess
             ? hipMemcpyAsync(b->d_by_size.p, b->by_size.data(), b->npose * sizeof(int),
@@ -2713,7 +2733,7 @@ int mmo_min_run_dev(mmo_min* z, double* dofs, int iters, double* e_out, void* st
     p.atom_order = c->d_sweep.p; p.rb_left = c->d_rb_left.p; p.rb_right = c->d_rb_right.p;
     p.rg_off = c->d_rg_off.p; p.rg_atoms = c->d_rg_atoms.p; p.pair_ij = c->d_pair_ij.p;
     p.pair_par = c->d_pair_par.p;
-    p.npose = b->npose; p.max_atoms = b->max_atoms; p.ndof_total = b->ndof; p.iters = iters;
+    p.npose = b->npose; p.max_atoms = b->max_atoms; p.max_rb = b->max_rb; p.max_rg = b->max_rg; p.ndof_total = b->ndof; p.iters = iters;
     p.m = z->m; p.pose_lig = b->d_pose_lig.p; p.dof_off = b->d_dof_off.p; p.order = b->d_by_size.p;
     p.x = dofs; p.lo = z->lo.p; p.hi = z->hi.p; p.S = z->S.p; p.Y = z->Y.p; p.rho = z->rho.p;
     p.st = z->st.p; p.e_out = e_out; p.queue = z->queue.p; p.intra = (z->flags & MMO_F_INTRA) != 0;
@@ -2741,6 +2761,15 @@ int mmo_min_run_dev(mmo_min* z, double* dofs, int iters, double* e_out, void* st
     const int blocks = std::max(1, std::min((b->npose + waves - 1) / waves, ncu * std::max(1, 16 / waves)));
     HIPCHK(c, launch_fill_int(z->queue.p, 1, 0, s));
     timer_begin(c, "min", s);
+    p.slots = min_slots(c, b);
+    p.fe = z->fe.p;
+    if (rec_lds && kind == kDofInterAtom && p.slots > 0 && z->fe.n > 0 &&
+        min_pooled_lds_bytes(p) <= kMaxLds - 128) {
+      const int nb = std::min(c->ncu, (b->npose + p.slots - 1) / p.slots);   // at most one per CU
+      HIPCHK(c, launch_min_pooled(p, nb, s));
+      timer_end(c, "min", s);
+      return MMO_OK;
+    }
     HIPCHK(c, launch_min_persist(p, kind, blocks, waves, rec_lds, s));
     timer_end(c, "min", s);
     return MMO_OK;
@@ -2794,7 +2823,7 @@ void mmo_min_destroy(mmo_min* z) {
                               &z->rho, &z->lo, &z->hi})
       v->release();
     z->st.release();
-    z->queue.release();
+    z->queue.release(); z->fe.release();
   }
   delete z;
 }
@@ -2848,6 +2877,7 @@ int mmo_tune_set(mmo_ctx* c, const char* key, double v) {
   else if (k == "cell_xsub" && iv >= 1 && iv <= 16) c->cell_xsub = iv;
   else if (k == "min_fused" && (iv == 0 || iv == 1)) c->min_fused = iv;
   else if (k == "min_f64" && (iv == 0 || iv == 1)) c->min_f64 = iv;
+  else if (k == "min_pooled" && iv >= 0 && iv <= 2 * kMinSlots) c->min_pooled = iv;
   else if (k == "min_waves" && iv >= 1 && iv <= 16) c->min_waves = iv;
   else if (k == "min_rec_lds" && (iv == 0 || iv == 1)) c->min_rec_lds = iv;
   else if (k == "mc_rec_lds" && (iv == 0 || iv == 1)) c->mc_rec_lds = iv;
@@ -2884,6 +2914,7 @@ double mmo_tune_get(mmo_ctx* c, const char* key) {
   if (k == "cell_xsub") return c->cell_xsub;
   if (k == "min_fused") return c->min_fused;
   if (k == "min_f64") return c->min_f64;
+  if (k == "min_pooled") return c->min_pooled;
   if (k == "min_waves") return c->min_waves;
   if (k == "min_rec_lds") return c->min_rec_lds;
   if (k == "mc_rec_lds") return c->mc_rec_lds;

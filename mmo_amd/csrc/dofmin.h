@@ -371,70 +371,15 @@ __device__ __forceinline__ double dof_pose(const DofEval& ev, const double* base
   return rad;
 }
 
-// E and dE/dDOF (lane i) of DOF vector x for one wavefront.  tx.. (LDS, 3 x max_atoms)
-// hold the conformer during the evaluation (the reverse pass returns them to the base
-// rows' values), hx.. (LDS) serve as the adjoint.  e_inter / e_intra receive the two
-// parts.  Returns E (+inf for a pose longer than 12 A after its torsions, NaN for an
-// interpolated pose outside the grid).
-template <int INTER>
-__device__ double dof_eval(const DofEval& ev, const double* base, double x, double* tx, double* ty,
-                           double* tz, double* hx, double* hy, double* hz, double& gdof,
-                           double& e_inter, double& e_intra, double& rad) {
+// The rest of an evaluation once h (LDS) holds dE_inter/dx: the rigid-body sums, E_intra (if
+// asked for, returned) and the reverse torsion pass; gdof (lane i) = dE/dDOF i.
+__device__ __forceinline__ double dof_adjoint(const DofEval& ev, const double* M, double sn, double cs,
+                                              double* tx, double* ty, double* tz, double* hx,
+                                              double* hy, double* hz, double& gdof) {
   const int lane = threadIdx.x & (kWave - 1);
   const LigInfo& li = ev.li;
   const int L = li.n_atoms;
-  double M[9], T[3], sn, cs;
-  rad = dof_pose(ev, base, x, tx, ty, tz, M, nullptr, nullptr, nullptr, T, sn, cs);
-  gdof = 0.0;
-  e_inter = e_intra = 0.0;
-  if (!(rad <= 12.0)) return __builtin_inf();   // Mol.Too_long (src/optim.ml:72-75)
-  auto posed = [&](int j, double& x0, double& y0, double& z0) {
-    const double a = tx[j], b = ty[j], c = tz[j];
-    x0 = (M[0] * a + M[1] * b + M[2] * c) + T[0];
-    y0 = (M[3] * a + M[4] * b + M[5] * c) + T[1];
-    z0 = (M[6] * a + M[7] * b + M[8] * c) + T[2];
-  };
-  // E_inter and dE/dx in the pose frame, into h
-  if (INTER == kDofInterAtom) {
-    int sat = 0;
-    auto at = [&](int j) { return ev.atom_order ? ev.atom_order[li.atom_base + j] : j; };
-    auto atom = [&](int j, LigPt& l, double& cq, double& ca, double& cb) {
-      const int ja = at(j);
-      double px, py, pz;
-      posed(ja, px, py, pz);
-      l = lig_pt(px, py, pz, ev.fr, &sat);
-      const LigAtom la = ev.latoms[li.atom_base + ja];
-      cq = la.keq; ca = la.a; cb = la.b;
-    };
-    auto gout = [&](int j, double gx, double gy, double gz) {
-      const int ja = at(j);
-      hx[ja] = gx; hy[ja] = gy; hz[ja] = gz;
-    };
-    double e_el = 0.0, e_vd = 0.0;
-    atom_sweep<true, decltype(atom)&, decltype(gout)&, true, true, 4>(
-        ev.cg, ev.s_cell, ev.s_pos, ev.s_ab, ev.rres, ev.fr, L, ev.wl, atom, gout, e_el, e_vd);
-    (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
-    e_inter = wave_sum(e_el + e_vd);
-  } else if (INTER == kDofInterF64) {
-    auto gout = [&](int j, double gx, double gy, double gz) { hx[j] = gx; hy[j] = gy; hz[j] = gz; };
-    e_inter = f64_sweep_grad(ev, L, posed, gout);
-  } else {
-    double e = 0.0;
-    int bad = 0;
-    for (int j = lane; j < L; j += kWave) {
-      double px, py, pz;
-      posed(j, px, py, pz);
-      bool ok = true;
-      double dg[3] = {0.0, 0.0, 0.0};
-      e += trilin<true>(ev.g, ev.latoms[li.atom_base + j].type, px - ev.g.ox, py - ev.g.oy,
-                        pz - ev.g.oz, ok, dg);
-      if (!ok) bad = 1;
-      hx[j] = dg[0]; hy[j] = dg[1]; hz[j] = dg[2];
-    }
-    e_inter = wave_sum(e);
-    if (__ballot(bad) != 0ull) e_inter = __builtin_nan("");
-  }
-  wave_lds_sync();
+  double e_intra = 0.0;
   // rigid-body part: dE/dt = sum g, dE/dangle = sum_q dM_q S_q with S = sum g c^T; then the
   // conformer-frame adjoint h = M^T g
   double tsx = 0.0, tsy = 0.0, tsz = 0.0, S[9];
@@ -517,7 +462,134 @@ __device__ double dof_eval(const DofEval& ev, const double* base, double x, doub
     }
     wave_lds_sync();
   }
+  return e_intra;
+}
+
+// E and dE/dDOF (lane i) of DOF vector x for one wavefront.  tx.. (LDS, 3 x max_atoms)
+// hold the conformer during the evaluation (the reverse pass returns them to the base
+// rows' values), hx.. (LDS) serve as the adjoint.  e_inter / e_intra receive the two
+// parts.  Returns E (+inf for a pose longer than 12 A after its torsions, NaN for an
+// interpolated pose outside the grid).
+template <int INTER>
+__device__ double dof_eval(const DofEval& ev, const double* base, double x, double* tx, double* ty,
+                           double* tz, double* hx, double* hy, double* hz, double& gdof,
+                           double& e_inter, double& e_intra, double& rad) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const LigInfo& li = ev.li;
+  const int L = li.n_atoms;
+  double M[9], T[3], sn, cs;
+  rad = dof_pose(ev, base, x, tx, ty, tz, M, nullptr, nullptr, nullptr, T, sn, cs);
+  gdof = 0.0;
+  e_inter = e_intra = 0.0;
+  if (!(rad <= 12.0)) return __builtin_inf();   // Mol.Too_long (src/optim.ml:72-75)
+  auto posed = [&](int j, double& x0, double& y0, double& z0) {
+    const double a = tx[j], b = ty[j], c = tz[j];
+    x0 = (M[0] * a + M[1] * b + M[2] * c) + T[0];
+    y0 = (M[3] * a + M[4] * b + M[5] * c) + T[1];
+    z0 = (M[6] * a + M[7] * b + M[8] * c) + T[2];
+  };
+  // E_inter and dE/dx in the pose frame, into h
+  if (INTER == kDofInterAtom) {
+    int sat = 0;
+    auto at = [&](int j) { return ev.atom_order ? ev.atom_order[li.atom_base + j] : j; };
+    auto atom = [&](int j, LigPt& l, double& cq, double& ca, double& cb) {
+      const int ja = at(j);
+      double px, py, pz;
+      posed(ja, px, py, pz);
+      l = lig_pt(px, py, pz, ev.fr, &sat);
+      const LigAtom la = ev.latoms[li.atom_base + ja];
+      cq = la.keq; ca = la.a; cb = la.b;
+    };
+    auto gout = [&](int j, double gx, double gy, double gz) {
+      const int ja = at(j);
+      hx[ja] = gx; hy[ja] = gy; hz[ja] = gz;
+    };
+    double e_el = 0.0, e_vd = 0.0;
+    atom_sweep<true, decltype(atom)&, decltype(gout)&, true, true, 4>(
+        ev.cg, ev.s_cell, ev.s_pos, ev.s_ab, ev.rres, ev.fr, L, ev.wl, atom, gout, e_el, e_vd);
+    (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
+    e_inter = wave_sum(e_el + e_vd);
+  } else if (INTER == kDofInterF64) {
+    auto gout = [&](int j, double gx, double gy, double gz) { hx[j] = gx; hy[j] = gy; hz[j] = gz; };
+    e_inter = f64_sweep_grad(ev, L, posed, gout);
+  } else {
+    double e = 0.0;
+    int bad = 0;
+    for (int j = lane; j < L; j += kWave) {
+      double px, py, pz;
+      posed(j, px, py, pz);
+      bool ok = true;
+      double dg[3] = {0.0, 0.0, 0.0};
+      e += trilin<true>(ev.g, ev.latoms[li.atom_base + j].type, px - ev.g.ox, py - ev.g.oy,
+                        pz - ev.g.oz, ok, dg);
+      if (!ok) bad = 1;
+      hx[j] = dg[0]; hy[j] = dg[1]; hz[j] = dg[2];
+    }
+    e_inter = wave_sum(e);
+    if (__ballot(bad) != 0ull) e_inter = __builtin_nan("");
+  }
+  wave_lds_sync();
+  e_intra = dof_adjoint(ev, M, sn, cs, tx, ty, tz, hx, hy, hz, gdof);
   return e_inter + e_intra;
+}
+
+// The unit of atoms 4 unit .. 4 unit + 3 (in the sweep's order) of a pose's FP32 gradient
+// sweep, as atom_sweep has it in dof_eval, for any wavefront: posed(j, x, y, z) gives atom j,
+// at[] its parameters (FP32) and index; dE/dx goes to h, the lanes' energies to fe_out[lane].
+template <class PosFn>
+__device__ __forceinline__ void dof_sweep_unit(const DofEval& ev, int n_atoms, int unit, PosFn&& posed,
+                                               const float4* at, double* hx, double* hy, double* hz,
+                                               float4* fe_out) {
+  constexpr int NA = 4;
+  const int lane = threadIdx.x & (kWave - 1);
+  const Frame& fr = ev.fr;
+  const PairK pk = pair_k(fr.inv_s2, fr.inv_s, ev.rres);
+  const int j0 = NA * unit;
+  const bool mine = lane < NA && j0 + lane < n_atoms;
+  LigPt l = lig_pt_zero();
+  float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  int ja = 0, sat = 0;
+  if (mine) {
+    c = at[j0 + lane];
+    ja = __float_as_int(c.w);
+    double px, py, pz;
+    posed(ja, px, py, pz);
+    l = lig_pt(px, py, pz, fr, &sat);
+  }
+  (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
+  LigPt lu[NA];
+  float c1[NA], fa[NA], fb[NA];
+  float sq[NA], s12[NA], s6[NA], fe[NA], fx[NA], fy[NA], fz[NA];
+#pragma unroll
+  for (int u = 0; u < NA; ++u) {
+    const int v = j0 + u < n_atoms ? u : 0;   // a short last unit repeats its first atom
+    lu[u].x = __builtin_amdgcn_readlane(l.x, v);
+    lu[u].y = __builtin_amdgcn_readlane(l.y, v);
+    lu[u].z = __builtin_amdgcn_readlane(l.z, v);
+    lu[u].rx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.rx), v));
+    lu[u].ry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.ry), v));
+    lu[u].rz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.rz), v));
+    c1[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.x), v));
+    fa[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.y), v));
+    fb[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.z), v));
+  }
+  sweep_pass<true, true, NA, false>(ev.cg, ev.s_cell, ev.s_pos, ev.s_ab, fr.inv_s, pk, ev.wl, lu, c1,
+                                    fa, fb, sq, s12, s6, fe, fx, fy, fz);
+  fe_out[lane] = make_float4(fe[0], fe[1], fe[2], fe[3]);
+  float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+#pragma unroll
+  for (int u = 0; u < NA; ++u) {
+    const float ux = wave_sum_f(fx[u]), uy = wave_sum_f(fy[u]), uz = wave_sum_f(fz[u]);
+    gx = lane == u ? ux : gx;
+    gy = lane == u ? uy : gy;
+    gz = lane == u ? uz : gz;
+  }
+  if (mine) {
+    const double gs = -2.0 * (double)fr.inv_s;
+    hx[ja] = gs * (double)gx;
+    hy[ja] = gs * (double)gy;
+    hz[ja] = gs * (double)gz;
+  }
 }
 
 }  // namespace mmo

@@ -337,7 +337,7 @@ struct MinPersistArgs {
   const int* rg_atoms;
   const uint32_t* pair_ij;
   const double4* pair_par;
-  int npose, max_atoms, ndof_total, iters, m;
+  int npose, max_atoms, max_rb, max_rg, ndof_total, iters, m;
   const int* pose_lig;
   const int* dof_off;
   const int* order;             // nullable: queue position -> pose (largest ligands first)
@@ -350,6 +350,8 @@ struct MinPersistArgs {
   MinPose* st;
   double* e_out;                // nullable: best energy per pose
   int* queue;
+  int slots;                    // pooled form: poses per workgroup and their units' energies,
+  float4* fe;                   // 64 per unit of 4 atoms, min_units(max_atoms) a slot
   int intra;
   double max_step, min_step, gtol, c1;
   Frame fr;
@@ -361,6 +363,12 @@ struct MinPersistArgs {
   GridDev g;
 };
 size_t min_persist_lds_bytes(const MinPersistArgs& a, int waves, bool rec_lds);
+// sweep units of a pose of n atoms (dof_sweep_unit)
+__host__ __device__ inline int min_units(int n) { return (n + 3) / 4; }
+// poses a workgroup of the pooled form may hold, and its LDS with `slots` of them
+constexpr int kMinSlots = 8;
+size_t min_pooled_lds_bytes(const MinPersistArgs& a);
+hipError_t launch_min_pooled(const MinPersistArgs& a, int nblocks, hipStream_t s);
 hipError_t launch_min_persist(const MinPersistArgs& a, int inter, int nblocks, int waves,
                               bool rec_lds, hipStream_t s);
 hipError_t launch_min_reset(MinPose* st, int npose, hipStream_t s);

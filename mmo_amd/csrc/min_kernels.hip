@@ -148,6 +148,212 @@ __global__ void __launch_bounds__(min_persist_waves(REC_LDS) * 64) k_min_persist
   }
 }
 
+// ------------------------------------------------------------------- pooled form
+// Few poses per CU leave k_min_persist waiting: a pose is one wavefront's chain of
+// evaluations (1,000 poses: 125 workgroups of 8, and 21 ms however many there are, the time
+// of the largest ligand).  Here a workgroup keeps `slots` poses, one wavefront each, and all
+// its wavefronts share the receptor sweeps of these poses, a unit of 4 atoms at a time, as
+// they become free; the units leave FP32 energies per lane in memory for the pose's
+// wavefront to add up in its atoms' order, so every sum has k_min_persist's bits.  Sweeps and
+// the rest alternate between workgroup barriers.
+// 100 iterations, ligands of 26 to 94 atoms, 3,000-atom receptor: 64 poses 16.3 -> 8.4 ms,
+// 500 21.4 -> 9.5, 1,000 21.4 -> 11.5, 1,500 22.3 -> 13.4, 2,000 22.0 -> 17.0 (4 slots, the
+// other half from the queue).  Of an evaluation's 260,000 cycles at 1,000 poses E_intra's
+// chain of FP64 LDS additions takes 95,000, the sweeps 94,000, the torsions and their adjoint
+// 43,000.  The additions as reads and writes of one diagonal at a time took 199,000.
+constexpr int kMinPooledWaves = 8;
+
+// per slot: the atoms' parameters and order, the conformer and the adjoint (FP64), the rigid
+// motion, the torsions (rg_off relative to the pose); then the wavefronts' sweep scratch
+__host__ __device__ inline size_t min_slot_lds_bytes(int max_atoms, int max_rb, int max_rg) {
+  return ((size_t)max_atoms * (6 * sizeof(double) + sizeof(float4)) + 12 * sizeof(double) +
+          (3 * (size_t)max_rb + 1 + max_rg) * sizeof(int) + 15) & ~(size_t)15;
+}
+
+__global__ void __launch_bounds__(kMinPooledWaves * 64) k_min_pooled(MinPersistArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  __shared__ int s_atoms[kMinSlots];   // atoms to sweep (0: none), kept until the next round
+  __shared__ int s_live[kMinSlots];    // the slot holds a pose
+  __shared__ int s_next;               // the next unit of this round
+  const RecPos* s_pos;
+  const RecAB* s_ab;
+  const int* s_cell;
+  load_receptor<true>(a.rpos, a.rab, a.nrec, a.cg, s_pos, s_ab, s_cell, smem);
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  char* slots = smem + receptor_lds_bytes<true>(a.nrec, a.cg);
+  const size_t slot_bytes = min_slot_lds_bytes(a.max_atoms, a.max_rb, a.max_rg);
+  const size_t units = min_units(a.max_atoms);
+  float4* fe = a.fe + (size_t)blockIdx.x * a.slots * units * kWave;
+  auto slot_at = [&](int s) { return reinterpret_cast<float4*>(slots + s * slot_bytes); };
+  auto slot_xyz = [&](int s) { return reinterpret_cast<double*>(slot_at(s) + a.max_atoms); };
+  auto slot_rt = [&](int s) { return slot_xyz(s) + 6 * (size_t)a.max_atoms; };
+  const MinCfg cfg{a.m, a.max_step, a.min_step, a.gtol, a.c1};
+  DofEval ev;
+  ev.latoms = a.latoms; ev.atom_order = a.atom_order;
+  ev.pair_ij = a.pair_ij; ev.pair_par = a.pair_par; ev.intra = a.intra != 0;
+  ev.fr = a.fr; ev.s_pos = s_pos; ev.s_ab = s_ab; ev.s_cell = s_cell; ev.rres = a.rres; ev.cg = a.cg;
+  ev.wl = reinterpret_cast<int*>(slots + a.slots * slot_bytes) + wv * kAtomSweepInts;
+  // wavefront w < slots keeps slot w's pose: its DOFs in the lanes, as in k_min_persist
+  const bool keeper = wv < a.slots;
+  float4* at = slot_at(keeper ? wv : 0);
+  double* tx = slot_xyz(keeper ? wv : 0);
+  double *ty = tx + a.max_atoms, *tz = ty + a.max_atoms;
+  double *hx = tz + a.max_atoms, *hy = hx + a.max_atoms, *hz = hy + a.max_atoms;
+  int* const rb_left = reinterpret_cast<int*>(slot_rt(keeper ? wv : 0) + 12);
+  int* const rb_right = rb_left + a.max_rb;
+  int* const rg_off = rb_right + a.max_rb;
+  int* const rg_atoms = rg_off + a.max_rb + 1;
+  ev.rb_left = rb_left; ev.rb_right = rb_right; ev.rg_off = rg_off; ev.rg_atoms = rg_atoms;
+  // a pose per slot dealt by size, to and fro over the workgroups; then from the queue
+  const int nb = gridDim.x, b = blockIdx.x;
+  int q = keeper ? wv * nb + ((wv & 1) ? nb - 1 - b : b) : a.npose;
+  bool live = false;
+  int p = 0, it = 0;
+  size_t i = 0;
+  bool act = false;
+  double lo = 0.0, hi = 0.0, xt = 0.0, x = 0.0, g = 0.0, d = 0.0;
+  const double* base = nullptr;
+  MinPose s{};
+  for (;;) {
+    double M[9], T[3], sn = 0.0, cs = 0.0, rad = 0.0;
+    if (keeper) {
+      if (!live && q < a.npose) {
+        live = true;
+        p = a.order ? a.order[q] : q;
+        ev.li = a.ligs[a.pose_lig[p]];
+        const int o = a.dof_off[p];
+        const int n = a.dof_off[p + 1] - o;
+        ev.ntors = n - 6;
+        act = lane < n;
+        i = (size_t)o + (act ? lane : 0);
+        base = a.lig_xyz + 3 * (size_t)ev.li.atom_base;
+        lo = (act && a.lo) ? a.lo[i] : -__builtin_inf();
+        hi = (act && a.hi) ? a.hi[i] : __builtin_inf();
+        s = MinPose{};
+        xt = act ? a.x[i] : 0.0;
+        x = g = d = 0.0;
+        it = 0;
+        for (int j = lane; j < ev.li.n_atoms; j += kWave) {
+          const int ja = a.atom_order ? a.atom_order[ev.li.atom_base + j] : j;
+          const LigAtom la = a.latoms[ev.li.atom_base + ja];
+          at[j] = make_float4((float)la.keq, (float)la.a, (float)la.b, __int_as_float(ja));
+        }
+        const int* off = a.rg_off + ev.li.rg_base;
+        const int g0 = off[0], ng = off[ev.ntors] - g0;
+        if (lane < ev.ntors) {
+          rb_left[lane] = a.rb_left[ev.li.rb_base + lane];
+          rb_right[lane] = a.rb_right[ev.li.rb_base + lane];
+        }
+        if (lane <= ev.ntors) rg_off[lane] = off[lane] - g0;
+        for (int m = lane; m < ng; m += kWave) rg_atoms[m] = a.rg_atoms[g0 + m];
+        ev.li.rb_base = ev.li.rg_base = 0;   // the staged torsions
+        wave_lds_sync();
+      }
+      if (live) {
+        rad = dof_pose(ev, base, xt, tx, ty, tz, M, nullptr, nullptr, nullptr, T, sn, cs);
+        double* rt = slot_rt(wv);
+        if (lane == 0) {
+          for (int k = 0; k < 9; ++k) rt[k] = M[k];
+          for (int k = 0; k < 3; ++k) rt[9 + k] = T[k];
+        }
+      }
+      if (lane == 0) {
+        s_live[wv] = live;
+        s_atoms[wv] = live && rad <= 12.0 ? ev.li.n_atoms : 0;   // Mol.Too_long
+      }
+    }
+    if (threadIdx.x == 0) s_next = 0;
+    __syncthreads();
+    bool any = false;
+    for (int k = 0; k < a.slots; ++k) any |= s_live[k] != 0;
+    if (!__builtin_amdgcn_readfirstlane((int)any)) break;   // the same for all wavefronts
+    for (;;) {
+      int u = 0;
+      if (lane == 0) u = atomicAdd(&s_next, 1);
+      u = __builtin_amdgcn_readlane(u, 0);
+      int sl = 0, n = 0;
+      for (; sl < a.slots; ++sl) {
+        n = __builtin_amdgcn_readfirstlane(s_atoms[sl]);
+        if (u < min_units(n)) break;
+        u -= min_units(n);
+      }
+      if (sl == a.slots) break;
+      const double* rt = slot_rt(sl);
+      double* sx = slot_xyz(sl);
+      const int A = a.max_atoms;
+      auto posed = [&](int j, double& x0, double& y0, double& z0) {
+        const double c0 = sx[j], c1 = sx[A + j], c2 = sx[2 * A + j];
+        x0 = (rt[0] * c0 + rt[1] * c1 + rt[2] * c2) + rt[9];
+        y0 = (rt[3] * c0 + rt[4] * c1 + rt[5] * c2) + rt[10];
+        z0 = (rt[6] * c0 + rt[7] * c1 + rt[8] * c2) + rt[11];
+      };
+      dof_sweep_unit(ev, n, u, posed, slot_at(sl), sx + 3 * A, sx + 4 * A, sx + 5 * A,
+                     fe + ((size_t)sl * units + u) * kWave);
+    }
+    __syncthreads();
+    if (live) {
+      double gt = 0.0, f = __builtin_inf();
+      if (rad <= 12.0) {
+        double e = 0.0;   // per lane, in the order of the atoms (as atom_sweep adds them)
+        const int L = ev.li.n_atoms;
+        const float4* mine = fe + (size_t)wv * units * kWave + lane;
+        constexpr int kAhead = 8;   // loads in flight
+        for (int u0 = 0; u0 < min_units(L); u0 += kAhead) {
+          float4 v[kAhead];
+#pragma unroll
+          for (int k = 0; k < kAhead; ++k)
+            if (u0 + k < min_units(L)) v[k] = mine[(size_t)(u0 + k) * kWave];
+#pragma unroll
+          for (int k = 0; k < kAhead; ++k) {
+            const int j = 4 * (u0 + k);
+            if (j < L) e += (double)v[k].x;
+            if (j + 1 < L) e += (double)v[k].y;
+            if (j + 2 < L) e += (double)v[k].z;
+            if (j + 3 < L) e += (double)v[k].w;
+          }
+        }
+        const double e_inter = wave_sum(e);
+        const double e_intra = dof_adjoint(ev, M, sn, cs, tx, ty, tz, hx, hy, hz, gt);
+        f = e_inter + e_intra;
+      }
+      xt = lbfgs_wave(s, x, g, d, xt, f, act ? gt : 0.0, rad, lo, hi, act, a.S + i, a.Y + i,
+                      (size_t)a.ndof_total, a.rho + p, (size_t)a.npose, cfg);
+      ++it;
+      if (it >= a.iters || __builtin_amdgcn_readfirstlane(s.status) != kMinRunning) {
+        if (act) a.x[i] = x;
+        int qv = 0;
+        if (lane == 0) {
+          a.st[p] = s;
+          if (a.e_out) a.e_out[p] = s.f;
+          qv = atomicAdd(a.queue, 1);
+        }
+        wave_lds_sync();   // all lanes meet here
+        q = a.slots * nb + __builtin_amdgcn_readlane(qv, 0);
+        live = false;
+      }
+    }
+  }
+}
+
+size_t min_pooled_lds_bytes(const MinPersistArgs& a) {
+  return receptor_lds_bytes<true>(a.nrec, a.cg) + a.slots * min_slot_lds_bytes(a.max_atoms, a.max_rb, a.max_rg) +
+         kMinPooledWaves * kAtomSweepInts * sizeof(int);
+}
+
+hipError_t launch_min_pooled(const MinPersistArgs& a, int nblocks, hipStream_t s) {
+  if (a.npose == 0) return hipSuccess;
+  const size_t lds = min_pooled_lds_bytes(a);
+  if (a.slots < 1 || a.slots > kMinSlots || a.slots > kMinPooledWaves || lds > kMaxLds)
+    return hipErrorInvalidValue;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_min_pooled),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)(kMaxLds - 128));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_min_pooled, dim3(nblocks), dim3(kMinPooledWaves * kWave), lds, s, a);
+  return hipGetLastError();
+}
+
 size_t min_persist_lds_bytes(const MinPersistArgs& a, int waves, bool rec_lds) {
   return (rec_lds ? receptor_lds_bytes<true>(a.nrec, a.cg) : 0) +
          (size_t)waves * min_wave_lds_bytes(a.max_atoms);

@@ -274,3 +274,37 @@ def test_dof_gradient_of_all_torsion_forms(sys0, n, kind):
                                             lig["rg_atoms"], d[p])[2]
                 scale = np.abs(J).sum(axis=(1, 2)) * np.abs(h).max()
                 np.testing.assert_array_less(np.abs(g[p] - (J * h).sum(axis=(1, 2))), 1e-9 * scale + 1e-12)
+
+
+@pytest.mark.parametrize("npose,iters", [(1, 1), (7, 30), (257, 12), (800, 5), (1793, 4), (2049, 2)])
+@pytest.mark.parametrize("intra", [False, True])
+def test_pooled_minimiser(sys0, npose, iters, intra):
+    """The minimiser whose workgroups pool their poses' sweeps (one to seven poses a CU, one or
+    several a workgroup, the rest from the queue) gives the one-wavefront form's points,
+    energies and decisions bit for bit: ligands of 1, 4, 5, 64, 65 atoms and the library's, poses
+    in contact, out of reach and too long; above its range the other form runs."""
+    import torch
+    from mmo_amd.minimize import Minimizer
+    ctx, lig, _ = sys0
+    rng = np.random.default_rng(npose)
+    ligs = [lig] + synth.library(5) + [_chain(n, 3, "facing", rng) for n in (1, 4, 5, 64, 65)]
+    ids = np.array([ctx.add_ligand(l) for l in ligs])
+    pick = rng.integers(0, len(ligs), npose)
+    b = ctx.batch(ids[pick])
+    start = np.concatenate([np.concatenate([rng.uniform(-12, 12, 3), rng.uniform(-3, 3, 3),
+                                            rng.uniform(-0.4, 0.4, len(ligs[k]["rb_left"]))]) for k in pick])
+    start[::7] *= 4.0   # among them poses beyond the cutoff
+    got = []
+    for pooled in (0, 8):
+        ctx.tune(min_pooled=pooled)
+        mz = Minimizer(b, flags=ff.F_INTER_SHIFTED | (ff.F_INTRA if intra else 0), max_step=0.3)
+        for _ in range(2):   # the second run starts from nothing of the first
+            d = torch.tensor(start, device="cuda:0")
+            e = mz.run(d, iters)
+            torch.cuda.synchronize()
+        got.append((e.cpu().numpy(), d.cpu().numpy(), mz.info()))
+    ctx.tune(min_pooled=8)
+    assert np.array_equal(got[0][0], got[1][0], equal_nan=True)
+    assert np.array_equal(got[0][1], got[1][1], equal_nan=True)
+    for k in got[0][2]:
+        assert np.array_equal(got[0][2][k], got[1][2][k], equal_nan=True), k
