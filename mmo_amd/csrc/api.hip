@@ -105,6 +105,10 @@ struct LigHost {
   std::vector<double> q;
   std::vector<int> anum, type;
   std::vector<uint32_t> pair_ij;
+  // the same by the torsions a pair feels, and their round masks (mc_pair_order), once made
+  std::vector<uint32_t> mc_ij;
+  std::vector<uint64_t> mc_mask;
+  bool mc_made = false;
   std::vector<int> rb_left, rb_right, rg_off, rg_atoms;
   std::vector<int> sweep;   // order in which the per-atom sweeps take the atoms
   bool free = false;        // torsions_free, and within kMaxFree*
@@ -183,6 +187,16 @@ struct mmo_ctx {
   DevBuf<double> d_lig_xyz;
   DevBuf<uint32_t> d_pair_ij;
   DevBuf<double4> d_pair_par;
+  // the chains' pair lists (McPairs), built when chains are first made
+  int mc_pairs_version = -1;   // lig_version they were uploaded for
+  std::vector<McPairs> mc_pairs;
+  DevBuf<McPairs> d_pe_lig;
+  DevBuf<uint32_t> d_pe_ij;
+  DevBuf<double2> d_pe_qa;
+  DevBuf<double> d_pe_b;
+  DevBuf<uint64_t> d_pe_mask;
+  int uff_version = 0;
+  int mc_keep_pairs = 1;       // chains keep their pair energies
   DevBuf<uint64_t> d_intra_bits;   // per atom i, bit d: the pair (i, i + d mod n) counts (free ligands)
   DevBuf<int64_t> d_bit_base;      // per ligand, into d_intra_bits
   DevBuf<int> d_sweep;          // per ligand at atom_base: the sweeps' atom order
@@ -246,6 +260,11 @@ struct mmo_mc {
   DevBuf<McState> d_st;
   DevBuf<double> d_conf, d_best, d_dr, d_undo;
   DevBuf<SwState> d_sw;
+  // pair energies kept per chain, valid for the UFF parameters of pe_uff (-1: not yet)
+  DevBuf<double> d_pe;
+  DevBuf<int64_t> d_pe_off;
+  DevBuf<uint64_t> d_pe_sel;
+  int pe_words = 0, pe_uff = -1;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   int graph_steps = 0;
@@ -502,6 +521,102 @@ int sync_ligands(mmo_ctx* c) {
   HIPCHK(c, hipStreamSynchronize(s));
   c->lig_dirty = false;
   ++c->lig_version;
+  return MMO_OK;
+}
+
+// A ligand's pairs for chains that keep pair energies (McPairs): by the set of torsions
+// that change a pair's distance, i.e. whose group holds one of its atoms, sets of few torsions
+// first; a torsion's mask names the rounds of 64 that hold such a pair.  Ligands whose lists
+// would take long to make get none.
+constexpr size_t kMcPairWork = 1u << 26;
+void mc_pair_order(LigHost& h) {
+  if (h.mc_made) return;
+  h.mc_made = true;
+  const int R = (int)h.rb_left.size();
+  const size_t np = h.pair_ij.size();
+  if (R == 0 || np == 0 || np * R > kMcPairWork || (size_t)R * h.n > kMcPairWork) return;
+  const int sw = (R + 63) / 64;
+  std::vector<uint64_t> in((size_t)h.n * sw, 0ull);   // per atom: the groups that hold it
+  for (int k = 0; k < R; ++k)
+    for (int m = h.rg_off[k]; m < h.rg_off[k + 1]; ++m)
+      in[(size_t)h.rg_atoms[m] * sw + k / 64] |= 1ull << (k % 64);
+  // atoms of the same groups form a class; per pair of classes the torsions it feels
+  std::map<std::vector<uint64_t>, int> classes;
+  std::vector<int> cls(h.n);
+  for (int j = 0; j < h.n; ++j)
+    cls[j] = classes.emplace(std::vector<uint64_t>(in.begin() + (size_t)j * sw, in.begin() + (size_t)(j + 1) * sw),
+                             (int)classes.size()).first->second;
+  const size_t nc = classes.size();
+  if (nc * nc > kMcPairWork) return;
+  std::vector<const uint64_t*> sig(nc);
+  for (const auto& [key, k] : classes) sig[k] = key.data();
+  std::map<std::pair<int, std::vector<uint64_t>>, std::vector<uint32_t>> by;
+  std::vector<std::vector<uint32_t>*> list_of(nc * nc, nullptr);
+  std::vector<uint64_t> key(sw);
+  for (uint32_t p : h.pair_ij) {
+    const int ca = cls[p & 0xffff], cb = cls[p >> 16];
+    std::vector<uint32_t>*& list = list_of[ca * nc + cb];
+    if (!list) {
+      int bits = 0;
+      for (int w = 0; w < sw; ++w) {
+        key[w] = sig[ca][w] ^ sig[cb][w];
+        bits += __builtin_popcountll(key[w]);
+      }
+      list = &by[{bits, key}];
+    }
+    list->push_back(p);
+  }
+  const size_t rounds = (np + kWave - 1) / kWave, words = (rounds + 63) / 64;
+  h.mc_ij.reserve(rounds * kWave);
+  h.mc_mask.assign((size_t)R * words, 0ull);
+  for (const auto& [k, list] : by) {
+    const size_t r0 = h.mc_ij.size() / kWave;
+    h.mc_ij.insert(h.mc_ij.end(), list.begin(), list.end());
+    const size_t r1 = (h.mc_ij.size() - 1) / kWave;
+    for (int b = 0; b < R; ++b)
+      if ((k.second[b / 64] >> (b % 64)) & 1)
+        for (size_t r = r0; r <= r1; ++r) h.mc_mask[(size_t)b * words + r / 64] |= 1ull << (r % 64);
+  }
+  h.mc_ij.resize(rounds * kWave, 0u);
+}
+
+// the registry's McPairs on the device (after sync_ligands)
+int sync_mc_pairs(mmo_ctx* c) {
+  if (c->mc_pairs_version == c->lig_version) return MMO_OK;
+  std::vector<uint32_t> ij;
+  std::vector<double4> pp;
+  std::vector<double2> qa;
+  std::vector<double> pb;
+  std::vector<uint64_t> mask;
+  c->mc_pairs.clear();
+  for (LigHost& h : c->ligs) {
+    mc_pair_order(h);
+    McPairs mp{};
+    mp.base = (int64_t)ij.size();
+    mp.mask_base = (int64_t)mask.size();
+    mp.rounds = (int)(h.mc_ij.size() / kWave);
+    mp.words = (mp.rounds + 63) / 64;
+    c->mc_pairs.push_back(mp);
+    int r = pair_params(c, h.mc_ij, h.q.data(), h.anum.data(), pp);
+    if (r) return r;
+    for (size_t p = 0; p < pp.size(); ++p) {
+      const bool in = p < h.pair_ij.size();   // the last round's filling has no energy
+      qa.push_back(in ? make_double2(pp[p].x, pp[p].y) : make_double2(0.0, 0.0));
+      pb.push_back(in ? pp[p].z : 0.0);
+    }
+    ij.insert(ij.end(), h.mc_ij.begin(), h.mc_ij.end());
+    mask.insert(mask.end(), h.mc_mask.begin(), h.mc_mask.end());
+  }
+  hipStream_t s = c->stream;
+  int r;
+  if ((r = upload(c, c->d_pe_lig, c->mc_pairs.data(), c->mc_pairs.size(), s)) ||
+      (r = upload(c, c->d_pe_ij, ij.data(), ij.size(), s)) ||
+      (r = upload(c, c->d_pe_qa, qa.data(), qa.size(), s)) ||
+      (r = upload(c, c->d_pe_b, pb.data(), pb.size(), s)) ||
+      (r = upload(c, c->d_pe_mask, mask.data(), mask.size(), s)))
+    return r;
+  HIPCHK(c, hipStreamSynchronize(s));
+  c->mc_pairs_version = c->lig_version;
   return MMO_OK;
 }
 
@@ -803,7 +918,8 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     c->grid_cells.release();
     c->rpos_s.release(); c->rab_s.release(); c->rres_s.release(); c->d_cells.release();
     c->d_ligs.release(); c->d_latoms.release(); c->d_lig_xyz.release();
-    c->d_pair_ij.release(); c->d_pair_par.release(); c->d_intra_bits.release(); c->d_bit_base.release(); c->d_sweep.release(); c->d_clash.release();
+    c->d_pair_ij.release(); c->d_pair_par.release();
+    c->d_pe_lig.release(); c->d_pe_ij.release(); c->d_pe_qa.release(); c->d_pe_b.release(); c->d_pe_mask.release(); c->d_intra_bits.release(); c->d_bit_base.release(); c->d_sweep.release(); c->d_clash.release();
     c->d_rb_left.release(); c->d_rb_right.release(); c->d_rg_off.release(); c->d_rg_atoms.release();
     c->s_xyz.release(); c->s_e.release(); c->s_g.release(); c->s_part.release();
     c->s_lig.release(); c->s_latom.release(); c->s_pij.release(); c->s_ppar.release();
@@ -832,6 +948,7 @@ int mmo_set_uff_table(mmo_ctx* c, const int32_t* anum, const double* x, const do
     t[anum[i]] = Uff{x[i], d[i]};
   }
   c->uff = t;
+  ++c->uff_version;
   c->lig_dirty = true;
   c->has_rec = false;   // receptor parameters depend on the table: upload again
   return MMO_OK;
@@ -1802,6 +1919,36 @@ int mmo_grid_compute(mmo_ctx* c, const int32_t* probe_anum, const double* probe_
 }
 
 // ------------------------------------------------------------------ Monte Carlo
+// Room for the chains' round energies, where they turn torsions and add E_intra: 16 bytes per
+// round (64 pairs) of each chain, 2 KB for a ligand of 132 atoms.  Above the bound, or without
+// that memory, the chains evaluate all pairs of every torsion proposal.
+constexpr size_t kMcPairBytes = (size_t)1 << 30;
+static int mc_keep_pairs(mmo_mc* m, hipStream_t s) {
+  mmo_ctx* c = m->ctx;
+  if (!(m->flags & kMcTweak) || !(m->flags & kMcIntraUff) || !c->mc_keep_pairs) return MMO_OK;
+  if (3 * (size_t)m->max_atoms * sizeof(double) > 65536) return MMO_OK;   // k_mc_pairs' LDS
+  int r;
+  if ((r = sync_ligands(c)) || (r = sync_mc_pairs(c))) return r;
+  std::vector<int64_t> off(m->nchain);
+  size_t total = 0;
+  int words = 1;
+  for (int k = 0; k < m->nchain; ++k) {
+    const McPairs& mp = c->mc_pairs[m->chain_lig[k]];
+    off[k] = (int64_t)total;
+    total += 2 * (size_t)mp.rounds;
+    words = std::max(words, mp.words);
+  }
+  if (total == 0 || total * sizeof(double) > kMcPairBytes) return MMO_OK;
+  if (m->d_pe.ensure(total) != hipSuccess) {
+    (void)hipGetLastError();
+    return MMO_OK;
+  }
+  std::vector<uint64_t> sel((size_t)m->nchain * words, 0ull);
+  m->pe_words = words;
+  if ((r = upload(c, m->d_pe_off, off.data(), off.size(), s))) return r;
+  return upload(c, m->d_pe_sel, sel.data(), sel.size(), s);
+}
+
 int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double* rot0,
                   const double* pos0, int inter_mode, int flags, const double* roi_center,
                   double roi_r, double temperature, uint64_t seed, int total_frames,
@@ -1921,6 +2068,10 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
     delete m;
     return r;
   }
+  if ((r = mc_keep_pairs(m, s))) {
+    delete m;
+    return r;
+  }
   hipError_t e = m->d_queue.ensure(1);
   if (e == hipSuccess) e = mc_prepare();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1931,6 +2082,10 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
   *out = m;
   return MMO_OK;
 }
+
+// before a run on stream s: the lists of this registry, and the energies of new chains or
+// changed parameters
+static int mc_fresh_pairs(mmo_mc* m, hipStream_t s);
 
 static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work) {
   mmo_ctx* c = m->ctx;
@@ -1957,7 +2112,27 @@ static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work) {
   a.min_min_step = 1e-10; a.min_gtol = m->min_gtol; a.min_c1 = 1e-4;
   a.min_base = m->d_min_base.p; a.min_S = m->d_min_S.p; a.min_Y = m->d_min_Y.p;
   a.min_rho = m->d_min_rho.p;
+  if (m->pe_words > 0 && m->min_iters == 0) {
+    a.pe_lig = c->d_pe_lig.p; a.pe_ij = c->d_pe_ij.p; a.pe_qa = c->d_pe_qa.p; a.pe_b = c->d_pe_b.p;
+    a.pe_mask = c->d_pe_mask.p; a.pe = m->d_pe.p; a.pe_off = m->d_pe_off.p;
+    a.pe_sel = m->d_pe_sel.p; a.pe_words = m->pe_words;
+  }
   return a;
+}
+
+static int mc_fresh_pairs(mmo_mc* m, hipStream_t s) {
+  mmo_ctx* c = m->ctx;
+  if (m->pe_words == 0) return MMO_OK;
+  int r = sync_mc_pairs(c);
+  if (r) return r;
+  if (m->min_iters > 0) {   // minimised proposals change the conformer otherwise
+    m->pe_uff = -1;
+    return MMO_OK;
+  }
+  if (m->pe_uff == c->uff_version) return MMO_OK;
+  HIPCHK(c, launch_mc_pairs(mc_args(m, 1, m->nchain, m->d_work.p), m->nchain, s));
+  m->pe_uff = c->uff_version;
+  return MMO_OK;
 }
 
 // launch shape: up to 8 chains (wavefronts) per workgroup; in the direct form the
@@ -1990,6 +2165,7 @@ int mmo_mc_run(mmo_mc* m, int nsteps, void* stream) {
   if (nsteps <= 0) return fail(c, MMO_ERR_BAD_ARG, "nsteps must be positive");
   if ((r = sync_ligands(c))) return r;
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  if ((r = mc_fresh_pairs(m, s))) return r;
   McArgs a = mc_args(m, nsteps, m->nchain, m->d_work.p);
   timer_begin(c, "mc", s);
   HIPCHK(c, mc_launch(m, a, m->nchain, s));
@@ -2005,6 +2181,7 @@ int mmo_mc_run_graph(mmo_mc* m, int nsteps, int nreplay, void* stream) {
   if (nsteps <= 0 || nreplay <= 0) return fail(c, MMO_ERR_BAD_ARG, "bad graph arguments");
   if ((r = sync_ligands(c))) return r;
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  if (m->pe_words > 0 && (r = sync_mc_pairs(c))) return r;
   // a graph holds the registry's device pointers: capture again when they may have moved
   if (m->gexec && (m->graph_steps != nsteps || m->graph_version != c->lig_version)) {
     (void)hipGraphExecDestroy(m->gexec);
@@ -2034,6 +2211,7 @@ int mmo_mc_run_graph(mmo_mc* m, int nsteps, int nreplay, void* stream) {
     HIPCHK(c, hipStreamWaitEvent(c->stream, ev, 0));
     (void)hipEventDestroy(ev);
   }
+  if ((r = mc_fresh_pairs(m, c->stream))) return r;
   timer_begin(c, "mc", c->stream);
   for (int k = 0; k < nreplay; ++k) HIPCHK(c, hipGraphLaunch(m->gexec, c->stream));
   timer_end(c, "mc", c->stream);
@@ -2055,6 +2233,7 @@ int mmo_mc_run_per_ligand(mmo_mc* m, int nsteps, void* stream) {
   if (nsteps <= 0) return fail(c, MMO_ERR_BAD_ARG, "nsteps must be positive");
   if ((r = sync_ligands(c))) return r;
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  if ((r = mc_fresh_pairs(m, s))) return r;
   timer_begin(c, "mc", s);
   for (const auto& gr : m->groups) {
     McArgs a = mc_args(m, nsteps, gr.second, m->d_work_by_lig.p + gr.first);
@@ -2171,6 +2350,7 @@ void mmo_mc_destroy(mmo_mc* m) {
     m->d_chain_lig.release(); m->d_chain_atom.release(); m->d_chain_rb.release();
     m->d_work.release(); m->d_work_by_lig.release(); m->d_queue.release(); m->d_st.release();
     m->d_conf.release(); m->d_best.release(); m->d_dr.release(); m->d_undo.release(); m->d_sw.release();
+    m->d_pe.release(); m->d_pe_off.release(); m->d_pe_sel.release();
     m->d_min_base.release(); m->d_min_S.release(); m->d_min_Y.release(); m->d_min_rho.release();
   }
   delete m;
@@ -2868,6 +3048,7 @@ int mmo_tune_set(mmo_ctx* c, const char* key, double v) {
   else if (k == "scan_lattice" && iv >= 0 && iv <= 2) c->scan_lattice = iv;
   else if (k == "scan_split" && iv >= 0 && iv <= (1 << 20)) c->scan_split = iv;
   else if (k == "grid_pack" && (iv == 0 || iv == 1)) c->grid_pack = iv;
+  else if (k == "mc_keep_pairs" && (iv == 0 || iv == 1)) c->mc_keep_pairs = iv;
   else if (k == "mc_waves_per_cu" && iv >= 1 && iv <= 32) c->mc_waves_per_cu = iv;
   else if (k == "mc_wg_waves" && iv >= 1 && iv <= 16) c->mc_wg_waves = iv;
   else if (k == "pose_cull" && (iv == 0 || iv == 1)) c->pose_cull = iv;
@@ -2905,6 +3086,7 @@ double mmo_tune_get(mmo_ctx* c, const char* key) {
   if (k == "cell_size") return c->cell_size;
   if (k == "cull_ok") return c->cull_ok ? 1.0 : 0.0;
   if (k == "cullp_ok") return c->cullp_ok ? 1.0 : 0.0;
+  if (k == "mc_keep_pairs") return c->mc_keep_pairs;
   if (k == "mc_waves_per_cu") return c->mc_waves_per_cu;
   if (k == "mc_wg_waves") return c->mc_wg_waves;
   if (k == "pose_cull") return c->pose_cull;

@@ -41,6 +41,14 @@ struct McState {
 };
 static_assert(sizeof(McState) % 8 == 0, "McState is copied as 32-bit words into 8-aligned LDS slots");
 
+// A ligand's interacting pairs in rounds of 64 (the last filled with pairs of no energy),
+// ordered by the torsions they feel; per torsion a mask of the rounds that hold such pairs.
+// rounds = 0: its chains evaluate all pairs.
+struct McPairs {
+  int64_t base, mask_base;   // first pair; first mask word
+  int rounds, words;         // words of a mask
+};
+
 struct McArgs {
   // ligands
   const LigInfo* ligs;
@@ -54,6 +62,17 @@ struct McArgs {
   const uint32_t* pair_ij;
   const double4* pair_par;
   int max_atoms;
+  // energies of the rounds kept per chain (pe null: none), 2 x rounds at pe_off, and which
+  // place of each round is the chain's (pe_words words per chain)
+  const McPairs* pe_lig;
+  const uint32_t* pe_ij;
+  const double2* pe_qa;         // ke qi qj, Ai Aj
+  const double* pe_b;           // 2 Bi Bj
+  const uint64_t* pe_mask;
+  double* pe;
+  const int64_t* pe_off;
+  uint64_t* pe_sel;
+  int pe_words;
   // chains
   int nwork;                 // chains to process in this launch
   const int* work;           // their indices, most expensive first
@@ -99,6 +118,8 @@ struct McArgs {
 int mc_max_waves(const McArgs& a);
 hipError_t launch_mc(const McArgs& a, int nblocks, int waves, bool rec_lds, hipStream_t s);
 size_t mc_lds_bytes(const McArgs& a, int waves, bool rec_lds);
+// the chains' kept energies from their conformers (3 max_atoms FP64 of LDS a chain)
+hipError_t launch_mc_pairs(const McArgs& a, int nchain, hipStream_t s);
 hipError_t mc_prepare();
 
 }  // namespace mmo

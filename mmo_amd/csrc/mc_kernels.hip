@@ -78,16 +78,6 @@ __device__ __forceinline__ void sw_reset(SwState& w) {
   w.head = w.count = w.acc = 0;
 }
 
-// Rot.of_axis_angle (src/rot.ml:121-146)
-__device__ __forceinline__ void axis_angle(double x, double y, double z, double th, double* m) {
-  double s, c;
-  sincos(th, &s, &c);
-  const double o = 1.0 - c;
-  m[0] = c + x * x * o;     m[1] = x * y * o - z * s; m[2] = x * z * o + y * s;
-  m[3] = x * y * o + z * s; m[4] = c + y * y * o;     m[5] = y * z * o - x * s;
-  m[6] = x * z * o - y * s; m[7] = y * z * o + x * s; m[8] = c + z * z * o;
-}
-
 // --------------------------------------------------------------- energies of a pose
 // The pose being scored (rotation, conformer centre, position) and the frame's Metropolis
 // uniform, in the chain's LDS slot: the energy sweeps read it from there, so none of it
@@ -139,8 +129,7 @@ __device__ double mc_inter_interp(const McArgs& a, const LigInfo& li, const Pose
          (double)cv[6] * (wlx * wly * wlz) + (double)cv[7] * (whx * wly * wlz);
   }
   e = wave_sum(e);
-  for (int off = 1; off < kWave; off <<= 1) bad |= __shfl_xor(bad, off, kWave);
-  return bad ? __builtin_nan("") : e;
+  return __ballot(bad) != 0ull ? __builtin_nan("") : e;
 }
 
 // shifted direct sum of the pose: FP32 pairs swept per 8-atom sub-block (pose_sweep);
@@ -241,6 +230,136 @@ __device__ double mc_intra(const McArgs& a, const LigInfo& li, const double* sx,
   return wave_sum(e);
 }
 
+// LDS writes of one wavefront made visible to its other lanes (the chain's conformer
+// buffers belong to one wavefront; the workgroup's other wavefronts run other chains)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// E_intra of a chain that turns one torsion at a time: only pairs with one atom in the turned
+// group change, so the energy of every round (64 pairs) is kept per chain and a proposal
+// evaluates the rounds that hold such pairs.  The pairs are listed by the torsions they feel
+// (McPairs, api.hip), which leaves 41 % of the rounds of ligands of 26 to 132 atoms to a
+// torsion (26 % for the largest; 25 % of the pairs).  A round's energy has two places: the
+// proposal's goes to the one that sel does not name, and accepting it flips the rounds' bits.
+// The sum is over all rounds in their order, whichever were evaluated.
+// A frame's latency bounds this form up to some 6,000 chains (96 chains alone take 60 % of
+// their time), and the pair sum was half of it: 8,100 pairs of a 132-atom ligand 28,000 cycles
+// alone and 57,000 with four wavefronts on a SIMD, now 8,000 to 20,000 and 24,000.  6,144
+// chains on the grids, 1,000 frames: 25.4 -> 17.8 ms (12,288: 38.9 -> 30.5).  Energies kept
+// per pair, not per round, were 22.9 ms (every frame reads them all back); the whole list with
+// the parameters formed from the atoms' in LDS 27.6.
+struct PairLoad {
+  uint32_t ij;
+  double2 qa;   // ke qi qj, Ai Aj
+  double b;     // 2 Bi Bj
+};
+__device__ __forceinline__ PairLoad load_pair(const McArgs& a, int64_t p) {
+  return {a.pe_ij[p], a.pe_qa[p], a.pe_b[p]};
+}
+__device__ __forceinline__ double mc_pair(const PairLoad& p, const double* sx, const double* sy,
+                                          const double* sz) {
+  const int i = p.ij & 0xffff, j = p.ij >> 16;
+  const double dx = sx[i] - sx[j], dy = sy[i] - sy[j], dz = sz[i] - sz[j];
+  const double r2 = dx * dx + dy * dy + dz * dz;
+  const double irr = rsqrt(fmax(r2, 1.0e-4));   // no branch around the refinement
+  const double ir = r2 >= 1.0e-4 ? irr : 100.0;   // 1 / max(r, 0.01)
+  const double uu = ir * ir, u3 = uu * uu * uu, u6 = u3 * u3;
+  return p.qa.x * ir + p.qa.y * u6 - p.b * u3;
+}
+
+// Sums of two rounds at once: the halves of the wavefront are exchanged first, so that the
+// other five steps of a wavefront sum serve both; lane 31 gets round 0's, lane 63 round 1's.
+__device__ __forceinline__ double two_round_sums(double v0, double v1) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v0), __double2loint(v1), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v0), __double2hiint(v1), false, false);
+  double v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  v += dpp_d<0x111>(v, 0.0);
+  v += dpp_d<0x112>(v, 0.0);
+  v += dpp_d<0x114>(v, 0.0);
+  v += dpp_d<0x118>(v, 0.0);
+  v += dpp_d<0x142, 0xa>(v, 0.0);
+  return v;
+}
+
+// a 64-bit word that all lanes hold, as a scalar
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (uint64_t)hi << 32 | lo;
+}
+
+// mask (nullable): the rounds to evaluate, per word of 64 rounds; sel: the rounds' places
+__device__ double mc_intra_table(const McArgs& a, const McPairs& mp, double* E, const uint64_t* sel,
+                                 const uint64_t* mask, const double* sx, const double* sy,
+                                 const double* sz) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double e = 0.0;
+  for (int w = 0; w < mp.words; ++w) {
+    const uint64_t s = uniform64(sel[w]), m = mask ? uniform64(mask[w]) : 0ull;
+    const int r0 = 64 * w;
+    // the next two rounds' pairs are fetched while two are evaluated
+    PairLoad next[2];
+    int nq[2];
+    uint64_t todo = m;
+    auto fetch = [&]() {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        // an odd last round is evaluated twice, to the same place
+        if (u == 0 || todo) nq[u] = __builtin_ctzll(todo);
+        else nq[u] = nq[0];
+        todo &= todo - 1;
+        next[u] = load_pair(a, mp.base + (int64_t)(r0 + nq[u]) * kWave + lane);
+      }
+    };
+    bool more = todo != 0;
+    if (more) fetch();
+    while (more) {
+      const PairLoad cur[2] = {next[0], next[1]};
+      const int q = lane < 32 ? nq[0] : nq[1];
+      more = todo != 0;
+      if (more) fetch();
+      const double v0 = mc_pair(cur[0], sx, sy, sz), v1 = mc_pair(cur[1], sx, sy, sz);
+      const double v = two_round_sums(v0, v1);
+      if ((lane & 31) == 31) E[((s >> q) & 1 ? 0 : mp.rounds) + r0 + q] = v;
+    }
+    wave_sync();
+    const uint64_t at = s ^ m;
+    if (r0 + lane < mp.rounds) e += E[((at >> lane) & 1 ? mp.rounds : 0) + r0 + lane];
+  }
+  return wave_sum(e);
+}
+
+// All rounds of every chain, to the places sel names: before a run's first launch, and when
+// the parameters have changed.  One wavefront per chain.
+__global__ void __launch_bounds__(64) k_mc_pairs(McArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  const int chain = blockIdx.x, lane = threadIdx.x;
+  const McPairs mp = a.pe_lig[a.chain_lig[chain]];
+  if (mp.rounds == 0) return;
+  double* sx = reinterpret_cast<double*>(smem);
+  double* sy = sx + a.max_atoms;
+  double* sz = sy + a.max_atoms;
+  const int L = a.ligs[a.chain_lig[chain]].n_atoms;
+  const double* conf = a.conf + 3 * (size_t)a.chain_atom[chain];
+  for (int j = lane; j < L; j += kWave) {
+    sx[j] = conf[3 * j]; sy[j] = conf[3 * j + 1]; sz[j] = conf[3 * j + 2];
+  }
+  __syncthreads();
+  double* E = a.pe + a.pe_off[chain];
+  const uint64_t* sel = a.pe_sel + (size_t)chain * a.pe_words;
+  for (int q0 = 0; q0 < mp.rounds; q0 += 2) {
+    const int q1 = min(q0 + 1, mp.rounds - 1);
+    const double v0 = mc_pair(load_pair(a, mp.base + (int64_t)q0 * kWave + lane), sx, sy, sz);
+    const double v1 = mc_pair(load_pair(a, mp.base + (int64_t)q1 * kWave + lane), sx, sy, sz);
+    const double v = two_round_sums(v0, v1);
+    const int q = lane < 32 ? q0 : q1;
+    if ((lane & 31) == 31) E[((sel[q / 64] >> (q % 64)) & 1 ? mp.rounds : 0) + q] = v;
+  }
+}
+
 struct RecView {
   const RecPos* pos;
   const RecAB* ab;
@@ -252,14 +371,6 @@ template <int INTER>
 __device__ double mc_inter(const McArgs& a, const LigInfo& li, const PoseView& v, const RecView& r) {
   if (INTER == kMcInterGrid) return mc_inter_interp(a, li, v);
   return mc_inter_direct<INTER>(a, li, v, r.pos, r.ab, r.cell, r.wl);
-}
-
-// LDS writes of one wavefront made visible to its other lanes (the chain's conformer
-// buffers belong to one wavefront; the workgroup's other wavefronts run other chains)
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // ------------------------------------------------- Monte Carlo-plus-minimisation
@@ -407,6 +518,12 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
     wave_sync();
     const bool flex = (a.flags & kMcTweak) && nrb > 0;
     const bool use_intra = (a.flags & kMcIntraUff) != 0;
+    // the chain's pair energies, if it keeps them
+    McPairs mp{};
+    if (!MIN && a.pe && use_intra && flex) mp = a.pe_lig[lig];
+    double* const pe = mp.rounds ? a.pe + a.pe_off[chain] : nullptr;
+    uint64_t* const sel = a.pe_sel + (size_t)chain * a.pe_words;
+    const uint64_t* mask = nullptr;   // rounds of the proposal's torsion
 
     if (!st.initialized) {
       // start pose: Mol.rotate_then_translate_copy centered_lig rot0 pos0, no
@@ -417,7 +534,8 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
       }
       wave_sync();
       const PoseView v{cx_, cy_, cz_, pose};
-      st.prev_e_intra = use_intra ? mc_intra(a, li, cx_, cy_, cz_) : 0.0;
+      st.prev_e_intra = mp.rounds ? mc_intra_table(a, mp, pe, sel, nullptr, cx_, cy_, cz_)
+                        : use_intra ? mc_intra(a, li, cx_, cy_, cz_) : 0.0;
       st.prev_e_inter = mc_inter<INTER>(a, li, v, rv);
       st.prev_e = st.prev_e_inter + st.prev_e_intra;
       st.best_e = st.prev_e;
@@ -431,16 +549,42 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
       st.initialized = 1;
     }
 
+    // the draws of frames draws_at .. draws_end - 1, in the lanes
+    constexpr int kDraws = kWave / 3;
+    double draw_a = 0.0, draw_b = 0.0, draw_s = 0.0, draw_c = 0.0;
+    int draws_at = 0, draws_end = 0;
     const int frame_end = min(st.frame + a.nsteps, a.total_frames);
     for (; st.frame < frame_end; ++st.frame) {
       const bool rigid = (st.frame & 1) == 0;
-      const uint4 r0 = philox(make_uint4((uint32_t)chain, (uint32_t)st.frame, 0u, 0x4D4D4F31u), a.seed_lo, a.seed_hi);
-      const uint4 r1 = philox(make_uint4((uint32_t)chain, (uint32_t)st.frame, 1u, 0x4D4D4F31u), a.seed_lo, a.seed_hi);
-      const uint4 r2 = philox(make_uint4((uint32_t)chain, (uint32_t)st.frame, 2u, 0x4D4D4F31u), a.seed_lo, a.seed_hi);
-      double u0, u1, u2, u3, u4, u5;
-      uniform2(r0, u0, u1);
-      uniform2(r1, u2, u3);
-      uniform2(r2, u4, u5);
+      const int frame = __builtin_amdgcn_readfirstlane(st.frame);
+      if (frame >= draws_end) {
+        // the numbers of the next kDraws frames (one draw for all of them where every frame had
+        // its three generator calls and a sincos in all lanes: a fifth of the vector
+        // instructions of a frame on the grids): lane 3 f + c draws pair c of frame f; lanes
+        // of pair 0 also take the frame's angle (rigid: Move.rand_rot, torsion:
+        // Move.rand_angle, src/move.ml:14-31) with the step sizes as they are now
+        const int f = frame + lane / 3;
+        const uint4 r = philox(make_uint4((uint32_t)chain, (uint32_t)f, (uint32_t)(lane % 3), 0x4D4D4F31u),
+                               a.seed_lo, a.seed_hi);
+        uniform2(r, draw_a, draw_b);
+        double u = draw_a, amp = st.max_rot;
+        if (f & 1) {
+          u = draw_b;
+          const int step = st.conf_step + ((f >> 1) - (frame >> 1));
+          const bool flip = step > 0 && step % kMcBlock == 0 && !(a.flags & kMcNoFlip);
+          amp = pi;
+          if (flex && !flip) {
+            const int i = (int)(draw_a * nrb);
+            amp = dr[i < nrb ? i : nrb - 1];
+          }
+        }
+        sincos(u * (2.0 * amp) - amp, &draw_s, &draw_c);
+        draws_at = frame;
+        draws_end = frame + kDraws;
+      }
+      const int dl = 3 * (frame - draws_at);
+      const double u0 = readlane_d(draw_a, dl), u1 = readlane_d(draw_b, dl);
+      const double ds = readlane_d(draw_s, dl), dc = readlane_d(draw_c, dl);
 
       // ---- proposal
       double nrot[9], npos[3], ccx, ccy, ccz;
@@ -457,15 +601,12 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
           // Mol.flip_rbond / tweak_rbond on a copy (src/lds.ml:784-795, src/mol.ml:635-647)
           int i = (int)(u0 * nrb);
           i = i < nrb ? i : nrb - 1;
-          const bool flip = st.conf_step > 0 && st.conf_step % kMcBlock == 0 && !(a.flags & kMcNoFlip);
-          const double amp = flip ? pi : dr[i];
-          const double ang = u1 * (2.0 * amp) - amp;   // Move.rand_angle, src/move.ml:14-16
           const int left = a.rb_left[li.rb_base + i], right = a.rb_right[li.rb_base + i];
           const double ox = cx_[right], oy = cy_[right], oz = cz_[right];
           const double vx = ox - cx_[left], vy = oy - cy_[left], vz = oz - cz_[left];
           const double mag = sqrt(vx * vx + vy * vy + vz * vz);
-          double Rm[9];
-          axis_angle(vx / mag, vy / mag, vz / mag, ang, Rm);
+          const Rod rod = rodrigues(vx / mag, vy / mag, vz / mag, ds, dc);
+          const double* Rm = rod.m;
           wave_sync();
           const int g0 = a.rg_off[li.rg_base + i], g1 = a.rg_off[li.rg_base + i + 1];
           for (int m = g0 + lane; m < g1; m += kWave) {
@@ -497,6 +638,7 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
           mg0 = g0;
           mg1 = g1;
           just_rotated = i;
+          mask = a.pe_mask + mp.mask_base + (size_t)i * mp.words;
         }
       } else {
         // Move.rand_rot: left-multiply the passive axis rotation Rot.rx / ry / rz
@@ -504,11 +646,9 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
         // p' = c p + s q and q' = c q - s p, with (p, q) = rows (1, 2) for x, (2, 0) for y,
         // (0, 1) for z.  Written with selects: a switch that built the 3x3 matrix per axis
         // was mis-lowered by hipcc (the -s entry of the z matrix came out 0).
-        const double th = u0 * (2.0 * st.max_rot) - st.max_rot;
         int ax = (int)(u1 * 3.0);
         ax = ax < 3 ? ax : 2;
-        double s, c;
-        sincos(th, &s, &c);
+        const double s = ds, c = dc;
         const bool ax0 = ax == 0, ax1 = ax == 1;
         for (int cc = 0; cc < 3; ++cc) {
           const double r0 = st.rot[cc], r1 = st.rot[3 + cc], r2 = st.rot[6 + cc];
@@ -520,6 +660,8 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
           nrot[6 + cc] = ax0 ? qn : (ax1 ? pn : r2);
         }
         // Move.rand_trans (src/move.ml:46-54)
+        const double u2 = readlane_d(draw_a, dl + 1), u3 = readlane_d(draw_b, dl + 1),
+                     u4 = readlane_d(draw_a, dl + 2);
         npos[0] = st.pos[0] + (u2 * 2.0 - 1.0) * st.max_trans;
         npos[1] = st.pos[1] + (u3 * 2.0 - 1.0) * st.max_trans;
         npos[2] = st.pos[2] + (u4 * 2.0 - 1.0) * st.max_trans;
@@ -532,7 +674,7 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
         for (int k = 0; k < 9; ++k) pose->m[k] = nrot[k];
         pose->c[0] = ccx; pose->c[1] = ccy; pose->c[2] = ccz;
         for (int k = 0; k < 3; ++k) pose->p[k] = npos[k];
-        pose->u = u5;
+        pose->u = readlane_d(draw_b, dl + 2);
       }
       wave_sync();
       asm volatile("" ::: "memory");
@@ -545,7 +687,9 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
         // the proposal, locally minimised; its centre is the pose centre of the ROI test
         curr_e = mc_minimize<INTER>(a, li, chain, flex, use_intra, v, rv, ml, st, mM, mT, cpos);
       } else {
-        if (!rigid && use_intra && flex) st.prev_e_intra = mc_intra(a, li, sx, sy, sz);
+        if (!rigid && use_intra && flex)
+          st.prev_e_intra = mp.rounds ? mc_intra_table(a, mp, pe, sel, mask, sx, sy, sz)
+                                      : mc_intra(a, li, sx, sy, sz);
         st.prev_e_inter = mc_inter<INTER>(a, li, v, rv);
         curr_e = st.prev_e_inter + st.prev_e_intra;
       }
@@ -568,6 +712,7 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
         // reset_run_params (src/lds.ml:632-648): the conformer is kept; the best pose
         // becomes the registered conformer at the start pose (best_lig := prev_lig :=
         // rotate_then_translate_copy centered_lig rot0 pos0, src/lds.ml:645-646)
+        if (st.max_rot != a.max_rot0) draws_end = 0;   // drawn with the old step size
         st.max_rot = a.max_rot0;
         st.max_trans = a.max_trans0;
         for (int k = 0; k < 9; ++k) { st.rot[k] = st.rot0[k]; st.best_rot[k] = (k % 4 == 0) ? 1.0 : 0.0; }
@@ -626,6 +771,7 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
             if (mg1 > mg0) {   // conf := conf' (already in place): keep it
               for (int k = 0; k < 3; ++k) st.center[k] = P.c[k];
               mg0 = mg1 = 0;
+              for (int w = lane; w < mp.words; w += kWave) sel[w] ^= mask[w];
             }
           }
         }
@@ -656,12 +802,14 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
         // adaptive rigid steps every 100 rigid frames (src/lds.ml:971-974, :586-600)
         if (rigid && st.rigid_step > 0 && st.rigid_step % kMcBlock == 0) {
           const double ar = sw_ratio(st.sw);
+          draws_end = 0;
           if (ar <= 0.45) { st.max_trans *= 0.95; st.max_rot *= 0.95; }
           else if (ar >= 0.55) { st.max_trans *= 1.05; st.max_rot = fmin(pi, 1.05 * st.max_rot); }
         }
         // adaptive torsion steps on the proposal's copy (src/lds.ml:976-979, :603-621):
         // kept only when the proposal was accepted (conf := conf')
         if (accept && flex && !rigid && st.conf_step > 0 && st.conf_step % (kMcBlock * nrb) == 0) {
+          draws_end = 0;
           for (int k = 0; k < nrb; ++k) {
             const double ar = sw_ratio(rsw[k]);
             if (ar <= 0.45) dr[k] = 0.95 * dr[k];
@@ -736,6 +884,11 @@ int mc_inter_kind(const McArgs& a) {
 }
 
 int mc_max_waves(const McArgs& a) { return mc_form_waves(mc_inter_kind(a), a.min_iters > 0); }
+
+hipError_t launch_mc_pairs(const McArgs& a, int nchain, hipStream_t s) {
+  hipLaunchKernelGGL(k_mc_pairs, dim3(nchain), dim3(kWave), 3 * (size_t)a.max_atoms * sizeof(double), s, a);
+  return hipGetLastError();
+}
 
 hipError_t launch_mc(const McArgs& a, int nblocks, int waves, bool rec_lds, hipStream_t s) {
   if (waves < 1 || waves > mc_max_waves(a)) return hipErrorInvalidValue;

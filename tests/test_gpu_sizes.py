@@ -308,3 +308,52 @@ def test_pooled_minimiser(sys0, npose, iters, intra):
     assert np.array_equal(got[0][1], got[1][1], equal_nan=True)
     for k in got[0][2]:
         assert np.array_equal(got[0][2][k], got[1][2][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("mode", ["grid", "direct"])
+@pytest.mark.parametrize("chains,frames", [(1, 9), (40, 130)])
+def test_chains_keep_round_energies(sys0, mode, chains, frames):
+    """Chains that keep the E_intra of every round of 64 pairs and evaluate those a torsion
+    changes follow the chains that evaluate all pairs: ligands without torsions, with no pairs,
+    with less than a round, with one and with several mask words, groups of any atoms; in one
+    run and in pieces, also through a graph.  Kept rounds hold pairs whose atoms turned
+    together since: distances equal to rounding, 12 x 2^-52 of a pair's energy; the energies
+    of these chains in contact agree to 1e-10 relative, the decisions are the same."""
+    from mmo_amd import mc
+    ctx, lig, _ = sys0
+    rng = np.random.default_rng(chains)
+    ligs = [lig] + synth.library(6) + [_chain(n, r, k, rng) for n, r, k in (
+        (1, 0, "nested"), (5, 2, "nested"), (40, 0, "nested"), (64, 6, "facing"),
+        (91, 9, "any"), (100, 12, "nested"))]
+    probe_a, probe_q, types = synth.grid_types(ligs, 10)
+    origin, gdims, gstep = synth.grid_spec((0.0, 0.0, 0.0), 64, 0.375)
+    ctx.compute_grids(probe_a, probe_q, gstep, gdims, origin, copy_out=False)
+    ids = np.array([ctx.add_ligand(l, types=t) for l, t in zip(ligs, types)])
+    pick = np.arange(chains) % len(ligs)
+    rot, pos = synth.random_rotations(rng, chains), rng.uniform(-1, 1, (chains, 3))
+
+    def make():
+        return mc.MonteCarlo(ctx, ids[pick], rot, pos, ff.INTERP if mode == "grid" else ff.SHIFTED,
+                             frames, flags=mc.TWEAK_RBONDS | mc.INTRA_UFF | mc.HARD_ROI,
+                             roi_center=(0.0, 0.0, 0.0), roi_r=8.0, seed=7)
+
+    def run(how):
+        m = make()
+        if how == "pieces":
+            m.run(1)
+            m.run_graph(1, 3)
+            m.run(frames - 4)
+        else:
+            m.run(frames)
+        return m.state()
+    ctx.tune(mc_keep_pairs=0)
+    want = run("whole")
+    ctx.tune(mc_keep_pairs=1)
+    whole, pieces = run("whole"), run("pieces")
+    for k in want:
+        a, b, c = (np.asarray(s[k]) for s in (want, whole, pieces))
+        assert np.array_equal(b, c, equal_nan=a.dtype.kind == "f"), k
+        if a.dtype.kind == "f":
+            np.testing.assert_allclose(b, a, rtol=1e-10, atol=1e-10, err_msg=k)
+        else:
+            assert np.array_equal(a, b), k
