@@ -1195,9 +1195,13 @@ static int plain_inter(mmo_ctx* c, int mode, const double* xs, const double* ys,
   if ((r = plain_setup(c, xs, ys, zs, q, anum, n, true))) return r;
   hipStream_t s = c->stream;
   const bool grad = gx != nullptr;
-  // one pose: split the receptor over block rows so the whole chip works on it
+  // one pose: a wavefront per 64 receptor atoms (the FP32 sums end there anyway), each lane
+  // no more ligand atoms than it must: the serial loop of a lane is the time of the launch.
+  // 75 against 3,000 atoms: slices of 256 and four atoms a lane 73 us, now 16 us
   InterLaunch L = inter_launch(c, mode, c->s_lig.p, c->s_latom.p, nullptr);
-  L.rslice = std::max(64, std::min(c->nrec, 256));
+  L.rslice = 64;
+  if (n <= kWave) L.k = 1;
+  else if (n <= 2 * kWave) L.k = 2;
   L.rtile = std::min(L.rtile, L.rslice);
   L.waves = 1;
   const int nslice = (c->nrec + L.rslice - 1) / L.rslice;

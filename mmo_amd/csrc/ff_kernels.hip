@@ -1092,18 +1092,19 @@ static hipError_t launch_inter_t(const InterArgs<Src>& a, int waves, hipStream_t
   return hipGetLastError();
 }
 
-// sums the gridDim.y partial outputs (slice-major) into out, in slice order
-__global__ void k_reduce_slices(const double* part, int nslice, size_t n, int stride, int ncomp,
-                                double* out) {
+// sums the gridDim.y partial outputs (slice-major) into out, in slice order: ncomp 1: the
+// energy, 3: with its two parts.  Eight slices' loads are in flight at once.
+template <int NCOMP>
+__global__ void k_reduce_slices(const double* part, int nslice, size_t n, int stride, double* out) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x) {
-    for (int c = 0; c < ncomp; ++c) {
-      if (ncomp == 1 && c > 0) break;
-      const int cc = (ncomp == 1) ? 0 : (c == 0 ? 0 : c + 1);   // 0, 2, 3
-      double acc = 0.0;
-      for (int y = 0; y < nslice; ++y) acc += part[(size_t)y * n * stride + i * stride + cc];
-      out[i * stride + cc] = acc;
-    }
+    double acc[NCOMP];
+    for (int c = 0; c < NCOMP; ++c) acc[c] = 0.0;
+    const double* p = part + i * stride;
+#pragma unroll 8
+    for (int y = 0; y < nslice; ++y, p += n * stride)
+      for (int c = 0; c < NCOMP; ++c) acc[c] += p[c == 0 ? 0 : c + 1];   // 0, 2, 3
+    for (int c = 0; c < NCOMP; ++c) out[i * stride + (c == 0 ? 0 : c + 1)] = acc[c];
   }
 }
 
@@ -1148,8 +1149,12 @@ hipError_t launch_inter_coords(const InterLaunch& L, const Tile* tiles, const in
   hipError_t err = launch_inter_any(L.mode, L.k, grad != nullptr, a, L.waves, s);
   if (err != hipSuccess || ny == 1 || (grad && !write_e)) return err;
   const int blocks = std::min(4096, (npose + 255) / 256);
-  hipLaunchKernelGGL(k_reduce_slices, dim3(blocks), dim3(256), 0, s, part, ny, (size_t)npose,
-                     e_stride, comp ? 3 : 1, e_out);
+  if (comp)
+    hipLaunchKernelGGL(k_reduce_slices<3>, dim3(blocks), dim3(256), 0, s, part, ny, (size_t)npose,
+                       e_stride, e_out);
+  else
+    hipLaunchKernelGGL(k_reduce_slices<1>, dim3(blocks), dim3(256), 0, s, part, ny, (size_t)npose,
+                       e_stride, e_out);
   return hipGetLastError();
 }
 

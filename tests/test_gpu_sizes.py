@@ -6,7 +6,7 @@ import pytest
 import oracle
 from mmo_amd import ff, synth
 
-from parity import assert_energy, inter_abs_sum
+from parity import assert_energy, assert_grad, inter_abs_sum
 
 pytestmark = pytest.mark.gpu
 
@@ -357,3 +357,30 @@ def test_chains_keep_round_energies(sys0, mode, chains, frames):
             np.testing.assert_allclose(b, a, rtol=1e-10, atol=1e-10, err_msg=k)
         else:
             assert np.array_equal(a, b), k
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 128, 131])
+@pytest.mark.parametrize("nrec", [1, 63, 64, 65, 577])
+def test_plain_forms_at_slice_edges(n, nrec):
+    """One pose against slices of 64 receptor atoms (one, a full one, one and a remainder, ten)
+    with one, two and four ligand atoms a lane: energy, its parts and gradient in both modes."""
+    _, rec = synth.config0()
+    rng = np.random.default_rng(n + nrec)
+    big = max(synth.library(24), key=lambda l: len(l["xs"]))
+    keep = np.arange(min(n, len(big["xs"])))
+    lig = {k: big[k][keep].copy() for k in ("xs", "ys", "zs", "q", "anum")}
+    at = np.argsort(np.hypot(rec["xs"], rec["ys"]) + np.abs(rec["zs"]))[:nrec]
+    part = {k: np.asarray(rec[k])[at].copy() for k in ("xs", "ys", "zs", "q", "anum")}
+    ctx = ff.Context(0)
+    ctx.set_receptor(part)
+    x = _rows(lig) + rng.uniform(-1, 1, 3)
+    lig.update(xs=x[:, 0].copy(), ys=x[:, 1].copy(), zs=x[:, 2].copy())
+    for mode, shifted in ((ff.SHIFTED, True), (ff.GLOBAL, False)):
+        s = inter_abs_sum(part, x, lig, shifted)
+        e, el, vd = ctx.ene_inter(lig, mode, components=True)
+        want, wel, wvd = oracle.ene_inter(part, lig, shifted=shifted, components=True)
+        assert_energy([e, el, vd], [want, wel, wvd], [s, s, s], what="plain %d x %d" % (n, nrec))
+        eg, g = ctx.ene_inter_grad(lig, mode)
+        ref, gref = oracle.grad_inter(part, lig, shifted=shifted)
+        assert_energy(eg, ref, s, what="plain gradient's energy")
+        assert_grad(g, gref, what="plain gradient %d x %d" % (n, nrec))
