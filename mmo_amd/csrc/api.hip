@@ -415,14 +415,17 @@ std::vector<int> clash_order(const std::vector<double>& xyz, int n) {
 int pair_params(mmo_ctx* c, const std::vector<uint32_t>& pij, const double* q,
                 const int32_t* anum, std::vector<double4>& out) {
   out.resize(pij.size());
+  std::vector<double> A, B;   // per atom, looked up once
   for (size_t p = 0; p < pij.size(); ++p) {
-    const int i = pij[p] & 0xffff, j = pij[p] >> 16;
-    double Ai, Bi, Aj, Bj;
-    int r = atom_ab(c, anum[i], &Ai, &Bi);
-    if (r) return r;
-    r = atom_ab(c, anum[j], &Aj, &Bj);
-    if (r) return r;
-    out[p] = make_double4(kElecWeight * q[i] * q[j], Ai * Aj, 2.0 * Bi * Bj, 0.0);
+    const size_t i = pij[p] & 0xffff, j = pij[p] >> 16;
+    while (A.size() <= std::max(i, j)) {
+      double Ak, Bk;
+      int r = atom_ab(c, anum[A.size()], &Ak, &Bk);
+      if (r) return r;
+      A.push_back(Ak);
+      B.push_back(Bk);
+    }
+    out[p] = make_double4(kElecWeight * q[i] * q[j], A[i] * A[j], 2.0 * B[i] * B[j], 0.0);
   }
   return MMO_OK;
 }
@@ -599,10 +602,10 @@ int sync_mc_pairs(mmo_ctx* c) {
     c->mc_pairs.push_back(mp);
     int r = pair_params(c, h.mc_ij, h.q.data(), h.anum.data(), pp);
     if (r) return r;
-    for (size_t p = 0; p < pp.size(); ++p) {
-      const bool in = p < h.pair_ij.size();   // the last round's filling has no energy
-      qa.push_back(in ? make_double2(pp[p].x, pp[p].y) : make_double2(0.0, 0.0));
-      pb.push_back(in ? pp[p].z : 0.0);
+    for (size_t p = h.pair_ij.size(); p < pp.size(); ++p) pp[p] = make_double4(0.0, 0.0, 0.0, 0.0);
+    for (const double4& v : pp) {
+      qa.push_back(make_double2(v.x, v.y));
+      pb.push_back(v.z);
     }
     ij.insert(ij.end(), h.mc_ij.begin(), h.mc_ij.end());
     mask.insert(mask.end(), h.mc_mask.begin(), h.mc_mask.end());
@@ -1953,6 +1956,8 @@ static int mc_keep_pairs(mmo_mc* m, hipStream_t s) {
   return upload(c, m->d_pe_sel, sel.data(), sel.size(), s);
 }
 
+static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work);
+
 int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double* rot0,
                   const double* pos0, int inter_mode, int flags, const double* roi_center,
                   double roi_r, double temperature, uint64_t seed, int total_frames,
@@ -1988,7 +1993,6 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
   m->chain_lig.assign(chain_lig, chain_lig + nchain);
   m->chain_atom.resize(nchain);
   m->chain_rb.resize(nchain);
-  std::vector<double> conf;
   std::vector<McState> st(nchain);
   const double deg = (4.0 * std::atan(1.0)) / 180.0;   // Math.to_radian
   for (int k = 0; k < nchain; ++k) {
@@ -2013,7 +2017,6 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
     m->natoms += h.n;
     m->nrb += (int)h.rb_left.size();
     m->max_atoms = std::max(m->max_atoms, h.n);
-    conf.insert(conf.end(), h.xyz.begin(), h.xyz.end());
     McState& s0 = st[k];
     std::memset(&s0, 0, sizeof(McState));
     for (int q = 0; q < 9; ++q) s0.rot0[q] = s0.rot[q] = rot0[9 * k + q];
@@ -2064,19 +2067,26 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
       (r = upload(c, m->d_work, m->work.data(), nchain, s)) ||
       (r = upload(c, m->d_work_by_lig, m->work_by_lig.data(), nchain, s)) ||
       (r = upload(c, m->d_st, st.data(), st.size(), s)) ||
-      (r = upload(c, m->d_conf, conf.data(), conf.size(), s)) ||
-      (r = upload(c, m->d_best, conf.data(), conf.size(), s)) ||
-      (r = upload(c, m->d_undo, conf.data(), conf.size(), s)) ||
       (r = upload(c, m->d_dr, dr.data(), dr.size(), s)) ||
       (r = upload(c, m->d_sw, sw.data(), sw.size(), s))) {
     delete m;
     return r;
   }
-  if ((r = mc_keep_pairs(m, s))) {
+  hipError_t e = hipSuccess;
+  for (DevBuf<double>* v : {&m->d_conf, &m->d_best, &m->d_undo})
+    if (e == hipSuccess) e = v->ensure(3 * (size_t)m->natoms);
+  if (e != hipSuccess) {
+    delete m;
+    return fail(c, MMO_ERR_NOMEM, "Monte Carlo conformers: %s", hipGetErrorString(e));
+  }
+  if ((r = sync_ligands(c)) || (r = mc_keep_pairs(m, s))) {
     delete m;
     return r;
   }
-  hipError_t e = m->d_queue.ensure(1);
+  // the registered conformers of every chain, from the registry (uploaded once a chain they
+  // were 22 MB for 6,144 chains: 3 ms of host copies)
+  e = launch_mc_start(mc_args(m, 1, nchain, m->d_work.p), nchain, s);
+  if (e == hipSuccess) e = m->d_queue.ensure(1);
   if (e == hipSuccess) e = mc_prepare();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {

@@ -120,6 +120,8 @@ hipError_t launch_mc(const McArgs& a, int nblocks, int waves, bool rec_lds, hipS
 size_t mc_lds_bytes(const McArgs& a, int waves, bool rec_lds);
 // the chains' kept energies from their conformers (3 max_atoms FP64 of LDS a chain)
 hipError_t launch_mc_pairs(const McArgs& a, int nchain, hipStream_t s);
+// every chain's conformer and best pose = its ligand's registered conformer
+hipError_t launch_mc_start(const McArgs& a, int nchain, hipStream_t s);
 hipError_t mc_prepare();
 
 }  // namespace mmo

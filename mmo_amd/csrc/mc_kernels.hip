@@ -885,6 +885,19 @@ int mc_inter_kind(const McArgs& a) {
 
 int mc_max_waves(const McArgs& a) { return mc_form_waves(mc_inter_kind(a), a.min_iters > 0); }
 
+__global__ void __launch_bounds__(64) k_mc_start(McArgs a) {
+  const int chain = blockIdx.x;
+  const LigInfo li = a.ligs[a.chain_lig[chain]];
+  const double* from = a.lig_xyz + 3 * (size_t)li.atom_base;
+  const size_t to = 3 * (size_t)a.chain_atom[chain];
+  for (int k = threadIdx.x; k < 3 * li.n_atoms; k += blockDim.x) a.conf[to + k] = a.best_xyz[to + k] = from[k];
+}
+
+hipError_t launch_mc_start(const McArgs& a, int nchain, hipStream_t s) {
+  hipLaunchKernelGGL(k_mc_start, dim3(nchain), dim3(kWave), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_mc_pairs(const McArgs& a, int nchain, hipStream_t s) {
   hipLaunchKernelGGL(k_mc_pairs, dim3(nchain), dim3(kWave), 3 * (size_t)a.max_atoms * sizeof(double), s, a);
   return hipGetLastError();
