@@ -184,6 +184,10 @@ int mmo_batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out, d
 int mmo_batch_dof_offsets(const mmo_batch* b, int32_t* dof_off /* npose+1 */);
 int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double* xyz_out,
                              double* e_out, double* gdof, double* radius_out, void* stream);
+/* After it: total[p] = e_out[4 p] + e_out[4 p + 1], or +inf where radius[p] > max_radius
+ * (Mol.Too_long); the gdof (nullable) of those poses becomes 0.  One launch. */
+int mmo_batch_dof_totals_dev(mmo_batch* b, const double* e_out, const double* radius,
+                             double max_radius, double* gdof, double* total, void* stream);
 
 /* --------------------------------------------------------------- rigid scan */
 /* Exhaustive rigid scan (Lds.exhaustive_rigid_ligand_docking, src/lds.ml:1040-1114,

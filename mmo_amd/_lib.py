@@ -49,6 +49,7 @@ SIGNATURES = {
     "mmo_batch_score_dev": (_i, [_p, _i, _p, _p, _p, _p]),
     "mmo_batch_score": (_i, [_p, _i, _p, _p, _p]),
     "mmo_batch_score_dofs_dev": (_i, [_p, _i, _p, _p, _p, _p, _p, _p]),
+    "mmo_batch_dof_totals_dev": (_i, [_p, _p, _p, _d, _p, _p, _p]),
     "mmo_scan_dev": (_i, [_p, _i, _i, _p, _i, _p, _i, _p, _p]),
     "mmo_set_vdw_mask": (_i, [_p, _p, _d, _i, _i, _i, _p]),
     "mmo_get_vdw_mask": (_i, [_p, _p]),

@@ -1811,6 +1811,19 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
   return MMO_OK;
 }
 
+int mmo_batch_dof_totals_dev(mmo_batch* b, const double* e_out, const double* radius,
+                             double max_radius, double* gdof, double* total, void* stream) {
+  if (!b) return fail(nullptr, MMO_ERR_BAD_ARG, "NULL batch");
+  mmo_ctx* c = b->ctx;
+  int r = check_ctx(c);
+  if (r) return r;
+  if (b->npose > 0 && (!e_out || !radius || !total))
+    return fail(c, MMO_ERR_BAD_ARG, "NULL energies, radii or totals");
+  HIPCHK(c, launch_dof_totals(e_out, radius, max_radius, b->d_dof_off.p, b->npose, gdof, total,
+                              (hipStream_t)stream));
+  return MMO_OK;
+}
+
 // ------------------------------------------------------------------ rigid scan
 int mmo_scan_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, int nrot,
                  const double* trans, int ntrans, double* e_out, void* stream) {

@@ -236,6 +236,9 @@ constexpr size_t kMaxLds = 160 * 1024;
 size_t dof_lds_bytes(const DofArgs& a, bool grad);
 hipError_t launch_apply_config(const DofArgs& a, hipStream_t s);
 hipError_t launch_dof_grad(const DofArgs& a, hipStream_t s);
+// total[p] = e[4 p] + e[4 p + 1]; beyond max_radius +inf, and gdof (nullable) 0
+hipError_t launch_dof_totals(const double* e, const double* radius, double max_radius,
+                             const int* dof_off, int npose, double* gdof, double* total, hipStream_t s);
 
 // -------------------------------------------------- rigid-scan filters, top-k
 struct ScanFilterArgs {

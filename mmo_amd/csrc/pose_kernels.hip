@@ -19,6 +19,8 @@
 //   a_bar    = sum_i (z_i x h_i) sin + h_i (a.z_i)(1-cos) + z_i (a.h_i)(1-cos),  z_i = x_i - p
 //   v_bar    = (I - a a^T) a_bar / |v|,  v = x_right - x_left
 //   right_bar += v_bar + p_bar,  left_bar -= v_bar.
+#include <algorithm>
+
 #include "common.h"
 #include "dof.h"
 #include "kernels.h"
@@ -533,6 +535,26 @@ hipError_t launch_dof_grad(const DofArgs& a, hipStream_t s) {
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_dof_grad<false>, dim3(a.npose), dim3(kWave), lds, s, a);
   }
+  return hipGetLastError();
+}
+
+__global__ void __launch_bounds__(256) k_dof_totals(const double* e, const double* radius, double max_radius,
+                                                    const int* dof_off, int npose, double* gdof,
+                                                    double* total) {
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < npose; p += gridDim.x * blockDim.x) {
+    const bool beyond = radius[p] > max_radius;
+    total[p] = beyond ? __builtin_inf() : e[4 * (size_t)p] + e[4 * (size_t)p + 1];
+    if (gdof && beyond)
+      for (int k = dof_off[p]; k < dof_off[p + 1]; ++k) gdof[k] = 0.0;
+  }
+}
+
+hipError_t launch_dof_totals(const double* e, const double* radius, double max_radius,
+                             const int* dof_off, int npose, double* gdof, double* total, hipStream_t s) {
+  if (npose == 0) return hipSuccess;
+  const int blocks = std::min((npose + 255) / 256, 2048);
+  hipLaunchKernelGGL(k_dof_totals, dim3(blocks), dim3(256), 0, s, e, radius, max_radius, dof_off, npose,
+                     gdof, total);
   return hipGetLastError();
 }
 

@@ -424,3 +424,11 @@ class Batch:
         self.ctx._check(lib.mmo_batch_score_dofs_dev(self.h, int(flags), p(dofs), p(xyz_out),
                                                      p(e_out), p(gdof), p(radius),
                                                      _stream_ptr(stream)))
+
+    def dof_totals_dev(self, e, radius, max_radius, total, gdof=None, stream=None):
+        """After score_dofs_dev: total = E_inter + E_intra, +inf (and a zero gradient) where
+        radius > max_radius."""
+        def p(t):
+            return ct.c_void_p(t.data_ptr()) if t is not None else None
+        self.ctx._check(lib.mmo_batch_dof_totals_dev(self.h, p(e), p(radius), float(max_radius),
+                                                     p(gdof), p(total), _stream_ptr(stream)))

@@ -384,3 +384,29 @@ def test_plain_forms_at_slice_edges(n, nrec):
         ref, gref = oracle.grad_inter(part, lig, shifted=shifted)
         assert_energy(eg, ref, s, what="plain gradient's energy")
         assert_grad(g, gref, what="plain gradient %d x %d" % (n, nrec))
+
+
+@pytest.mark.parametrize("npose", [1, 16, 257])
+def test_dof_totals(sys0, npose):
+    """Totals and gradients of poses within and beyond a length limit, with radii equal to it,
+    infinite and NaN, are what the same torch operations give."""
+    import torch
+    ctx, lig, _ = sys0
+    rng = np.random.default_rng(npose)
+    ligs = [lig, _chain(5, 0, "nested", rng), _chain(40, 7, "nested", rng)]
+    b = ctx.batch(np.array([ctx.add_ligand(l) for l in ligs])[np.arange(npose) % 3])
+    dev = torch.device("cuda:0")
+    e = torch.tensor(rng.normal(size=(npose, 4)), device=dev)
+    rad = torch.tensor(rng.choice([3.0, 12.0, np.nextafter(12.0, 13.0), np.inf, np.nan, 40.0], npose), device=dev)
+    g = torch.tensor(rng.normal(size=int(b.dof_off[-1])), device=dev)
+    e[0, 0] = float("nan")
+    pose = torch.repeat_interleave(torch.arange(npose), torch.tensor(np.diff(b.dof_off).astype(np.int64))).to(dev)
+    beyond = rad > 12.0
+    want = torch.where(beyond, torch.full_like(rad, float("inf")), e[:, 0] + e[:, 1])
+    gwant = g.masked_fill(beyond[pose], 0.0)
+    total = torch.empty_like(rad)
+    b.dof_totals_dev(e, rad, 12.0, total)
+    assert torch.equal(total.nan_to_num(7.0, 8.0), want.nan_to_num(7.0, 8.0))
+    total.zero_()
+    b.dof_totals_dev(e, rad, 12.0, total, g)
+    assert torch.equal(total.nan_to_num(7.0, 8.0), want.nan_to_num(7.0, 8.0)) and torch.equal(g, gwant)
