@@ -774,9 +774,9 @@ __global__ void __launch_bounds__(1024) k_grid(GridArgs a, CellGrid cg) {
   const int* s_cell;
   load_receptor<LDS>(a.rpos, a.rab, a.nrec, cg, s_pos, s_ab, s_cell, smem);
   const int lane = threadIdx.x & (kWave - 1);
-  const int brick = blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
-  const int bx = (a.nx + 3) / 4, by = (a.ny + 3) / 4, bz = (a.nz + 3) / 4;
-  if (brick >= bx * by * bz) return;
+  const int brick = a.brick0 + blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
+  const int bx = (a.nx + 3) / 4, by = (a.ny + 3) / 4;
+  if (brick >= a.brick1) return;
   const int ib = brick % bx, jb = (brick / bx) % by, kb = brick / (bx * by);
   const int i = ib * 4 + (lane & 3), j = jb * 4 + ((lane >> 2) & 3), k = kb * 4 + (lane >> 4);
   const bool inside = i < a.nx && j < a.ny && k < a.nz;
@@ -1338,8 +1338,11 @@ hipError_t launch_interp_scan_list(const InterpLaunch& L, int lig, const double*
   return hipGetLastError();
 }
 
-hipError_t launch_grid(const GridArgs& a, const CellGrid& cg, bool in_lds, hipStream_t s) {
-  const int bricks = ((a.nx + 3) / 4) * ((a.ny + 3) / 4) * ((a.nz + 3) / 4);
+hipError_t launch_grid(GridArgs a, const CellGrid& cg, bool in_lds, int kb0, int kb1, hipStream_t s) {
+  const int row = ((a.nx + 3) / 4) * ((a.ny + 3) / 4);
+  a.brick0 = row * kb0;
+  a.brick1 = row * kb1;
+  const int bricks = a.brick1 - a.brick0;
   const int waves = 16;
   const int blocks = (bricks + waves - 1) / waves;
   if (in_lds) {

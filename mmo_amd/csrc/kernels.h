@@ -105,6 +105,7 @@ struct GridArgs {
   int ntypes;
   double max_e;                  // clamp (Params.max_E = 1e5, src/params.ml:26)
   float* out;                    // ntypes * nvox, index i + j nx + k nx ny
+  int brick0, brick1;   // the launch's bricks
 };
 
 struct DofArgs {
@@ -187,7 +188,8 @@ constexpr int kDesolvNodes = 256;
 hipError_t launch_desolv(const DesolvArgs& a, bool pose, hipStream_t s);
 hipError_t launch_fill(double* p, size_t n, double v, hipStream_t s);
 hipError_t launch_fill_int(int* p, size_t n, int v, hipStream_t s);
-hipError_t launch_grid(const GridArgs& a, const CellGrid& cg, bool in_lds, hipStream_t s);
+// the bricks (4^3 nodes) of rows kb0 .. kb1 - 1 in z
+hipError_t launch_grid(GridArgs a, const CellGrid& cg, bool in_lds, int kb0, int kb1, hipStream_t s);
 // one pose per wavefront, shifted form, receptor culled per 8-atom sub-block
 struct PoseCullArgs {
   const double* xyz;        // rows (x, y, z), pose-major
