@@ -1905,7 +1905,7 @@ struct Segment {
 // faults of fresh memory: 84 MB of grids in 8.0 ms.  Here several threads take the segments
 // in pieces, each through a pinned piece of its own, on a stream of the copies: 2.8 ms.
 constexpr int kDrainThreads = 8;
-constexpr size_t kDrainPiece = 1u << 20, kDrainMin = 8u << 20;
+constexpr size_t kDrainPiece = 1u << 20, kDrainMin = 10u << 20;
 
 // what the copies need, kept by the context; false: not to be had
 static bool drain_ready(mmo_ctx* c) {
@@ -2000,8 +2000,12 @@ int mmo_grid_compute(mmo_ctx* c, const int32_t* probe_anum, const double* probe_
   timer_begin(c, "grid", s);
   if (out && bytes >= kDrainMin && drain_ready(c)) {
     // slabs of z, so that the host takes the first while the next are computed: the launches
-    // take 2.1 ms for 128^3 nodes, the whole call 5.1 ms in one slab, 3.7 in four
-    const int nslab = std::min(4, (nz + 3) / 4);
+    // take 2.1 ms for 128^3 nodes, the whole call 5.1 ms in one slab, 3.7 in four.  A slab
+    // has 8 wavefronts (bricks) per SIMD: launches of less take as long as a full one (0.14
+    // ms; 64^3 nodes, 10 MB: four slabs 1.25 ms, one 0.85, the runtime's copy 0.96, and at 60^3
+    // 0.84 against 0.79)
+    const size_t bricks = (size_t)((nx + 3) / 4) * ((ny + 3) / 4) * ((nz + 3) / 4);
+    const int nslab = (int)std::max<size_t>(1, std::min<size_t>({4, bricks / 8192, (size_t)(nz + 3) / 4}));
     std::vector<Segment> segs;
     std::vector<hipEvent_t> ev(nslab, nullptr);
     hipError_t e = hipSuccess;
