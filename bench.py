@@ -239,7 +239,7 @@ def bench_interp(ctx, lig, rots, trans, steps, warmup):
             "grid_precompute_ms": grid_ms, "grid_precompute_wall_s": grid_s,
             "poses_inside_grid": inside, "poses_out_of_grid": npose - inside,
             "gather_GBs": 32.0 * lookups / (avg * 1e-3) / 1e9,
-            "roofline": gather_roofline(32.0 * lookups, avg, "k_interp (scan)",
+            "roofline": gather_roofline(32.0 * lookups, avg, "k_interp_lattice (scan)",
                                         traffic=measured_traffic("k_interp scan"),
                                         algorithmic_TFLOPs=ops / (avg * 1e-3) / 1e12,
                                         executed=executed_tflops("k_interp scan", npose, avg)),
@@ -366,10 +366,10 @@ def bench_egrad(ctx, ligs, ids, rec, poses_per_lig=4, reps=20, cpu=True):
     out = {"batched": n / tb, "per_ligand": n / tp, "speedup": tp / tb, "unit": "poses/s",
            "poses": n, "ligands": len(ids), "ms_batched": tb * 1e3, "ms_per_ligand": tp * 1e3,
            "dtype": "fp32 pairs, fp64 per-pose sums and DOF chain",
-           "roofline": valu_roofline(flop, kernel_ms, "k_pose_cull<grad> (per-atom sweep)",
+           "roofline": valu_roofline(flop, kernel_ms, "k_pose_units<grad> (units of four atoms)",
                                      flop_per_pose=flop / n,
                                      in_cutoff_pairs_per_pose=float(n_in.mean()),
-                                     executed=executed_tflops("k_pose_cull egrad", n, kernel_ms),
+                                     executed=executed_tflops("k_pose_units egrad", n, kernel_ms),
                                      note="the pose kernel of the batched step; the step also "
                                           "runs the DOF chain and the FP64 intra kernels")}
     if cpu:

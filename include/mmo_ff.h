@@ -415,15 +415,18 @@ int mmo_fixed_point_bits(const mmo_ctx* ctx);
  * wavefront; same energies), "scan_lattice" (interpolated scans of translations that form a
  * lattice: 0 the general kernel, 1 the lattice kernel by a rule on sizes, 2 whenever it can),
  * "cell_size" (applies to the next mmo_set_receptor), "mc_waves_per_cu",
- * "pose_waves" (batches: wavefronts per workgroup), "pose_cull" (1: batches in
- * the shifted form run one wavefront per pose with a culled receptor sweep; 0: tiles of
- * poses over the whole receptor), "pose_sweep" (that sweep: 1 lanes over the receptor
- * atoms near each ligand atom, 0 per 8-atom sub-block), "mc_sweep" (the same choice for
+ * "pose_waves" (batches with pose_sweep 0: wavefronts per workgroup), "pose_cull" (1:
+ * batches in the shifted form sweep the receptor near each pose; 0: tiles of
+ * poses over the whole receptor), "pose_sweep" (that sweep: 1 units of four ligand atoms,
+ * lanes over the receptor atoms near them; 0 one wavefront per pose, per 8-atom sub-block), "mc_sweep" (the same choice for
  * the Monte Carlo direct sum), "row_clip" (scan and grid sweeps clip cell rows longer
  * than this many atoms to the cutoff sphere's x chord), "cell_xsub" (the pose and Monte
  * Carlo sweeps use cells up to this many times narrower along x, fewer when the receptor
  * and that cell table would pass 96 KiB; applies to the next mmo_set_receptor),
- * "mc_wg_waves" (Monte Carlo chains per workgroup).  No counterpart in the reference. */
+ * "mc_wg_waves" (Monte Carlo chains per workgroup), "mc_keep_pairs" (1: chains made from
+ * now on keep the E_intra of every 64 pairs and evaluate those a torsion changes; 0: all
+ * pairs), "min_pooled" (minimisers made from now on: workgroups share their poses' sweeps
+ * up to this many poses per CU; 0: never; same results).  No counterpart in the reference. */
 int mmo_tune_set(mmo_ctx* ctx, const char* key, double value);
 double mmo_tune_get(mmo_ctx* ctx, const char* key);
 

@@ -15,7 +15,7 @@ The library exposes its launch shapes as context settings (`Context.tune`):
                           next set_receptor)
   plain batches           inter_k (1, 2, 4, 8), inter_waves (1-4), inter_rtile (receptor
                           atoms per LDS tile)
-  batches (pose culled)   pose_waves (wavefronts per workgroup, 1-16)
+  batches (pose_sweep 0)  pose_waves (wavefronts per workgroup, 1-16)
   Monte Carlo             mc_wg_waves (chains per workgroup, 1-16), mc_waves_per_cu
                           (resident chains per CU, 1-32)
 
