@@ -425,7 +425,8 @@ int mmo_fixed_point_bits(const mmo_ctx* ctx);
  * and that cell table would pass 96 KiB; applies to the next mmo_set_receptor),
  * "mc_wg_waves" (Monte Carlo chains per workgroup), "mc_keep_pairs" (1: chains made from
  * now on keep the E_intra of every 64 pairs and evaluate those a torsion changes; 0: all
- * pairs), "min_pooled" (minimisers made from now on: workgroups share their poses' sweeps
+ * pairs), "mc_pool" (direct chains made from now on: workgroups share their chains' sweeps
+ * up to this many chains per CU; 0: never; same results), "min_pooled" (minimisers made from now on: workgroups share their poses' sweeps
  * up to this many poses per CU; 0: never; same results).  No counterpart in the reference. */
 int mmo_tune_set(mmo_ctx* ctx, const char* key, double value);
 double mmo_tune_get(mmo_ctx* ctx, const char* key);

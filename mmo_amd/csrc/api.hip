@@ -198,6 +198,7 @@ struct mmo_ctx {
   DevBuf<double> d_pe_b;
   DevBuf<uint64_t> d_pe_mask;
   int uff_version = 0;
+  int mc_pool = 12;            // chains per CU up to which workgroups pool their sweeps
   int mc_keep_pairs = 1;       // chains keep their pair energies
   DevBuf<uint64_t> d_intra_bits;   // per atom i, bit d: the pair (i, i + d mod n) counts (free ligands)
   DevBuf<int64_t> d_bit_base;      // per ligand, into d_intra_bits
@@ -270,6 +271,7 @@ struct mmo_mc {
   DevBuf<int64_t> d_pe_off;
   DevBuf<uint64_t> d_pe_sel;
   int pe_words = 0, pe_uff = -1;
+  DevBuf<float4> d_pool;   // pooled sweeps: their units' sums
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   int graph_steps = 0;
@@ -2078,6 +2080,7 @@ static int mc_keep_pairs(mmo_mc* m, hipStream_t s) {
 
 static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work);
 
+static int mc_pool_slots(const mmo_ctx* c, int nwork, int max_atoms);
 int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double* rot0,
                   const double* pos0, int inter_mode, int flags, const double* roi_center,
                   double roi_r, double temperature, uint64_t seed, int total_frames,
@@ -2203,6 +2206,11 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
     delete m;
     return r;
   }
+  // pooled sweeps, where there may be some; without the memory the chains do without
+  if (inter_mode == MMO_SHIFTED && mc_pool_slots(c, nchain, m->max_atoms) > 0 &&
+      m->d_pool.ensure((size_t)mc_pool_slots(c, nchain, m->max_atoms) * c->ncu *
+                       ((m->max_atoms + 3) / 4) * 3 * kWave) != hipSuccess)
+    (void)hipGetLastError();
   // the registered conformers of every chain, from the registry (uploaded once a chain they
   // were 22 MB for 6,144 chains: 3 ms of host copies)
   e = launch_mc_start(mc_args(m, 1, nchain, m->d_work.p), nchain, s);
@@ -2271,7 +2279,19 @@ static int mc_fresh_pairs(mmo_mc* m, hipStream_t s) {
 
 // launch shape: up to 8 chains (wavefronts) per workgroup; in the direct form the
 // workgroup stages the receptor in LDS when it fits next to the conformers
-static hipError_t mc_launch(mmo_mc* m, const McArgs& a, int nwork, hipStream_t s) {
+// Chains per workgroup of the pooled form for nwork chains (0: each wavefront sweeps for its own
+// chain): all of them at once, up to 12 a CU, one workgroup per CU.  3,000 chains (12 a CU) take
+// 12.8 against 15.4 ms a 100 frames; more keep every wavefront busy by themselves (4,096 chains
+// through 8 slots 17.3 against 16.0).  The units' sums (3 KiB per 4 atoms) stay within a bound.
+constexpr size_t kMcPoolBytes = (size_t)384 << 20;
+static int mc_pool_slots(const mmo_ctx* c, int nwork, int max_atoms) {
+  const int slots = (nwork + c->ncu - 1) / c->ncu;
+  if (slots > std::min(c->mc_pool, kMcPoolSlots)) return 0;
+  const size_t bytes = (size_t)slots * c->ncu * ((max_atoms + 3) / 4) * 3 * kWave * sizeof(float4);
+  return bytes <= kMcPoolBytes ? slots : 0;
+}
+
+static hipError_t mc_launch(mmo_mc* m, McArgs a, int nwork, hipStream_t s) {
   int dev = 0, ncu = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -2284,6 +2304,17 @@ static hipError_t mc_launch(mmo_mc* m, const McArgs& a, int nwork, hipStream_t s
     rec_lds = false;
     waves = wmax;
     while (waves > 1 && mc_lds_bytes(a, waves, false) > cap) --waves;
+  }
+  if (rec_lds && mc_can_pool(a) && m->d_pool.n > 0) {
+    a.pool_slots = mc_pool_slots(m->ctx, nwork, m->max_atoms);
+    while (waves > 1 && mc_lds_bytes(a, waves, true) > cap) --waves;
+    const size_t need = (size_t)a.pool_slots * m->ctx->ncu * ((m->max_atoms + 3) / 4) * 3 * kWave;
+    if (a.pool_slots > 0 && waves > a.pool_slots && need <= m->d_pool.n) {
+      a.pool = m->d_pool.p;
+      const int nb = std::min(m->ctx->ncu, (nwork + a.pool_slots - 1) / a.pool_slots);
+      return launch_mc(a, nb, waves, true, s);
+    }
+    a.pool_slots = 0;
   }
   // at least one workgroup per CU; more when the residency setting allows
   const int resident = ncu * std::max(1, m->ctx->mc_waves_per_cu / waves);
@@ -2484,7 +2515,7 @@ void mmo_mc_destroy(mmo_mc* m) {
     m->d_chain_lig.release(); m->d_chain_atom.release(); m->d_chain_rb.release();
     m->d_work.release(); m->d_work_by_lig.release(); m->d_queue.release(); m->d_st.release();
     m->d_conf.release(); m->d_best.release(); m->d_dr.release(); m->d_undo.release(); m->d_sw.release();
-    m->d_pe.release(); m->d_pe_off.release(); m->d_pe_sel.release();
+    m->d_pool.release(); m->d_pe.release(); m->d_pe_off.release(); m->d_pe_sel.release();
     m->d_min_base.release(); m->d_min_S.release(); m->d_min_Y.release(); m->d_min_rho.release();
   }
   delete m;
@@ -3182,6 +3213,7 @@ int mmo_tune_set(mmo_ctx* c, const char* key, double v) {
   else if (k == "scan_lattice" && iv >= 0 && iv <= 2) c->scan_lattice = iv;
   else if (k == "scan_split" && iv >= 0 && iv <= (1 << 20)) c->scan_split = iv;
   else if (k == "grid_pack" && (iv == 0 || iv == 1)) c->grid_pack = iv;
+  else if (k == "mc_pool" && iv >= 0 && iv <= kMcPoolSlots) c->mc_pool = iv;
   else if (k == "mc_keep_pairs" && (iv == 0 || iv == 1)) c->mc_keep_pairs = iv;
   else if (k == "mc_waves_per_cu" && iv >= 1 && iv <= 32) c->mc_waves_per_cu = iv;
   else if (k == "mc_wg_waves" && iv >= 1 && iv <= 16) c->mc_wg_waves = iv;
@@ -3220,6 +3252,7 @@ double mmo_tune_get(mmo_ctx* c, const char* key) {
   if (k == "cell_size") return c->cell_size;
   if (k == "cull_ok") return c->cull_ok ? 1.0 : 0.0;
   if (k == "cullp_ok") return c->cullp_ok ? 1.0 : 0.0;
+  if (k == "mc_pool") return c->mc_pool;
   if (k == "mc_keep_pairs") return c->mc_keep_pairs;
   if (k == "mc_waves_per_cu") return c->mc_waves_per_cu;
   if (k == "mc_wg_waves") return c->mc_wg_waves;

@@ -49,6 +49,9 @@ struct McPairs {
   int rounds, words;         // words of a mask
 };
 
+// chains a workgroup of the pooled form may run
+constexpr int kMcPoolSlots = 12;
+
 struct McArgs {
   // ligands
   const LigInfo* ligs;
@@ -104,6 +107,10 @@ struct McArgs {
   // local minimisation after every proposal (Monte Carlo-plus-minimisation): min_iters
   // L-BFGS evaluations over the proposal's DOFs; per chain the base rows (like conf),
   // history S, Y (min_m slots of 64 lanes) and rho (min_m)
+  // pooled sweeps (pool_slots > 0): chains per workgroup and their units' sums, 3 x 64 float4
+  // per unit, (max_atoms + 3) / 4 units a slot
+  int pool_slots;
+  float4* pool;
   int min_iters, min_m;
   double min_max_step, min_min_step, min_gtol, min_c1;
   double* min_base;
@@ -116,6 +123,8 @@ struct McArgs {
 // the receptor and its cell table to LDS (they must fit next to the conformers)
 // wavefronts per workgroup the Monte Carlo kernel is compiled for (the launch bound)
 int mc_max_waves(const McArgs& a);
+int mc_inter_kind(const McArgs& a);
+bool mc_can_pool(const McArgs& a);
 hipError_t launch_mc(const McArgs& a, int nblocks, int waves, bool rec_lds, hipStream_t s);
 size_t mc_lds_bytes(const McArgs& a, int waves, bool rec_lds);
 // the chains' kept energies from their conformers (3 max_atoms FP64 of LDS a chain)

@@ -373,6 +373,88 @@ __device__ double mc_inter(const McArgs& a, const LigInfo& li, const PoseView& v
   return mc_inter_direct<INTER>(a, li, v, r.pos, r.ab, r.cell, r.wl);
 }
 
+// ---------------------------------------------------------------- pooled sweeps
+// With few chains per CU a chain's frame is one wavefront's sweep after another (96 chains of
+// 26 to 132 atoms: 225,000 of 240,000 cycles a frame) while the CU's other wavefronts have
+// none.  POOL: the first `slots` wavefronts of a workgroup run chains and all of them share the
+// sweeps, a unit of four atoms at a time from an LDS counter, between two barriers a frame.  A
+// unit leaves its FP32 sums per lane in memory (3 KiB) and the chain's wavefront adds them in
+// the atoms' order, as atom_sweep does: every energy keeps its bits.
+// 100 frames in the direct form, 3,000-atom receptor: 5 chains 7.9 -> 2.6 ms, 96 17.0 -> 3.9, 1,000
+// 14.8 -> 6.5, 2,000 14.8 -> 9.7, 3,000 15.4 -> 12.8.
+struct PoolLds {
+  int atoms[kMcPoolSlots], base[kMcPoolSlots];   // of the pose to sweep, 0: none
+  int live[kMcPoolSlots];
+  int next;
+};
+
+// One unit: atoms 4 u .. 4 u + 3 (in the sweep's order) of a pose of n atoms.
+__device__ __forceinline__ void pool_unit(const McArgs& a, const PoseView& v, int n, int atom_base, int u,
+                                          const RecView& rv, float4* out) {
+  constexpr int NA = 4;
+  const int lane = threadIdx.x & (kWave - 1);
+  const Frame& fr = a.fr;
+  const PairK pk = pair_k(fr.inv_s2, fr.inv_s, a.rres);
+  const int j0 = NA * u;
+  LigPt l = lig_pt_zero();
+  int sat = 0;
+  if (lane < NA && j0 + lane < n) {
+    const int ja = a.atom_order ? a.atom_order[atom_base + j0 + lane] : j0 + lane;
+    double x, y, z;
+    v.at(ja, x, y, z);
+    l = lig_pt(x, y, z, fr, &sat);
+  }
+  (void)sat;   // saturated atoms stay beyond the cutoff of every receptor atom
+  LigPt lu[NA];
+  float c1[NA] = {}, fa[NA] = {}, fb[NA] = {};
+  float sq[NA], s12[NA], s6[NA], fe[NA], fx[NA], fy[NA], fz[NA];
+#pragma unroll
+  for (int k = 0; k < NA; ++k) {
+    const int s = j0 + k < n ? k : 0;   // a short last unit repeats its first atom
+    lu[k].x = __builtin_amdgcn_readlane(l.x, s);
+    lu[k].y = __builtin_amdgcn_readlane(l.y, s);
+    lu[k].z = __builtin_amdgcn_readlane(l.z, s);
+    lu[k].rx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.rx), s));
+    lu[k].ry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.ry), s));
+    lu[k].rz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.rz), s));
+  }
+  sweep_pass<false, true, NA, false>(a.cg, rv.cell, rv.pos, rv.ab, fr.inv_s, pk, rv.wl, lu, c1, fa, fb,
+                                     sq, s12, s6, fe, fx, fy, fz);
+  out[lane] = make_float4(sq[0], sq[1], sq[2], sq[3]);
+  out[kWave + lane] = make_float4(s12[0], s12[1], s12[2], s12[3]);
+  out[2 * kWave + lane] = make_float4(s6[0], s6[1], s6[2], s6[3]);
+}
+
+// The pose's energy from its units, in atom_sweep's order.
+__device__ __forceinline__ double pool_energy(const McArgs& a, const LigInfo& li, const float4* units) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double e_el = 0.0, e_vd = 0.0;
+  for (int jb = 0; jb < li.n_atoms; jb += kWave) {
+    double mq = 0.0, ma = 0.0, mb = 0.0;
+    if (jb + lane < li.n_atoms) {
+      const int ja = a.atom_order ? a.atom_order[li.atom_base + jb + lane] : jb + lane;
+      const LigAtom la = a.latoms[li.atom_base + ja];
+      mq = la.keq; ma = la.a; mb = la.b;
+    }
+    const int nj = min(kWave, li.n_atoms - jb);
+    const float4* p = units + (size_t)(jb / 4) * 3 * kWave + lane;
+#pragma unroll 2
+    for (int jj = 0; jj < nj; jj += 4, p += 3 * kWave) {
+      const float4 q = p[0], t12 = p[kWave], t6 = p[2 * kWave];
+      const float sq[4] = {q.x, q.y, q.z, q.w}, s12[4] = {t12.x, t12.y, t12.z, t12.w},
+                  s6[4] = {t6.x, t6.y, t6.z, t6.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (jj + u >= nj) break;
+        e_el = fma((double)sq[u], readlane_d(mq, jj + u), e_el);
+        e_vd = fma((double)s12[u], readlane_d(ma, jj + u), e_vd);
+        e_vd = fma(-2.0 * (double)s6[u], readlane_d(mb, jj + u), e_vd);
+      }
+    }
+  }
+  return wave_sum(e_el + e_vd);
+}
+
 // ------------------------------------------------- Monte Carlo-plus-minimisation
 // LDS of one chain's minimiser (after the chain slots): the minimised conformer and the
 // adjoint, 6 x max_atoms FP64
@@ -448,7 +530,7 @@ __device__ double mc_minimize(const McArgs& a, const LigInfo& li, int chain, boo
 // (15.4 M against 14.2 M steps/s) and for the grid form (225 M against 203 M).
 __host__ __device__ constexpr int mc_form_waves(int, bool min) { return min ? 8 : 16; }
 
-template <bool REC_LDS, int INTER, bool MIN>
+template <bool REC_LDS, int INTER, bool MIN, bool POOL = false>
 __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a, int rec_bytes) {
   extern __shared__ __align__(16) char mc_lds[];
   RecView rv;
@@ -477,12 +559,61 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
   }
   const double pi = 3.14159265358979311600;       // 4 atan 1 (src/math.ml:13)
 
-  for (;;) {
+  // POOL: shared by the workgroup; a round = the units of every published pose.  False once no
+  // wavefront runs a chain: the same for all of them, and the last time any of them asks.
+  PoolLds& pl = *reinterpret_cast<PoolLds*>(
+      reinterpret_cast<int*>(reinterpret_cast<McPose*>(s_st + nwv) + nwv) + nwv * kAtomSweepInts);
+  const size_t pool_units = (a.max_atoms + 3) / 4;
+  float4* const pool = POOL ? a.pool + (size_t)blockIdx.x * a.pool_slots * pool_units * 3 * kWave : nullptr;
+  auto pool_round = [&]() __attribute__((always_inline)) {
+    if (threadIdx.x == 0) pl.next = 0;
+    __syncthreads();
+    int any = 0;
+    for (int k = 0; k < a.pool_slots; ++k) any |= pl.live[k];
+    if (!__builtin_amdgcn_readfirstlane(any)) return false;
+    for (;;) {
+      int u = 0;
+      if (lane == 0) u = atomicAdd(&pl.next, 1);
+      u = __builtin_amdgcn_readlane(u, 0);
+      int sl = 0, n = 0;
+      for (; sl < a.pool_slots; ++sl) {
+        n = __builtin_amdgcn_readfirstlane(pl.atoms[sl]);
+        if (u < (n + 3) / 4) break;
+        u -= (n + 3) / 4;
+      }
+      if (sl == a.pool_slots) break;
+      const double* c = reinterpret_cast<const double*>(mc_lds + rec_bytes) + (size_t)sl * 3 * a.max_atoms;
+      const PoseView v{c, c + a.max_atoms, c + 2 * a.max_atoms, reinterpret_cast<McPose*>(s_st + nwv) + sl};
+      pool_unit(a, v, n, __builtin_amdgcn_readfirstlane(pl.base[sl]), u, rv,
+                pool + ((size_t)sl * pool_units + u) * 3 * kWave);
+    }
+    __syncthreads();
+    return true;
+  };
+  auto inter = [&](const LigInfo& li, const PoseView& v) __attribute__((always_inline)) {
+    if constexpr (!POOL) {
+      return mc_inter<INTER>(a, li, v, rv);
+    } else {
+      if (lane == 0) { pl.atoms[wv] = li.n_atoms; pl.base[wv] = li.atom_base; }
+      (void)pool_round();
+      return pool_energy(a, li, pool + (size_t)wv * pool_units * 3 * kWave);
+    }
+  };
+  bool first = true;   // POOL: the first chains are dealt, to and fro over the workgroups
+  const bool keeper = !POOL || wv < a.pool_slots;
+  if (POOL && keeper && lane == 0) pl.live[wv] = 1;
+
+  for (; keeper;) {
     // the next chain: lane 0 takes it from the queue; readlane makes it a scalar, so the
     // loop exit is uniform
     int qv = 0;
-    if (lane == 0) qv = atomicAdd(a.queue, 1);
-    const int q = __builtin_amdgcn_readlane(qv, 0);
+    if (lane == 0 && !(POOL && first)) qv = atomicAdd(a.queue, 1);
+    int q = __builtin_amdgcn_readlane(qv, 0);
+    if (POOL) {
+      const int nb = gridDim.x, b = blockIdx.x, w = __builtin_amdgcn_readfirstlane(wv);
+      q = first ? w * nb + ((w & 1) ? nb - 1 - b : b) : a.pool_slots * nb + q;
+      first = false;
+    }
     if (q >= a.nwork) break;
     const int chain = a.work[q];
     // the chain's state in this wavefront's LDS slot (wave-uniform values)
@@ -536,7 +667,7 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
       const PoseView v{cx_, cy_, cz_, pose};
       st.prev_e_intra = mp.rounds ? mc_intra_table(a, mp, pe, sel, nullptr, cx_, cy_, cz_)
                         : use_intra ? mc_intra(a, li, cx_, cy_, cz_) : 0.0;
-      st.prev_e_inter = mc_inter<INTER>(a, li, v, rv);
+      st.prev_e_inter = inter(li, v);
       st.prev_e = st.prev_e_inter + st.prev_e_intra;
       st.best_e = st.prev_e;
       for (int k = 0; k < 9; ++k) { st.rot[k] = st.rot0[k]; st.best_rot[k] = st.rot0[k]; }
@@ -690,7 +821,7 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
         if (!rigid && use_intra && flex)
           st.prev_e_intra = mp.rounds ? mc_intra_table(a, mp, pe, sel, mask, sx, sy, sz)
                                       : mc_intra(a, li, sx, sy, sz);
-        st.prev_e_inter = mc_inter<INTER>(a, li, v, rv);
+        st.prev_e_inter = inter(li, v);
         curr_e = st.prev_e_inter + st.prev_e_intra;
       }
       asm volatile("" ::: "memory");
@@ -834,6 +965,11 @@ __global__ void __launch_bounds__(mc_form_waves(INTER, MIN) * 64) k_mc(McArgs a,
     }
     wave_sync();
   }
+  if constexpr (POOL) {
+    if (keeper && lane == 0) { pl.live[wv] = 0; pl.atoms[wv] = 0; }
+    while (pool_round()) {
+    }
+  }
 }
 
 __global__ void k_mc_reset_queue(int* q) {
@@ -848,7 +984,7 @@ size_t mc_lds_bytes(const McArgs& a, int waves, bool rec_lds) {
   const size_t conf = ((size_t)waves * 3 * a.max_atoms * sizeof(double) + 15) & ~(size_t)15;
   const size_t mins = a.min_iters > 0 ? (size_t)waves * 6 * a.max_atoms * sizeof(double) : 0;
   return rec + conf + (size_t)waves * (sizeof(McState) + sizeof(McPose) + kAtomSweepInts * sizeof(int)) +
-         mins;
+         mins + (a.pool_slots > 0 ? (sizeof(PoolLds) + 15) & ~(size_t)15 : 0);
 }
 
 template <bool R, int I>
@@ -873,6 +1009,9 @@ hipError_t mc_prepare() {
   if (e == hipSuccess) e = mc_allow_lds<false, kMcInterSub>(cap);
   if (e == hipSuccess) e = mc_allow_lds<false, kMcInterF64>(cap);
   if (e == hipSuccess) e = mc_allow_lds<false, kMcInterGrid>(cap);
+  if (e == hipSuccess)
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mc<true, kMcInterAtom, false, true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, cap);
   return e;
 }
 
@@ -882,6 +1021,8 @@ int mc_inter_kind(const McArgs& a) {
   // the minimiser's gradients come from the per-atom sweep
   return (a.sweep == 1 || a.min_iters > 0) ? kMcInterAtom : kMcInterSub;
 }
+
+bool mc_can_pool(const McArgs& a) { return mc_inter_kind(a) == kMcInterAtom && a.min_iters == 0; }
 
 int mc_max_waves(const McArgs& a) { return mc_form_waves(mc_inter_kind(a), a.min_iters > 0); }
 
@@ -913,7 +1054,10 @@ hipError_t launch_mc(const McArgs& a, int nblocks, int waves, bool rec_lds, hipS
   const dim3 g(nblocks), b(waves * kWave);
   const int key = mc_inter_kind(a) + (rec_lds ? 8 : 0) + (a.min_iters > 0 ? 16 : 0);
   switch (key) {
-    case kMcInterAtom + 8: hipLaunchKernelGGL((k_mc<true, kMcInterAtom, false>), g, b, lds, s, a, rec_bytes); break;
+    case kMcInterAtom + 8:
+      if (a.pool_slots > 0) hipLaunchKernelGGL((k_mc<true, kMcInterAtom, false, true>), g, b, lds, s, a, rec_bytes);
+      else hipLaunchKernelGGL((k_mc<true, kMcInterAtom, false>), g, b, lds, s, a, rec_bytes);
+      break;
     case kMcInterSub + 8: hipLaunchKernelGGL((k_mc<true, kMcInterSub, false>), g, b, lds, s, a, rec_bytes); break;
     case kMcInterF64 + 8: hipLaunchKernelGGL((k_mc<true, kMcInterF64, false>), g, b, lds, s, a, rec_bytes); break;
     case kMcInterAtom: hipLaunchKernelGGL((k_mc<false, kMcInterAtom, false>), g, b, lds, s, a, 0); break;

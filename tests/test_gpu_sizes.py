@@ -432,3 +432,41 @@ def test_large_grids_reach_the_host_whole(sys0, dims, ntypes):
         one = ctx.compute_grids(anum[t:t + 1], q[t:t + 1], step, (dims[0], dims[1], cut), origin, **kw)
         assert one.nbytes < 10 << 20
         assert np.array_equal(one[0], whole[t][:cut]) and np.any(one != 0)
+
+
+@pytest.mark.parametrize("chains,frames", [(1, 7), (257, 40), (1100, 6), (3072, 4)])
+def test_pooled_chains(sys0, chains, frames):
+    """Direct chains whose workgroups pool their sweeps (one to twelve chains a CU) have the
+    states of chains that each sweep alone, bit for bit, in one run, in pieces, through a graph
+    and one launch per ligand: ligands of 1, 4, 5, 64, 65 atoms and the library's, chains that
+    leave the region, chains that end too long."""
+    from mmo_amd import mc
+    ctx, lig, _ = sys0
+    rng = np.random.default_rng(chains)
+    long = _chain(18, 6, "nested", rng)
+    ligs = [lig] + synth.library(4) + [_chain(n, min(n - 1, 2) if n > 4 else 0, "nested", rng)
+                                       for n in (1, 4, 5, 64, 65)] + [long]
+    ids = np.array([ctx.add_ligand(l) for l in ligs])
+    pick = rng.integers(0, len(ligs), chains)
+    rot, pos = synth.random_rotations(rng, chains), rng.uniform(-6, 6, (chains, 3))
+    got = []
+    for pool, how in ((0, "run"), (12, "run"), (12, "pieces"), (12, "ligand")):
+        ctx.tune(mc_pool=pool)
+        m = mc.MonteCarlo(ctx, ids[pick], rot, pos, ff.SHIFTED, frames,
+                          flags=mc.TWEAK_RBONDS | mc.INTRA_UFF | mc.HARD_ROI,
+                          roi_center=(0.0, 0.0, 0.0), roi_r=7.0, seed=11)
+        if how == "run":
+            m.run(frames)
+        elif how == "ligand":
+            m.run_per_ligand(frames)
+        else:
+            m.run(1)
+            m.run_graph(1, 2)
+            m.run(frames - 3)
+        got.append((m.state(), m.coords()))
+    ctx.tune(mc_pool=12)
+    for st, xyz in got[1:]:
+        for k, v in got[0][0].items():
+            a, b = np.asarray(v), np.asarray(st[k])
+            assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f"), k
+        assert all(np.array_equal(x, y) for x, y in zip(got[0][1][1], xyz[1]))
