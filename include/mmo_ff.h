@@ -167,7 +167,8 @@ enum {
  * grad: device FP64 (n_atoms_total x 3) or NULL.  Out-of-grid poses (INTERP) get
  * NaN in e_out[p*4+0].  GLOBAL sums atoms anywhere (those outside the fixed-point
  * window, ~64 A from the receptor centre, through FP64 pairs); non-finite atoms give
- * NaN. */
+ * NaN.  Calls on one batch with buffers of their own may run on several streams at once,
+ * and in captured graphs, but for those with MMO_F_INTER_GLOBAL, which share the batch's. */
 int mmo_batch_score_dev(mmo_batch* b, int flags, const double* xyz, double* e_out,
                         double* grad, void* stream);
 /* Host-pointer variant (copies in and out; synchronous). */
@@ -180,7 +181,9 @@ int mmo_batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out, d
  * Writes coordinates to xyz_out (n_atoms_total x 3, nullable), energies to e_out,
  * and with MMO_F_GRAD dE/dDOF to gdof (same layout as dofs).  radius_out (nullable,
  * npose) gets the enclosing radius after the torsions (Mol.check_elongation_exn uses
- * > 12 A as Too_long, src/optim.ml:75).  All pointers are device pointers. */
+ * > 12 A as Too_long, src/optim.ml:75).  All pointers are device pointers.  Calls with
+ * MMO_F_GRAD, and those without xyz_out, keep coordinates in the batch: on one batch the
+ * caller orders them. */
 int mmo_batch_dof_offsets(const mmo_batch* b, int32_t* dof_off /* npose+1 */);
 int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double* xyz_out,
                              double* e_out, double* gdof, double* radius_out, void* stream);

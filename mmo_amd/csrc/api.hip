@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <system_error>
@@ -95,6 +96,21 @@ struct DevBuf {
     n = 0;
   }
 };
+
+// an event that several objects hold; left alone in a forked child, as all device state
+using Event = std::shared_ptr<std::remove_pointer<hipEvent_t>::type>;
+hipError_t make_event(Event& ev) {
+  hipEvent_t e = nullptr;
+  const hipError_t err = hipEventCreate(&e);
+  const pid_t pid = getpid();
+  if (err == hipSuccess)
+    ev = Event(e, [pid](hipEvent_t v) {
+      if (getpid() == pid) (void)hipEventDestroy(v);
+    });
+  return err;
+}
+// the events around the last launch of a kernel family: `last` is `own`, or its caller's
+struct Timer { Event first, own, last; };
 
 // ligands the adjoint without a serial pass takes: a bound on the host's check, and on the
 // n^2 bits of interacting pairs (above, a pose does not fit in LDS with its E_intra)
@@ -248,7 +264,7 @@ struct mmo_ctx {
   bool drain_failed = false;
   // tuning
   int inter_k = 4, inter_waves = 4, inter_rtile = 2048;
-  std::map<std::string, std::pair<hipEvent_t, hipEvent_t>> ev;
+  std::map<std::string, Timer> ev;
   std::map<std::string, float> last_ms;   // -2: pending
 };
 
@@ -282,6 +298,15 @@ struct mmo_mc {
   DevBuf<double> d_min_base, d_min_S, d_min_Y, d_min_rho;
 };
 
+// Room for the unit energies of one call on a batch (take_unit_sums).
+struct UnitSums {
+  DevBuf<double> part;          // 2 per unit
+  hipStream_t stream = nullptr;
+  bool used = false, captured = false;
+  unsigned long long capture = 0;   // captured: the capture's id
+  Event done;                   // after the last call's reader (not captured)
+};
+
 struct mmo_batch {
   mmo_ctx* ctx = nullptr;
   int device = 0;      // the context's, kept so that destruction never reads the context
@@ -299,6 +324,7 @@ struct mmo_batch {
   int nunits = 0;
   DevBuf<UnitAtom> d_units;
   DevBuf<int> d_unit_off;
+  std::vector<std::unique_ptr<UnitSums>> sums;
   DevBuf<Tile> d_tiles;
   DevBuf<double> d_xyz, d_e, d_g, d_part, d_conf;
 };
@@ -693,11 +719,14 @@ void plan_tiles(const std::vector<int>& pose_lig, const std::vector<LigHost>* li
 
 // HIP events bracketing the last launch of each kernel family, on its stream
 void timer_begin(mmo_ctx* c, const char* name, hipStream_t s) {
-  (void)hipEventRecord(c->ev[name].first, s);
+  (void)hipEventRecord(c->ev[name].first.get(), s);
 }
-void timer_end(mmo_ctx* c, const char* name, hipStream_t s) {
-  (void)hipEventRecord(c->ev[name].second, s);
+// done: an event of the caller's to record instead of the timer's own
+hipError_t timer_end(mmo_ctx* c, const char* name, hipStream_t s, const Event& done = nullptr) {
+  Timer& t = c->ev[name];
+  t.last = done ? done : t.own;
   c->last_ms[name] = -2.0f;   // resolved by mmo_last_kernel_ms
+  return hipEventRecord(t.last.get(), s);
 }
 
 // plain one-ligand helper: uploads coordinates and a one-entry ligand table
@@ -908,12 +937,12 @@ int mmo_ctx_create(int device, mmo_ctx** out) {
     return fail(nullptr, MMO_ERR_DEVICE, "stream creation failed");
   }
   for (const char* k : {"inter", "interp", "intra", "grid", "mc", "min"}) {
-    hipEvent_t a = nullptr, b = nullptr;
-    if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) {
+    Timer& t = c->ev[k];
+    if (make_event(t.first) != hipSuccess || make_event(t.own) != hipSuccess) {
       delete c;
       return fail(nullptr, MMO_ERR_DEVICE, "event creation failed");
     }
-    c->ev[k] = {a, b};
+    t.last = t.own;
   }
   *out = c;
   return MMO_OK;
@@ -940,10 +969,6 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     c->s_tk.release(); c->s_keep.release(); c->d_mask_cells.release();
     c->s_list.release(); c->s_nkept.release(); c->d_desolv.release(); c->d_rec64.release();
     c->s_dvox.release(); c->s_datoms.release(); c->s_dpart.release();
-    for (auto& kv : c->ev) {
-      (void)hipEventDestroy(kv.second.first);
-      (void)hipEventDestroy(kv.second.second);
-    }
     (void)hipStreamDestroy(c->stream);
   }
   delete c;
@@ -1487,6 +1512,63 @@ static int deal_batch(mmo_batch* b, int waves, hipStream_t s) {
   return MMO_OK;
 }
 
+// Unit energies lie between the kernel that makes them and the one that adds them up, so every
+// call in flight has its own: a buffer per stream, for up to kUnitStreams streams; those beyond
+// take the one used longest ago, after its reader (the event that ends the call's timer: one
+// of its own would be 4 us a call).  A capture's calls keep their buffers (one per stream of
+// the capture) until the batch goes, since its graph may run at any time.  The first buffer
+// comes with the batch: a first call, also a captured one, allocates nothing.
+constexpr size_t kUnitStreams = 4;
+
+static int add_unit_sums(mmo_batch* b) {
+  std::unique_ptr<UnitSums> u(new UnitSums());
+  HIPCHK(b->ctx, u->part.ensure(2 * (size_t)b->nunits));
+  const hipError_t e = make_event(u->done);
+  if (e != hipSuccess) u->part.release();
+  HIPCHK(b->ctx, e);
+  b->sums.push_back(std::move(u));
+  return MMO_OK;
+}
+
+// the buffer of a call on stream s, whose reader the caller follows with a record of `done`
+static int take_unit_sums(mmo_batch* b, hipStream_t s, UnitSums** out) {
+  mmo_ctx* c = b->ctx;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(s, &status, &id) != hipSuccess) (void)hipGetLastError();
+  const bool captured = status == hipStreamCaptureStatusActive;
+  UnitSums *mine = nullptr, *fresh = nullptr, *oldest = nullptr;
+  size_t streams = 0;
+  for (auto& u : b->sums) {   // the longest unused first
+    if (!u->used) fresh = u.get();
+    else if (u->captured == captured && u->stream == s && (!captured || u->capture == id)) mine = u.get();
+    else if (!u->captured && !oldest) oldest = u.get();
+    streams += u->used && !u->captured;
+  }
+  if (!mine && !fresh && (captured || streams < kUnitStreams)) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // allocation within a capture
+    if (captured) HIPCHK(c, hipThreadExchangeStreamCaptureMode(&mode));
+    const int r = add_unit_sums(b);
+    if (captured) HIPCHK(c, hipThreadExchangeStreamCaptureMode(&mode));
+    if (r == MMO_OK) fresh = b->sums.back().get();
+    else if (captured || !oldest) return r;
+    else (void)hipGetLastError();
+  }
+  UnitSums* u = mine ? mine : fresh ? fresh : oldest;
+  // (also on one stream: its handle may have passed to another since)
+  if (u->used && !u->captured) HIPCHK(c, hipStreamWaitEvent(s, u->done.get(), 0));
+  u->used = true;
+  u->captured = captured;
+  u->capture = id;
+  u->stream = s;
+  if (!captured) {
+    auto at = std::find_if(b->sums.begin(), b->sums.end(), [&](const auto& v) { return v.get() == u; });
+    std::rotate(at, at + 1, b->sums.end());
+  }
+  *out = u;
+  return MMO_OK;
+}
+
 int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch** out) {
   int r = check_ctx(c);
   if (r) return r;
@@ -1547,7 +1629,7 @@ int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch**
     b->nunits = unit_off[npose];
   }
   hipStream_t s = c->stream;
-  if ((r = upload(c, b->d_units, units.data(), units.size(), s)) ||
+  if ((r = add_unit_sums(b)) || (r = upload(c, b->d_units, units.data(), units.size(), s)) ||
       (r = upload(c, b->d_unit_off, unit_off.data(), unit_off.size(), s)) ||
       (r = upload(c, b->d_pose_lig, b->pose_lig.data(), npose, s)) ||
       (r = upload(c, b->d_atom_off, b->atom_off.data(), npose + 1, s)) ||
@@ -1573,6 +1655,7 @@ void mmo_batch_destroy(mmo_batch* b) {
     b->d_pose_lig.release(); b->d_atom_off.release(); b->d_dof_off.release(); b->d_perm.release();
     b->d_order.release(); b->d_by_size.release();
     b->d_units.release(); b->d_unit_off.release();
+    for (auto& u : b->sums) u->part.release();
     b->d_tiles.release(); b->d_xyz.release(); b->d_e.release(); b->d_g.release(); b->d_part.release();
     b->d_conf.release();
   }
@@ -1593,9 +1676,9 @@ int mmo_batch_dof_offsets(const mmo_batch* b, int32_t* off) {
   return MMO_OK;
 }
 
-// sum_later: the caller adds up the units' energies (b->d_part) of a shifted gradient itself
+// later: room for the units' energies of a shifted gradient, which the caller adds up itself
 static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out, double* grad,
-                       hipStream_t s, bool sum_later = false) {
+                       hipStream_t s, double* later = nullptr) {
   mmo_ctx* c = b->ctx;
   const int inter = flags & (MMO_F_INTER_SHIFTED | MMO_F_INTER_GLOBAL | MMO_F_INTER_INTERP);
   if (inter && (inter & (inter - 1)))
@@ -1625,8 +1708,9 @@ static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out
     PoseUnitArgs a{};
     a.xyz = xyz; a.units = b->d_units.p; a.nunits = b->nunits; a.latoms = c->d_latoms.p;
     a.rres = c->rres.p;
-    HIPCHK(c, b->d_part.ensure(2 * (size_t)b->nunits));
-    a.part = b->d_part.p;
+    UnitSums* sums = nullptr;
+    if (!later && (r = take_unit_sums(b, s, &sums))) return r;
+    a.part = later ? later : sums->part.p;
     timer_begin(c, "inter", s);
     if (!want_grad || comp) {
       a.pairs = comp ? 1 : 0;
@@ -1637,10 +1721,11 @@ static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out
       a.grad = grad;
       if (comp) a.part = nullptr;   // the energies are written
       HIPCHK(c, launch_pose_units(L, a, true, c->ncu, s));
-      if (!comp && !sum_later)
+      if (!comp && !later)
         HIPCHK(c, launch_pose_sum(a.part, b->d_unit_off.p, b->npose, false, false, e_out, s));
     }
-    timer_end(c, "inter", s);
+    const hipError_t e = timer_end(c, "inter", s, sums ? sums->done : nullptr);
+    if (sums) HIPCHK(c, e);
   } else if (pose_first) {
     // one wavefront per pose over the culled receptor, 8-atom sub-blocks
     InterLaunch L = inter_launch(c, MMO_SHIFTED, c->d_ligs.p, c->d_latoms.p, c->d_lig_xyz.p);
@@ -1806,7 +1891,9 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
       }
     }
     const bool sum_later = g && (score_flags & MMO_F_INTER_SHIFTED) && c->pose_cull && c->pose_sweep == 1;
-    if ((r = batch_score(b, bflags, xyz, e_out, gx, s, sum_later))) return r;
+    // these calls share the batch's conformers and gradient, so they share the units' energies
+    if (sum_later) HIPCHK(c, b->d_part.ensure((size_t)b->nunits));
+    if ((r = batch_score(b, bflags, xyz, e_out, gx, s, sum_later ? b->d_part.p : nullptr))) return r;
     if (g) {
       if (sum_later) {
         a.part = b->d_part.p; a.unit_off = b->d_unit_off.p; a.e_sum = e_out;
@@ -3178,10 +3265,10 @@ double mmo_last_kernel_ms(mmo_ctx* c, const char* kernel) {
   auto it = c->last_ms.find(kernel);
   if (it == c->last_ms.end()) return -1.0;
   if (it->second == -2.0f) {
-    auto& e = c->ev[kernel];
-    if (hipEventSynchronize(e.second) != hipSuccess) return -1.0;
+    const Timer& t = c->ev[kernel];
+    if (hipEventSynchronize(t.last.get()) != hipSuccess) return -1.0;
     float ms = -1.0f;
-    if (hipEventElapsedTime(&ms, e.first, e.second) != hipSuccess) return -1.0;
+    if (hipEventElapsedTime(&ms, t.first.get(), t.last.get()) != hipSuccess) return -1.0;
     it->second = ms;
   }
   return it->second;
