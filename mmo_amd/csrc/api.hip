@@ -15,6 +15,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <system_error>
 #include <thread>
@@ -302,9 +303,9 @@ struct mmo_mc {
 struct UnitSums {
   DevBuf<double> part;          // 2 per unit
   hipStream_t stream = nullptr;
-  bool used = false, captured = false;
-  unsigned long long capture = 0;   // captured: the capture's id
-  Event done;                   // after the last call's reader (not captured)
+  bool used = false;
+  std::optional<unsigned long long> capture;   // a capture's: its id
+  Event done;                   // after the last call's reader (not a capture's)
 };
 
 struct mmo_batch {
@@ -369,6 +370,15 @@ int atom_ab(mmo_ctx* c, int anum, double* A, double* B) {
   *A = sd * x3 * x3;
   *B = sd * x3;
   return MMO_OK;
+}
+
+// the id of the capture that stream s is part of, if it is being captured
+std::optional<unsigned long long> capture_id(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(s, &status, &id) != hipSuccess) (void)hipGetLastError();
+  if (status != hipStreamCaptureStatusActive) return std::nullopt;
+  return id;
 }
 
 template <class T>
@@ -1533,17 +1543,15 @@ static int add_unit_sums(mmo_batch* b) {
 // the buffer of a call on stream s, whose reader the caller follows with a record of `done`
 static int take_unit_sums(mmo_batch* b, hipStream_t s, UnitSums** out) {
   mmo_ctx* c = b->ctx;
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  unsigned long long id = 0;
-  if (hipStreamGetCaptureInfo(s, &status, &id) != hipSuccess) (void)hipGetLastError();
-  const bool captured = status == hipStreamCaptureStatusActive;
+  const std::optional<unsigned long long> id = capture_id(s);
+  const bool captured = id.has_value();
   UnitSums *mine = nullptr, *fresh = nullptr, *oldest = nullptr;
   size_t streams = 0;
   for (auto& u : b->sums) {   // the longest unused first
     if (!u->used) fresh = u.get();
-    else if (u->captured == captured && u->stream == s && (!captured || u->capture == id)) mine = u.get();
-    else if (!u->captured && !oldest) oldest = u.get();
-    streams += u->used && !u->captured;
+    else if (u->stream == s && u->capture == id) mine = u.get();
+    else if (!u->capture && !oldest) oldest = u.get();
+    streams += u->used && !u->capture;
   }
   if (!mine && !fresh && (captured || streams < kUnitStreams)) {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // allocation within a capture
@@ -1556,9 +1564,8 @@ static int take_unit_sums(mmo_batch* b, hipStream_t s, UnitSums** out) {
   }
   UnitSums* u = mine ? mine : fresh ? fresh : oldest;
   // (also on one stream: its handle may have passed to another since)
-  if (u->used && !u->captured) HIPCHK(c, hipStreamWaitEvent(s, u->done.get(), 0));
+  if (u->used && !u->capture) HIPCHK(c, hipStreamWaitEvent(s, u->done.get(), 0));
   u->used = true;
-  u->captured = captured;
   u->capture = id;
   u->stream = s;
   if (!captured) {
@@ -2301,6 +2308,10 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
   // the registered conformers of every chain, from the registry (uploaded once a chain they
   // were 22 MB for 6,144 chains: 3 ms of host copies)
   e = launch_mc_start(mc_args(m, 1, nchain, m->d_work.p), nchain, s);
+  if (e == hipSuccess && m->pe_words > 0) {
+    e = launch_mc_pairs(mc_args(m, 1, nchain, m->d_work.p), nchain, s);
+    m->pe_uff = c->uff_version;
+  }
   if (e == hipSuccess) e = m->d_queue.ensure(1);
   if (e == hipSuccess) e = mc_prepare();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -2311,10 +2322,6 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
   *out = m;
   return MMO_OK;
 }
-
-// before a run on stream s: the lists of this registry, and the energies of new chains or
-// changed parameters
-static int mc_fresh_pairs(mmo_mc* m, hipStream_t s);
 
 static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work) {
   mmo_ctx* c = m->ctx;
@@ -2349,6 +2356,8 @@ static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work) {
   return a;
 }
 
+// before a run on stream s: the lists of this registry, and the kept energies where the
+// parameters have changed or the chains have been minimised
 static int mc_fresh_pairs(mmo_mc* m, hipStream_t s) {
   mmo_ctx* c = m->ctx;
   if (m->pe_words == 0) return MMO_OK;
@@ -2360,7 +2369,7 @@ static int mc_fresh_pairs(mmo_mc* m, hipStream_t s) {
   }
   if (m->pe_uff == c->uff_version) return MMO_OK;
   HIPCHK(c, launch_mc_pairs(mc_args(m, 1, m->nchain, m->d_work.p), m->nchain, s));
-  m->pe_uff = c->uff_version;
+  if (!capture_id(s)) m->pe_uff = c->uff_version;   // recorded only: to do when it is run
   return MMO_OK;
 }
 
