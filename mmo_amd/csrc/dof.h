@@ -121,8 +121,10 @@ __device__ __forceinline__ LayerWeights layer_weights(const AxisCell& x, const A
 __device__ __forceinline__ double layer_value(const LayerWeights& w, float a, float b, float c, float d) {
   return fma((double)d, w.w01, fma((double)c, w.w11, fma((double)b, w.w10, (double)a * w.w00)));
 }
+// (a sum of the layers, not a step from one to the other: two infinite layers stay infinite)
 __device__ __forceinline__ double between_layers(double b0, double b1, double w) {
-  return fma(w, b1 - b0, b0);
+#pragma clang fp contract(off)   // 1 - w as it stands: w may be a product
+  return fma(w, b1, (1.0 - w) * b0);
 }
 // coordinate of R c + T along one row r of R (Rot.rotate, src/rot.ml:97-100, then translate)
 __device__ __forceinline__ double rotate_shift(const double* r, const double* c, double t) {
