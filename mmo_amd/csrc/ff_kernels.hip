@@ -940,7 +940,10 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<Src> a) {
         const AxisCell cx = axis_cell(a.g, rotate_shift(R, c, T[0]) - a.g.ox, a.g.nx),
                        cy = axis_cell(a.g, rotate_shift(R + 3, c, T[1]) - a.g.oy, a.g.ny),
                        cz = axis_cell(a.g, rotate_shift(R + 6, c, T[2]) - a.g.oz, a.g.nz);
-        if (!(cx.in && cy.in && cz.in)) bad = 1;
+        if (!(cx.in && cy.in && cz.in)) {   // NaN whatever the other atoms give
+          bad = 1;
+          break;
+        }
         float v[8];
         grid_corners<CELLS>(a.g, a.latoms[li.atom_base + j].type, cx.i, cy.i, cz.i, v);
         const LayerWeights lw = layer_weights(cx, cy);
