@@ -882,14 +882,16 @@ bool translation_lattice(const double* trans, int ntrans, std::vector<double>& a
 
 // Whether an interpolated scan takes the lattice kernel (k_interp_lattice): translations that
 // form a lattice whose z ascend by at most 4 grid layers, grids within a 31-bit buffer, and
-// enough work.  SIMD cycles per ligand atom, measured on 75 atoms and 64^3 grids: a 64-pose
-// tile of the general kernel 579; a wavefront of the lattice kernel about 250 for the x, y
-// and z weights, 130 a layer (its two node pairs a lane, at 4 lanes a cycle) and 27 a z, so
-// it gains where the columns fill their wavefronts and z shares layers: ms general / lattice,
-// 4,608 rotations: 20^3 at 0.5 A 10.18 / 3.88, 16^3 at 0.25 4.02 / 1.03, 9 x 9 x 40 at 0.2
-// 3.18 / 1.07, 10^3 at 1.0 2.11 / 1.74, but 5 x 5 x 1 0.075 / 0.098.  A wavefront walks its z
-// one after the other (250 us a 20-long column), so below 2,048 wavefronts the general
-// kernel's shorter ones win: 128 rotations of 20^3 (896) 0.32 / 0.35, 512 (3,584) 1.27 / 0.53.
+// enough work.  SIMD cycles per ligand atom, measured on 23, 75 and 131 atoms and 64^3 grids:
+// a 64-pose tile of the general kernel 579; a wavefront of the lattice kernel about 150 for
+// the x, y and z weights, 130 a layer (its two node pairs a lane, at 4 lanes a cycle) and 8 a
+// z, so it gains where the columns fill their wavefronts and z shares layers.  It is a chain of
+// layers, so fewer than 2,800 wavefronts take the time of that many (0.17 ms for 10 z at 0.5
+// A, 75 atoms).  ms general / lattice, 1,500 rotations: 20^3 at 0.5 A 3.21 / 1.35, at 0.75 A
+// 3.58 / 2.01, 20 x 20 x 21 3.61 / 2.07, 24 z 3.95 / 2.34, at 1 A (half of them outside the
+// grid) 2.73 / 2.32, 2.73 / 2.44 and 2.78 / 2.66; 21 x 21 x 1 0.20 / 0.17, 5^3 0.067 / 0.104,
+// 8 x 8 x 2 0.061 / 0.065, 9 x 9 x 21 at 1 A 1.00 / 1.00; 128 rotations of 20^3 0.29 / 0.18,
+// 64 0.156 / 0.177, 512 of 8^3 0.079 / 0.136, 1,500 of 8^3 0.22 / 0.15.
 bool lattice_scan(const mmo_ctx* c, int nrot, const double* trans, int ntrans,
                   std::vector<double>& axes, LatticeArgs& la) {
   const size_t grid_bytes = c->g.nvox * c->ntypes * sizeof(float);
@@ -897,14 +899,20 @@ bool lattice_scan(const mmo_ctx* c, int nrot, const double* trans, int ntrans,
       !translation_lattice(trans, ntrans, axes, la.n, la.stride))
     return false;
   la.nrot = nrot; la.ntrans = ntrans; la.g = c->g; la.grid_bytes = (uint32_t)grid_bytes;
-  const int nz = la.n[2], zc = std::min(nz, kLatticeZ);
+  const int nz = la.n[2];
   const double* z = axes.data() + la.n[0] + la.n[1];
   for (int k = 1; k < nz; ++k)   // also false for a z that is not a number
     if (!(z[k] >= z[k - 1] && (z[k] - z[k - 1]) * c->g.ods <= 4.0)) return false;
   if (c->scan_lattice == 2) return true;
-  const double layers = nz > 1 ? (z[nz - 1] - z[0]) * c->g.ods * (zc - 1) / (nz - 1) + 2.0 : 2.0;
-  const double units = (double)lattice_units(la), tiles = (double)nrot * ((ntrans + kWave - 1) / kWave);
-  return units >= 2048.0 && 1.15 * units * (250.0 + 130.0 * layers + 27.0 * zc) < 579.0 * tiles;
+  const int ztiles = lattice_tiles(nz);
+  double cycles = 0.0;   // of one column tile's wavefronts
+  for (int t = 0; t < ztiles; ++t) {
+    int z0, zn;
+    lattice_tile(nz, t, z0, zn);
+    cycles += 150.0 + 130.0 * ((z[z0 + zn - 1] - z[z0]) * c->g.ods + 2.0) + 8.0 * zn;
+  }
+  const double units = std::max((double)lattice_units(la), 2800.0);
+  return 1.15 * (units / ztiles) * cycles < 579.0 * nrot * ((ntrans + kWave - 1) / kWave);
 }
 
 }  // namespace
