@@ -809,15 +809,15 @@ InterLaunch scan_launch(mmo_ctx* c, int mode, int scan_cull) {
 // the 75-atom ligand and the 3000-atom receptor, ms per launch: 125 tiles 2.70 / 0.14, 1,000
 // 2.74 / 0.77, 4,000 3.91 / 2.73, 8,000 6.61 / 5.39, 12,000 9.30 / 8.08; the filtered scan
 // of one tile 2.7 / 0.08.  Beyond that the scratch (8 bytes per atom and pose) costs more
-// memory than the last, partly filled round of wavefronts is worth.
-int split_scan(mmo_ctx* c, InterLaunch& L, int lig_id, size_t ntiles) {
+// memory than the last, partly filled round of wavefronts is worth.  Without that memory the
+// scan is not split.
+void split_scan(mmo_ctx* c, InterLaunch& L, int lig_id, size_t ntiles) {
   constexpr size_t kMaxPart = (size_t)1 << 26;   // doubles (512 MiB)
   L.n_atoms = c->ligs[lig_id].n;
-  if (L.cull < 4 || ntiles > (size_t)c->scan_split || L.n_atoms * ntiles * kWave > kMaxPart)
-    return MMO_OK;
-  HIPCHK(c, c->s_scan_part.ensure(L.n_atoms * ntiles * kWave));
-  L.part = c->s_scan_part.p;
-  return MMO_OK;
+  if (L.cull < 4 || L.n_atoms < 2 || ntiles > (size_t)c->scan_split || L.n_atoms * ntiles * kWave > kMaxPart)
+    return;
+  if (c->s_scan_part.ensure(L.n_atoms * ntiles * kWave) == hipSuccess) L.part = c->s_scan_part.p;
+  else (void)hipGetLastError();
 }
 
 // translations in Morton order of their per-axis ranks: 64 consecutive slots form a
@@ -1986,7 +1986,7 @@ int mmo_scan_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, int nrot,
     timer_end(c, "interp", s);
   } else {
     InterLaunch L = scan_launch(c, mode, c->scan_cull);
-    if ((r = split_scan(c, L, lig_id, (size_t)nrot * ((ntrans + kWave - 1) / kWave)))) return r;
+    split_scan(c, L, lig_id, (size_t)nrot * ((ntrans + kWave - 1) / kWave));
     timer_begin(c, "inter", s);
     HIPCHK(c, launch_inter_scan(L, lig_id, d_rot, nrot, d_trans, c->s_tperm.p, ntrans, e_out, s));
     timer_end(c, "inter", s);
@@ -3012,7 +3012,7 @@ int mmo_scan_filtered_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, 
       // the scan's own culled kernel (the list form has no unculled one): the kept poses'
       // energies are those of mmo_scan_dev, bit for bit
       InterLaunch L = scan_launch(c, MMO_SHIFTED, c->scan_cull ? c->scan_cull : 2);
-      if ((r = split_scan(c, L, lig_id, ((size_t)nk + kWave - 1) / kWave))) return r;
+      split_scan(c, L, lig_id, ((size_t)nk + kWave - 1) / kWave);
       timer_begin(c, "inter", s);
       HIPCHK(c, launch_inter_scan_list(L, lig_id, a.rots, a.trans, c->s_tperm.p, ntrans, c->s_list.p,
                                        nk, e_out, s));
