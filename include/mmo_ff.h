@@ -430,7 +430,9 @@ int mmo_fixed_point_bits(const mmo_ctx* ctx);
  * now on keep the E_intra of every 64 pairs and evaluate those a torsion changes; 0: all
  * pairs), "mc_pool" (direct chains made from now on: workgroups share their chains' sweeps
  * up to this many chains per CU; 0: never; same results), "min_pooled" (minimisers made from now on: workgroups share their poses' sweeps
- * up to this many poses per CU; 0: never; same results).  No counterpart in the reference. */
+ * up to this many poses per CU; 0: never; same results).  mmo_tune_get also knows
+ * "mc_pooled_slots" and "min_pooled_slots": the chains or poses per workgroup of the last such
+ * launch, 0 where it was not pooled.  No counterpart in the reference. */
 int mmo_tune_set(mmo_ctx* ctx, const char* key, double value);
 double mmo_tune_get(mmo_ctx* ctx, const char* key);
 

@@ -217,6 +217,7 @@ struct mmo_ctx {
   int uff_version = 0;
   int mc_pool = 12;            // chains per CU up to which workgroups pool their sweeps
   int mc_keep_pairs = 1;       // chains keep their pair energies
+  int mc_last_pooled = 0, min_last_pooled = 0;   // slots of the last launch's pooled form (0: another form)
   DevBuf<uint64_t> d_intra_bits;   // per atom i, bit d: the pair (i, i + d mod n) counts (free ligands)
   DevBuf<int64_t> d_bit_base;      // per ligand, into d_intra_bits
   DevBuf<int> d_sweep;          // per ligand at atom_base: the sweeps' atom order
@@ -731,12 +732,12 @@ void plan_tiles(const std::vector<int>& pose_lig, const std::vector<LigHost>* li
 void timer_begin(mmo_ctx* c, const char* name, hipStream_t s) {
   (void)hipEventRecord(c->ev[name].first.get(), s);
 }
-// done: an event of the caller's to record instead of the timer's own
-hipError_t timer_end(mmo_ctx* c, const char* name, hipStream_t s, const Event& done = nullptr) {
+// done: an event of the caller's to record instead of the timer's own; whether it was recorded
+bool timer_end(mmo_ctx* c, const char* name, hipStream_t s, const Event& done = nullptr) {
   Timer& t = c->ev[name];
   t.last = done ? done : t.own;
   c->last_ms[name] = -2.0f;   // resolved by mmo_last_kernel_ms
-  return hipEventRecord(t.last.get(), s);
+  return hipEventRecord(t.last.get(), s) == hipSuccess;
 }
 
 // plain one-ligand helper: uploads coordinates and a one-entry ligand table
@@ -1739,8 +1740,8 @@ static int batch_score(mmo_batch* b, int flags, const double* xyz, double* e_out
       if (!comp && !later)
         HIPCHK(c, launch_pose_sum(a.part, b->d_unit_off.p, b->npose, false, false, e_out, s));
     }
-    const hipError_t e = timer_end(c, "inter", s, sums ? sums->done : nullptr);
-    if (sums) HIPCHK(c, e);
+    if (!timer_end(c, "inter", s, sums ? sums->done : nullptr) && sums)
+      return fail(c, MMO_ERR_DEVICE, "event record: %s", hipGetErrorString(hipGetLastError()));
   } else if (pose_first) {
     // one wavefront per pose over the culled receptor, 8-atom sub-blocks
     InterLaunch L = inter_launch(c, MMO_SHIFTED, c->d_ligs.p, c->d_latoms.p, c->d_lig_xyz.p);
@@ -2182,7 +2183,10 @@ static int mc_keep_pairs(mmo_mc* m, hipStream_t s) {
 
 static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work);
 
-static int mc_pool_slots(const mmo_ctx* c, int nwork, int max_atoms);
+struct McShape { int waves; bool rec_lds; int pool_slots, pool_waves; };
+static McShape mc_shape(const mmo_mc* m, McArgs a, int nwork);
+static size_t mc_pool_sums(const mmo_ctx* c, int slots, int max_atoms);
+
 int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double* rot0,
                   const double* pos0, int inter_mode, int flags, const double* roi_center,
                   double roi_r, double temperature, uint64_t seed, int total_frames,
@@ -2308,10 +2312,10 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
     delete m;
     return r;
   }
-  // pooled sweeps, where there may be some; without the memory the chains do without
-  if (inter_mode == MMO_SHIFTED && mc_pool_slots(c, nchain, m->max_atoms) > 0 &&
-      m->d_pool.ensure((size_t)mc_pool_slots(c, nchain, m->max_atoms) * c->ncu *
-                       ((m->max_atoms + 3) / 4) * 3 * kWave) != hipSuccess)
+  // pooled sweeps, where the chains' launches will have some (a run in a caller's capture cannot
+  // allocate them); without the memory the chains do without
+  const McShape shape = mc_shape(m, mc_args(m, 1, nchain, m->d_work.p), nchain);
+  if (shape.pool_slots > 0 && m->d_pool.ensure(mc_pool_sums(c, shape.pool_slots, m->max_atoms)) != hipSuccess)
     (void)hipGetLastError();
   // the registered conformers of every chain, from the registry (uploaded once a chain they
   // were 22 MB for 6,144 chains: 3 ms of host copies)
@@ -2381,49 +2385,57 @@ static int mc_fresh_pairs(mmo_mc* m, hipStream_t s) {
   return MMO_OK;
 }
 
-// launch shape: up to 8 chains (wavefronts) per workgroup; in the direct form the
-// workgroup stages the receptor in LDS when it fits next to the conformers
 // Chains per workgroup of the pooled form for nwork chains (0: each wavefront sweeps for its own
 // chain): all of them at once, up to 12 a CU, one workgroup per CU.  3,000 chains (12 a CU) take
 // 12.8 against 15.4 ms a 100 frames; more keep every wavefront busy by themselves (4,096 chains
 // through 8 slots 17.3 against 16.0).  The units' sums (3 KiB per 4 atoms) stay within a bound.
 constexpr size_t kMcPoolBytes = (size_t)384 << 20;
+static size_t mc_pool_sums(const mmo_ctx* c, int slots, int max_atoms) {   // float4
+  return (size_t)slots * c->ncu * ((max_atoms + 3) / 4) * 3 * kWave;
+}
 static int mc_pool_slots(const mmo_ctx* c, int nwork, int max_atoms) {
   const int slots = (nwork + c->ncu - 1) / c->ncu;
   if (slots > std::min(c->mc_pool, kMcPoolSlots)) return 0;
-  const size_t bytes = (size_t)slots * c->ncu * ((max_atoms + 3) / 4) * 3 * kWave * sizeof(float4);
-  return bytes <= kMcPoolBytes ? slots : 0;
+  return mc_pool_sums(c, slots, max_atoms) * sizeof(float4) <= kMcPoolBytes ? slots : 0;
+}
+
+// launch shape: up to 8 chains (wavefronts) per workgroup; in the direct form the
+// workgroup stages the receptor in LDS when it fits next to the conformers
+static McShape mc_shape(const mmo_mc* m, McArgs a, int nwork) {
+  const size_t cap = 160 * 1024;
+  McShape g{};
+  g.rec_lds = m->inter_mode != MMO_INTERP && m->ctx->cullp_ok && m->ctx->mc_rec_lds;
+  const int wmax = std::min(mc_max_waves(a), m->ctx->mc_wg_waves);
+  g.waves = wmax;
+  while (g.waves > 1 && mc_lds_bytes(a, g.waves, g.rec_lds) > cap) --g.waves;
+  if (g.rec_lds && (g.waves < std::min(4, wmax) || mc_lds_bytes(a, g.waves, g.rec_lds) > cap)) {
+    g.rec_lds = false;
+    g.waves = wmax;
+    while (g.waves > 1 && mc_lds_bytes(a, g.waves, false) > cap) --g.waves;
+  }
+  if (g.rec_lds && mc_can_pool(a)) {
+    a.pool_slots = mc_pool_slots(m->ctx, nwork, m->max_atoms);
+    g.pool_waves = g.waves;
+    while (g.pool_waves > 1 && mc_lds_bytes(a, g.pool_waves, true) > cap) --g.pool_waves;
+    if (g.pool_waves > a.pool_slots) g.pool_slots = a.pool_slots;
+  }
+  return g;
 }
 
 static hipError_t mc_launch(mmo_mc* m, McArgs a, int nwork, hipStream_t s) {
-  int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  const size_t cap = 160 * 1024;
-  bool rec_lds = m->inter_mode != MMO_INTERP && m->ctx->cullp_ok && m->ctx->mc_rec_lds;
-  const int wmax = std::min(mc_max_waves(a), m->ctx->mc_wg_waves);
-  int waves = wmax;
-  while (waves > 1 && mc_lds_bytes(a, waves, rec_lds) > cap) --waves;
-  if (rec_lds && (waves < std::min(4, wmax) || mc_lds_bytes(a, waves, rec_lds) > cap)) {
-    rec_lds = false;
-    waves = wmax;
-    while (waves > 1 && mc_lds_bytes(a, waves, false) > cap) --waves;
-  }
-  if (rec_lds && mc_can_pool(a) && m->d_pool.n > 0) {
-    a.pool_slots = mc_pool_slots(m->ctx, nwork, m->max_atoms);
-    while (waves > 1 && mc_lds_bytes(a, waves, true) > cap) --waves;
-    const size_t need = (size_t)a.pool_slots * m->ctx->ncu * ((m->max_atoms + 3) / 4) * 3 * kWave;
-    if (a.pool_slots > 0 && waves > a.pool_slots && need <= m->d_pool.n) {
-      a.pool = m->d_pool.p;
-      const int nb = std::min(m->ctx->ncu, (nwork + a.pool_slots - 1) / a.pool_slots);
-      return launch_mc(a, nb, waves, true, s);
-    }
-    a.pool_slots = 0;
+  mmo_ctx* c = m->ctx;
+  const McShape g = mc_shape(m, a, nwork);
+  c->mc_last_pooled = 0;
+  if (g.pool_slots > 0 && mc_pool_sums(c, g.pool_slots, m->max_atoms) <= m->d_pool.n) {
+    a.pool_slots = c->mc_last_pooled = g.pool_slots;
+    a.pool = m->d_pool.p;
+    const int nb = std::min(c->ncu, (nwork + a.pool_slots - 1) / a.pool_slots);
+    return launch_mc(a, nb, g.pool_waves, true, s);
   }
   // at least one workgroup per CU; more when the residency setting allows
-  const int resident = ncu * std::max(1, m->ctx->mc_waves_per_cu / waves);
-  const int blocks = std::max(1, std::min((nwork + waves - 1) / waves, resident));
-  return launch_mc(a, blocks, waves, rec_lds, s);
+  const int resident = c->ncu * std::max(1, c->mc_waves_per_cu / g.waves);
+  const int blocks = std::max(1, std::min((nwork + g.waves - 1) / g.waves, resident));
+  return launch_mc(a, blocks, g.waves, g.rec_lds, s);
 }
 
 int mmo_mc_run(mmo_mc* m, int nsteps, void* stream) {
@@ -3130,7 +3142,8 @@ int mmo_min_create(mmo_batch* b, int history, int flags, const double* lo, const
   if (e == hipSuccess) e = z->queue.ensure(1);
   // without this buffer the minimiser takes another form
   const size_t unit_fe = (size_t)min_units(b->max_atoms) * kWave;
-  if (e == hipSuccess && inter == MMO_F_INTER_SHIFTED && min_slots(c, b) > 0)
+  if (e == hipSuccess && inter == MMO_F_INTER_SHIFTED && c->min_fused && !c->min_f64 && c->cullp_ok &&
+      c->min_rec_lds && min_slots(c, b) > 0)
     if (z->fe.ensure((size_t)min_slots(c, b) * c->ncu * unit_fe) != hipSuccess) (void)hipGetLastError();
   if (e == hipSuccess && b->d_by_size.n < (size_t)b->npose)
     e = b->d_by_size.ensure(b->npose) == hipSuccess
@@ -3212,9 +3225,11 @@ int mmo_min_run_dev(mmo_min* z, double* dofs, int iters, double* e_out, void* st
     timer_begin(c, "min", s);
     p.slots = min_slots(c, b);
     p.fe = z->fe.p;
+    c->min_last_pooled = 0;
     if (rec_lds && kind == kDofInterAtom && p.slots > 0 && z->fe.n > 0 &&
         min_pooled_lds_bytes(p) <= kMaxLds - 128) {
       const int nb = std::min(c->ncu, (b->npose + p.slots - 1) / p.slots);   // at most one per CU
+      c->min_last_pooled = p.slots;
       HIPCHK(c, launch_min_pooled(p, nb, s));
       timer_end(c, "min", s);
       return MMO_OK;
@@ -3357,6 +3372,8 @@ double mmo_tune_get(mmo_ctx* c, const char* key) {
   if (k == "cull_ok") return c->cull_ok ? 1.0 : 0.0;
   if (k == "cullp_ok") return c->cullp_ok ? 1.0 : 0.0;
   if (k == "mc_pool") return c->mc_pool;
+  if (k == "mc_pooled_slots") return c->mc_last_pooled;
+  if (k == "min_pooled_slots") return c->min_last_pooled;
   if (k == "mc_keep_pairs") return c->mc_keep_pairs;
   if (k == "mc_waves_per_cu") return c->mc_waves_per_cu;
   if (k == "mc_wg_waves") return c->mc_wg_waves;
