@@ -1253,9 +1253,14 @@ static int plain_inter(mmo_ctx* c, int mode, const double* xs, const double* ys,
   const bool grad = gx != nullptr;
   // one pose: a wavefront per 64 receptor atoms (the FP32 sums end there anyway), each lane
   // no more ligand atoms than it must: the serial loop of a lane is the time of the launch.
-  // 75 against 3,000 atoms: slices of 256 and four atoms a lane 73 us, now 16 us
+  // 75 against 3,000 atoms: slices of 256 and four atoms a lane 73 us, now 16 us.  On large
+  // receptors the slices' sums and their additions to one gradient cost more than the loop: from
+  // 32,768 atoms on larger slices, up to 256.  us a call, slices of 64 / 128 / 256, energy and
+  // gradient of 75 atoms: 15,000 atoms 97 92 110, 126 125 145; 60,000 140 116 122, 193 161 165;
+  // 120,000 200 151 139, 297 211 189; 1,000,000 1145 643 393, 1696 930 550 (of 1,000 atoms 1619
+  // 1087 865, 2438 1657 1601; 512 would be slower for those from 250,000 atoms down).
   InterLaunch L = inter_launch(c, mode, c->s_lig.p, c->s_latom.p, nullptr);
-  L.rslice = 64;
+  L.rslice = 64 * std::min(4, (c->nrec + 32767) / 32768);
   if (n <= kWave) L.k = 1;
   else if (n <= 2 * kWave) L.k = 2;
   L.rtile = std::min(L.rtile, L.rslice);
