@@ -2788,6 +2788,7 @@ int mmo_set_vdw_mask(mmo_ctx* c, const double* radii, double step, int nx, int n
                   c->rec_anum[a]);
     bitmask_atom(mask, dims, o, step, &c->rec_host[3 * (size_t)a], rad, true);
   }
+  c->has_mask = false;   // until both buffers are those of the new grid
   if ((r = upload(c, c->d_mask, mask.data(), mask.size(), c->stream))) return r;
   HIPCHK(c, c->d_mask_cells.ensure(mask.size()));
   HIPCHK(c, launch_mask_cells(c->d_mask.p, c->d_mask_cells.p, nx, ny, nz, c->stream));
