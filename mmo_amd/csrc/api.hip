@@ -12,12 +12,12 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <optional>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -2063,7 +2063,7 @@ static int drain_segments(mmo_ctx* c, void* out, const void* src, const std::vec
   for (int t = 1; t < kDrainThreads; ++t) {
     try {
       th[t] = std::thread(drain, t);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {   // no thread, or no memory for one
     }
   }
   drain(0);
