@@ -1522,8 +1522,9 @@ static int pose_cull_waves(const mmo_ctx* c, int npose) {
   return std::max(1, std::min(c->pose_waves, (npose + 255) / 256));
 }
 
-// Deals the batch's slot order for workgroups of `waves` wavefronts (pose_sweep = 0; again
-// only if the workgroup shape changes).  The host copy stays in the batch while
+// Deals the batch's slot order for workgroups of `waves` wavefronts (pose_sweep = 0: at the
+// batch's creation, or by the first call that needs it; again only if the workgroup shape
+// changes).  The host copy stays in the batch while
 // the upload may be in flight; a re-deal first waits for the previous upload.
 static int deal_batch(mmo_batch* b, int waves, hipStream_t s) {
   if (b->order_waves == waves) return MMO_OK;
@@ -1656,7 +1657,8 @@ int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch**
       (r = upload(c, b->d_atom_off, b->atom_off.data(), npose + 1, s)) ||
       (r = upload(c, b->d_dof_off, b->dof_off.data(), npose + 1, s)) ||
       (r = upload(c, b->d_perm, b->perm.data(), npose, s)) ||
-      (r = upload(c, b->d_tiles, b->tiles.data(), b->tiles.size(), s))) {
+      (r = upload(c, b->d_tiles, b->tiles.data(), b->tiles.size(), s)) ||
+      (c->pose_cull && c->pose_sweep == 0 && (r = deal_batch(b, pose_cull_waves(c, npose), s)))) {
     delete b;
     return r;
   }

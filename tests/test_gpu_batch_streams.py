@@ -132,3 +132,27 @@ def test_captured_calls(setup):
         for k in range(2):
             assert torch.equal(outs[k][0], want[k][0]) and torch.equal(outs[k][1], want[k][1])
     assert ctx is b.ctx
+
+
+def test_captured_first_call_of_the_sub_block_kernel(setup):
+    """A batch made with pose_sweep = 0 has its slot order: its first call can be captured."""
+    import torch
+    ctx = setup[0]
+    ctx.tune(pose_sweep=0)
+    try:
+        b, ligs = _batch(setup, 300)
+        x = _poses(ligs, 1)
+        (e, g), (we, wg) = _buffers(b, True), _buffers(b, True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            b.score_dev(x, e, g, flags=FLAGS | ff.F_GRAD)
+        for k in range(3):
+            x.copy_(_poses(ligs, 2 + k))
+            b.score_dev(x, we, wg, flags=FLAGS | ff.F_GRAD)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(e, we) and torch.equal(g, wg)
+    finally:
+        ctx.tune(pose_sweep=1)
