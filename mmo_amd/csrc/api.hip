@@ -3010,7 +3010,7 @@ int mmo_scan_filtered_dev(mmo_ctx* c, int lig_id, int mode, const double* rots, 
   if ((r = upload(c, c->s_tperm, tperm.data(), tperm.size(), s))) return r;
   const int n = nrot * ntrans;
   const size_t groups = scan_keep_groups(nrot, ntrans);
-  HIPCHK(c, c->s_keep.ensure(groups * (kKeepSlots / 64)));
+  HIPCHK(c, c->s_keep.ensure(groups * scan_keep_tiles(nrot, ntrans)));
   HIPCHK(c, c->s_list.ensure(n));
   HIPCHK(c, c->s_nkept.ensure(groups + 1));
   // the kept slots in the scan's pose order (so that consecutive kept poses stay in the

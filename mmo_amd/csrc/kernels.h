@@ -266,6 +266,7 @@ struct ScanFilterArgs {
   int nx, ny, nz;
   const uint8_t* skip;        // per translation: 1 = skipped (ROI / centre clash)
   int atom_clash;             // test every atom's 8 corners
+  int tiles;                  // scan_keep_tiles (set by the launch)
   double* e;                  // scan energies, set to +inf for skipped poses (all, before scoring)
 };
 hipError_t launch_scan_filter(const ScanFilterArgs& a, hipStream_t s);
@@ -274,10 +275,10 @@ hipError_t launch_mask_cells(const uint32_t* mask, uint32_t* cells, int nx, int 
                              hipStream_t s);
 // Filter before scoring: list[0 .. *total) = the slots of the scan's pose order (rotation r,
 // translation tperm[slot - r * ntrans]) that the filters keep, in order; every a.e = +inf.
-constexpr int kKeepSlots = 2048;   // slots of one workgroup
-size_t scan_keep_groups(int nrot, int ntrans);
+int scan_keep_tiles(int nrot, int ntrans);       // of 64 slots each: a workgroup's
+size_t scan_keep_groups(int nrot, int ntrans);   // workgroups
 struct KeepScratch {
-  uint64_t* words;            // kKeepSlots / 64 per workgroup: keep flags
+  uint64_t* words;            // scan_keep_tiles per workgroup: keep flags
   unsigned* count;            // per workgroup
   unsigned* total;
   int* list;

@@ -109,26 +109,29 @@ __device__ __forceinline__ bool cell_clash(const ScanFilterArgs& a, uint32_t v) 
 // a coordinate of the clash test: one that is not finite is outside every grid
 __device__ __forceinline__ double clash_coord(double v) { return fabs(v) <= 1e300 ? v : 1e300; }
 
-// A workgroup takes kKeepSlots slots of the scan's pose order, 64 per wavefront at a time
+// A workgroup takes a.tiles x 64 slots of the scan's pose order, 64 per wavefront at a time
 // (one 64-bit word of keep flags).  TILED (at least 64 translations): the slots of one
 // rotation (workgroup = rotation, then its share of the translations), whose rotated atoms
 // R c are formed once in LDS, so that a pose's atom costs three additions instead of the
 // whole transform; else consecutive slots of any rotations, each lane forming its own.
-constexpr int kKeepTiles = kKeepSlots / 64;
+// 32 tiles share the rotated atoms; scans that would fill fewer than 2,048 workgroups (8 a CU) so
+// take fewer, down to one a wavefront: 40,000 poses of a 5-atom ligand 79 us with 32, 53 now, of 38
+// atoms 94 and 63.
+constexpr int kKeepTiles = 32;
 
 template <bool TILED>
 struct KeepSlots {
-  int nrot, ntrans, per_rot;   // per_rot: workgroups per rotation (TILED)
+  int nrot, ntrans, size, per_rot;   // slots of a workgroup; workgroups per rotation (TILED)
   __device__ KeepSlots(const ScanFilterArgs& a)
-      : nrot(a.nrot), ntrans(a.ntrans), per_rot((a.ntrans + kKeepSlots - 1) / kKeepSlots) {}
+      : nrot(a.nrot), ntrans(a.ntrans), size(64 * a.tiles), per_rot((a.ntrans + size - 1) / size) {}
   // slot `lane` of the workgroup's tile q: its rotation and translation slot; false: none
   __device__ bool at(int q, int lane, int& r, int& ts) const {
     if (TILED) {
       r = blockIdx.x / per_rot;
-      ts = (blockIdx.x - r * per_rot) * kKeepSlots + q * 64 + lane;
+      ts = (blockIdx.x - r * per_rot) * size + q * 64 + lane;
       return ts < ntrans;
     }
-    const size_t slot = (size_t)blockIdx.x * kKeepSlots + q * 64 + lane;
+    const size_t slot = (size_t)blockIdx.x * size + q * 64 + lane;
     if (slot >= (size_t)nrot * ntrans) return false;
     r = (int)(slot / ntrans);
     ts = (int)(slot - (size_t)r * ntrans);
@@ -164,11 +167,11 @@ __global__ void __launch_bounds__(256) k_scan_filter(ScanFilterArgs a, const int
     }
   }
   __syncthreads();
-  for (int q = wave; q < kKeepTiles; q += 4) {
+  for (int q = wave; q < a.tiles; q += 4) {
     int r = 0, ts = 0;
     const bool in = slots.at(q, lane, r, ts);
     if (__ballot(in) == 0ull) {
-      if (KEEP && lane == 0) words[(size_t)blockIdx.x * kKeepTiles + q] = 0ull;
+      if (KEEP && lane == 0) words[(size_t)blockIdx.x * a.tiles + q] = 0ull;
       continue;
     }
     const int t = in ? (tperm ? tperm[ts] : ts) : 0;
@@ -198,7 +201,7 @@ __global__ void __launch_bounds__(256) k_scan_filter(ScanFilterArgs a, const int
     if (KEEP) {
       const uint64_t w = __ballot(keep);
       if (lane == 0) {
-        words[(size_t)blockIdx.x * kKeepTiles + q] = w;
+        words[(size_t)blockIdx.x * a.tiles + q] = w;
         if (w) atomicAdd(&s_count, (unsigned)__popcll(w));
       }
     } else if (in && !keep) {
@@ -222,7 +225,7 @@ __global__ void __launch_bounds__(64) k_keep_list(ScanFilterArgs a, const uint64
   // nothing kept here: the next workgroup (or the end of the list) starts at the same place
   if ((blockIdx.x + 1 < gridDim.x ? start[blockIdx.x + 1] : *total) == first) return;
   unsigned base = first;
-  const uint64_t mine = lane < kKeepTiles ? words[(size_t)blockIdx.x * kKeepTiles + lane] : 0ull;
+  const uint64_t mine = lane < a.tiles ? words[(size_t)blockIdx.x * a.tiles + lane] : 0ull;
   for (uint64_t any = __ballot(mine != 0ull); any; any &= any - 1) {
     const int q = __builtin_ctzll(any);
     const uint64_t w = __shfl((unsigned long long)mine, q, 64);
@@ -234,14 +237,23 @@ __global__ void __launch_bounds__(64) k_keep_list(ScanFilterArgs a, const uint64
   }
 }
 
+static size_t keep_groups(int nrot, int ntrans, int tiles) {
+  const int size = 64 * tiles;
+  return ntrans >= 64 ? (size_t)nrot * ((ntrans + size - 1) / size)
+                      : ((size_t)nrot * ntrans + size - 1) / size;
+}
+int scan_keep_tiles(int nrot, int ntrans) {
+  int tiles = kKeepTiles;
+  while (tiles > 4 && keep_groups(nrot, ntrans, tiles) < 2048) tiles /= 2;
+  return tiles;
+}
 size_t scan_keep_groups(int nrot, int ntrans) {
-  return ntrans >= 64 ? (size_t)nrot * ((ntrans + kKeepSlots - 1) / kKeepSlots)
-                      : ((size_t)nrot * ntrans + kKeepSlots - 1) / kKeepSlots;
+  return keep_groups(nrot, ntrans, scan_keep_tiles(nrot, ntrans));
 }
 
 template <bool TILED>
-static hipError_t scan_filter_t(const ScanFilterArgs& a, const int* tperm, const KeepScratch* w,
-                                hipStream_t s) {
+static hipError_t scan_filter_t(ScanFilterArgs a, const int* tperm, const KeepScratch* w, hipStream_t s) {
+  a.tiles = scan_keep_tiles(a.nrot, a.ntrans);
   const size_t groups = scan_keep_groups(a.nrot, a.ntrans);
   const size_t lds = a.atom_clash ? (size_t)3 * a.n_atoms * sizeof(double) : 0;
   if (!w) {
