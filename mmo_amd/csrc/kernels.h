@@ -287,14 +287,14 @@ hipError_t launch_scan_keep(const ScanFilterArgs& a, const int* tperm, const Kee
                             hipStream_t s);
 
 constexpr int kTopkMax = 2048;
-constexpr int kTopkCand = 4096;   // keys the select leaves to the final sort (>= kTopkMax)
+constexpr int kTopkCand = 4096;   // keys the select leaves to the final sort, at most (>= kTopkMax)
 constexpr int kTopkPasses = 5;       // digits of the select
 constexpr int kTopkHist = kTopkPasses * 8192;
 struct TopkState {
   uint64_t prefix, mask;      // the selected high bits and which they are
   uint64_t rem, k;            // keys still to be taken among those matching the prefix; of k
-  unsigned done;              // the keys at or below the prefix fit the candidate list
-  unsigned pad;
+  unsigned limit;             // candidates to end at (topk_limit)
+  unsigned done;              // no more keys than that are at or below the prefix
 };
 struct TopkScratch {
   TopkState* st;              // kTopkPasses + 1

@@ -10,7 +10,7 @@
 // Top-k (the TopKeeper of src/lds.ml:1055-1064, :1110-1113, lowest energies first):
 // an MSB-first radix select over order-preserving 64-bit keys of the energies narrows the
 // k-th smallest key down by 13 bits a pass (at most 5 passes) until no more than
-// kTopkCand keys are at or below the prefix; those are gathered, and one workgroup sorts
+// topk_limit keys are at or below the prefix; those are gathered, and one workgroup sorts
 // them by (energy, index) and keeps the first k.  Where more than that many keys are equal
 // to the k-th, the passes resolve all 64 bits and the equal keys are taken in index order
 // (so ties resolve to the lowest pose indices).  NaN sorts as the largest value.
@@ -355,14 +355,14 @@ __device__ TopkState topk_next(const TopkState& p, const unsigned* hist, int shi
   r.mask |= (uint64_t)((1 << bits) - 1) << shift;
   r.rem = s[nw + 1];
   // keys below the prefix: k - rem
-  r.done = p.k - r.rem + s[nw + 2] <= (uint64_t)kTopkCand ? 1u : 0u;
+  r.done = p.k - r.rem + s[nw + 2] <= (uint64_t)p.limit ? 1u : 0u;
   return r;
 }
 
-__global__ void k_topk_init(TopkState* st, unsigned* hist, unsigned* count, uint64_t k) {
+__global__ void k_topk_init(TopkState* st, unsigned* hist, unsigned* count, uint64_t k, unsigned limit) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
-    st[0] = TopkState{0ull, 0ull, k, k, 0u, 0u};
+    st[0] = TopkState{0ull, 0ull, k, k, limit, 0u};
     *count = 0u;
   }
   if (i < kTopkHist) hist[i] = 0u;
@@ -511,19 +511,29 @@ __global__ void __launch_bounds__(1024) k_topk_sort(const TopkState* st, const u
   }
 }
 
+// The sort of the candidates takes 25, 45 and 91 us for 1,024, 2,048 and 4,096 of them, a pass 6
+// us up to some 4 M energies and 60 us for 36.9 M: few energies (or, for large k, as many as the
+// list holds) are sorted at once, and up to 4 M the passes go on until they have left 1,024 (or
+// k) candidates, beyond until the list holds them.  20,000 energies of seven values, k = 1 or 100: 159 us with 4,096, 75 and 84 now;
+// 4,096 energies, k = 1, sorted at once 112 to 121, 75 to 80 by passes; 3,000,000 normally distributed, k = 100, 196 and 75.
+constexpr int kTopkSort = 2048;
+static unsigned topk_limit(size_t n, int k) {
+  return n <= ((size_t)1 << 22) ? std::max(1024, k) : kTopkCand;
+}
+
 hipError_t launch_topk(const double* e, size_t n, int k, double* out_e, int64_t* out_i,
                        TopkScratch w, hipStream_t s) {
   if (k <= 0 || n == 0) return hipSuccess;
   // LDS: kTopkCand keys and indices (64 KiB, the most a launch may ask for without the
   // kernel's limit being raised)
   constexpr size_t lds = (size_t)kTopkCand * (sizeof(uint64_t) + sizeof(int64_t));
-  if (n <= (size_t)kTopkCand) {
+  if (n <= (size_t)kTopkSort || (n <= (size_t)kTopkCand && k > kTopkSort / 2)) {
     hipLaunchKernelGGL(k_topk_sort, dim3(1), dim3(1024), lds, s, w.st, w.count, w.cand_e, w.cand_i, e,
                        (int)n, k, out_e, out_i);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_topk_init, dim3(kTopkHist / 1024), dim3(1024), 0, s, w.st, w.hist, w.count,
-                     (uint64_t)k);
+                     (uint64_t)k, topk_limit(n, k));
   const int blocks = (int)std::min<size_t>(512, (n + 4 * kTopkThreads - 1) / (4 * kTopkThreads));
   int shift = 64;
   for (int p = 0; p < kTopkPasses; ++p) {
