@@ -314,7 +314,8 @@ struct mmo_batch {
   int device = 0;      // the context's, kept so that destruction never reads the context
   pid_t pid = 0;
   int npose = 0, natoms = 0, ndof = 0, ntiles = 0, max_atoms = 0, max_rb = 0, max_rg = 0;
-  bool free = true;    // every ligand's torsions are free (LigHost)
+  int n_free = 0, max_free_atoms = 0;   // poses whose ligands' torsions are free (LigHost)
+  DevBuf<int> d_dof_poses;   // where only some are: those, then the others
   std::vector<int> pose_lig, atom_off, dof_off, perm;
   std::vector<Tile> tiles;
   // poses by ligand size, largest first, and the pose kernel's slot order dealt from it
@@ -1503,7 +1504,9 @@ int mmo_ligand_add(mmo_ctx* c, const double* xs, const double* ys, const double*
   } else {
     h.rg_off.assign(1, 0);
   }
-  h.free = torsions_free(h);
+  // (fewer than 8 atoms without torsions are the general adjoint's: 16,384 poses of one atom 108 us
+  // against 155, of 6 atoms 161 against 167, but of 8 atoms with two torsions 192 against 182)
+  h.free = (n >= 8 || nrb > 0) && torsions_free(h);
   c->ligs.push_back(std::move(h));
   c->lig_dirty = true;
   *lig_id = (int)c->ligs.size() - 1;
@@ -1621,7 +1624,10 @@ int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch**
     }
     b->max_atoms = std::max(b->max_atoms, c->ligs[l].n);
     b->max_rb = std::max(b->max_rb, (int)c->ligs[l].rb_left.size());
-    b->free &= c->ligs[l].free;
+    if (c->ligs[l].free) {
+      ++b->n_free;
+      b->max_free_atoms = std::max(b->max_free_atoms, c->ligs[l].n);
+    }
     b->max_rg = std::max(b->max_rg, c->ligs[l].rg_off.back());
   }
   b->atom_off[npose] = (int)na;
@@ -1650,8 +1656,15 @@ int mmo_batch_create(mmo_ctx* c, const int32_t* pose_lig, int npose, mmo_batch**
     }
     b->nunits = unit_off[npose];
   }
+  std::vector<int> dof_poses;
+  if (b->n_free > 0 && b->n_free < npose) {
+    dof_poses.resize(npose);
+    int at[2] = {0, b->n_free};
+    for (int p = 0; p < npose; ++p) dof_poses[at[c->ligs[pose_lig[p]].free ? 0 : 1]++] = p;
+  }
   hipStream_t s = c->stream;
-  if ((r = add_unit_sums(b)) || (r = upload(c, b->d_units, units.data(), units.size(), s)) ||
+  if ((!dof_poses.empty() && (r = upload(c, b->d_dof_poses, dof_poses.data(), npose, s))) ||
+      (r = add_unit_sums(b)) || (r = upload(c, b->d_units, units.data(), units.size(), s)) ||
       (r = upload(c, b->d_unit_off, unit_off.data(), unit_off.size(), s)) ||
       (r = upload(c, b->d_pose_lig, b->pose_lig.data(), npose, s)) ||
       (r = upload(c, b->d_atom_off, b->atom_off.data(), npose + 1, s)) ||
@@ -1680,7 +1693,7 @@ void mmo_batch_destroy(mmo_batch* b) {
     b->d_units.release(); b->d_unit_off.release();
     for (auto& u : b->sums) u->part.release();
     b->d_tiles.release(); b->d_xyz.release(); b->d_e.release(); b->d_g.release(); b->d_part.release();
-    b->d_conf.release();
+    b->d_conf.release(); b->d_dof_poses.release();
   }
   delete b;
 }
@@ -1887,7 +1900,7 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
                 "ligands too large for the DOF kernels: %zu bytes of LDS per pose (limit %zu)",
                 dof_lds_bytes(a, g), kMaxLds);
   HIPCHK(c, launch_apply_config(a, s));
-  a.free_torsions = g && b->free;   // after the limit, which is the general adjoint's
+  a.poses = b->d_dof_poses.p; a.n_free = b->n_free; a.max_free_atoms = b->max_free_atoms;
   const int score_flags = flags & ~MMO_F_COMPONENTS;
   if (score_flags & ~MMO_F_GRAD) {
     if (!e_out) return fail(c, MMO_ERR_BAD_ARG, "NULL energy buffer");
@@ -1907,7 +1920,7 @@ int mmo_batch_score_dofs_dev(mmo_batch* b, int flags, const double* dofs, double
         ai.latoms = c->d_latoms.p;
         ai.intra_bits = c->d_intra_bits.p;
         ai.bit_base = c->d_bit_base.p;
-        if (dof_lds_bytes(ai, true) <= kMaxLds) {
+        if (b->n_free == b->npose || dof_lds_bytes(ai, true) <= kMaxLds) {
           a = ai;
           bflags &= ~MMO_F_INTRA;
         }

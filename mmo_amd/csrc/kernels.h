@@ -144,8 +144,10 @@ struct DofArgs {
   int e_stride;
   const uint32_t* pair_ij;
   const double4* pair_par;      // ke qi qj, Ai Aj, 2 Bi Bj
-  // every ligand's torsions are free (LigHost): the adjoint then needs no serial pass
-  int free_torsions;
+  // the first n_free of `poses` (nullptr: of all, in order) have ligands whose torsions are free
+  // (LigHost), of at most max_free_atoms: their adjoint needs no serial pass
+  const int* poses;
+  int n_free, max_free_atoms;
   const LigAtom* latoms;
   const uint64_t* intra_bits;   // per ligand at bit_base: each atom's pairs (intra_ring)
   const int64_t* bit_base;

@@ -209,8 +209,8 @@ template <bool INTRA>
 __global__ void __launch_bounds__(INTRA ? kDofWaves * kWave : kWave) k_dof_grad(DofArgs a) {
   extern __shared__ __align__(16) char smem[];
   __shared__ double s_part[kDofWaves];
-  const int pose = blockIdx.x;
-  if (pose >= a.npose) return;
+  if ((int)blockIdx.x >= a.npose - a.n_free) return;
+  const int pose = a.poses ? a.poses[a.n_free + blockIdx.x] : a.n_free + blockIdx.x;
   const LigInfo li = a.ligs[a.pose_lig[pose]];
   const int L = li.n_atoms, tid = threadIdx.x, lane = tid & (kWave - 1);
   double* sx = reinterpret_cast<double*>(smem);
@@ -394,8 +394,8 @@ __global__ void __launch_bounds__(kFreeThreads) k_dof_grad_free(DofArgs a) {
   extern __shared__ __align__(16) char smem[];
   __shared__ double s_part[kFreeThreads / kWave];
   __shared__ double s_sn[3], s_cs[3];
-  const int pose = blockIdx.x;
-  if (pose >= a.npose) return;
+  if ((int)blockIdx.x >= a.n_free) return;
+  const int pose = a.poses ? a.poses[blockIdx.x] : blockIdx.x;
   const int lig = a.pose_lig[pose];
   const LigInfo li = a.ligs[lig];
   const int L = li.n_atoms, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
@@ -486,11 +486,10 @@ __global__ void __launch_bounds__(kFreeThreads) k_dof_grad_free(DofArgs a) {
 
 // LDS of k_dof_grad_free: coordinates and adjoint; with E_intra a copy per wavefront, too
 static size_t dof_free_lds_bytes(const DofArgs& a) {
-  return dof_coord_bytes(a.max_atoms, a.e_intra ? 6 + 3 * (kFreeThreads / kWave) : 6);
+  return dof_coord_bytes(a.max_free_atoms, a.e_intra ? 6 + 3 * (kFreeThreads / kWave) : 6);
 }
 
 size_t dof_lds_bytes(const DofArgs& a, bool grad) {
-  if (grad && a.free_torsions) return dof_free_lds_bytes(a);
   const int arrays = grad ? (a.e_intra ? 6 + 3 * kDofWaves : 6) : 3;
   return dof_coord_bytes(a.max_atoms, arrays) + torsion_lds_bytes(a.max_rb, a.max_rg);
 }
@@ -516,24 +515,30 @@ hipError_t launch_apply_config(const DofArgs& a, hipStream_t s) {
 
 hipError_t launch_dof_grad(const DofArgs& a, hipStream_t s) {
   if (a.npose == 0) return hipSuccess;
-  const size_t lds = dof_lds_bytes(a, true);
-  if (lds > kMaxLds) return hipErrorInvalidConfiguration;
-  if (a.free_torsions && a.e_intra) {
-    hipError_t e = lds_limit(&k_dof_grad_free<true>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dof_grad_free<true>, dim3(a.npose), dim3(kFreeThreads), lds, s, a);
-  } else if (a.free_torsions) {
-    hipError_t e = lds_limit(&k_dof_grad_free<false>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dof_grad_free<false>, dim3(a.npose), dim3(kFreeThreads), lds, s, a);
-  } else if (a.e_intra) {
-    hipError_t e = lds_limit(&k_dof_grad<true>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dof_grad<true>, dim3(a.npose), dim3(kDofWaves * kWave), lds, s, a);
-  } else {
-    hipError_t e = lds_limit(&k_dof_grad<false>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dof_grad<false>, dim3(a.npose), dim3(kWave), lds, s, a);
+  hipError_t e = hipSuccess;
+  if (a.n_free > 0) {
+    const size_t lds = dof_free_lds_bytes(a);
+    if (lds > kMaxLds) return hipErrorInvalidConfiguration;
+    const dim3 grid(a.n_free), block(kFreeThreads);
+    if (a.e_intra) {
+      if ((e = lds_limit(&k_dof_grad_free<true>, lds)) != hipSuccess) return e;
+      hipLaunchKernelGGL(k_dof_grad_free<true>, grid, block, lds, s, a);
+    } else {
+      if ((e = lds_limit(&k_dof_grad_free<false>, lds)) != hipSuccess) return e;
+      hipLaunchKernelGGL(k_dof_grad_free<false>, grid, block, lds, s, a);
+    }
+  }
+  if (a.n_free < a.npose) {
+    const size_t lds = dof_lds_bytes(a, true);
+    if (lds > kMaxLds) return hipErrorInvalidConfiguration;
+    const dim3 grid(a.npose - a.n_free);
+    if (a.e_intra) {
+      if ((e = lds_limit(&k_dof_grad<true>, lds)) != hipSuccess) return e;
+      hipLaunchKernelGGL(k_dof_grad<true>, grid, dim3(kDofWaves * kWave), lds, s, a);
+    } else {
+      if ((e = lds_limit(&k_dof_grad<false>, lds)) != hipSuccess) return e;
+      hipLaunchKernelGGL(k_dof_grad<false>, grid, dim3(kWave), lds, s, a);
+    }
   }
   return hipGetLastError();
 }

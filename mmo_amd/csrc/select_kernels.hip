@@ -514,8 +514,9 @@ __global__ void __launch_bounds__(1024) k_topk_sort(const TopkState* st, const u
 // The sort of the candidates takes 25, 45 and 91 us for 1,024, 2,048 and 4,096 of them, a pass 6
 // us up to some 4 M energies and 60 us for 36.9 M: few energies (or, for large k, as many as the
 // list holds) are sorted at once, and up to 4 M the passes go on until they have left 1,024 (or
-// k) candidates, beyond until the list holds them.  20,000 energies of seven values, k = 1 or 100: 159 us with 4,096, 75 and 84 now;
-// 4,096 energies, k = 1, sorted at once 112 to 121, 75 to 80 by passes; 3,000,000 normally distributed, k = 100, 196 and 75.
+// k) candidates, beyond until the list holds them.  20,000 energies of seven values, k = 1 or 100:
+// 159 us with 4,096, 75 and 84 now; 4,096 energies, k = 1, sorted at once 112 to 121, 75 to 80
+// by passes; 3,000,000 normally distributed, k = 100, 196 and 75.
 constexpr int kTopkSort = 2048;
 static unsigned topk_limit(size_t n, int k) {
   return n <= ((size_t)1 << 22) ? std::max(1024, k) : kTopkCand;
