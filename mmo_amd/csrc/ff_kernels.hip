@@ -649,6 +649,29 @@ __global__ void __launch_bounds__(256) k_pose_units(PoseUnitArgs a, Frame fr, co
   }
 }
 
+// a wavefront per pose
+__global__ void __launch_bounds__(256) k_unit_list(const int* pose_lig, const int* atom_off, const int* unit_off,
+                                                   int npose, const UnitLig* ligs, const int* sweep,
+                                                   UnitAtom* units) {
+  const int p = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  if (p >= npose) return;
+  const UnitLig l = ligs[pose_lig[p]];
+  UnitAtom* mine = units + (size_t)kUnitAtoms * unit_off[p];
+  const int slots = kUnitAtoms * (unit_off[p + 1] - unit_off[p]);
+  for (int j = threadIdx.x & (kWave - 1); j < slots; j += kWave) {
+    const int at = j < l.n_atoms ? sweep[l.sweep_at + j] : 0;
+    mine[j] = j < l.n_atoms ? UnitAtom{atom_off[p] + at, l.atom_base + at} : UnitAtom{-1, 0};
+  }
+}
+
+hipError_t launch_unit_list(const int* pose_lig, const int* atom_off, const int* unit_off, int npose,
+                            const UnitLig* ligs, const int* sweep, UnitAtom* units, hipStream_t s) {
+  if (npose == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_unit_list, dim3((npose + 3) / 4), dim3(256), 0, s, pose_lig, atom_off, unit_off, npose,
+                     ligs, sweep, units);
+  return hipGetLastError();
+}
+
 hipError_t launch_pose_units(const InterLaunch& L, const PoseUnitArgs& args, bool grad, int ncu,
                              hipStream_t s) {
   PoseUnitArgs a = args;

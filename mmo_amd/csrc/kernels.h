@@ -227,6 +227,10 @@ hipError_t launch_pose_cull(const InterLaunch& L, const PoseCullArgs& a, bool gr
 // shifted form per unit of kUnitAtoms ligand atoms (consecutive in the sweep order)
 constexpr int kUnitAtoms = 4;
 struct UnitAtom { int row, latom; };   // coordinate row, ligand-atom index; row < 0: none
+// the units of a batch, from its poses' ligands: atoms, first ligand atom, place in `sweep`
+struct UnitLig { int n_atoms, atom_base, sweep_at; };
+hipError_t launch_unit_list(const int* pose_lig, const int* atom_off, const int* unit_off, int npose,
+                            const UnitLig* ligs, const int* sweep, UnitAtom* units, hipStream_t s);
 struct PoseUnitArgs {
   const double* xyz;        // rows (x, y, z)
   const UnitAtom* units;    // kUnitAtoms per unit, pose-major
