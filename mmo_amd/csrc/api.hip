@@ -419,10 +419,30 @@ int upload(mmo_ctx* c, DevBuf<T>& b, const T* src, size_t n, hipStream_t s) {
 // terminal neighbours (hydrogens, halogens) right after it, so that a group of
 // consecutive atoms is a compact piece of the molecule.  Fragments follow one another.
 std::vector<int> sweep_order(const int32_t* dists, int n) {
-  std::vector<std::vector<int>> nb(n);
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j)
-      if (i != j && dists[i + (size_t)j * n] == 1) nb[i].push_back(j);
+  // the neighbours of every atom, ascending, one after the other; bonds are few, so the matrix is
+  // looked through 16 entries at a time
+  std::vector<std::pair<int, int>> bonds;
+  std::vector<int> first(n + 1, 0);
+  bonds.reserve(4 * (size_t)n);
+  for (int j = 0; j < n; ++j) {
+    const int32_t* d = dists + (size_t)j * n;
+    for (int i0 = 0; i0 < n; i0 += 16) {
+      const int i1 = std::min(n, i0 + 16);
+      int any = 0;
+      if (i1 - i0 == 16)
+        for (int i = 0; i < 16; ++i) any |= d[i0 + i] == 1;
+      else
+        for (int i = i0; i < i1; ++i) any |= d[i] == 1;
+      for (int i = i0; any && i < i1; ++i)
+        if (d[i] == 1 && i != j) {
+          bonds.push_back({i, j});
+          ++first[i + 1];
+        }
+    }
+  }
+  for (int i = 0; i < n; ++i) first[i + 1] += first[i];
+  std::vector<int> nb(bonds.size()), fill(first.begin(), first.end() - 1);
+  for (const auto& [i, j] : bonds) nb[fill[i]++] = j;
   std::vector<int> order;
   std::vector<char> seen(n, 0);
   std::vector<int> stack;
@@ -434,15 +454,17 @@ std::vector<int> sweep_order(const int32_t* dists, int n) {
       const int a = stack.back();
       stack.pop_back();
       order.push_back(a);
-      for (int b : nb[a])   // terminal neighbours now
-        if (!seen[b] && nb[b].size() <= 1) {
+      for (int k = first[a]; k < first[a + 1]; ++k) {   // terminal neighbours now
+        const int b = nb[k];
+        if (!seen[b] && first[b + 1] - first[b] <= 1) {
           seen[b] = 1;
           order.push_back(b);
         }
-      for (auto it = nb[a].rbegin(); it != nb[a].rend(); ++it)   // branches next, lowest first
-        if (!seen[*it]) {
-          seen[*it] = 1;
-          stack.push_back(*it);
+      }
+      for (int k = first[a + 1] - 1; k >= first[a]; --k)   // branches next, lowest first
+        if (!seen[nb[k]]) {
+          seen[nb[k]] = 1;
+          stack.push_back(nb[k]);
         }
     }
   }
@@ -455,6 +477,7 @@ std::vector<uint32_t> intra_pairs(const int32_t* dists, int n) {
   // hold distinct i and distinct j, so the lanes of one wavefront add their gradient
   // terms to distinct LDS words instead of all to atom i's.
   std::vector<uint32_t> out;
+  out.reserve(std::min((size_t)n * (n - 1) / 2, (size_t)1 << 16));
   for (int d = 1; d < n; ++d)
     for (int i = 0; i + d < n; ++i) {
       const int j = i + d;
@@ -469,15 +492,18 @@ std::vector<int> clash_order(const std::vector<double>& xyz, int n) {
   double c[3] = {0.0, 0.0, 0.0};
   for (int j = 0; j < n; ++j)
     for (int k = 0; k < 3; ++k) c[k] += xyz[3 * j + k] / n;
-  std::vector<std::pair<double, int>> far(n);
+  std::vector<uint64_t> far(n);   // the bits of a distance (not negative: in its order), then the atom
   for (int j = 0; j < n; ++j) {
     double d2 = 0.0;
     for (int k = 0; k < 3; ++k) d2 += (xyz[3 * j + k] - c[k]) * (xyz[3 * j + k] - c[k]);
-    far[j] = {std::isfinite(d2) ? -d2 : 0.0, j};
+    const float d = std::isfinite(d2) ? (float)d2 : 0.0f;
+    uint32_t bits;
+    std::memcpy(&bits, &d, sizeof bits);
+    far[j] = (uint64_t)~bits << 32 | (uint32_t)j;
   }
   std::sort(far.begin(), far.end());
   std::vector<int> order(n);
-  for (int j = 0; j < n; ++j) order[j] = far[j].second;
+  for (int j = 0; j < n; ++j) order[j] = (int)(uint32_t)far[j];
   return order;
 }
 
@@ -1448,31 +1474,30 @@ int mmo_ene_intra_grad(mmo_ctx* c, const double* xs, const double* ys, const dou
 // Rotation groups that are each one side of their bond, all seen from one end of the
 // molecule, are of this kind; groups facing each other are not.
 static bool torsions_free(const LigHost& h) {
-  const int R = (int)h.rb_left.size();
+  const int R = (int)h.rb_left.size(), W = (h.n + 63) / 64;
   if (h.n > kMaxFreeAtoms || (size_t)R * (h.rg_atoms.size() + R + h.n) > kMaxFreeWork) return false;
-  std::vector<char> in(h.n);
-  for (int k = 0; k < R; ++k) {
-    std::fill(in.begin(), in.end(), 0);
+  std::vector<uint64_t> groups((size_t)R * W, 0ull);
+  auto has = [&](int k, int j) { return (groups[(size_t)k * W + j / 64] >> (j % 64)) & 1; };
+  for (int k = 0; k < R; ++k)
     for (int m = h.rg_off[k]; m < h.rg_off[k + 1]; ++m) {
-      if (in[h.rg_atoms[m]]) return false;   // an atom listed twice
-      in[h.rg_atoms[m]] = 1;
+      const int j = h.rg_atoms[m];
+      if (has(k, j)) return false;   // an atom listed twice
+      groups[(size_t)k * W + j / 64] |= 1ull << (j % 64);
     }
+  for (int k = 0; k < R; ++k) {
     const int size = h.rg_off[k + 1] - h.rg_off[k];
     const int l = h.rb_left[k], r = h.rb_right[k];
     for (int q = k + 1; q < R; ++q) {
       const int lq = h.rb_left[q], rq = h.rb_right[q];
       int shared = 0;
-      bool has_l = false, has_r = false;   // ends of k in group q
-      for (int m = h.rg_off[q]; m < h.rg_off[q + 1]; ++m) {
-        shared += in[h.rg_atoms[m]];
-        has_l |= h.rg_atoms[m] == l;
-        has_r |= h.rg_atoms[m] == r;
-      }
-      const bool apart = shared == 0 && !in[lq] && !in[rq] && !has_l && !has_r;
+      for (int w = 0; w < W; ++w)
+        shared += __builtin_popcountll(groups[(size_t)k * W + w] & groups[(size_t)q * W + w]);
+      const bool has_l = has(q, l), has_r = has(q, r);   // ends of k in group q
+      const bool apart = shared == 0 && !has(k, lq) && !has(k, rq) && !has_l && !has_r;
       const bool carried = shared == size && (has_l || l == lq || l == rq) &&
                            (has_r || r == lq || r == rq);
       const bool within = shared == h.rg_off[q + 1] - h.rg_off[q] && !has_l && !has_r &&
-                          (in[lq] || lq == l || lq == r) && (in[rq] || rq == l || rq == r);
+                          (has(k, lq) || lq == l || lq == r) && (has(k, rq) || rq == l || rq == r);
       if (!apart && !carried && !within) return false;
     }
   }
