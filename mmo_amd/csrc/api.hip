@@ -147,7 +147,7 @@ struct LigHost {
   std::vector<int> anum, type;
   std::vector<uint32_t> pair_ij;
   // the same by the torsions a pair feels, and their round masks (mc_pair_order), once made
-  std::vector<uint32_t> mc_ij;
+  std::vector<uint32_t> mc_index;   // kNoPair: filled up
   std::vector<uint64_t> mc_mask;
   bool mc_made = false;
   std::vector<int> rb_left, rb_right, rg_off, rg_atoms;
@@ -231,11 +231,12 @@ struct mmo_ctx {
   // the chains' pair lists (McPairs), built when chains are first made
   int mc_pairs_version = -1;   // lig_version they were uploaded for
   std::vector<McPairs> mc_pairs;
-  DevBuf<McPairs> d_pe_lig;
+  DevBuf<char> pe_block;   // what the views are parts of
+  View<McPairs> d_pe_lig;
   DevBuf<uint32_t> d_pe_ij;
   DevBuf<double2> d_pe_qa;
   DevBuf<double> d_pe_b;
-  DevBuf<uint64_t> d_pe_mask;
+  View<uint64_t> d_pe_mask;
   int uff_version = 0;
   int mc_pool = 12;            // chains per CU up to which workgroups pool their sweeps
   int mc_keep_pairs = 1;       // chains keep their pair energies
@@ -639,80 +640,103 @@ void mc_pair_order(LigHost& h) {
     for (int m = h.rg_off[k]; m < h.rg_off[k + 1]; ++m)
       in[(size_t)h.rg_atoms[m] * sw + k / 64] |= 1ull << (k % 64);
   // atoms of the same groups form a class; per pair of classes the torsions it feels
-  std::map<std::vector<uint64_t>, int> classes;
-  std::vector<int> cls(h.n);
-  for (int j = 0; j < h.n; ++j)
-    cls[j] = classes.emplace(std::vector<uint64_t>(in.begin() + (size_t)j * sw, in.begin() + (size_t)(j + 1) * sw),
-                             (int)classes.size()).first->second;
-  const size_t nc = classes.size();
+  auto set_of = [&](int j) { return in.data() + (size_t)j * sw; };
+  auto less = [&](int a, int b) { return std::lexicographical_compare(set_of(a), set_of(a) + sw, set_of(b), set_of(b) + sw); };
+  std::vector<int> by_set(h.n), cls(h.n), first;   // first: an atom of each class
+  for (int j = 0; j < h.n; ++j) by_set[j] = j;
+  std::sort(by_set.begin(), by_set.end(), less);
+  for (int k = 0; k < h.n; ++k) {
+    if (k == 0 || less(by_set[k - 1], by_set[k])) first.push_back(by_set[k]);
+    cls[by_set[k]] = (int)first.size() - 1;
+  }
+  const size_t nc = first.size();
   if (nc * nc > kMcPairWork) return;
-  std::vector<const uint64_t*> sig(nc);
-  for (const auto& [key, k] : classes) sig[k] = key.data();
-  std::map<std::pair<int, std::vector<uint64_t>>, std::vector<uint32_t>> by;
-  std::vector<std::vector<uint32_t>*> list_of(nc * nc, nullptr);
-  std::vector<uint64_t> key(sw);
-  for (uint32_t p : h.pair_ij) {
-    const int ca = cls[p & 0xffff], cb = cls[p >> 16];
-    std::vector<uint32_t>*& list = list_of[ca * nc + cb];
-    if (!list) {
-      int bits = 0;
-      for (int w = 0; w < sw; ++w) {
-        key[w] = sig[ca][w] ^ sig[cb][w];
-        bits += __builtin_popcountll(key[w]);
-      }
-      list = &by[{bits, key}];
+  // the pairs of each two classes; those that feel the same torsions are one list
+  std::vector<uint32_t> count(nc * nc, 0u), place(np);
+  for (size_t p = 0; p < np; ++p) {
+    const size_t a = cls[h.pair_ij[p] & 0xffff], b = cls[h.pair_ij[p] >> 16];
+    place[p] = (uint32_t)(a < b ? a * nc + b : b * nc + a);
+    ++count[place[p]];
+  }
+  std::vector<uint64_t> key;   // of each two classes present: torsions, which, and the two's number
+  const size_t len = sw + 2;
+  for (size_t q = 0; q < nc * nc; ++q) {
+    if (count[q] == 0) continue;
+    key.resize(key.size() + len);
+    uint64_t* k = key.data() + key.size() - len;
+    for (int w = 0; w < sw; ++w) {
+      k[1 + w] = set_of(first[q / nc])[w] ^ set_of(first[q % nc])[w];
+      k[0] += __builtin_popcountll(k[1 + w]);
     }
-    list->push_back(p);
+    k[len - 1] = q;
   }
+  std::vector<const uint64_t*> order(key.size() / len);
+  for (size_t k = 0; k < order.size(); ++k) order[k] = key.data() + k * len;
+  std::sort(order.begin(), order.end(), [&](const uint64_t* a, const uint64_t* b) {
+    return std::lexicographical_compare(a, a + len, b, b + len);
+  });
   const size_t rounds = (np + kWave - 1) / kWave, words = (rounds + 63) / 64;
-  h.mc_ij.reserve(rounds * kWave);
+  h.mc_index.assign(rounds * kWave, kNoPair);
   h.mc_mask.assign((size_t)R * words, 0ull);
-  for (const auto& [k, list] : by) {
-    const size_t r0 = h.mc_ij.size() / kWave;
-    h.mc_ij.insert(h.mc_ij.end(), list.begin(), list.end());
-    const size_t r1 = (h.mc_ij.size() - 1) / kWave;
-    for (int b = 0; b < R; ++b)
-      if ((k.second[b / 64] >> (b % 64)) & 1)
-        for (size_t r = r0; r <= r1; ++r) h.mc_mask[(size_t)b * words + r / 64] |= 1ull << (r % 64);
+  std::vector<uint32_t> list_of(nc * nc, 0u), at;
+  uint32_t next = 0;
+  for (size_t k = 0; k < order.size();) {
+    const uint64_t* set = order[k] + 1;
+    const size_t r0 = next / kWave;
+    at.push_back(next);
+    for (; k < order.size() && std::equal(set, set + sw, order[k] + 1); ++k) {
+      list_of[order[k][len - 1]] = (uint32_t)at.size() - 1;
+      next += count[order[k][len - 1]];
+    }
+    const size_t r1 = (next - 1) / kWave;
+    for (int w = 0; w < sw; ++w)
+      for (uint64_t left = set[w]; left; left &= left - 1) {
+        uint64_t* mask = h.mc_mask.data() + (size_t)(64 * w + __builtin_ctzll(left)) * words;
+        for (size_t r = r0; r <= r1; ++r) mask[r / 64] |= 1ull << (r % 64);
+      }
   }
-  h.mc_ij.resize(rounds * kWave, 0u);
+  for (size_t p = 0; p < np; ++p) h.mc_index[at[list_of[place[p]]]++] = (uint32_t)p;
 }
 
-// the registry's McPairs on the device (after sync_ligands)
+// The registry's McPairs on the device (after sync_ligands).  The host orders the pairs once a
+// ligand; a kernel takes the pairs and their parameters from the registry's in that order.  Made
+// and uploaded by the host they were 1.5 ms of the first chains of 48 new ligands.
 int sync_mc_pairs(mmo_ctx* c) {
   if (c->mc_pairs_version == c->lig_version) return MMO_OK;
-  std::vector<uint32_t> ij;
-  std::vector<double4> pp;
-  std::vector<double2> qa;
-  std::vector<double> pb;
+  std::vector<uint32_t> index;
   std::vector<uint64_t> mask;
-  c->mc_pairs.clear();
+  size_t pair_base = 0, total = 0;
   for (LigHost& h : c->ligs) {
     mc_pair_order(h);
+    total += h.mc_index.size();
+  }
+  index.reserve(total);
+  c->mc_pairs.clear();
+  for (LigHost& h : c->ligs) {
     McPairs mp{};
-    mp.base = (int64_t)ij.size();
+    mp.base = (int64_t)index.size();
     mp.mask_base = (int64_t)mask.size();
-    mp.rounds = (int)(h.mc_ij.size() / kWave);
+    if (pair_base + h.pair_ij.size() < kNoPair) {   // the registry's pairs by 32-bit numbers
+      mp.rounds = (int)(h.mc_index.size() / kWave);
+      for (uint32_t p : h.mc_index) index.push_back(p == kNoPair ? p : (uint32_t)pair_base + p);
+      mask.insert(mask.end(), h.mc_mask.begin(), h.mc_mask.end());
+    }
     mp.words = (mp.rounds + 63) / 64;
     c->mc_pairs.push_back(mp);
-    int r = pair_params(c, h.mc_ij, h.q.data(), h.anum.data(), pp);
-    if (r) return r;
-    for (size_t p = h.pair_ij.size(); p < pp.size(); ++p) pp[p] = make_double4(0.0, 0.0, 0.0, 0.0);
-    for (const double4& v : pp) {
-      qa.push_back(make_double2(v.x, v.y));
-      pb.push_back(v.z);
-    }
-    ij.insert(ij.end(), h.mc_ij.begin(), h.mc_ij.end());
-    mask.insert(mask.end(), h.mc_mask.begin(), h.mc_mask.end());
+    pair_base += h.pair_ij.size();
   }
   hipStream_t s = c->stream;
-  int r;
-  if ((r = upload(c, c->d_pe_lig, c->mc_pairs.data(), c->mc_pairs.size(), s)) ||
-      (r = upload(c, c->d_pe_ij, ij.data(), ij.size(), s)) ||
-      (r = upload(c, c->d_pe_qa, qa.data(), qa.size(), s)) ||
-      (r = upload(c, c->d_pe_b, pb.data(), pb.size(), s)) ||
-      (r = upload(c, c->d_pe_mask, mask.data(), mask.size(), s)))
-    return r;
+  UploadBlock up;
+  View<uint32_t> d_index;
+  up.add(c->mc_pairs.data(), c->mc_pairs.size(), c->d_pe_lig);
+  up.add(mask.data(), mask.size(), c->d_pe_mask);
+  up.add(index.data(), index.size(), d_index);
+  HIPCHK(c, up.send(c->pe_block, s));
+  HIPCHK(c, c->d_pe_ij.ensure(index.size()));
+  HIPCHK(c, c->d_pe_qa.ensure(index.size()));
+  HIPCHK(c, c->d_pe_b.ensure(index.size()));
+  HIPCHK(c, launch_mc_pair_list(d_index.p, index.size(), c->d_pair_ij.p, c->d_pair_par.p, c->d_pe_ij.p,
+                                c->d_pe_qa.p, c->d_pe_b.p, s));
   HIPCHK(c, hipStreamSynchronize(s));
   c->mc_pairs_version = c->lig_version;
   return MMO_OK;
@@ -1030,7 +1054,7 @@ void mmo_ctx_destroy(mmo_ctx* c) {
     if (c->drain_stream) (void)hipStreamDestroy(c->drain_stream);
     c->d_ligs.release(); c->d_latoms.release(); c->d_lig_xyz.release();
     c->d_pair_ij.release(); c->d_pair_par.release();
-    c->d_pe_lig.release(); c->d_pe_ij.release(); c->d_pe_qa.release(); c->d_pe_b.release(); c->d_pe_mask.release(); c->d_intra_bits.release(); c->d_bit_base.release(); c->d_sweep.release(); c->d_clash.release();
+    c->pe_block.release(); c->d_pe_ij.release(); c->d_pe_qa.release(); c->d_pe_b.release(); c->d_intra_bits.release(); c->d_bit_base.release(); c->d_sweep.release(); c->d_clash.release();
     c->d_rb_left.release(); c->d_rb_right.release(); c->d_rg_off.release(); c->d_rg_atoms.release();
     c->s_xyz.release(); c->s_e.release(); c->s_g.release(); c->s_part.release();
     c->s_lig.release(); c->s_latom.release(); c->s_pij.release(); c->s_ppar.release();

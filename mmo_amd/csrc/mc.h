@@ -49,6 +49,11 @@ struct McPairs {
   int rounds, words;         // words of a mask
 };
 
+// their pairs and parameters from the registry's, by the numbers in `index` (kNoPair: no energy)
+constexpr uint32_t kNoPair = ~0u;
+hipError_t launch_mc_pair_list(const uint32_t* index, size_t n, const uint32_t* pair_ij, const double4* pair_par,
+                               uint32_t* ij, double2* qa, double* b, hipStream_t s);
+
 // chains a workgroup of the pooled form may run
 constexpr int kMcPoolSlots = 12;
 

@@ -1034,6 +1034,26 @@ __global__ void __launch_bounds__(64) k_mc_start(McArgs a) {
   for (int k = threadIdx.x; k < 3 * li.n_atoms; k += blockDim.x) a.conf[to + k] = a.best_xyz[to + k] = from[k];
 }
 
+__global__ void __launch_bounds__(256) k_mc_pair_list(const uint32_t* index, size_t n, const uint32_t* pair_ij,
+                                                      const double4* pair_par, uint32_t* ij, double2* qa,
+                                                      double* b) {
+  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const uint32_t p = index[k];
+  const double4 v = p == kNoPair ? make_double4(0.0, 0.0, 0.0, 0.0) : pair_par[p];
+  ij[k] = p == kNoPair ? 0u : pair_ij[p];
+  qa[k] = make_double2(v.x, v.y);
+  b[k] = v.z;
+}
+
+hipError_t launch_mc_pair_list(const uint32_t* index, size_t n, const uint32_t* pair_ij, const double4* pair_par,
+                               uint32_t* ij, double2* qa, double* b, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_mc_pair_list, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, index, n, pair_ij, pair_par,
+                     ij, qa, b);
+  return hipGetLastError();
+}
+
 hipError_t launch_mc_start(const McArgs& a, int nchain, hipStream_t s) {
   hipLaunchKernelGGL(k_mc_start, dim3(nchain), dim3(kWave), 0, s, a);
   return hipGetLastError();
