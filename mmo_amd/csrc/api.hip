@@ -303,14 +303,17 @@ struct mmo_mc {
   double beta = 0.0, roi[3] = {0.0, 0.0, 0.0}, roi_r = 0.0;
   std::vector<int> chain_lig, chain_atom, chain_rb, work, work_by_lig;
   std::vector<std::pair<int, int>> groups;   // (first, count) in work_by_lig per ligand
-  DevBuf<int> d_chain_lig, d_chain_atom, d_chain_rb, d_work, d_work_by_lig, d_queue;
+  DevBuf<char> block;        // what the views are parts of, and of `rows`
+  DevBuf<double> rows;
+  View<int> d_chain_lig, d_chain_atom, d_chain_rb, d_work, d_work_by_lig;
+  DevBuf<int> d_queue;
   DevBuf<McState> d_st;
-  DevBuf<double> d_conf, d_best, d_dr, d_undo;
+  View<double> d_conf, d_best, d_dr, d_undo;
   DevBuf<SwState> d_sw;
   // pair energies kept per chain, valid for the UFF parameters of pe_uff (-1: not yet)
   DevBuf<double> d_pe;
-  DevBuf<int64_t> d_pe_off;
-  DevBuf<uint64_t> d_pe_sel;
+  View<int64_t> d_pe_off;
+  View<uint64_t> d_pe_sel;
   int pe_words = 0, pe_uff = -1;
   DevBuf<float4> d_pool;   // pooled sweeps: their units' sums
   hipGraph_t graph = nullptr;
@@ -2264,7 +2267,7 @@ int mmo_grid_compute(mmo_ctx* c, const int32_t* probe_anum, const double* probe_
 // round (64 pairs) of each chain, 2 KB for a ligand of 132 atoms.  Above the bound, or without
 // that memory, the chains evaluate all pairs of every torsion proposal.
 constexpr size_t kMcPairBytes = (size_t)1 << 30;
-static int mc_keep_pairs(mmo_mc* m, hipStream_t s) {
+static int mc_keep_pairs(mmo_mc* m, UploadBlock& up) {
   mmo_ctx* c = m->ctx;
   if (!(m->flags & kMcTweak) || !(m->flags & kMcIntraUff) || !c->mc_keep_pairs) return MMO_OK;
   if (3 * (size_t)m->max_atoms * sizeof(double) > 65536) return MMO_OK;   // k_mc_pairs' LDS
@@ -2286,8 +2289,9 @@ static int mc_keep_pairs(mmo_mc* m, hipStream_t s) {
   }
   std::vector<uint64_t> sel((size_t)m->nchain * words, 0ull);
   m->pe_words = words;
-  if ((r = upload(c, m->d_pe_off, off.data(), off.size(), s))) return r;
-  return upload(c, m->d_pe_sel, sel.data(), sel.size(), s);
+  up.add(off.data(), off.size(), m->d_pe_off);
+  up.add(sel.data(), sel.size(), m->d_pe_sel);
+  return MMO_OK;
 }
 
 static McArgs mc_args(mmo_mc* m, int nsteps, int nwork, const int* work);
@@ -2377,8 +2381,6 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
     }
   }
   std::vector<double> dr(std::max(m->nrb, 1), 5.0 * deg);   // Params.max_rbond_rot
-  std::vector<SwState> sw(std::max(m->nrb, 1));
-  std::memset(sw.data(), 0, sw.size() * sizeof(SwState));
   // processing order: most expensive chains first (atoms and intra pairs)
   m->work.resize(nchain);
   for (int k = 0; k < nchain; ++k) m->work[k] = k;
@@ -2399,27 +2401,33 @@ int mmo_mc_create(mmo_ctx* c, const int32_t* chain_lig, int nchain, const double
     k = e;
   }
   hipStream_t s = c->stream;
-  if ((r = upload(c, m->d_chain_lig, m->chain_lig.data(), nchain, s)) ||
-      (r = upload(c, m->d_chain_atom, m->chain_atom.data(), nchain, s)) ||
-      (r = upload(c, m->d_chain_rb, m->chain_rb.data(), nchain, s)) ||
-      (r = upload(c, m->d_work, m->work.data(), nchain, s)) ||
-      (r = upload(c, m->d_work_by_lig, m->work_by_lig.data(), nchain, s)) ||
-      (r = upload(c, m->d_st, st.data(), st.size(), s)) ||
-      (r = upload(c, m->d_dr, dr.data(), dr.size(), s)) ||
-      (r = upload(c, m->d_sw, sw.data(), sw.size(), s))) {
+  UploadBlock up;
+  up.add(m->chain_lig.data(), nchain, m->d_chain_lig);
+  up.add(m->chain_atom.data(), nchain, m->d_chain_atom);
+  up.add(m->chain_rb.data(), nchain, m->d_chain_rb);
+  up.add(m->work.data(), nchain, m->d_work);
+  up.add(m->work_by_lig.data(), nchain, m->d_work_by_lig);
+  up.add(dr.data(), dr.size(), m->d_dr);
+  if ((r = mc_keep_pairs(m, up)) || (r = upload(c, m->d_st, st.data(), st.size(), s))) {
     delete m;
     return r;
   }
-  hipError_t e = hipSuccess;
-  for (DevBuf<double>* v : {&m->d_conf, &m->d_best, &m->d_undo})
-    if (e == hipSuccess) e = v->ensure(3 * (size_t)m->natoms);
+  const size_t rows = 3 * (size_t)m->natoms, nsw = std::max(m->nrb, 1);
+  hipError_t e = up.send(m->block, s);
+  if (e == hipSuccess) e = m->rows.ensure(3 * rows);
+  if (e == hipSuccess) e = m->d_sw.ensure(nsw);
   if (e != hipSuccess) {
     delete m;
     return fail(c, MMO_ERR_NOMEM, "Monte Carlo conformers: %s", hipGetErrorString(e));
   }
-  if ((r = sync_ligands(c)) || (r = mc_keep_pairs(m, s))) {
+  m->d_conf.p = m->rows.p;
+  m->d_best.p = m->rows.p + rows;
+  m->d_undo.p = m->rows.p + 2 * rows;
+  static_assert(sizeof(SwState) % sizeof(int) == 0, "cleared as words");
+  e = launch_fill_int(reinterpret_cast<int*>(m->d_sw.p), nsw * (sizeof(SwState) / sizeof(int)), 0, s);
+  if (e != hipSuccess) {
     delete m;
-    return r;
+    return fail(c, MMO_ERR_DEVICE, "Monte Carlo setup: %s", hipGetErrorString(e));
   }
   // pooled sweeps, where the chains' launches will have some (a run in a caller's capture cannot
   // allocate them); without the memory the chains do without
@@ -2737,10 +2745,8 @@ void mmo_mc_destroy(mmo_mc* m) {
     (void)hipDeviceSynchronize();
     if (m->gexec) (void)hipGraphExecDestroy(m->gexec);
     if (m->graph) (void)hipGraphDestroy(m->graph);
-    m->d_chain_lig.release(); m->d_chain_atom.release(); m->d_chain_rb.release();
-    m->d_work.release(); m->d_work_by_lig.release(); m->d_queue.release(); m->d_st.release();
-    m->d_conf.release(); m->d_best.release(); m->d_dr.release(); m->d_undo.release(); m->d_sw.release();
-    m->d_pool.release(); m->d_pe.release(); m->d_pe_off.release(); m->d_pe_sel.release();
+    m->block.release(); m->rows.release(); m->d_queue.release(); m->d_st.release();
+    m->d_sw.release(); m->d_pool.release(); m->d_pe.release();
     m->d_min_base.release(); m->d_min_S.release(); m->d_min_Y.release(); m->d_min_rho.release();
   }
   delete m;
