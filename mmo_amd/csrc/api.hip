@@ -2522,7 +2522,12 @@ static McShape mc_shape(const mmo_mc* m, McArgs a, int nwork) {
   const size_t cap = 160 * 1024;
   McShape g{};
   g.rec_lds = m->inter_mode != MMO_INTERP && m->ctx->cullp_ok && m->ctx->mc_rec_lds;
-  const int wmax = std::min(mc_max_waves(a), m->ctx->mc_wg_waves);
+  int wmax = std::min(mc_max_waves(a), m->ctx->mc_wg_waves);
+  // Few minimising chains: one a SIMD, on more CUs, rather than eight a workgroup on a few.  Two
+  // long chains on a SIMD take their time from each other, and which two meet differs from build
+  // to build: ms per 8 frames, eight a workgroup (two builds) and this: 64 chains on the grids
+  // 2.11, 2.34, 1.96, 200 2.07, 2.37, 1.97; 500 direct 7.86, 8.96, 7.14, 1,000 8.12, 9.13, 7.26.
+  if (a.min_iters > 0) wmax = std::min(wmax, std::max(4, (nwork + m->ctx->ncu - 1) / m->ctx->ncu));
   g.waves = wmax;
   while (g.waves > 1 && mc_lds_bytes(a, g.waves, g.rec_lds) > cap) --g.waves;
   if (g.rec_lds && (g.waves < std::min(4, wmax) || mc_lds_bytes(a, g.waves, g.rec_lds) > cap)) {
