@@ -97,9 +97,14 @@ hipError_t launch_mask_cells(const uint32_t* mask, uint32_t* cells, int nx, int 
 // Whether an atom at (x, y, z) has a protein-volume voxel among its 8 corners.  Corners
 // outside the grid count as free: the conversion truncates as int_of_float and saturates,
 // so 0 <= i < nx - 1 is the cell test (coordinates are finite, see clash_coord).
+__device__ __forceinline__ uint32_t trunc_sat(double v) {
+  int i;   // the instruction: a conversion out of int's range is undefined in C++
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(i) : "v"(v));
+  return (uint32_t)i;
+}
 __device__ __forceinline__ uint32_t atom_cell(const ScanFilterArgs& a, double x, double y, double z) {
-  const uint32_t i = (uint32_t)(int)((x - a.ox) * a.inv_step), j = (uint32_t)(int)((y - a.oy) * a.inv_step),
-                 k = (uint32_t)(int)((z - a.oz) * a.inv_step);
+  const uint32_t i = trunc_sat((x - a.ox) * a.inv_step), j = trunc_sat((y - a.oy) * a.inv_step),
+                 k = trunc_sat((z - a.oz) * a.inv_step);
   if (!(i < (uint32_t)a.nx - 1u && j < (uint32_t)a.ny - 1u && k < (uint32_t)a.nz - 1u)) return ~0u;
   return i + (uint32_t)a.nx * (j + (uint32_t)a.ny * k);   // fewer than 2^31 voxels
 }
