@@ -758,7 +758,6 @@ InterLaunch inter_launch(mmo_ctx* c, int mode, const LigInfo* ligs, const LigAto
   L.cull_k = c->cull_k;
   L.row_chunk = c->scan_chunk;
   L.row_filter = c->row_filter;
-  L.atom_order = nullptr;
   L.n_atoms = 0;
   L.part = nullptr;
   L.cg = c->cg;
@@ -863,7 +862,6 @@ InterLaunch scan_launch(mmo_ctx* c, int mode, int scan_cull) {
     L.rpos = c->rpos_s.p; L.rab = c->rab_s.p; L.rres = c->rres_s.p;
     L.row_chunk = c->scan_chunk;
     L.row_filter = c->row_filter;
-    L.atom_order = c->d_sweep.p;
     return L;
   }
   if (mode == MMO_SHIFTED && scan_cull) {

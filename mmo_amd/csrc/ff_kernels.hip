@@ -111,7 +111,6 @@ struct InterArgs {
   int write_e;        // GRAD kernel: also write E
   int rslice;         // receptor atoms per gridDim.y slice
   int npose_total;    // for partial outputs when gridDim.y > 1
-  const int* atom_order;   // nullable: per ligand at atom_base, the sweeps' atom order
   // k_scan_rows with few tiles: gridDim.y = the ligand's atoms, one per wavefront, their
   // energies to part[(atom * ntiles + tile) * 64 + lane] for k_scan_sum (nullptr: one
   // wavefront sums all atoms of its tile)
@@ -1163,7 +1162,7 @@ hipError_t launch_inter_coords(const InterLaunch& L, const Tile* tiles, const in
   a.src.xyz = xyz; a.src.atom_off = atom_off; a.src.tiles = tiles; a.src.perm = perm;
   a.ntiles = ntiles; a.fr = L.fr; a.rpos = L.rpos; a.rab = L.rab; a.rres = L.rres; a.nrec = L.nrec;
   a.rtile = L.rtile; a.ligs = L.ligs; a.latoms = L.latoms; a.lig_xyz = L.lig_xyz;
-  a.e_stride = e_stride; a.grad = grad; a.write_e = write_e; a.atom_order = nullptr;
+  a.e_stride = e_stride; a.grad = grad; a.write_e = write_e;
   a.part = nullptr;
   a.rslice = L.rslice > 0 ? L.rslice : L.nrec;
   a.npose_total = npose;
@@ -1280,7 +1279,7 @@ hipError_t launch_inter_scan(const InterLaunch& L, int lig, const double* rots, 
   a.ntiles = nrot * a.src.tiles_per_rot; a.fr = L.fr; a.rpos = L.rpos; a.rab = L.rab; a.rres = L.rres;
   a.nrec = L.nrec; a.rtile = L.rtile; a.ligs = L.ligs; a.latoms = L.latoms;
   a.lig_xyz = L.lig_xyz; a.e_out = e_out; a.e_stride = 1; a.e_comp = nullptr; a.grad = nullptr;
-  a.write_e = 1; a.rslice = L.nrec; a.npose_total = nrot * ntrans; a.atom_order = L.atom_order;
+  a.write_e = 1; a.rslice = L.nrec; a.npose_total = nrot * ntrans;
   a.part = L.part;
   if (L.cull) return launch_cull(L, a, s);
   return launch_inter_any(L.mode, L.k, false, a, L.waves, s);
@@ -1296,7 +1295,7 @@ hipError_t launch_inter_scan_list(const InterLaunch& L, int lig, const double* r
   a.ntiles = (nlist + kWave - 1) / kWave; a.fr = L.fr; a.rpos = L.rpos; a.rab = L.rab;
   a.rres = L.rres; a.nrec = L.nrec; a.rtile = L.rtile; a.ligs = L.ligs; a.latoms = L.latoms;
   a.lig_xyz = L.lig_xyz; a.e_out = e_out; a.e_stride = 1; a.e_comp = nullptr; a.grad = nullptr;
-  a.write_e = 1; a.rslice = L.nrec; a.npose_total = nlist; a.atom_order = L.atom_order;
+  a.write_e = 1; a.rslice = L.nrec; a.npose_total = nlist;
   a.part = L.part;
   return launch_cull(L, a, s);
 }

@@ -19,7 +19,6 @@ struct InterLaunch {
   int cull_k;          // ligand atoms per lane in the culled kernel (1, 2, 4)
   int row_chunk;       // k_scan_rows: receptor atoms fetched at once (4 or 8)
   int row_filter;      // k_scan_rows: far rows' atoms tested against the box first (0 / 1)
-  const int* atom_order;   // nullable: per ligand at atom_base, the sweeps' atom order
   // k_scan_rows: atoms of the scan's ligand; with `part` (n_atoms x 64 x tiles doubles) one
   // of them per wavefront
   int n_atoms;
