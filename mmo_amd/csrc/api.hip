@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <exception>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -104,18 +105,18 @@ template <class T>
 struct View { T* p = nullptr; };
 struct UploadBlock {
   std::vector<char> bytes;
-  std::vector<std::pair<size_t, void**>> at;
+  std::vector<std::pair<size_t, std::function<void(char*)>>> at;
   template <class T>
   void add(const T* src, size_t n, View<T>& out) {
     const size_t o = (bytes.size() + 15) & ~(size_t)15;
     bytes.resize(o + std::max<size_t>(n, 1) * sizeof(T));
     if (n) std::memcpy(bytes.data() + o, src, n * sizeof(T));
-    at.push_back({o, reinterpret_cast<void**>(&out.p)});
+    at.push_back({o, [&out](char* p) { out.p = reinterpret_cast<T*>(p); }});
   }
   hipError_t send(DevBuf<char>& to, hipStream_t s) {
     hipError_t e = to.ensure(bytes.size());
     if (e != hipSuccess) return e;
-    for (auto& v : at) *v.second = to.p + v.first;
+    for (auto& v : at) v.second(to.p + v.first);
     return hipMemcpyAsync(to.p, bytes.data(), bytes.size(), hipMemcpyHostToDevice, s);
   }
 };
