@@ -981,12 +981,19 @@ bool lattice_scan(const mmo_ctx* c, int nrot, const double* trans, int ntrans,
   const double* z = axes.data() + la.n[0] + la.n[1];
   for (int k = 1; k < nz; ++k)   // also false for a z that is not a number
     if (!(z[k] >= z[k - 1] && (z[k] - z[k - 1]) * c->g.ods <= 4.0)) return false;
+  la.ztile = kLatticeZ;
+  const size_t short_units = lattice_units(la);
+  la.ztile = kLatticeLongZ;
+  const size_t long_units = lattice_units(la);
+  if (long_units == short_units || (z[nz - 1] - z[0]) * c->g.ods > 2.25 * (nz - 1) ||
+      (long_units < kLatticeLongUnits && !(long_units <= 5120 && short_units > 6000)))
+    la.ztile = kLatticeZ;
   if (c->scan_lattice == 2) return true;
-  const int ztiles = lattice_tiles(nz);
+  const int ztiles = lattice_tiles(nz, la.ztile);
   double cycles = 0.0;   // of one column tile's wavefronts
   for (int t = 0; t < ztiles; ++t) {
     int z0, zn;
-    lattice_tile(nz, t, z0, zn);
+    lattice_tile(nz, la.ztile, t, z0, zn);
     cycles += 150.0 + 130.0 * ((z[z0 + zn - 1] - z[z0]) * c->g.ods + 2.0) + 8.0 * zn;
   }
   const double units = std::max((double)lattice_units(la), 2800.0);

@@ -1004,14 +1004,14 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<Src> a) {
 // same bits as k_interp gives the pose.
 // Bound: the address rate of the two gathered pairs a layer (16 cycles each per CU; reading
 // the corners one by one, as k_interp does, takes 8 of them a pose).  36.9 M poses, 75 atoms,
-// 64^3 grids: 3.89 ms, k_interp 9.6 ms.
+// 64^3 grids: 3.85 ms, k_interp 9.6 ms.
 template <int ZC>
 __global__ void __launch_bounds__(256) k_interp_lattice(LatticeArgs a) {
   typedef float pair_f __attribute__((ext_vector_type(2)));
   typedef unsigned pair_u __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & (kWave - 1);
   const int nx = a.n[0], ny = a.n[1], nz = a.n[2];
-  const int col_tiles = (nx * ny + kWave - 1) / kWave, z_tiles = lattice_tiles(nz);
+  const int col_tiles = (nx * ny + kWave - 1) / kWave, z_tiles = lattice_tiles(nz, ZC);
   const int unit = uniformi(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave);
   const int rot = unit / (col_tiles * z_tiles);
   if (rot >= a.nrot) return;
@@ -1021,7 +1021,7 @@ __global__ void __launch_bounds__(256) k_interp_lattice(LatticeArgs a) {
   const bool col_ok = col < nx * ny;
   const int iy = col_ok ? col / nx : 0, ix = col_ok ? col - iy * nx : 0;
   int z0, zn;
-  lattice_tile(nz, zt, z0, zn);
+  lattice_tile(nz, ZC, zt, z0, zn);
   const double tx = a.axes[ix], ty = a.axes[nx + iy];
   const double tz = a.axes[nx + ny + z0 + (lane < zn ? lane : 0)];   // lane = z
   const LigInfo li = a.ligs[a.lig];
@@ -1090,10 +1090,11 @@ __global__ void __launch_bounds__(256) k_interp_lattice(LatticeArgs a) {
 }
 
 hipError_t launch_interp_lattice(const LatticeArgs& a, hipStream_t s) {
-  constexpr int ZC = kLatticeZ;
   const size_t units = lattice_units(a);
   if (units == 0) return hipSuccess;
-  hipLaunchKernelGGL((k_interp_lattice<ZC>), dim3((unsigned)((units + 3) / 4)), dim3(4 * kWave), 0, s, a);
+  const dim3 grid((unsigned)((units + 3) / 4)), block(4 * kWave);
+  if (a.ztile == kLatticeLongZ) hipLaunchKernelGGL((k_interp_lattice<kLatticeLongZ>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_interp_lattice<kLatticeZ>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 

@@ -59,6 +59,7 @@ struct LatticeArgs {
   const double* rots;          // nrot x 9
   const double* axes;          // the n[0] x, n[1] y and n[2] z values
   int nrot, ntrans, n[3], stride[3];   // translation of (i, j, k) = i stride[0] + ...
+  int ztile;                   // z positions of one wavefront, at most
   GridDev g;
   uint32_t grid_bytes;         // of all types' grids together (below 2 GiB)
   const LigInfo* ligs;
@@ -71,17 +72,26 @@ struct LatticeArgs {
 // kernel at steps of 0.375, 0.5, 0.75 and 1 A (8 to 40 z, 23 to 131 atoms, mean): 10 2.71, 2.14, 1.92,
 // 1.32 times its speed, 12 2.77, 2.17, 1.93, 1.31, 13 2.77, 2.16, 1.91, 1.31, 16 (5 wavefronts)
 // 2.67, 2.08, 1.84, 1.26, 20 2.62, 2.02, 1.81, 1.25, 24 (4 wavefronts) 2.81, 2.10, 1.84, 1.25
-constexpr int kLatticeZ = 12;
+// Up to 20 (5 wavefronts) instead where that saves tiles, the z are at most 2.25 layers apart, so
+// that the two layers read again at each border count, and the wavefronts are at least 20,480 (four
+// rounds of the chip) or one round in these tiles (5,120) but more or nearly so in the others
+// (6,000 of 7,168): 4,608 rotations of 20^3 at 0.5 A 3.94 -> 3.85 ms; 5,120 to 16,000 rotations of
+// 16 x 16 columns, 23 to 131 atoms, 13 z 9 to 24 % less time at 0.375, 0.5 and 0.56 A, 4 to 12 % at 0.75,
+// 20 z 0 to 12 % and -5 to 4 %, 28 to 40 z 4 to 16 %; in one round 9 to 29 %.  With other numbers of
+// wavefronts the shorter chain counts: 13 to 20 z of 200 rotations take 0.55 to 0.65 times as long in
+// two tiles; at 1 A and 3,000 rotations 0.85 to 0.98.
+constexpr int kLatticeZ = 12, kLatticeLongZ = 20;
+constexpr size_t kLatticeLongUnits = 20480;
 // The z axis in as few tiles as that allows, of equal length but for one: tile t's first z and
 // their number
-__host__ __device__ inline int lattice_tiles(int nz) { return (nz + kLatticeZ - 1) / kLatticeZ; }
-__host__ __device__ inline void lattice_tile(int nz, int t, int& z0, int& zn) {
-  const int tiles = lattice_tiles(nz), len = nz / tiles, longer = nz - len * tiles;
+__host__ __device__ inline int lattice_tiles(int nz, int ztile) { return (nz + ztile - 1) / ztile; }
+__host__ __device__ inline void lattice_tile(int nz, int ztile, int t, int& z0, int& zn) {
+  const int tiles = lattice_tiles(nz, ztile), len = nz / tiles, longer = nz - len * tiles;
   z0 = t * len + (t < longer ? t : longer);
   zn = len + (t < longer ? 1 : 0);
 }
 inline size_t lattice_units(const LatticeArgs& a) {
-  return (size_t)a.nrot * (((size_t)a.n[0] * a.n[1] + kWave - 1) / kWave) * lattice_tiles(a.n[2]);
+  return (size_t)a.nrot * (((size_t)a.n[0] * a.n[1] + kWave - 1) / kWave) * lattice_tiles(a.n[2], a.ztile);
 }
 hipError_t launch_interp_lattice(const LatticeArgs& a, hipStream_t s);
 
