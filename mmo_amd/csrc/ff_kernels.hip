@@ -953,38 +953,46 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<Src> a) {
   double e = 0.0;
   int bad = 0;
   if (pose_ok) {
-    for (int j = aslot; j < li.n_atoms; j += split) {
-      if constexpr (std::is_base_of<ScanSrc, Src>::value) {
-        const int r = pose / a.src.ntrans, tr = pose - r * a.src.ntrans;
-        const double* R = a.src.rots + 9 * (size_t)r;
-        const double* T = a.src.trans + 3 * (size_t)tr;
+    if constexpr (std::is_base_of<ScanSrc, Src>::value) {
+      const int r = pose / a.src.ntrans, tr = pose - r * a.src.ntrans;
+      const double* R = a.src.rots + 9 * (size_t)r;
+      const double* T = a.src.trans + 3 * (size_t)tr;
+      auto add = [&](int j) {
         const double* c = a.lig_xyz + 3 * (size_t)(li.atom_base + j);
         const AxisCell cx = axis_cell(a.g, rotate_shift(R, c, T[0]) - a.g.ox, a.g.nx),
                        cy = axis_cell(a.g, rotate_shift(R + 3, c, T[1]) - a.g.oy, a.g.ny),
                        cz = axis_cell(a.g, rotate_shift(R + 6, c, T[2]) - a.g.oz, a.g.nz);
-        if (!(cx.in && cy.in && cz.in)) {   // NaN whatever the other atoms give
-          bad = 1;
-          break;
-        }
+        bad |= !(cx.in && cy.in && cz.in);
         float v[8];
         grid_corners<CELLS>(a.g, a.latoms[li.atom_base + j].type, cx.i, cy.i, cz.i, v);
         const LayerWeights lw = layer_weights(cx, cy);
         e += between_layers(layer_value(lw, v[0], v[1], v[2], v[3]),
                             layer_value(lw, v[4], v[5], v[6], v[7]), cz.w);
-        continue;
+      };
+      // a pose with an atom outside the grid is NaN whatever its other atoms give.  Asked once for
+      // two atoms: after each, launches of one wavefront a SIMD take 4 to 7 % longer (100 x 5^3 poses,
+      // 131 atoms 87 -> 81 us a call); four at once hold 74 VGPRs, 4,608 x 10^3 poses 5 % longer
+      int j = aslot;
+      for (; j + split < li.n_atoms && !bad; j += 2 * split) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) add(j + u * split);
       }
-      double x, y, z;
-      a.src.pos(pose, pslot, j, li, a.latoms, a.lig_xyz, x, y, z);
-      const int ty = a.type_override ? a.type_override[j] : a.latoms[li.atom_base + j].type;
-      bool ok = true;
-      double dg[3] = {0.0, 0.0, 0.0};
-      e += trilin<GRAD, CELLS>(a.g, ty, x - a.g.ox, y - a.g.oy, z - a.g.oz, ok, dg);
-      if (!ok) bad = 1;
-      if (GRAD) {
-        double* gr = a.grad + 3 * (size_t)a.src.row(pose, j);
-        if (!ok) dg[0] = dg[1] = dg[2] = __builtin_nan("");
-        if (a.grad_accumulate) { gr[0] += dg[0]; gr[1] += dg[1]; gr[2] += dg[2]; }
-        else { gr[0] = dg[0]; gr[1] = dg[1]; gr[2] = dg[2]; }
+      for (; j < li.n_atoms && !bad; j += split) add(j);
+    } else {
+      for (int j = aslot; j < li.n_atoms; j += split) {
+        double x, y, z;
+        a.src.pos(pose, pslot, j, li, a.latoms, a.lig_xyz, x, y, z);
+        const int ty = a.type_override ? a.type_override[j] : a.latoms[li.atom_base + j].type;
+        bool ok = true;
+        double dg[3] = {0.0, 0.0, 0.0};
+        e += trilin<GRAD, CELLS>(a.g, ty, x - a.g.ox, y - a.g.oy, z - a.g.oz, ok, dg);
+        if (!ok) bad = 1;
+        if (GRAD) {
+          double* gr = a.grad + 3 * (size_t)a.src.row(pose, j);
+          if (!ok) dg[0] = dg[1] = dg[2] = __builtin_nan("");
+          if (a.grad_accumulate) { gr[0] += dg[0]; gr[1] += dg[1]; gr[2] += dg[2]; }
+          else { gr[0] = dg[0]; gr[1] = dg[1]; gr[2] = dg[2]; }
+        }
       }
     }
   }
