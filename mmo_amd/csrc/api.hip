@@ -1337,16 +1337,20 @@ static int plain_inter(mmo_ctx* c, int mode, const double* xs, const double* ys,
   const bool grad = gx != nullptr;
   // one pose: a wavefront per 64 receptor atoms (the FP32 sums end there anyway), each lane
   // no more ligand atoms than it must: the serial loop of a lane is the time of the launch.
-  // 75 against 3,000 atoms: slices of 256 and four atoms a lane 73 us, now 16 us.  On large
-  // receptors the slices' sums and their additions to one gradient cost more than the loop: from
-  // 32,768 atoms on larger slices, up to 256.  us a call, slices of 64 / 128 / 256, energy and
-  // gradient of 75 atoms: 15,000 atoms 97 92 110, 126 125 145; 60,000 140 116 122, 193 161 165;
-  // 120,000 200 151 139, 297 211 189; 1,000,000 1145 643 393, 1696 930 550 (of 1,000 atoms 1619
-  // 1087 865, 2438 1657 1601; 512 would be slower for those from 250,000 atoms down).
+  // 75 against 3,000 atoms: slices of 256 and four atoms a lane 73 us, now 16 us.  A slice costs
+  // its sums (and its additions to one gradient, the more the more ligand atoms), its loop
+  // slice x k x passes pairs a lane, so the best length goes with the root of receptor atoms
+  // over pairs a lane.  us a call, slices of 64 / 128 / 256, energy and gradient: 75 ligand atoms,
+  // 15,000 receptor atoms 91 91 106, 118 118 142; 120,000 196 143 134, 286 198 177; 1,000,000 1184 658
+  // 397, 1720 929 550; 1,000, 15,000 170 225 351, 255 326 518; 120,000 292 282 389, 560 482 593;
+  // 1,000,000 1612 1095 870, 2375 1698 1522; 5,000, 120,000 680 879 1539, 1305 1436 2413; 1,000,000
+  // 3629 3099 2986, 7129 5118 5343.
   InterLaunch L = inter_launch(c, mode, c->s_lig.p, c->s_latom.p, nullptr);
-  L.rslice = 64 * std::min(4, (c->nrec + 32767) / 32768);
   if (n <= kWave) L.k = 1;
   else if (n <= 2 * kWave) L.k = 2;
+  const int pairs = (n + L.k * kWave - 1) / (L.k * kWave) * L.k;   // ligand atoms of a lane
+  const double length = std::sqrt(c->nrec * (1.0 + n / (grad ? 2000.0 : 6000.0)) / pairs);
+  L.rslice = length < 90.0 ? 64 : length < 157.0 ? 128 : length < 222.0 ? 192 : 256;
   L.rtile = std::min(L.rtile, L.rslice);
   L.waves = 1;
   const int nslice = (c->nrec + L.rslice - 1) / L.rslice;

@@ -1,6 +1,7 @@
 """One pose against large receptors."""
 import numpy as np
 import pytest
+from scipy.spatial import cKDTree
 
 import oracle
 from mmo_amd import ff, synth
@@ -13,8 +14,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nrec", [32768, 32769, 98305])
 @pytest.mark.parametrize("atoms", [30, 131])
 def test_plain_forms_at_slice_lengths(nrec, atoms):
-    """Receptors on either side of the sizes at which the slices of one pose grow from 64 atoms to
-    128 and 256, the last slice with one atom: energy, parts and gradient, both modes."""
+    """Slices of one pose of 128, 192 and 256 receptor atoms, whole ones and with a last one of one
+    atom: energy, parts and gradient, both modes."""
     base = synth.config4_receptor()
     rng = np.random.default_rng(nrec + atoms)
     x = np.concatenate([np.stack([base["xs"], base["ys"], base["zs"]], 1) + 62.0 * np.array(s)
@@ -38,3 +39,31 @@ def test_plain_forms_at_slice_lengths(nrec, atoms):
         want, gwant = oracle.grad_inter(rec, lig, shifted=shifted)
         assert_energy(e, want, s, what="plain gradient's energy")
         assert_grad(g, gwant, what="plain gradient")
+
+
+@pytest.mark.parametrize("nrec, atoms", [(8200, 40), (20001, 1000), (60001, 300)])
+def test_plain_forms_of_many_ligand_atoms(nrec, atoms):
+    """Slices that depend on the ligand's atoms too (64 and 128, the last with a remainder): energy,
+    parts and gradient against the oracle."""
+    base = synth.config4_receptor()
+    rng = np.random.default_rng(atoms + nrec)
+    x = np.concatenate([np.stack([base["xs"], base["ys"], base["zs"]], 1) + 62.0 * np.array(s)
+                        for s in ((0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 0), (1, 0, 1), (0, 1, 1), (1, 1, 1))])
+    pick = np.sort(rng.permutation(len(x))[:nrec])
+    x = x[pick]
+    rec = {"xs": x[:, 0].copy(), "ys": x[:, 1].copy(), "zs": x[:, 2].copy(),
+           "q": np.tile(base["q"], 8)[pick], "anum": np.tile(base["anum"], 8)[pick].astype(np.int32)}
+    ctx = ff.Context(0)
+    ctx.set_receptor(rec)
+    p = rng.uniform(0.0, 62.0, (50 * atoms, 3))
+    p = p[cKDTree(x).query(p)[0] > 1.8][:atoms]   # no clash hides the other pairs
+    assert len(p) == atoms
+    lig = {"xs": p[:, 0].copy(), "ys": p[:, 1].copy(), "zs": p[:, 2].copy(),
+           "q": rng.uniform(-0.3, 0.3, atoms), "anum": rng.choice([1, 6, 7, 8], atoms).astype(np.int32)}
+    s = inter_abs_sum(rec, p, lig, True)
+    got = ctx.ene_inter(lig, ff.SHIFTED, components=True)
+    assert_energy(got, oracle.ene_inter(rec, lig, shifted=True, components=True), [s, s, s], what="plain")
+    e, g = ctx.ene_inter_grad(lig, ff.SHIFTED)
+    want, gwant = oracle.grad_inter(rec, lig, shifted=True)
+    assert_energy(e, want, s, what="plain gradient's energy")
+    assert_grad(g, gwant, what="plain gradient")
