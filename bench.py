@@ -39,6 +39,7 @@ PEAK_HBM_GBS = 8000.0
 # L2 read bandwidth: 16 channels of 128 B per clock in each XCD's L2, 8 XCDs, 2.4 GHz
 # (the L2 structure AMD documents for CDNA 3, kept on CDNA 4; no MI355X figure is published)
 PEAK_L2_GBS = 8 * 16 * 128 * 2.4
+PEAK_GATHERS = 256 * 2.4 / 16   # G wavefront gathers/s: 256 CUs, 16 cycles each
 N_ROT, N_TRANS_SIDE, TRANS_STEP = 4608, 20, 0.5
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 
@@ -104,6 +105,21 @@ def gather_roofline(nbytes, kernel_ms, kernel, traffic=None, **more):
         r["beyond_l2_GBs"] = traffic / (kernel_ms * 1e-3) / 1e9
         r["beyond_l2_frac_of_hbm"] = r["beyond_l2_GBs"] / PEAK_HBM_GBS
     r.update(more)
+    return r
+
+
+def address_roofline(nposes, kernel_ms, kernel, record):
+    """Scattered loads: a CU's address unit takes 4 of a wavefront's 64 addresses a cycle, so a
+    gathered load occupies it for 16 cycles.  The loads of the workload are those counted
+    (SQ_INSTS_VMEM_RD per pose); `traffic` is the bytes per launch beyond L2, as elsewhere."""
+    loads = record.get("gathers_per_pose")
+    rate = loads * nposes / (kernel_ms * 1e-3) / 1e9 if loads else None
+    r = {"bound": "address unit", "achieved": rate, "peak": PEAK_GATHERS, "unit": "G wavefront gathers/s",
+         "frac": rate / PEAK_GATHERS if rate else None, "kernel": kernel, "kernel_ms": kernel_ms,
+         "traffic": record.get("bytes_per_launch")}
+    if r["traffic"]:
+        r["beyond_l2_GBs"] = r["traffic"] / (kernel_ms * 1e-3) / 1e9
+        r["beyond_l2_frac_of_hbm"] = r["beyond_l2_GBs"] / PEAK_HBM_GBS
     return r
 
 
@@ -238,11 +254,10 @@ def bench_interp(ctx, lig, rots, trans, steps, warmup):
             "grids": "10 x 64^3 FP32 at 0.375 A (%.1f MB)" % (10 * 64 ** 3 * 4 / 1e6),
             "grid_precompute_ms": grid_ms, "grid_precompute_wall_s": grid_s,
             "poses_inside_grid": inside, "poses_out_of_grid": npose - inside,
-            "gather_GBs": 32.0 * lookups / (avg * 1e-3) / 1e9,
-            "roofline": gather_roofline(32.0 * lookups, avg, "k_interp_lattice (scan)",
-                                        traffic=measured_traffic("k_interp scan"),
-                                        algorithmic_TFLOPs=ops / (avg * 1e-3) / 1e12,
-                                        executed=executed_tflops("k_interp scan", npose, avg)),
+            "lookups_per_s": lookups / (avg * 1e-3),
+            "algorithmic_TFLOPs": ops / (avg * 1e-3) / 1e12,
+            "roofline": address_roofline(npose, avg, "k_interp_lattice (scan)",
+                                         counter_record("k_interp scan")),
             "note": "poses with an atom outside the grid return NaN and are counted"}
 
 

@@ -2227,7 +2227,8 @@ int mmo_grid_compute(mmo_ctx* c, const int32_t* probe_anum, const double* probe_
   timer_begin(c, "grid", s);
   if (out && bytes >= kDrainMin && drain_ready(c)) {
     // slabs of z, so that the host takes the first while the next are computed: the launches
-    // take 2.1 ms for 128^3 nodes, the whole call 5.1 ms in one slab, 3.7 in four.  A slab
+    // take 2.1 ms for 128^3 nodes, the whole call 5.1 ms in one slab, 3.7
+    // (alone) to 4.8 (between other work) in four.  A slab
     // has 8 wavefronts (bricks) per SIMD: launches of less take as long as a full one (0.14
     // ms; 64^3 nodes, 10 MB: four slabs 1.25 ms, one 0.85, the runtime's copy 0.96, and at 60^3
     // 0.84 against 0.79)
